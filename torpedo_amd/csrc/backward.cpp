@@ -66,8 +66,7 @@ extern "C" int tpd_backward(tpd_ctx* c, const float* d_dL_dimage, float* d_grad_
     const uint32_t gx = (W + kTile - 1) / kTile, gy = (H + kTile - 1) / kTile;
     if (c->last_pairs > 0) {
         BackwardArgs a{};
-        a.ranges = c->d_ranges;
-        a.tile_order = c->d_tile_order;
+        a.jobs = c->d_jobs;
         a.vals = c->sorted_vals;
         a.splats = c->d_splats;
         a.width = W;
@@ -80,6 +79,7 @@ extern "C" int tpd_backward(tpd_ctx* c, const float* d_dL_dimage, float* d_grad_
         a.partials = b->partials;
         a.final_T = c->d_final_T;
         a.final_last = c->d_final_last;
+        a.tile_last = c->d_tile_last;
         launch_blend_bwd(a, s);
     }
     if (c->profile) hipEventRecord(b->ev[1], s);

@@ -59,7 +59,9 @@ struct BatchState {
     uint64_t* d_ikeys_alt = nullptr; size_t cap_ikeys_alt = 0;
     uint32_t* d_ivals_alt = nullptr; size_t cap_ivals_alt = 0;
     uint2* d_ranges = nullptr; size_t cap_ranges = 0;
-    uint32_t* d_tile_order = nullptr; size_t cap_tile_order = 0;
+    uint32_t* d_tile_hist = nullptr; size_t cap_tile_hist = 0;
+    TileJob* d_jobs = nullptr; size_t cap_jobs = 0;          // the blend's blocks, heaviest tiles first
+    int32_t* d_tile_last = nullptr; size_t cap_tile_last = 0;  // per block and wave, frames kept for a backward
     float* d_image = nullptr; size_t cap_image = 0;
     // per pixel final transmittance and last blended splat, written by frames kept for a backward
     float* d_final_T = nullptr; size_t cap_final_T = 0;
@@ -135,7 +137,7 @@ void batch_release(tpd_ctx* c) {
     release(b->d_splats); release(b->d_tiles); release(b->d_offsets); release(b->d_rects);
     release(b->d_ikeys); release(b->d_ivals); release(b->d_ikeys_alt); release(b->d_ivals_alt);
     release(b->d_full_keys); release(b->d_eval_count);
-    release(b->d_ranges); release(b->d_tile_order); release(b->d_image); release(b->d_rgba8);
+    release(b->d_ranges); release(b->d_tile_hist); release(b->d_jobs); release(b->d_tile_last); release(b->d_image); release(b->d_rgba8);
     release(b->d_final_T); release(b->d_final_last);
     release(b->d_keys); release(b->d_vals); release(b->d_keys_alt); release(b->d_vals_alt);
     release(b->ws.desc); release(b->ws.partials); release(b->ws.offsets); release(b->ws.tickets);
@@ -253,7 +255,9 @@ static int build_layout(tpd_ctx* c, BatchState* b) {
         (e = grow(b->d_ikeys_alt, b->cap_ikeys_alt, it)) != hipSuccess ||
         (e = grow(b->d_ivals_alt, b->cap_ivals_alt, it)) != hipSuccess ||
         (e = grow(b->d_ranges, b->cap_ranges, std::max<size_t>(tiles, 1))) != hipSuccess ||
-        (e = grow(b->d_tile_order, b->cap_tile_order, std::max<size_t>(tile_order_words(tiles), 1))) != hipSuccess ||
+        (e = grow(b->d_tile_hist, b->cap_tile_hist, std::max<size_t>(tile_hist_words(tiles), 1))) != hipSuccess ||
+        (e = grow(b->d_jobs, b->cap_jobs, std::max<size_t>(tiles, 1))) != hipSuccess ||
+        (e = grow(b->d_tile_last, b->cap_tile_last, std::max<size_t>(kBlendWaves * tiles, 1))) != hipSuccess ||
         (e = grow(b->d_image, b->cap_image, std::max<size_t>(3 * pix, 1))) != hipSuccess ||
         (e = grow(b->d_final_T, b->cap_final_T, std::max<size_t>(pix, 1))) != hipSuccess ||
         (e = grow(b->d_final_last, b->cap_final_last, std::max<size_t>(pix, 1))) != hipSuccess ||
@@ -420,9 +424,7 @@ static BatchArgs forward_args(BatchState* b, bool keep_bwd) {
 static BatchBlendArgs blend_args(BatchState* b) {
     BatchBlendArgs a{};
     a.views = b->d_views;
-    a.tile_view = b->d_tile_view;
-    a.tile_order = b->d_tile_order;
-    a.ranges = b->d_ranges;
+    a.jobs = b->d_jobs;
     a.vals = b->sorted_vals;
     a.splats = b->d_splats;
     a.ntiles = b->ntiles;
@@ -433,6 +435,7 @@ static BatchBlendArgs blend_args(BatchState* b) {
     a.partials = b->d_partials;
     a.final_T = b->d_final_T;
     a.final_last = b->d_final_last;
+    a.tile_last = b->d_tile_last;
     return a;
 }
 
@@ -487,7 +490,7 @@ static void record_forward(BatchState* b, bool keep_bwd, hipStream_t s, bool eve
                   2 * ((b->nitems + kEmitBlockItems - 1) / kEmitBlockItems), &b->d_counters[kCtrScanTicket], s, b->cap,
                   b->lo_bits(),
                   b->lo_bits(), kCtrSortPairs);
-    launch_tile_order(b->d_ranges, b->ntiles, b->d_counters, b->d_tile_order, s);
+    launch_tile_order(b->d_ranges, b->ntiles, b->d_counters, b->d_tile_hist, b->d_jobs, 0, b->d_tile_view, b->d_views, s);
     if (events) hipEventRecord(b->ev[5], s);
     BatchBlendArgs ba = blend_args(b);
     if (!keep_bwd) {  // a forward-only frame stores no per-pixel state for the backward

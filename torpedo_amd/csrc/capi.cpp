@@ -57,7 +57,9 @@ int ensure_image_buffers(tpd_ctx* c) {
     const size_t npix = (size_t)c->cam.width * c->cam.height;
     hipError_t e;
     if ((e = grow(c->d_ranges, c->cap_ranges, std::max<size_t>(ntiles, 1))) != hipSuccess ||
-        (e = grow(c->d_tile_order, c->cap_tile_order, std::max<size_t>(tile_order_words(ntiles), 1))) != hipSuccess)
+        (e = grow(c->d_tile_hist, c->cap_tile_hist, std::max<size_t>(tile_hist_words(ntiles), 1))) != hipSuccess ||
+        (e = grow(c->d_jobs, c->cap_jobs, std::max<size_t>(ntiles, 1))) != hipSuccess ||
+        (e = grow(c->d_tile_last, c->cap_tile_last, std::max<size_t>(kBlendWaves * ntiles, 1))) != hipSuccess)
         return hip_fail(e, "alloc ranges");
     if ((e = grow(c->d_image, c->cap_image, std::max<size_t>(3 * npix, 1))) != hipSuccess)
         return hip_fail(e, "alloc image");
@@ -188,7 +190,9 @@ int tpd_destroy(tpd_ctx* c) {
     release(c->ws.offsets);
     release(c->ws.tickets);
     release(c->d_ranges);
-    release(c->d_tile_order);
+    release(c->d_tile_hist);
+    release(c->d_jobs);
+    release(c->d_tile_last);
     release(c->d_image);
     release(c->d_rgba8);
     release(c->d_final_T);
@@ -396,7 +400,11 @@ int tpd_read_tile_order(tpd_ctx* c, uint32_t* order) {
     if (!c->rendered) return fail(TPD_ERR_STATE, "tpd_read_tile_order: nothing rendered");
     if (c->n == 0) return fail(TPD_ERR_STATE, "tpd_read_tile_order: an empty scene blends no tiles");
     const size_t ntiles = (size_t)((c->cam.width + 15) / 16) * ((c->cam.height + 15) / 16);
-    return copy_back(c, order, c->d_tile_order, sizeof(uint32_t) * ntiles);
+    std::vector<TileJob> jobs(ntiles);
+    const int rc = copy_back(c, jobs.data(), c->d_jobs, sizeof(TileJob) * ntiles);
+    const uint32_t gx = (c->cam.width + 15) / 16;
+    for (size_t t = 0; rc == TPD_OK && t < ntiles; ++t) order[t] = (jobs[t].txy >> 16) * gx + (jobs[t].txy & 0xFFFFu);
+    return rc;
 }
 
 int tpd_synchronize(tpd_ctx* c) {

@@ -23,10 +23,11 @@ namespace tpd {
 
 __global__ __launch_bounds__(kTilePixels) void k_blend_bwd(const BackwardArgs a) {
     __shared__ BlendBwdLds lds;
-    const uint32_t tile = a.tile_order ? a.tile_order[blockIdx.x] : xcd_remap(blockIdx.x, gridDim.x);
-    const TileView tv{tile % a.gx, tile / a.gx, a.width, a.height, a.gx, a.gy, 0};
-    blend_bwd_tile(lds, tv, a.ranges[tile], a.vals, a.splats, a.dL_dimg, a.offsets, a.partials, a.final_T,
-                   a.final_last);
+    const TileJob j = a.jobs[blockIdx.x];
+    const int4 last = reinterpret_cast<const int4*>(a.tile_last)[blockIdx.x];
+    const TileView tv{j.txy & 0xFFFFu, j.txy >> 16, a.width, a.height, a.gx, a.gy, 0};
+    blend_bwd_tile(lds, tv, make_uint2(j.start, j.end), a.vals, a.splats, a.dL_dimg, a.offsets, a.partials, a.final_T,
+                   a.final_last, last);
 }
 
 void launch_blend_bwd(const BackwardArgs& a, hipStream_t s) {

@@ -498,49 +498,46 @@ void launch_batch_emit(const BatchArgs& a, hipStream_t s) {
 
 // ------------------------------------------------------------------ blend, forward and backward
 
-__device__ __forceinline__ TileView batch_tile_view(const BatchViewDev* __restrict__ views,
-                                                    const uint32_t* __restrict__ tile_view, uint32_t tile) {
-    const BatchViewDev& vw = views[tile_view[tile]];
-    const uint32_t local = tile - vw.tile_base;
-    return TileView{local % vw.gx, local / vw.gx, vw.cam.width, vw.cam.height, vw.gx, vw.gy, vw.pix_base};
+__device__ __forceinline__ TileView batch_tile_view(const BatchViewDev* __restrict__ views, const TileJob& j) {
+    const BatchViewDev& vw = views[j.view];
+    return TileView{j.txy & 0xFFFFu, j.txy >> 16, vw.cam.width, vw.cam.height, vw.gx, vw.gy, vw.pix_base};
 }
 
 // COUNT: also adds the evaluated pixel-splat pairs to a.eval_count (a separate launch for the
 // FLOP count, so that the frame's own blend is timed without the counting).
 template <bool COUNT>
 __global__ __launch_bounds__(kTilePixels) void k_batch_blend(const BatchBlendArgs a,
-                                                             const BatchViewDev* __restrict__ views,
-                                                             const uint32_t* __restrict__ tile_view) {
+                                                             const BatchViewDev* __restrict__ views) {
     __shared__ BlendLds lds;
+    const TileJob j = a.jobs[blockIdx.x];  // loaded beside the flag (meaningless after an overflow)
     if (a.counters[kCtrOverflow]) return;  // the frame is rendered again with larger buffers
-    const uint32_t tile = a.tile_order ? a.tile_order[blockIdx.x] : xcd_remap(blockIdx.x, gridDim.x);
-    const TileView tv = batch_tile_view(views, tile_view, tile);
-    blend_tile<COUNT>(lds, tv, a.ranges[tile], a.vals, a.splats, a.image, a.rgba8, a.eval_count, a.final_T,
-                      a.final_last);
+    const TileView tv = batch_tile_view(views, j);
+    blend_tile<COUNT>(lds, tv, make_uint2(j.start, j.end), a.vals, a.splats, a.image, a.rgba8, a.eval_count, a.final_T,
+                      a.final_last, a.tile_last + 4 * (size_t)blockIdx.x);
 }
 
 void launch_batch_blend(const BatchBlendArgs& a, hipStream_t s) {
     if (a.ntiles == 0) return;
     if (a.eval_count)
-        hipLaunchKernelGGL(k_batch_blend<true>, dim3(a.ntiles), dim3(kTilePixels), 0, s, a, a.views, a.tile_view);
+        hipLaunchKernelGGL(k_batch_blend<true>, dim3(a.ntiles), dim3(kTilePixels), 0, s, a, a.views);
     else
-        hipLaunchKernelGGL(k_batch_blend<false>, dim3(a.ntiles), dim3(kTilePixels), 0, s, a, a.views, a.tile_view);
+        hipLaunchKernelGGL(k_batch_blend<false>, dim3(a.ntiles), dim3(kTilePixels), 0, s, a, a.views);
 }
 
 __global__ __launch_bounds__(kTilePixels) void k_batch_blend_bwd(const BatchBlendArgs a,
-                                                                 const BatchViewDev* __restrict__ views,
-                                                                 const uint32_t* __restrict__ tile_view) {
+                                                                 const BatchViewDev* __restrict__ views) {
     __shared__ BlendBwdLds lds;
+    const TileJob j = a.jobs[blockIdx.x];
+    const int4 last = reinterpret_cast<const int4*>(a.tile_last)[blockIdx.x];
     if (a.counters[kCtrOverflow]) return;
-    const uint32_t tile = a.tile_order ? a.tile_order[blockIdx.x] : xcd_remap(blockIdx.x, gridDim.x);
-    const TileView tv = batch_tile_view(views, tile_view, tile);
-    blend_bwd_tile(lds, tv, a.ranges[tile], a.vals, a.splats, a.dL_dimg, a.offsets, a.partials, a.final_T,
-                   a.final_last);
+    const TileView tv = batch_tile_view(views, j);
+    blend_bwd_tile(lds, tv, make_uint2(j.start, j.end), a.vals, a.splats, a.dL_dimg, a.offsets, a.partials, a.final_T,
+                   a.final_last, last);
 }
 
 void launch_batch_blend_bwd(const BatchBlendArgs& a, hipStream_t s) {
     if (a.ntiles == 0) return;
-    hipLaunchKernelGGL(k_batch_blend_bwd, dim3(a.ntiles), dim3(kTilePixels), 0, s, a, a.views, a.tile_view);
+    hipLaunchKernelGGL(k_batch_blend_bwd, dim3(a.ntiles), dim3(kTilePixels), 0, s, a, a.views);
 }
 
 // ------------------------------------------------------------------ preprocess backward

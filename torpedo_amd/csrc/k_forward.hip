@@ -300,7 +300,9 @@ __global__ __launch_bounds__(kOrderChunk) void k_tile_class_count(const uint2* _
 
 __global__ __launch_bounds__(kOrderChunk) void k_tile_order(const uint2* __restrict__ ranges, uint32_t ntiles,
                                                             const uint32_t* counters, const uint32_t* __restrict__ hist,
-                                                            uint32_t* __restrict__ order) {
+                                                            TileJob* __restrict__ jobs, uint32_t grid_width,
+                                                            const uint32_t* __restrict__ tile_view,
+                                                            const BatchViewDev* __restrict__ views) {
     __shared__ uint32_t slot[kTileClasses], total[kTileClasses], cstart[kTileClasses];
     const uint32_t tid = threadIdx.x, lane = __lane_id(), wave = tid / kWave, chunks = gridDim.x;
     if (counters && counters[kCtrOverflow]) return;
@@ -331,29 +333,37 @@ __global__ __launch_bounds__(kOrderChunk) void k_tile_order(const uint2* __restr
     const uint32_t t = blockIdx.x * kOrderChunk + tid;
     const uint32_t cls = t < ntiles ? tile_class(ranges, t) : 0u;
     const uint32_t pos = claim_class_slot(slot, cls, t < ntiles);
-    if (t < ntiles) order[cstart[cls] + xcd_unmap(pos - cstart[cls], total[cls])] = t;
+    if (t >= ntiles) return;
+    const uint2 r = ranges[t];
+    uint32_t v = 0, local = t, gx = grid_width;
+    if (grid_width == 0) {
+        v = tile_view[t];
+        local = t - views[v].tile_base;
+        gx = views[v].gx;
+    }
+    const uint32_t ty = local / gx;
+    jobs[cstart[cls] + xcd_unmap(pos - cstart[cls], total[cls])] = TileJob{(local - ty * gx) | ty << 16, r.x, r.y, v};
 }
 
-void launch_tile_order(const uint2* ranges, uint32_t ntiles, const uint32_t* counters, uint32_t* order, hipStream_t s) {
+void launch_tile_order(const uint2* ranges, uint32_t ntiles, const uint32_t* counters, uint32_t* hist, TileJob* jobs,
+                       uint32_t grid_width, const uint32_t* tile_view, const BatchViewDev* views, hipStream_t s) {
     if (ntiles == 0) return;
     const uint32_t chunks = (ntiles + kOrderChunk - 1) / kOrderChunk;
-    uint32_t* hist = order + ntiles;
     hipLaunchKernelGGL(k_tile_class_count, dim3(chunks), dim3(kOrderChunk), 0, s, ranges, ntiles, counters, hist);
     hipLaunchKernelGGL(k_tile_order, dim3(chunks), dim3(kOrderChunk), 0, s, ranges, ntiles, counters,
-                       (const uint32_t*)hist, order);
+                       (const uint32_t*)hist, jobs, grid_width, tile_view, views);
 }
 
 // ------------------------------------------------------------------ blend
 
-// blend.slang:22-105.  One 16x16 tile per 256-thread block (blend_tile); block indices are
-// spread so that neighbouring tiles share an XCD's L2.
+// blend.slang:22-105.  One 16x16 tile per 256-thread block (blend_tile).
 template <bool COUNT>
 __global__ __launch_bounds__(kTilePixels) void k_blend(const BlendArgs a) {
     __shared__ BlendLds lds;
-    const uint32_t tile = a.tile_order ? a.tile_order[blockIdx.x] : xcd_remap(blockIdx.x, gridDim.x);
-    const TileView tv{tile % a.gx, tile / a.gx, a.width, a.height, a.gx, 0, 0};
-    blend_tile<COUNT>(lds, tv, a.ranges[tile], a.vals, a.splats, a.image, a.rgba8, a.eval_count, a.final_T,
-                      a.final_last);
+    const TileJob j = a.jobs[blockIdx.x];
+    const TileView tv{j.txy & 0xFFFFu, j.txy >> 16, a.width, a.height, a.gx, 0, 0};
+    blend_tile<COUNT>(lds, tv, make_uint2(j.start, j.end), a.vals, a.splats, a.image, a.rgba8, a.eval_count, a.final_T,
+                      a.final_last, a.tile_last + 4 * (size_t)blockIdx.x);
 }
 
 void launch_blend(const BlendArgs& a, hipStream_t s) {

@@ -115,11 +115,10 @@ int render_forward(tpd_ctx* c, hipStream_t s) {
     const uint32_t nd = (c->n + kPreBlock - 1) / kPreBlock;
     launch_ranges(c->sorted_keys, c->d_counters, P, ntiles, c->d_ranges, c->d_scan_desc, nd,
                   &c->d_counters[kCtrScanTicket], s, 0xFFFFFFFFu, c->key_drop, c->lo_bits);
-    launch_tile_order(c->d_ranges, ntiles, nullptr, c->d_tile_order, s);
+    launch_tile_order(c->d_ranges, ntiles, nullptr, c->d_tile_hist, c->d_jobs, gx, nullptr, nullptr, s);
     if (c->profile) hipEventRecord(c->ev[5], s);
     BlendArgs b{};
-    b.ranges = c->d_ranges;
-    b.tile_order = c->d_tile_order;
+    b.jobs = c->d_jobs;
     b.vals = c->sorted_vals;
     b.splats = c->d_splats;
     b.width = W;
@@ -131,6 +130,7 @@ int render_forward(tpd_ctx* c, hipStream_t s) {
     b.eval_count = nullptr;  // counted on request, by blending the frame once more
     b.final_T = c->d_final_T;  // kept for a backward of this frame
     b.final_last = c->d_final_last;
+    b.tile_last = c->d_tile_last;
     launch_blend(b, s);
     c->last_blend = b;
     c->has_blend = true;

@@ -16,7 +16,6 @@ struct TileView {
     uint64_t pix_base;
 };
 
-constexpr uint32_t kBlendWaves = kTilePixels / kWave;  // 4 waves, one 8x8 quadrant each
 constexpr uint32_t kQuad = 8;
 constexpr uint32_t kSub = 4;                              // 4x4-pixel sub-blocks ...
 constexpr uint32_t kSubBlocks = kTilePixels / (kSub * kSub);  // ... 16 per tile, one per 16-lane row
@@ -39,8 +38,7 @@ struct BlendLds {
 
 struct BlendBwdLds {
     BlendLds s;
-    double acc[kTilePixels][kSplatGrads];   // per staged splat: the tile's gradient sums (see blend_bwd_tile)
-    int32_t last;
+    double acc[kTilePixels + 1][kSplatGrads];  // per staged splat (and the sentinel): the tile's gradient sums
 };
 
 __device__ __forceinline__ float4 slot4(const float4* arr, uint32_t off) {
@@ -176,13 +174,14 @@ __device__ __forceinline__ uint32_t blend_stage_loaded(BlendLds& s, const TileVi
 // different splats.  COUNT adds up the pixel-splat pairs whose power is evaluated (for the FLOP
 // roofline; sentinel entries are not counted).  With final_T / final_last, each pixel's final
 // transmittance and the sorted index of the last splat it blended (-1: none) are stored for the
-// backward, which then need not run the composite again.
+// backward, which then need not run the composite again, and the largest index of each wave in
+// tile_last[0 .. 3], from which the backward knows where to start before it has a pixel's.
 template <bool COUNT>
 __device__ __forceinline__ void blend_tile(BlendLds& s, const TileView& tv, uint2 range,
                                            const uint32_t* __restrict__ vals, const Splat* __restrict__ splats,
                                            float* __restrict__ image, uint8_t* __restrict__ rgba8,
-                                           uint64_t* eval_count, float* __restrict__ final_T = nullptr,
-                                           int32_t* __restrict__ final_last = nullptr) {
+                                           uint64_t* eval_count, float* __restrict__ final_T,
+                                           int32_t* __restrict__ final_last, int32_t* __restrict__ tile_last) {
     const uint32_t tid = threadIdx.x, wave = tid / kWave, lane = __lane_id();
     uint32_t pxl, pyl;
     tile_pixel(tv, pxl, pyl);
@@ -253,6 +252,10 @@ __device__ __forceinline__ void blend_tile(BlendLds& s, const TileView& tv, uint
             if (live == 0) break;
         }
     }
+    if (final_T) {
+        const int32_t m = wave_max(last);
+        if (lane == 0) tile_last[wave] = m;
+    }
     if (COUNT) {
         const uint64_t sum = wave_sum_u64(evals);
         if (lane == 0) atomicAdd(reinterpret_cast<unsigned long long*>(eval_count), (unsigned long long)sum);
@@ -299,7 +302,8 @@ __device__ __forceinline__ void store_pair_partial(const TileView& tv, uint32_t 
 }
 
 // Backward of one tile.  The forward frame stored each pixel's final transmittance and last
-// contributor (blend_tile's final_T / final_last); the tile's splats are walked back to front
+// contributor (blend_tile's final_T / final_last) and each wave's last contributor (tile_last); the
+// tile's splats are walked back to front
 // recovering T_i = T_{i+1} / (1 - a_i) and the colour accumulated behind each splat, producing per splat dL/d(image x, y), dL/d(conic a, b, c), dL/d(rgb), dL/d(opacity).
 // Each 16-lane row (one 4x4 sub-block) sums its lanes with DPP row operations in a fixed order;
 // the rows' sums for a splat (at most one per sub-block, 16 in all) are added in LDS with float64
@@ -311,11 +315,21 @@ __device__ __forceinline__ void store_pair_partial(const TileView& tv, uint32_t 
 // of the tile in g's rectangle, so no global atomics are needed, and the per-Gaussian sum over
 // its tiles runs in tile order.  Every pair of the tile's range is written (zeros behind the last
 // contributor), so the partials need no clearing beforehand.
+//
+// Bound: VALU issue (6.2e9 wave instructions x 4 cycles over 1,024 SIMDs = the kernel's time in a
+// step of 64 views, 46.5M pixels and 62.9M pairs).  An entry's update is about 100 instructions: only
+// what changes the pixel's state or reads the upstream gradient runs under the lanes' mask, the
+// colour behind is advanced where alpha and 1 - alpha are at hand, products shared with the power are
+// kept, and the nine row sums end in two masked LDS additions (130 instructions with every value
+// zeroed and formed under the mask, three additions, and the splat's colour carried to the next
+// update).  A tile has few rounds, so its first loads are kept to a chain of three: the tile's job and
+// tile_last by block index, then the values, then the records and offsets.  Together, that step's
+// k_batch_blend_bwd 9.81 -> 8.39 ms, k_blend_bwd at 3M Gaussians / 1920x1080 0.96 -> 0.87 ms.
 __device__ __forceinline__ void blend_bwd_tile(BlendBwdLds& L, const TileView& tv, uint2 range,
                                                const uint32_t* __restrict__ vals, const Splat* __restrict__ splats,
                                                const float* __restrict__ dL_dimg, const uint32_t* __restrict__ offsets,
                                                float* __restrict__ partials, const float* __restrict__ final_T,
-                                               const int32_t* __restrict__ final_last) {
+                                               const int32_t* __restrict__ final_last, const int4 tile_last) {
     constexpr uint32_t kG = kSplatGrads;
     const uint32_t tid = threadIdx.x, wave = tid / kWave, lane = __lane_id();
     uint32_t pxl, pyl;
@@ -323,9 +337,12 @@ __device__ __forceinline__ void blend_bwd_tile(BlendBwdLds& L, const TileView& t
     const bool inside = pxl < tv.width && pyl < tv.height;
     const float fx = (float)pxl, fy = (float)pyl;
     BlendLds& s = L.s;
-    if (tid == 0) L.last = -1;
     for (uint32_t x = tid; x < kTilePixels * kG; x += kTilePixels) (&L.acc[0][0])[x] = 0.0;
     const uint16_t* list = s.list[sub_block_of(wave, lane >> 4)];
+    // what the lane keeps and adds of a row's nine sums (entry_update)
+    const bool b0 = (lane & 1u) != 0u, b1 = (lane & 2u) != 0u;
+    const bool first_quad = (lane & 12u) == 0u, last_lane = (lane & 15u) == 15u, adds = first_quad || last_lane;
+    const uint32_t acc_lane2 = last_lane ? 128u : (b0 ? 64u : 0u) + (b1 ? 32u : 0u);
 
     // The forward frame stored each pixel's final transmittance and last blended splat.
     float T = 1.0f;
@@ -335,17 +352,7 @@ __device__ __forceinline__ void blend_bwd_tile(BlendBwdLds& L, const TileView& t
         T = final_T[o];
         last = final_last[o];
     }
-    __syncthreads();  // L.last initialised
-    if (last >= 0) atomicMax(&L.last, last);
-    __syncthreads();
-    const int32_t block_last = L.last;
-    // Pairs behind the tile's last contributor (all of them when no pixel blended anything) get
-    // zero gradients.
-    const uint32_t zero_from = block_last < 0 ? range.x
-                                              : range.x + (((uint32_t)block_last - range.x) / kTilePixels + 1u) * kTilePixels;
-    for (uint32_t k = zero_from + tid; k < range.y; k += kTilePixels)
-        store_pair_partial(tv, vals[k], splats, offsets, partials, nullptr);
-    if (block_last < 0) return;  // uniform
+    const int32_t block_last = max(max(tile_last.x, tile_last.y), max(tile_last.z, tile_last.w));
 
     // ---- back to front
     float g_r = 0.0f, g_g = 0.0f, g_b = 0.0f;
@@ -355,8 +362,7 @@ __device__ __forceinline__ void blend_bwd_tile(BlendBwdLds& L, const TileView& t
         g_b = dL_dimg[o * 3 + 2];
     }
     float acc_r = 0.0f, acc_g = 0.0f, acc_b = 0.0f;  // colour accumulated behind the current splat
-    float last_alpha = 0.0f, last_r = 0.0f, last_g = 0.0f, last_b = 0.0f;
-    const uint32_t first_chunk = ((uint32_t)block_last - range.x) / kTilePixels;
+    const int32_t first_chunk = block_last < 0 ? -1 : (int32_t)(((uint32_t)block_last - range.x) / kTilePixels);
     // Loads a chunk ahead, as the forward does: while chunk c is walked, the record and the offset of
     // this thread's splat of chunk c - 1 and the value of chunk c - 2 are in flight.  The offset gives
     // the pair's pre-sort position once the record is there, so the partial sums of the thread's slot
@@ -367,11 +373,12 @@ __device__ __forceinline__ void blend_bwd_tile(BlendBwdLds& L, const TileView& t
     const auto offset_of = [&](int32_t c, uint32_t g) -> uint32_t {
         return c >= 0 && range.x + (uint32_t)c * kTilePixels + tid < range.y ? offsets[g] : 0u;
     };
-    uint32_t g_next = value_of((int32_t)first_chunk);
-    StagedSplat next = load_staged(splats, g_next, range.x + first_chunk * kTilePixels + tid, range.y);
-    uint32_t off_next = offset_of((int32_t)first_chunk, g_next);
-    uint32_t g_after = value_of((int32_t)first_chunk - 1);
-    for (int32_t chunk = (int32_t)first_chunk; chunk >= 0; --chunk) {
+    uint32_t g_next = value_of(first_chunk);
+    StagedSplat next = load_staged(splats, g_next, range.x + (uint32_t)first_chunk * kTilePixels + tid,
+                                   first_chunk < 0 ? 0u : range.y);
+    uint32_t off_next = offset_of(first_chunk, g_next);
+    uint32_t g_after = value_of(first_chunk - 1);
+    for (int32_t chunk = first_chunk; chunk >= 0; --chunk) {
         const uint32_t base = range.x + (uint32_t)chunk * kTilePixels;
         const StagedSplat cur = next;
         const size_t pos = cur.valid ? pair_position(tv, cur.sp.xyzr, off_next) : 0;
@@ -385,84 +392,72 @@ __device__ __forceinline__ void blend_bwd_tile(BlendBwdLds& L, const TileView& t
         // Two list entries per step, back to front: both splats' powers, exponentials and alphas
         // are formed first (none depends on the transmittance), then the two updates run in order.
         // A step past the list's start reads the sentinel entry, which no lane takes.
-        const auto entry_update = [&](uint32_t off, const float4& A, const float4& B, float dx, float dy,
+        const int32_t last_off = (last - (int32_t)base) * (int32_t)kSlotBytes;  // of the last blended splat
+        const auto entry_update = [&](uint32_t off, const float4& A, float cdy, float adx, float bdx, float dx, float dy,
                                       float G, float raw, float alpha, uint64_t updm) {
-            const uint32_t j = off / kSlotBytes;
-            const bool upd = lane_on(updm);
-            float v[kG];
-#pragma unroll
-            for (uint32_t q = 0; q < kG; ++q) v[q] = 0.0f;
-            if (upd) {
+            float p = 0.0f, v5 = 0.0f, v6 = 0.0f, v7 = 0.0f, v8 = 0.0f;
+            if (lane_on(updm)) {
                 const float4 C = slot4(s.c, off);
                 // transmittance in front of this splat: 1 - alpha >= 0.01, so the hardware reciprocal
                 // (about 1 ulp) stands in for the correctly rounded division (the gradients are
                 // checked against float64, not bit for bit; plain and batched frames run this same code)
-                T = T * __builtin_amdgcn_rcpf(1.0f - alpha);
-                acc_r = last_alpha * last_r + (1.0f - last_alpha) * acc_r;
-                acc_g = last_alpha * last_g + (1.0f - last_alpha) * acc_g;
-                acc_b = last_alpha * last_b + (1.0f - last_alpha) * acc_b;
+                const float om = 1.0f - alpha;
+                T = T * __builtin_amdgcn_rcpf(om);
                 const float w = alpha * T;
-                v[5] = w * g_r;
-                v[6] = w * g_g;
-                v[7] = w * g_b;
+                v5 = w * g_r;
+                v6 = w * g_g;
+                v7 = w * g_b;
                 const float dL_dalpha = T * ((C.x - acc_r) * g_r + (C.y - acc_g) * g_g + (C.z - acc_b) * g_b);
-                last_alpha = alpha;
-                last_r = C.x; last_g = C.y; last_b = C.z;
-                if (raw < 0.99f) {  // unclamped: alpha = o * G
-                    v[8] = dL_dalpha * G;
-                    const float dL_dpower = dL_dalpha * alpha;
-                    v[0] = dL_dpower * (-A.z * dx - A.w * dy);
-                    v[1] = dL_dpower * (-B.x * dy - A.w * dx);
-                    v[2] = dL_dpower * (-0.5f * dx * dx);
-                    v[3] = dL_dpower * (-dx * dy);
-                    v[4] = dL_dpower * (-0.5f * dy * dy);
-                }
+                const bool unclamped = raw < 0.99f;  // alpha = o * G
+                v8 = unclamped ? dL_dalpha * G : 0.0f;
+                p = unclamped ? dL_dalpha * alpha : 0.0f;  // dL/dpower
+                acc_r = alpha * C.x + om * acc_r;
+                acc_g = alpha * C.y + om * acc_g;
+                acc_b = alpha * C.z + om * acc_b;
             }
-            // Row sums.  v[0..7] by a reduce-scatter: lanes exchange half of their values with the
+            // Position and conic gradients, in every lane (p is 0 where the splat is not taken).
+            // Multiplying by a power of two does not round, so -0.5 moves freely.
+            const float hp = -0.5f * p;
+            const float v0 = p * (-adx - A.w * dy), v1 = p * (-cdy - bdx);
+            const float v2 = hp * (dx * dx), v3 = -p * (dx * dy), v4 = hp * (dy * dy);
+            // Row sums.  v0 .. v7 by a reduce-scatter: lanes exchange half of their values with the
             // lane across bit 0, then across bit 1 (quad_perm), keeping the halves whose index bits
             // match their own, and the four quads of the row add up by rotations; lane (b0, b1) of
-            // every quad then holds the row sums of values 4 b0 + 2 b1 + {0, 1}, and the first quad
-            // adds them into the tile's float64 sums (2 LDS atomics per row instead of 8).  v[8] by a
-            // plain row reduction.  The order of every addition is fixed.
-            const bool b0 = (lane & 1u) != 0u, b1 = (lane & 2u) != 0u;
-            float x[4];
-#pragma unroll
-            for (uint32_t k = 0; k < 4; ++k) {
-                const float send = b0 ? v[k] : v[4 + k], keep = b0 ? v[4 + k] : v[k];
-                x[k] = keep + dpp_f32<0xB1>(send);  // quad_perm [1, 0, 3, 2]
-            }
-            float y[2];
-#pragma unroll
-            for (uint32_t m = 0; m < 2; ++m) {
-                const float send = b1 ? x[m] : x[2 + m], keep = b1 ? x[2 + m] : x[m];
-                y[m] = keep + dpp_f32<0x4E>(send);  // quad_perm [2, 3, 0, 1]
-            }
-#pragma unroll
-            for (uint32_t m = 0; m < 2; ++m) {
-                y[m] += dpp_f32<0x124>(y[m]);  // row_ror:4
-                y[m] += dpp_f32<0x128>(y[m]);  // row_ror:8
-            }
-            const float s8 = row_sum16(v[8]);
-            if (j < kTilePixels) {
-                if ((lane & 12u) == 0u) {
-                    const uint32_t q0 = (b0 ? 4u : 0u) + (b1 ? 2u : 0u);
-                    if (y[0] != 0.0f) atomicAdd(&L.acc[j][q0], (double)y[0]);
-                    if (y[1] != 0.0f) atomicAdd(&L.acc[j][q0 + 1u], (double)y[1]);
-                }
-                if ((lane & 15u) == 15u && s8 != 0.0f) atomicAdd(&L.acc[j][8], (double)s8);
-            }
+            // every quad then holds the row sums of values 4 b0 + 2 b1 + {0, 1}.  v8 by a plain row
+            // reduction.  The order of every addition is fixed.
+            const float x0 = (b0 ? v4 : v0) + dpp_mov<0xB1>(b0 ? v0 : v4);  // quad_perm [1, 0, 3, 2]
+            const float x1 = (b0 ? v5 : v1) + dpp_mov<0xB1>(b0 ? v1 : v5);
+            const float x2 = (b0 ? v6 : v2) + dpp_mov<0xB1>(b0 ? v2 : v6);
+            const float x3 = (b0 ? v7 : v3) + dpp_mov<0xB1>(b0 ? v3 : v7);
+            float y0 = (b1 ? x2 : x0) + dpp_mov<0x4E>(b1 ? x0 : x2);        // quad_perm [2, 3, 0, 1]
+            float y1 = (b1 ? x3 : x1) + dpp_mov<0x4E>(b1 ? x1 : x3);
+            y0 += dpp_mov<0x124>(y0);  // row_ror:4
+            y1 += dpp_mov<0x124>(y1);
+            y0 += dpp_mov<0x128>(y0);  // row_ror:8
+            y1 += dpp_mov<0x128>(y1);
+            const float s8 = row_sum16(v8);
+            // Into the tile's float64 sums: the row's first quad adds y0 and y1, its last lane v8's
+            // sum beside y0 (acc_lane2: twice the byte offset of the lane's first value; a slot's row of
+            // sums is 9/2 times its slot offset).
+            const float z = last_lane ? s8 : y0;
+            static_assert(2 * kG * sizeof(double) == 9 * kSlotBytes, "acc_lane2");
+            char* const acc = reinterpret_cast<char*>(&L.acc[0][0]) + ((__umul24(off, 9u) + acc_lane2) >> 1);
+            if (adds && z != 0.0f) atomicAdd(reinterpret_cast<double*>(acc), (double)z);
+            if (first_quad && y1 != 0.0f) atomicAdd(reinterpret_cast<double*>(acc) + 1, (double)y1);
         };
         for (int32_t i = (int32_t)walk - 1; i >= 0; i -= 2) {
             const uint32_t o1 = list[i], o2 = i >= 1 ? list[i - 1] : kSentinel;
-            // lanes whose last blended splat lies at or behind the entry (256 = the sentinel)
-            const uint64_t mine1 = ballot((int32_t)(base + o1 / kSlotBytes) <= last);
-            const uint64_t mine2 = ballot((int32_t)(base + o2 / kSlotBytes) <= last);
+            // lanes whose last blended splat lies at or behind the entry
+            const uint64_t mine1 = ballot((int32_t)o1 <= last_off);
+            const uint64_t mine2 = ballot((int32_t)o2 <= last_off);
             if ((mine1 | mine2) == 0) continue;
             const float4 A1 = slot4(s.a, o1), B1 = slot4(s.b, o1);
             const float4 A2 = slot4(s.a, o2), B2 = slot4(s.b, o2);
             const float dx1 = A1.x - fx, dy1 = A1.y - fy, dx2 = A2.x - fx, dy2 = A2.y - fy;
-            const float p1 = -0.5f * ((A1.z * dx1) * dx1 + (B1.x * dy1) * dy1) - (A1.w * dx1) * dy1;
-            const float p2 = -0.5f * ((A2.z * dx2) * dx2 + (B2.x * dy2) * dy2) - (A2.w * dx2) * dy2;
+            const float adx1 = A1.z * dx1, bdx1 = A1.w * dx1, cdy1 = B1.x * dy1;
+            const float adx2 = A2.z * dx2, bdx2 = A2.w * dx2, cdy2 = B2.x * dy2;
+            const float p1 = -0.5f * (adx1 * dx1 + cdy1 * dy1) - bdx1 * dy1;
+            const float p2 = -0.5f * (adx2 * dx2 + cdy2 * dy2) - bdx2 * dy2;
             const uint64_t act1 = ballot(p1 <= 0.0f) & ballot(!(p1 < B1.y)) & mine1;
             const uint64_t act2 = ballot(p2 <= 0.0f) & ballot(!(p2 < B2.y)) & mine2;
             if ((act1 | act2) == 0) continue;
@@ -471,8 +466,8 @@ __device__ __forceinline__ void blend_bwd_tile(BlendBwdLds& L, const TileView& t
             const float alpha1 = raw1 < 0.99f ? raw1 : 0.99f, alpha2 = raw2 < 0.99f ? raw2 : 0.99f;
             const uint64_t updm1 = act1 & ballot(!(alpha1 < 1.0f / 255.0f));
             const uint64_t updm2 = act2 & ballot(!(alpha2 < 1.0f / 255.0f));
-            if (updm1 != 0) entry_update(o1, A1, B1, dx1, dy1, G1, raw1, alpha1, updm1);
-            if (updm2 != 0) entry_update(o2, A2, B2, dx2, dy2, G2, raw2, alpha2, updm2);
+            if (updm1 != 0) entry_update(o1, A1, cdy1, adx1, bdx1, dx1, dy1, G1, raw1, alpha1, updm1);
+            if (updm2 != 0) entry_update(o2, A2, cdy2, adx2, bdx2, dx2, dy2, G2, raw2, alpha2, updm2);
         }
         __syncthreads();
         if (cur.valid) {
@@ -485,6 +480,10 @@ __device__ __forceinline__ void blend_bwd_tile(BlendBwdLds& L, const TileView& t
             store_partial_at(pos, partials, out);
         }
     }
+    // Pairs behind the tile's last contributor (all of them when no pixel blended anything) get
+    // zero gradients.
+    for (uint32_t k = range.x + (uint32_t)(first_chunk + 1) * kTilePixels + tid; k < range.y; k += kTilePixels)
+        store_pair_partial(tv, vals[k], splats, offsets, partials, nullptr);
 }
 
 }  // namespace tpd

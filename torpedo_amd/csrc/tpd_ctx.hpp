@@ -58,7 +58,9 @@ struct tpd_ctx {
 
     // image
     uint2* d_ranges = nullptr; size_t cap_ranges = 0;
-    uint32_t* d_tile_order = nullptr; size_t cap_tile_order = 0;
+    uint32_t* d_tile_hist = nullptr; size_t cap_tile_hist = 0;
+    tpd::TileJob* d_jobs = nullptr; size_t cap_jobs = 0;         // the blend's blocks, heaviest tiles first
+    int32_t* d_tile_last = nullptr; size_t cap_tile_last = 0;    // per block and wave, for the backward
     float* d_image = nullptr; size_t cap_image = 0;
     uint8_t* d_rgba8 = nullptr; size_t cap_rgba8 = 0;
     // per pixel final transmittance and last blended splat of the frame, for the backward

@@ -16,6 +16,7 @@ constexpr uint32_t kTile = 16;                 // BLOCK_X = BLOCK_Y (splat.slang
 constexpr uint32_t kTilePixels = kTile * kTile;
 constexpr uint32_t kPreBlock = 256;            // Gaussians per preprocess partition (WORKGROUP_SIZE)
 constexpr uint32_t kWave = 64;
+constexpr uint32_t kBlendWaves = kTilePixels / kWave;  // the blend: 4 waves, one 8x8 quadrant each
 
 // Camera uniform block (splat.slang:18-22) plus the image size the reference reads from the target.
 struct CameraParams {
@@ -447,24 +448,27 @@ __device__ __forceinline__ uint64_t wave_sum_u64(uint64_t v) {
     return v;
 }
 
-// The value of another lane of the wave by a DPP move (CTRL: quad_perm, row rotation, ...; every
-// lane must be active).
+// Largest value of the wave's 64 lanes, in every lane.
+__device__ __forceinline__ int32_t wave_max(int32_t v) {
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) v = max(v, __shfl_xor(v, d, 64));
+    return v;
+}
+
+// The value of another lane of the wave by a DPP move (CTRL: quad_perm, row rotation, mirror, ...,
+// which give every lane a source; every lane must be active).
 template <int CTRL>
-__device__ __forceinline__ float dpp_f32(float v) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false));
+__device__ __forceinline__ float dpp_mov(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
 }
 
 // Sum over each row of 16 lanes with DPP moves only: quad_perm [1,0,3,2] and [2,3,0,1] -> quad
 // sums, row_half_mirror -> 8-lane sums, row_mirror -> every lane holds its row's sum.
 __device__ __forceinline__ float row_sum16(float v) {
-    int x = __builtin_bit_cast(int, v);
-    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, x, 0xB1, 0xF, 0xF, false));
-    x = __builtin_bit_cast(int, v);
-    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, x, 0x4E, 0xF, 0xF, false));
-    x = __builtin_bit_cast(int, v);
-    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, x, 0x141, 0xF, 0xF, false));
-    x = __builtin_bit_cast(int, v);
-    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, x, 0x140, 0xF, 0xF, false));
+    v += dpp_mov<0xB1>(v);
+    v += dpp_mov<0x4E>(v);
+    v += dpp_mov<0x141>(v);
+    v += dpp_mov<0x140>(v);
     return v;
 }
 
@@ -478,15 +482,9 @@ __device__ __forceinline__ void store_relaxed(T* p, T v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Logical block index remapped so that each of the 8 XCDs (which receive workgroups round-robin)
-// works on one contiguous range of the index space; neighbouring tiles then share an L2.
-__device__ __forceinline__ uint32_t xcd_remap(uint32_t b, uint32_t nb) {
-    const uint32_t q = nb / 8u, r = nb % 8u;
-    const uint32_t xcd = b % 8u, pos = b / 8u;
-    return xcd < r ? xcd * (q + 1u) + pos : r * (q + 1u) + (xcd - r) * q + pos;
-}
-
-// The inverse: the block position (0 .. nb - 1) that xcd_remap maps to logical index r.
+// The block position (0 .. nb - 1) of logical index r, such that each of the 8 XCDs (which receive
+// workgroups round-robin) works on one contiguous range of the index space; neighbouring tiles then
+// share an L2.
 __host__ __device__ __forceinline__ uint32_t xcd_unmap(uint32_t r, uint32_t nb) {
     const uint32_t q = nb / 8u, m = nb % 8u;
     uint32_t xcd, pos;

@@ -53,9 +53,16 @@ struct ForwardArgs {
     uint32_t ntiles;
 };
 
+// A block of the blend: one tile, its sorted pairs and (in a batch) its view, in the launch order of
+// launch_tile_order.  One 16-byte load by block index tells the block all it needs.
+struct alignas(16) TileJob {
+    uint32_t txy;         // tile column | tile row << 16, inside the view
+    uint32_t start, end;  // the tile's range of the sorted pairs
+    uint32_t view;        // batch: the tile's view (0 in a plain frame)
+};
+
 struct BlendArgs {
-    const uint2* ranges;
-    const uint32_t* tile_order;  // block -> tile (heaviest first, launch_tile_order), or null
+    const TileJob* jobs;         // per block (heaviest tiles first)
     const uint32_t* vals;
     const Splat* splats;
     uint32_t width, height, gx, ntiles;
@@ -64,11 +71,11 @@ struct BlendArgs {
     uint64_t* eval_count;    // when non-null, incremented by the number of evaluated pixel-splat pairs
     float* final_T;          // H x W final transmittance, for the backward (or null)
     int32_t* final_last;     // H x W sorted index of the last blended splat, -1 for none (or null)
+    int32_t* tile_last;      // with final_T: per block and wave, the largest final_last
 };
 
 struct BackwardArgs {
-    const uint2* ranges;
-    const uint32_t* tile_order;  // the forward frame's block -> tile order, or null
+    const TileJob* jobs;         // the forward frame's
     const uint32_t* vals;
     const Splat* splats;
     uint32_t width, height, gx, gy, ntiles;
@@ -78,6 +85,7 @@ struct BackwardArgs {
                              // conic a, b, c, r, g, b, opacity); every pair is written
     const float* final_T;    // the forward frame's per-pixel final transmittance
     const int32_t* final_last;  // and last blended splat
+    const int32_t* tile_last;   // and its last blended splat per block and wave
 };
 
 struct PreBackwardArgs {
@@ -121,14 +129,15 @@ void launch_full_keys(const uint32_t* keys32, uint32_t drop, uint32_t lo_bits, c
 void launch_blend(const BlendArgs& a, hipStream_t s);
 // The tiles in launch order for the blend: classes of pair count (bit length) from the heaviest
 // down, empty tiles last, so that the longest tiles start first and the short ones fill the tail.
-// counters (optional): nothing is done after a pair overflow.  `order` holds
-// tile_order_words(ntiles) words: the order, then the per-chunk class counts.
+// counters (optional): nothing is done after a pair overflow.  `jobs` receives a job per tile in
+// that order; `hist` is scratch for the per-chunk class counts.  grid_width > 0: the tile columns of
+// the one view; 0: tile t belongs to view tile_view[t] of views.
 constexpr uint32_t kOrderChunk = 1024;  // tiles per block
 constexpr uint32_t kTileClasses = 33;   // pair-count bit lengths 0 .. 32
-inline size_t tile_order_words(size_t ntiles) {
-    return ntiles + kTileClasses * ((ntiles + kOrderChunk - 1) / kOrderChunk);
-}
-void launch_tile_order(const uint2* ranges, uint32_t ntiles, const uint32_t* counters, uint32_t* order, hipStream_t s);
+inline size_t tile_hist_words(size_t ntiles) { return kTileClasses * ((ntiles + kOrderChunk - 1) / kOrderChunk); }
+struct BatchViewDev;
+void launch_tile_order(const uint2* ranges, uint32_t ntiles, const uint32_t* counters, uint32_t* hist, TileJob* jobs,
+                       uint32_t grid_width, const uint32_t* tile_view, const BatchViewDev* views, hipStream_t s);
 
 // ------------------------------------------------------------------ batched rendering
 //
@@ -211,9 +220,7 @@ struct BatchArgs {
 
 struct BatchBlendArgs {
     const BatchViewDev* views;
-    const uint32_t* tile_view;    // view of each global tile
-    const uint32_t* tile_order;   // block -> tile (heaviest first), or null
-    const uint2* ranges;
+    const TileJob* jobs;          // per block (heaviest tiles first)
     const uint32_t* vals;
     const Splat* splats;
     uint32_t ntiles;
@@ -225,6 +232,7 @@ struct BatchBlendArgs {
     float* partials;              // backward: P x 9 per pair
     float* final_T;               // per pixel final transmittance: written by a forward kept for the
     int32_t* final_last;          // backward, read by it (with the last blended splat); or null
+    int32_t* tile_last;           // the largest final_last per block and wave, likewise
     uint64_t* eval_count;         // forward: evaluated pixel-splat pairs are added here, or null
 };
 
