@@ -36,7 +36,7 @@ struct BatchState {
     std::vector<uint32_t> h_scene_views, h_block_scene, h_tile_view;
     uint32_t nblocks = 0, nitems = 0, ntiles = 0, nmats = 0, max_ent = 1;
     uint64_t npix = 0;
-    uint32_t item_shape = 0;  // radix block shape of the item sort (ws.shape: that of the pair sort)
+    uint32_t item_shape = kShapeAuto;  // radix block shape of the item sort (ws.shape: that of the pair sort)
 
     // device tables
     BatchSceneDev* d_scenes = nullptr; size_t cap_scenes = 0;
@@ -106,7 +106,6 @@ struct BatchState {
     bool rendered = false;      // last frame validated
     bool kept_bwd_state = false;
     uint32_t last_pairs = 0;
-    bool items_dropped = false;  // the recorded frame's item sort drops the culled items
     uint32_t last_kept = 0;      // the last frame's items kept by its item sort (the visible ones)
     hipEvent_t ev[11] = {};  // eager stage events [0..6], frame bracket [7], [8], after each sort's histogram [9], [10]
     bool timed = false;
@@ -152,7 +151,7 @@ static BatchState* state(tpd_ctx* c) {
     if (!c->batch) {
         c->batch = new BatchState();
         c->batch->ws.shape = c->ws.shape;  // the context's radix block shape until tuned separately
-        c->batch->item_shape = c->ws.shape;
+        c->batch->item_shape = c->item_shape;
     }
     return c->batch;
 }
@@ -264,7 +263,7 @@ static int build_layout(tpd_ctx* c, BatchState* b) {
         (e = grow(b->d_rgba8, b->cap_rgba8, std::max<size_t>(4 * pix, 1))) != hipSuccess)
         return hip_fail(e, "tpd_batch: alloc");
     // look-back descriptors: the emission's, then the item offsets' (frames kept for a backward)
-    const size_t nparts = 2 * std::max<size_t>((items + kEmitBlockItems - 1) / kEmitBlockItems, 1);
+    const size_t nparts = std::max<size_t>(emit_parts((uint32_t)items) + item_offset_parts((uint32_t)items), 1);
     if (!b->d_scan_desc || b->cap_scan_desc < nparts) {
         if ((e = grow(b->d_scan_desc, b->cap_scan_desc, nparts)) != hipSuccess) return hip_fail(e, "tpd_batch: alloc");
     }
@@ -367,6 +366,9 @@ static int ensure_partials(BatchState* b, size_t pairs) {
 
 static uint32_t tile_key_bits(const BatchState* b) { return bit_length(b->ntiles > 1 ? b->ntiles - 1 : 1); }
 
+static uint32_t item_shape_of(const BatchState* b) { return sort_shape_for(b->item_shape, b->nitems, 8); }
+static uint32_t pair_shape_of(const BatchState* b) { return sort_shape_for(b->ws.shape, b->cap, 4); }
+
 static BatchArgs forward_args(BatchState* b, bool keep_bwd) {
     BatchArgs a{};
     a.scenes = b->d_scenes;
@@ -378,6 +380,7 @@ static BatchArgs forward_args(BatchState* b, bool keep_bwd) {
     a.nitems = b->nitems;
     a.mats = b->d_mats;
     a.scan_desc = b->d_scan_desc;
+    a.scan_desc2 = b->d_scan_desc + emit_parts(b->nitems);
     a.counters = b->d_counters;
     a.cap = b->cap;
     a.splats = b->d_splats;
@@ -385,34 +388,27 @@ static BatchArgs forward_args(BatchState* b, bool keep_bwd) {
     a.offsets = keep_bwd ? b->d_offsets : nullptr;
     a.rects = b->d_rects;
     a.item_keys = b->d_ikeys;
-    a.item_vals = b->d_ivals;
     a.lo_bits = b->lo_bits();
     a.lo_base = b->lo_base();
-    // the item sort's digit counts come from the item kernel when its passes fit the LDS histograms
-    const uint32_t ipasses = sort_shape_passes(b->item_shape, a.lo_bits);
-    if (b->nitems && ipasses <= kMaxCountedPasses) {
-        const uint32_t ibits = sort_shape_bits(b->item_shape);
-        const uint32_t iparts = (b->nitems + sort_shape_keys(b->item_shape) - 1) / sort_shape_keys(b->item_shape);
+    if (b->nitems) {
+        // the item sort's digit counts come from the item kernel (at most 4 passes: 31 bits)
+        const uint32_t ishape = item_shape_of(b), ikeys = sort_shape_keys(ishape);
         a.hist_counts = b->ws.partials;
         a.hist_desc0 = b->ws.desc;
         a.hist_tickets = b->ws.tickets;
-        a.hist_bits = ibits;
-        a.hist_passes = ipasses;
-        a.hist_desc0_words = iparts << ibits;
-        // and the pair sort's from the items' tile rectangles, when its passes fit too
-        const uint32_t pshape = b->ws.shape, pbits = sort_shape_bits(pshape);
-        const uint32_t ppasses = sort_shape_passes(pshape, tile_key_bits(b));
-        if (b->cap && ppasses >= 1 && ppasses <= kMaxCountedPairPasses) {
-            const uint32_t pparts = (b->cap + sort_shape_keys(pshape) - 1) / sort_shape_keys(pshape);
+        a.hist_bits = sort_shape_bits(ishape);
+        a.hist_plan = sort_digit_plan(ishape, a.lo_bits);
+        a.hist_desc0_words = ((b->nitems + ikeys - 1) / ikeys) << a.hist_bits;
+        // and the pair sort's from the items' tile rectangles, when its passes fit the LDS histograms
+        const uint32_t pshape = pair_shape_of(b), pkeys = sort_shape_keys(pshape);
+        const DigitPlan plan = sort_digit_plan(pshape, tile_key_bits(b));
+        if (b->cap && plan.passes <= kMaxCountedPairPasses) {
             a.pair_counts = b->ws.partials + kPairCountRow;
-            a.pair_bits = pbits;
-            a.pair_passes = ppasses;
-            a.pair_desc0_words = pparts << pbits;
+            a.pair_bits = sort_shape_bits(pshape);
+            a.pair_plan = plan;
+            a.pair_desc0_words = ((b->cap + pkeys - 1) / pkeys) << a.pair_bits;
         }
     }
-    // with its counts from the item kernel the item sort drops the culled items and its first pass
-    // takes each item's index as its value: the item kernel writes no values
-    if (a.hist_counts) a.item_vals = nullptr;
     a.keys = b->d_keys;
     a.vals = b->d_vals;
     a.ranges = b->d_ranges;
@@ -449,47 +445,38 @@ static void record_forward(BatchState* b, bool keep_bwd, hipStream_t s, bool eve
     launch_batch_items(a, s);
     launch_batch_item_offsets(a, s);  // frames kept for a backward only (a.offsets set)
     if (events) hipEventRecord(b->ev[1], s);
-    b->item_passes = b->nitems ? sort_shape_passes(b->item_shape, b->lo_bits()) : 0;
+    b->item_passes = a.hist_plan.passes;
+    const uint32_t key_bits = tile_key_bits(b), ishape = item_shape_of(b), pshape = pair_shape_of(b);
+    b->pair_passes = sort_shape_passes(pshape, key_bits);
     bool items_alt = false;
+    if (b->nitems) launch_sort_offsets(b->ws, ishape, a.hist_plan.passes, pshape, a.pair_plan.passes, b->d_counters, nullptr, s);
+    if (events) hipEventRecord(b->ev[9], s);
     if (b->nitems) {
         // 64-bit keys ordered by their low lo_bits bits (the depth key); the high word (the item's
-        // emission record) rides along.  The item sort has a block shape of its own.
-        const uint32_t pair_shape = b->ws.shape;
-        b->ws.shape = b->item_shape;
-        // with the counts from the item kernel, which counts the visible items only, the first
-        // pass drops the culled items (zero high word) and the rest of the frame runs on the
-        // visible ones (their number in kCtrItemsKept)
-        const bool counted = a.hist_counts != nullptr;
-        b->items_dropped = counted;
-        items_alt = launch_sort_pairs(b->ws, b->d_ikeys, b->d_ivals, b->d_ikeys_alt, b->d_ivals_alt, nullptr,
-                                      b->nitems, b->lo_bits(), s, events ? b->ev[9] : nullptr, 32u, nullptr, 0u,
-                                      counted, counted ? &b->d_counters[kCtrItemsKept] : nullptr);
-        a.kept_items = counted ? &b->d_counters[kCtrItemsKept] : nullptr;
-        b->ws.shape = pair_shape;
-    } else if (events)
-        hipEventRecord(b->ev[9], s);
+        // emission record) rides along.  The first pass drops the culled items (zero high word) and the
+        // rest of the frame runs on the visible ones (their number in kCtrItemsKept).
+        a.kept_items = &b->d_counters[kCtrItemsKept];
+        items_alt = launch_sort_items(b->ws, ishape, b->d_ikeys, b->d_ivals, b->d_ikeys_alt, b->d_ivals_alt, b->nitems,
+                                      b->lo_bits(), a.kept_items, s);
+    }
     b->sorted_items = items_alt ? b->d_ivals_alt : b->d_ivals;
     if (events) hipEventRecord(b->ev[2], s);
     a.sorted_items = b->sorted_items;
     a.sorted_keys64 = items_alt ? b->d_ikeys_alt : b->d_ikeys;
     launch_batch_emit(a, s);
     if (events) hipEventRecord(b->ev[3], s);
-    const uint32_t key_bits = tile_key_bits(b);
-    b->pair_passes = sort_shape_passes(b->ws.shape, key_bits);
+    if (events) hipEventRecord(b->ev[10], s);
     // kCtrSortPairs is P, or 0 after an overflow: the counted digits then cover pairs that were
     // never written, and the sort and the ranges must not run on them
-    const bool in_alt = launch_sort_pairs32(b->ws, b->d_keys, b->d_vals, b->d_keys_alt, b->d_vals_alt,
-                                            &b->d_counters[kCtrSortPairs], b->cap, key_bits, s,
-                                            events ? b->ev[10] : nullptr, a.pair_counts != nullptr);
+    const bool in_alt = launch_sort_pairs32(b->ws, pshape, b->d_keys, b->d_vals, b->d_keys_alt, b->d_vals_alt,
+                                            &b->d_counters[kCtrSortPairs], b->cap, key_bits, s, a.pair_counts != nullptr);
     b->sorted_keys = in_alt ? b->d_keys_alt : b->d_keys;
     b->sorted_vals = in_alt ? b->d_vals_alt : b->d_vals;
     if (events) hipEventRecord(b->ev[4], s);
-    // the keys are global tiles (a shift of 0 past key_drop = lo_bits); lo_bits also tells the
-    // ranges kernel whether the items were sorted on the depth window
-    launch_ranges(b->sorted_keys, b->d_counters, b->cap, b->ntiles, b->d_ranges, b->d_scan_desc,
-                  2 * ((b->nitems + kEmitBlockItems - 1) / kEmitBlockItems), &b->d_counters[kCtrScanTicket], s, b->cap,
-                  b->lo_bits(),
-                  b->lo_bits(), kCtrSortPairs);
+    // lo_bits tells the ranges kernel whether the items were sorted on the depth window
+    launch_ranges(b->sorted_keys, b->d_counters, b->cap, b->d_ranges, b->d_scan_desc,
+                  emit_parts(b->nitems) + item_offset_parts(b->nitems), &b->d_counters[kCtrScanTicket], s, b->cap,
+                  b->lo_bits());
     launch_tile_order(b->d_ranges, b->ntiles, b->d_counters, b->d_tile_hist, b->d_jobs, 0, b->d_tile_view, b->d_views, s);
     if (events) hipEventRecord(b->ev[5], s);
     BatchBlendArgs ba = blend_args(b);
@@ -602,7 +589,7 @@ static int validate(tpd_ctx* c, BatchState* b) {
         if (P > kMaxSortKeys) return fail(TPD_ERR_CAPACITY, "tpd_batch: more than 2^30 - 1 tile/Gaussian pairs");
         if (!b->h_counters[kCtrOverflow]) {
             b->last_pairs = P;
-            b->last_kept = b->items_dropped ? b->h_counters[kCtrItemsKept] : b->nitems;
+            b->last_kept = b->h_counters[kCtrItemsKept];
             b->rendered = true;
             b->kept_bwd_state = b->pending_mode != 0;
             return TPD_OK;
@@ -914,8 +901,7 @@ int tpd_batch_read_pairs(tpd_ctx* c, uint64_t* keys, uint32_t* vals, uint32_t ca
         // from the tile and the depth of each value's splat
         e = grow(b->d_full_keys, b->cap_full_keys, b->last_pairs);
         if (e == hipSuccess) {
-            launch_full_keys(b->sorted_keys, 0u, 0u, b->sorted_vals, b->d_splats, b->last_pairs, b->d_full_keys,
-                             c->stream);
+            launch_full_keys(b->sorted_keys, b->sorted_vals, b->d_splats, b->last_pairs, b->d_full_keys, c->stream);
             e = hipStreamSynchronize(c->stream);
         }
         if (e == hipSuccess) e = hipMemcpy(keys, b->d_full_keys, sizeof(uint64_t) * b->last_pairs, hipMemcpyDeviceToHost);
@@ -928,8 +914,8 @@ int tpd_batch_read_pairs(tpd_ctx* c, uint64_t* keys, uint32_t* vals, uint32_t ca
 int tpd_batch_get_sort_shapes(tpd_ctx* c, uint32_t* item_shape, uint32_t* pair_shape) {
     if (!c || !item_shape || !pair_shape) return fail(TPD_ERR_INVALID, "tpd_batch_get_sort_shapes: bad argument");
     const BatchState* b = state(c);
-    *item_shape = b->item_shape;
-    *pair_shape = b->ws.shape;
+    *item_shape = item_shape_of(b);
+    *pair_shape = pair_shape_of(b);
     return TPD_OK;
 }
 

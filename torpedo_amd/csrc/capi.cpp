@@ -40,10 +40,16 @@ int ensure_scene_buffers(tpd_ctx* c) {
     if ((e = grow(c->d_splats, c->cap_splats, n)) != hipSuccess) return hip_fail(e, "alloc splats");
     if ((e = grow(c->d_tiles, c->cap_tiles, n)) != hipSuccess) return hip_fail(e, "alloc tiles");
     if ((e = grow(c->d_offsets, c->cap_offsets, n)) != hipSuccess) return hip_fail(e, "alloc offsets");
-    const size_t nd = (n + kPreBlock - 1) / kPreBlock;
+    if ((e = grow(c->d_ikeys, c->cap_ikeys, n)) != hipSuccess || (e = grow(c->d_ikeys_alt, c->cap_ikeys_alt, n)) != hipSuccess ||
+        (e = grow(c->d_ivals, c->cap_ivals, n)) != hipSuccess || (e = grow(c->d_ivals_alt, c->cap_ivals_alt, n)) != hipSuccess ||
+        (e = grow(c->d_rects, c->cap_rects, n)) != hipSuccess)
+        return hip_fail(e, "alloc items");
+    if ((e = grow(c->d_scan_desc2, c->cap_scan_desc2, item_offset_parts((uint32_t)n))) != hipSuccess)
+        return hip_fail(e, "alloc scan desc");
+    const size_t nd = emit_parts((uint32_t)n);
     if (!c->d_scan_desc || c->cap_scan_desc < nd) {
         if ((e = grow(c->d_scan_desc, c->cap_scan_desc, nd)) != hipSuccess) return hip_fail(e, "alloc scan desc");
-        if ((e = hipMemsetAsync(c->d_scan_desc, 0, c->cap_scan_desc * sizeof(uint64_t), c->stream)) != hipSuccess)
+        if ((e = hipMemset(c->d_scan_desc, 0, c->cap_scan_desc * sizeof(uint64_t))) != hipSuccess)
             return hip_fail(e, "clear scan desc");
     }
     const size_t ne = std::max<uint32_t>(c->n_ent, 1u);
@@ -74,8 +80,7 @@ int ensure_image_buffers(tpd_ctx* c) {
 // Pair buffers and the sort workspace for `pairs` pairs (grown with 25% headroom).
 int ensure_pair_buffers(tpd_ctx* c, size_t pairs) {
     pairs = std::max<size_t>(pairs, 1);
-    if (c->cap_keys >= pairs && c->cap_vals >= pairs && c->cap_keys_alt >= pairs && c->cap_vals_alt >= pairs &&
-        (!c->keep_unsorted || c->cap_keys_dbg >= pairs))
+    if (c->cap_keys >= pairs && c->cap_vals >= pairs && c->cap_keys_alt >= pairs && c->cap_vals_alt >= pairs)
         return TPD_OK;
     const double h = 1.25;
     hipError_t e;
@@ -83,11 +88,7 @@ int ensure_pair_buffers(tpd_ctx* c, size_t pairs) {
     if ((e = grow(c->d_vals, c->cap_vals, pairs, h)) != hipSuccess) return hip_fail(e, "alloc vals");
     if ((e = grow(c->d_keys_alt, c->cap_keys_alt, pairs, h)) != hipSuccess) return hip_fail(e, "alloc keys");
     if ((e = grow(c->d_vals_alt, c->cap_vals_alt, pairs, h)) != hipSuccess) return hip_fail(e, "alloc vals");
-    if (c->keep_unsorted) {
-        if ((e = grow(c->d_keys_dbg, c->cap_keys_dbg, pairs, h)) != hipSuccess) return hip_fail(e, "alloc keys");
-        if ((e = grow(c->d_vals_dbg, c->cap_vals_dbg, pairs, h)) != hipSuccess) return hip_fail(e, "alloc vals");
-    }
-    return ensure_sort_workspace(c, c->cap_keys);
+    return ensure_sort_workspace(c, std::max<size_t>(c->cap_keys, c->n));
 }
 
 int ensure_sort_workspace(tpd_ctx* c, size_t pairs) {
@@ -156,9 +157,14 @@ int tpd_create(tpd_ctx** out, const tpd_config* cfg) {
         return hip_fail(e, "hipHostMalloc");
     }
     if ((e = hipMalloc(&c->d_counters, sizeof(uint32_t) * kCtrCount)) != hipSuccess ||
-        (e = hipMemsetAsync(c->d_counters, 0, sizeof(uint32_t) * kCtrCount, c->stream)) != hipSuccess) {
+        (e = hipMemset(c->d_counters, 0, sizeof(uint32_t) * kCtrCount)) != hipSuccess) {
         tpd_destroy(c);
         return hip_fail(e, "alloc counters");
+    }
+    std::memset(c->h_counters, 0, sizeof(uint32_t) * kCtrCount);
+    if ((e = hipHostGetDevicePointer(reinterpret_cast<void**>(&c->d_host_counters), c->h_counters, 0)) != hipSuccess) {
+        tpd_destroy(c);
+        return hip_fail(e, "hipHostGetDevicePointer");
     }
     *out = c;
     return TPD_OK;
@@ -178,6 +184,13 @@ int tpd_destroy(tpd_ctx* c) {
     release(c->d_tiles);
     release(c->d_offsets);
     release(c->d_scan_desc);
+    release(c->d_scan_desc2);
+    release(c->d_ikeys);
+    release(c->d_ikeys_alt);
+    release(c->d_ivals);
+    release(c->d_ivals_alt);
+    release(c->d_rects);
+    release(c->d_full_keys);
     release(c->d_counters);
     release(c->d_keys);
     release(c->d_vals);
@@ -247,6 +260,7 @@ int tpd_upload(tpd_ctx* c, const float* gaussians, uint32_t n, const uint32_t* e
     }
     c->have_scene = true;
     c->rendered = false;
+    c->depth_wide = false;
     return ensure_scene_buffers(c);
 }
 
@@ -353,6 +367,10 @@ int tpd_read_splats(tpd_ctx* c, float* out) {
     if ((rc = copy_back(c, tiles.data(), c->d_tiles, n * sizeof(uint32_t))) != TPD_OK) return rc;
     for (size_t i = 0; i < n; ++i) {
         float* o = out + 12 * i;
+        if (tiles[i] == 0) {  // a culled Gaussian has no record
+            std::fill(o, o + 12, 0.0f);
+            continue;
+        }
         o[0] = sp[i].rgb.x; o[1] = sp[i].rgb.y; o[2] = sp[i].rgb.z;
         std::memcpy(&o[3], &tiles[i], 4);
         o[4] = sp[i].xyzr.x; o[5] = sp[i].xyzr.y; o[6] = sp[i].xyzr.z; o[7] = sp[i].xyzr.w;
@@ -365,6 +383,7 @@ int tpd_read_tiles(tpd_ctx* c, uint32_t* counts, uint32_t* offsets) {
     if (!check_ctx(c) || !counts) return fail(TPD_ERR_INVALID, "tpd_read_tiles: bad argument");
     if (!c->rendered) return fail(TPD_ERR_STATE, "tpd_read_tiles: nothing rendered");
     int rc = copy_back(c, counts, c->d_tiles, sizeof(uint32_t) * (size_t)c->n);
+    if (rc == TPD_OK && offsets) rc = ensure_offsets(c, c->stream);
     if (rc == TPD_OK && offsets) rc = copy_back(c, offsets, c->d_offsets, sizeof(uint32_t) * (size_t)c->n);
     return rc;
 }
@@ -374,14 +393,14 @@ int tpd_read_pairs(tpd_ctx* c, uint64_t* keys, uint32_t* vals, uint32_t capacity
     if (!c->rendered) return fail(TPD_ERR_STATE, "tpd_read_pairs: nothing rendered");
     if (capacity < c->last_pairs) return fail(TPD_ERR_INVALID, "tpd_read_pairs: capacity below pair count");
     if (unsorted && !c->keep_unsorted) return fail(TPD_ERR_STATE, "tpd_read_pairs: keep_unsorted was not set");
-    const uint64_t* k = unsorted ? c->d_keys_dbg : c->sorted_keys;
+    const uint64_t* k = c->d_keys_dbg;
     const uint32_t* v = unsorted ? c->d_vals_dbg : c->sorted_vals;
-    if (!unsorted && c->key_drop != kKeysWide && c->last_pairs) {
-        // the sort left 32-bit keys: rebuild the 64-bit ones in the other (free) key buffer
-        uint64_t* full = c->sorted_keys == c->d_keys ? c->d_keys_alt : c->d_keys;
-        launch_full_keys(reinterpret_cast<const uint32_t*>(c->sorted_keys), c->key_drop, c->lo_bits, c->sorted_vals,
-                         c->d_splats, c->last_pairs, full, c->stream);
-        k = full;
+    if (!unsorted && c->last_pairs) {
+        // the sorted keys are tiles: the 64-bit ones are rebuilt with the depth of each value's splat
+        const hipError_t e = grow(c->d_full_keys, c->cap_full_keys, c->last_pairs);
+        if (e != hipSuccess) return hip_fail(e, "tpd_read_pairs");
+        launch_full_keys(c->sorted_keys, c->sorted_vals, c->d_splats, c->last_pairs, c->d_full_keys, c->stream);
+        k = c->d_full_keys;
     }
     int rc = copy_back(c, keys, k, sizeof(uint64_t) * (size_t)c->last_pairs);
     if (rc == TPD_OK) rc = copy_back(c, vals, v, sizeof(uint32_t) * (size_t)c->last_pairs);
@@ -428,14 +447,19 @@ int tpd_set_profiling(tpd_ctx* c, int enable) {
 int tpd_get_stage_times(tpd_ctx* c, float* ms, uint32_t* passes) {
     if (!check_ctx(c) || !ms) return fail(TPD_ERR_INVALID, "tpd_get_stage_times: bad argument");
     if (!c->profile || !c->rendered || c->n == 0) return fail(TPD_ERR_STATE, "tpd_get_stage_times: no profiled frame");
-    hipError_t e = hipEventSynchronize(c->ev[6]);
+    hipError_t e = hipEventSynchronize(c->ev[7]);
     if (e != hipSuccess) return hip_fail(e, "hipEventSynchronize");
-    const int from[6] = {0, 2, 3, 4, 5, 0};
-    const int to[6] = {1, 3, 4, 5, 6, 6};
-    for (int k = 0; k < 6; ++k) {
-        e = hipEventElapsedTime(&ms[k], c->ev[from[k]], c->ev[to[k]]);
-        if (e != hipSuccess) return hip_fail(e, "hipEventElapsedTime");
-    }
+    // items, digit offsets, item passes, emission, pair passes, ranges + tile order, blend
+    float d[7];
+    for (int k = 0; k < 7; ++k)
+        if ((e = hipEventElapsedTime(&d[k], c->ev[k], c->ev[k + 1])) != hipSuccess)
+            return hip_fail(e, "hipEventElapsedTime");
+    ms[0] = d[0] + d[3];
+    ms[1] = d[1];
+    ms[2] = d[2] + d[4];
+    ms[3] = d[5];
+    ms[4] = d[6];
+    if ((e = hipEventElapsedTime(&ms[5], c->ev[0], c->ev[7])) != hipSuccess) return hip_fail(e, "hipEventElapsedTime");
     if (passes) *passes = c->last_passes;
     return TPD_OK;
 }
@@ -508,7 +532,7 @@ int tpd_sort_pairs(tpd_ctx* c, uint64_t* d_keys, uint32_t* d_vals, uint64_t* d_k
     int rc = ensure_sort_workspace(c, n);
     if (rc != TPD_OK) return rc;
     hipStream_t s = pick_stream(c, stream);
-    *in_alt = launch_sort_pairs(c->ws, d_keys, d_vals, d_keys_alt, d_vals_alt, nullptr, n, key_bits, s) ? 1 : 0;
+    *in_alt = launch_sort_pairs(c->ws, d_keys, d_vals, d_keys_alt, d_vals_alt, n, key_bits, s) ? 1 : 0;
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return hip_fail(e, "sort launch");
     return TPD_OK;

@@ -74,9 +74,13 @@ __global__ __launch_bounds__(kPreBwdBlock) void k_preprocess_bwd(const PreBackwa
     const uint32_t tiles = valid ? a.tiles[i] : 0u;
     if (tiles > 0) {
         sum_pair_partials(a.partials + (size_t)a.offsets[i] * 9, tiles, gr);
-        const uint32_t e = a.ent_idx ? a.ent_idx[i] : 0u;
-        accumulate_param_grads(s_rec + threadIdx.x * kRecStride, a.ent[e].vm, a.ent[e].pvm, a.cam, a.sh_degree, gr,
-                               gm, gls, gq, gop, gsh);
+        const float* const rec = s_rec + threadIdx.x * kRecStride;
+        if (a.ent_idx) {
+            const EntityMats& m = a.ent[a.ent_idx[i]];
+            accumulate_param_grads(rec, m.vm, m.pvm, a.cam, a.sh_degree, gr, gm, gls, gq, gop, gsh);
+        } else {
+            accumulate_param_grads(rec, a.mats0.vm, a.mats0.pvm, a.cam, a.sh_degree, gr, gm, gls, gq, gop, gsh);
+        }
     }
     if (valid && a.g2d)
 #pragma unroll

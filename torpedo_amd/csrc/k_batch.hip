@@ -67,15 +67,14 @@ struct ItemCountLds {
 // Row r's w tiles are consecutive, so their pass-0 digits are the circular run of w digits from
 // d0 = first tile mod R: +1 at d0 and -1 at (d0 + w) mod R in the difference array, whose prefix
 // sums then fall one short on every digit for each time the run passes digit R - 1, i.e.
-// (d0 + w) >> bits times; that number goes into all0 (the thread's share of pair_all).  A higher
+// (d0 + w) / R times; that number goes into all0 (the thread's share of pair_all).  A higher
 // pass adds the whole rectangle to one digit when its first and last tile share that digit's
 // prefix, else each row's segments.
 __device__ __forceinline__ void count_pair_digits(ItemCountLds& L, uint32_t& all0, uint32_t tile0, uint32_t gx,
-                                                  uint32_t w, uint32_t h, uint32_t bits, uint32_t passes) {
-    const uint32_t dmask = (1u << bits) - 1u;
+                                                  uint32_t w, uint32_t h, const DigitPlan& plan) {
     const uint32_t last = tile0 + (h - 1u) * gx + (w - 1u);
-    for (uint32_t q = 1; q < passes; ++q) {
-        const uint32_t sh = q * bits;
+    for (uint32_t q = 1; q < plan.passes; ++q) {
+        const uint32_t sh = plan.shift[q], dmask = (1u << (plan.shift[q + 1] - sh)) - 1u;
         if ((tile0 >> sh) == (last >> sh)) {
             atomicAdd(&L.pair[q][(tile0 >> sh) & dmask], w * h);
             continue;
@@ -90,6 +89,7 @@ __device__ __forceinline__ void count_pair_digits(ItemCountLds& L, uint32_t& all
             }
         }
     }
+    const uint32_t bits = plan.shift[1], dmask = (1u << bits) - 1u;
     uint32_t t0 = tile0;
     for (uint32_t r = 0; r < h; ++r, t0 += gx) {
         const uint32_t d0 = t0 & dmask;
@@ -99,19 +99,97 @@ __device__ __forceinline__ void count_pair_digits(ItemCountLds& L, uint32_t& all
     }
 }
 
-// One Gaussian's items, for every view of its scene (the body of k_batch_items); with L, the
-// digits of each item key (and, with a.pair_counts, of each visible item's pair keys) are counted
-// in the block's LDS histograms.  The record's 3D covariance is computed once for all views.
-// ENT: the scene has entities (a per-Gaussian entity index); without, every Gaussian of the block
-// uses the view's first entity matrices, a block-uniform address (scalar loads).
+// Clears the block's counters and its share of what the frame's sorts need cleared: the item sort's
+// first descriptors, the tickets, and all tile ranges.
+__device__ __forceinline__ void begin_items(const BatchArgs& a, ItemCountLds& L) {
+    const uint32_t tid = threadIdx.x, gid = blockIdx.x * kPreBlock + tid, nthreads = gridDim.x * kPreBlock;
+    for (uint32_t t = gid; t < a.ntiles; t += nthreads) a.ranges[t] = make_uint2(0u, 0u);
+    for (uint32_t x = gid; x < a.hist_desc0_words; x += nthreads) a.hist_desc0[x] = 0u;
+    if (blockIdx.x == 0 && tid < kMaxPasses && a.hist_tickets) a.hist_tickets[tid] = 0u;
+    for (uint32_t x = tid; x < kMaxCountedPasses * kMaxRadix; x += kPreBlock) (&L.item[0][0])[x] = 0u;
+    if (a.pair_counts) {
+        for (uint32_t x = tid; x < kMaxCountedPairPasses * kMaxRadix; x += kPreBlock) (&L.pair[0][0])[x] = 0u;
+        for (uint32_t x = tid; x < kMaxRadix; x += kPreBlock) L.pair_diff[x] = 0u;
+        if (tid == 0) L.pair_all = 0u;
+    }
+    __syncthreads();
+}
+
+// One item in one view: its key (and rectangle record, and tile count for the backward), and the
+// digits of its key and of its pairs' keys in the block's counts.  The splat is written already.
+__device__ __forceinline__ void put_item(const BatchArgs& a, ItemCountLds& L, uint32_t& all0, uint32_t item, bool vis,
+                                         const Projected& p, uint32_t tile_base, uint32_t gx) {
+    const uint32_t culled_key = (1u << a.lo_bits) - 1u;  // lo_bits is 27 or 31
+    uint64_t key = culled_key;
+    if (vis) {
+        const uint32_t tile0 = tile_base + (uint32_t)p.y0 * gx + (uint32_t)p.x0;
+        const uint32_t w = (uint32_t)(p.x1 - p.x0), h = (uint32_t)(p.y1 - p.y0);
+        const uint32_t r32 = inline_rect(tile0, gx, w, h);
+        if (r32 == kRectLookup) a.rects[item] = pack_emit_rect(tile0, gx, w, h);
+        const uint32_t k32 = (as_uint(p.vz) - a.lo_base) & culled_key;
+        key = ((uint64_t)r32 << 32) | k32;
+        if (a.pair_counts) count_pair_digits(L, all0, tile0, gx, w, h, a.pair_plan);
+        for (uint32_t q = 0; q < a.hist_plan.passes; ++q)  // the item sort drops the culled items
+            atomicAdd(&L.item[q][(k32 >> a.hist_plan.shift[q]) &
+                                 ((1u << (a.hist_plan.shift[q + 1] - a.hist_plan.shift[q])) - 1u)], 1u);
+    }
+    a.item_keys[item] = key;
+    if (a.tiles) a.tiles[item] = p.tiles;
+}
+
+// Adds the block's digit counts to the sorts' (copy blockIdx mod kCountCopies).
+__device__ __forceinline__ void flush_item_counts(const BatchArgs& a, ItemCountLds& L, uint32_t all0) {
+    const uint32_t tid = threadIdx.x, lane = __lane_id(), wave = tid / kWave;
+    const bool pairs = a.pair_counts != nullptr;
+    if (pairs) {
+        const uint32_t s_all = wave_incl_scan(all0);
+        if (lane == kWave - 1 && s_all) atomicAdd(&L.pair_all, s_all);
+    }
+    __syncthreads();
+    const uint32_t R = 1u << a.hist_bits;
+    const size_t copy = (blockIdx.x % kCountCopies) * (kMaxPasses * kMaxRadix);
+    uint32_t* counts = a.hist_counts + copy;
+    for (uint32_t x = tid; x < a.hist_plan.passes * R; x += kPreBlock) {
+        const uint32_t v = L.item[x / R][x % R];
+        if (v) atomicAdd(&counts[x], v);  // x = pass * R + digit, the layout of the sort's counts
+    }
+    if (!pairs) return;
+    // pass 0 of the pair keys: pair_all plus the inclusive prefix sum of the difference array
+    // (modulo 2^32, where its negative entries live); each thread takes PR / 256 consecutive
+    // digits (PR = 256 or 512), of which the plan may use fewer
+    const uint32_t PR = 1u << a.pair_bits, per = PR / kPreBlock, used = 1u << a.pair_plan.shift[1];
+    uint32_t dv[2] = {0u, 0u}, local = 0;
+    for (uint32_t i = 0; i < per; ++i) {
+        dv[i] = L.pair_diff[tid * per + i];
+        local += dv[i];
+    }
+    const uint32_t incl = wave_incl_scan(local);
+    if (lane == kWave - 1) L.wave_sum[wave] = incl;
+    __syncthreads();
+    uint32_t run = incl - local + L.pair_all;
+    for (uint32_t w = 0; w < wave; ++w) run += L.wave_sum[w];
+    for (uint32_t i = 0; i < per; ++i) {
+        run += dv[i];
+        L.pair[0][tid * per + i] = tid * per + i < used ? run : 0u;
+    }
+    __syncthreads();
+    uint32_t* pcounts = a.pair_counts + copy;
+    for (uint32_t x = tid; x < a.pair_plan.passes * PR; x += kPreBlock) {
+        const uint32_t v = L.pair[x / PR][x % PR];
+        if (v) atomicAdd(&pcounts[x], v);
+    }
+}
+
+// One Gaussian's items, for every view of its scene.  The record's 3D covariance is computed once for
+// all views.  ENT: the scene has entities (a per-Gaussian entity index); without, every Gaussian of the
+// block uses the view's first entity matrices, a block-uniform address (scalar loads).
 template <bool ENT>
 __device__ __forceinline__ void items_of_gaussian(const BatchArgs& a, const BatchSceneDev& sc,
                                                   const BatchViewDev* __restrict__ views,
                                                   const uint32_t* __restrict__ scene_views,
                                                   const EntityMats* __restrict__ mats, uint32_t g,
-                                                  ItemCountLds* L, uint32_t& all0) {
+                                                  ItemCountLds& L, uint32_t& all0) {
     const uint32_t e = ENT ? sc.ent_idx[g] : 0u;
-    const uint32_t culled_key = a.lo_bits >= 32 ? 0xFFFFFFFFu : (1u << a.lo_bits) - 1u;
 
     // The record is read once and kept in registers for every view.
     float rec[60];
@@ -129,111 +207,105 @@ __device__ __forceinline__ void items_of_gaussian(const BatchArgs& a, const Batc
         const uint32_t item = vw.item_base + g;
         Projected p;
         const bool vis = project_in_view(rec, cov, mats[vw.mat_base + (ENT ? e : 0u)], vw, sc.sh_degree, p);
-        uint64_t key = culled_key;
         if (vis) {
-            store_splat(a.splats + item, true, p, ot);
-            const uint32_t tile0 = vw.tile_base + (uint32_t)p.y0 * vw.gx + (uint32_t)p.x0;
-            const uint32_t w = (uint32_t)(p.x1 - p.x0), h = (uint32_t)(p.y1 - p.y0);
-            const uint32_t r32 = inline_rect(tile0, vw.gx, w, h);
-            if (r32 == kRectLookup) a.rects[item] = pack_emit_rect(tile0, vw.gx, w, h);
-            key = ((uint64_t)r32 << 32) | ((as_uint(p.vz) - a.lo_base) & culled_key);
+            store_splat(a.splats + item, p, ot);
             depth_out |= depth_outside_window(p.vz);
-            if (L && a.pair_counts) count_pair_digits(*L, all0, tile0, vw.gx, w, h, a.pair_bits, a.pair_passes);
         }
-        a.item_keys[item] = key;
-        if (a.item_vals) a.item_vals[item] = item;
-        if (a.tiles) a.tiles[item] = p.tiles;
-        if (L && vis) {  // the item sort drops the culled items in its first pass
-            const uint32_t k32 = (uint32_t)key;  // the depth key: the bits the item sort orders by
-            const uint32_t dmask = (1u << a.hist_bits) - 1u;
-            for (uint32_t q = 0; q < a.hist_passes; ++q)
-                atomicAdd(&L->item[q][(k32 >> (q * a.hist_bits)) & dmask], 1u);
-        }
+        put_item(a, L, all0, item, vis, p, vw.tile_base, vw.gx);
     }
     if (depth_out) atomicOr(&a.counters[kCtrDepthOut], 1u);
 }
 
 // Per (Gaussian, view) item: project, write the splat record of a visible item, its emission
-// record (and tile count for the backward) and its depth key and index for the item sort.
-// Each block reads its 256 Gaussian records once, for all views of their scene.  With
-// a.hist_counts it also counts the item keys' digits for the item sort in LDS and adds its counts
-// into the sort's digit counts (the sort's own histogram pass, a second read of every key, is then
-// left out), and clears the first pass's look-back descriptors and the tickets; with
-// a.pair_counts likewise the digits of the pair keys the emission will write (every tile of each
-// visible item's rectangle), for the pair sort.  The block also clears its share of the tile
-// ranges, and block 0 the pair sort's count, which the emission sets.
+// record (and tile count for the backward) and its depth key for the item sort.
+// Each block reads its 256 Gaussian records once, for all views of their scene.  It also counts in
+// LDS the digits of the item keys (of the visible items) and, with a.pair_counts, of the pair keys
+// the emission will write (every tile of each visible item's rectangle), and adds its counts into the
+// sorts' digit counts: neither sort reads its keys for them.
 __global__ __launch_bounds__(kPreBlock) void k_batch_items(const BatchArgs a, const BatchSceneDev* __restrict__ scenes,
                                                            const BatchViewDev* __restrict__ views,
                                                            const uint32_t* __restrict__ scene_views,
                                                            const uint32_t* __restrict__ block_scene,
                                                            const EntityMats* __restrict__ mats) {
     __shared__ ItemCountLds L;
-    const uint32_t tid = threadIdx.x, lane = __lane_id(), wave = tid / kWave;
-    for (uint32_t t = blockIdx.x * kPreBlock + tid; t < a.ntiles; t += gridDim.x * kPreBlock)
-        a.ranges[t] = make_uint2(0u, 0u);
-    if (blockIdx.x == 0 && tid == 0) a.counters[kCtrSortPairs] = 0u;
+    begin_items(a, L);
     const uint32_t b = blockIdx.x;
+    if (b == 0 && threadIdx.x == 0) a.counters[kCtrSortPairs] = 0u;  // set by the emission
     if (b >= a.nblocks) return;  // the one block of a batch without Gaussians only clears
-    const bool counting = a.hist_counts != nullptr;  // block-uniform
-    const bool pairs = counting && a.pair_counts != nullptr;
-    if (counting) {
-        for (uint32_t x = blockIdx.x * kPreBlock + tid; x < a.hist_desc0_words; x += gridDim.x * kPreBlock)
-            a.hist_desc0[x] = 0u;
-        if (b == 0 && tid < kMaxPasses) a.hist_tickets[tid] = 0u;
-        for (uint32_t x = tid; x < kMaxCountedPasses * kMaxRadix; x += kPreBlock) (&L.item[0][0])[x] = 0u;
-        if (pairs) {
-            for (uint32_t x = tid; x < kMaxCountedPairPasses * kMaxRadix; x += kPreBlock) (&L.pair[0][0])[x] = 0u;
-            for (uint32_t x = tid; x < kMaxRadix; x += kPreBlock) L.pair_diff[x] = 0u;
-            if (tid == 0) L.pair_all = 0u;
-        }
-        __syncthreads();
-    }
     const BatchSceneDev& sc = scenes[block_scene[b]];
-    const uint32_t g = (b - sc.first_block) * kPreBlock + tid;
+    const uint32_t g = (b - sc.first_block) * kPreBlock + threadIdx.x;
     uint32_t all0 = 0;
     if (g < sc.n) {
         if (sc.ent_idx)
-            items_of_gaussian<true>(a, sc, views, scene_views, mats, g, counting ? &L : nullptr, all0);
+            items_of_gaussian<true>(a, sc, views, scene_views, mats, g, L, all0);
         else
-            items_of_gaussian<false>(a, sc, views, scene_views, mats, g, counting ? &L : nullptr, all0);
+            items_of_gaussian<false>(a, sc, views, scene_views, mats, g, L, all0);
     }
-    if (!counting) return;
-    if (pairs) {
-        const uint32_t s_all = wave_incl_scan(all0);
-        if (lane == kWave - 1 && s_all) atomicAdd(&L.pair_all, s_all);
+    flush_item_counts(a, L, all0);
+}
+
+// The plain frame's items: Gaussian i is item i.  A grid of at most kFrameBlocks blocks (four per CU,
+// what the registers allow) strides over the Gaussians, 256 at a time, so that a block adds its counts
+// to the sorts' once.  Also sums the frame's pair count.
+constexpr uint32_t kFrameBlocks = 1024;
+__global__ __launch_bounds__(kPreBlock) void k_frame_items(const FrameArgs f) {
+    __shared__ ItemCountLds L;
+    __shared__ uint64_t s_total[kPreBlock / kWave];
+    const BatchArgs& a = f.b;
+    begin_items(a, L);
+    const uint32_t tid = threadIdx.x;
+    uint32_t all0 = 0;
+    uint64_t total = 0;
+    bool depth_out = false;
+    for (uint32_t i = blockIdx.x * kPreBlock + tid; i < f.n; i += gridDim.x * kPreBlock) {
+        // The record into registers at once, 16-byte loads when the records are 16-byte aligned.
+        const float* g = f.gauss + (size_t)i * 60;
+        float rec[60];
+        if ((reinterpret_cast<uintptr_t>(f.gauss) & 15u) == 0u) {  // uniform
+            const float4* r4 = reinterpret_cast<const float4*>(g);
+#pragma unroll
+            for (int q = 0; q < 15; ++q) {
+                const float4 t = r4[q];
+                rec[4 * q + 0] = t.x; rec[4 * q + 1] = t.y; rec[4 * q + 2] = t.z; rec[4 * q + 3] = t.w;
+            }
+        } else {
+#pragma unroll
+            for (int q = 0; q < 60; ++q) rec[q] = g[q];
+        }
+        Projected p;
+        const float fx = (0.5f * (float)f.cam.width) * f.cam.focal_ndc[0];
+        const float fy = (0.5f * (float)f.cam.height) * f.cam.focal_ndc[1];
+        bool vis;
+        if (f.ent_idx) {
+            const EntityMats& m = f.ent[f.ent_idx[i]];
+            vis = project_gaussian(rec, m.vm, m.pvm, f.cam.view, fx, fy, f.cam.width, f.cam.height, f.gx, f.gy,
+                                   f.sh_degree, p);
+        } else {
+            vis = project_gaussian(rec, f.mats0.vm, f.mats0.pvm, f.cam.view, fx, fy, f.cam.width, f.cam.height, f.gx,
+                                   f.gy, f.sh_degree, p);
+        }
+        if (vis) {
+            store_splat(a.splats + i, p, opacity_terms(p.opacity));
+            depth_out |= depth_outside_window(p.vz);
+            total += p.tiles;
+        }
+        put_item(a, L, all0, i, vis, p, 0u, f.gx);
     }
-    __syncthreads();
-    const uint32_t R = 1u << a.hist_bits;
-    uint32_t* counts = a.hist_counts + (b % kCountCopies) * (kMaxPasses * kMaxRadix);
-    for (uint32_t x = tid; x < a.hist_passes * R; x += kPreBlock) {
-        const uint32_t v = L.item[x / R][x % R];
-        if (v) atomicAdd(&counts[x], v);  // x = pass * R + digit, the layout of the sort's counts
+    if (ballot(depth_out) != 0 && __lane_id() == 0) atomicOr(&a.counters[kCtrDepthOut], 1u);
+    total = wave_sum_u64(total);
+    if (__lane_id() == 0) s_total[tid / kWave] = total;
+    flush_item_counts(a, L, all0);  // (its barriers order s_total too)
+    if (tid == 0) {
+        total = 0;
+        for (uint32_t w = 0; w < kPreBlock / kWave; ++w) total += s_total[w];
+        atomicAdd(reinterpret_cast<unsigned long long*>(a.counters + kCtrTotal64), (unsigned long long)total);
     }
-    if (!pairs) return;
-    // pass 0 of the pair keys: pair_all plus the inclusive prefix sum of the difference array
-    // (modulo 2^32, where its negative entries live); each thread takes R / 256 consecutive
-    // digits (R = 256 or 512)
-    const uint32_t PR = 1u << a.pair_bits, per = PR / kPreBlock;
-    uint32_t dv[2] = {0u, 0u}, local = 0;
-    for (uint32_t i = 0; i < per; ++i) {
-        dv[i] = L.pair_diff[tid * per + i];
-        local += dv[i];
-    }
-    const uint32_t incl = wave_incl_scan(local);
-    if (lane == kWave - 1) L.wave_sum[wave] = incl;
-    __syncthreads();
-    uint32_t run = incl - local + L.pair_all;
-    for (uint32_t w = 0; w < wave; ++w) run += L.wave_sum[w];
-    for (uint32_t i = 0; i < per; ++i) {
-        run += dv[i];
-        L.pair[0][tid * per + i] = run;
-    }
-    __syncthreads();
-    uint32_t* pcounts = a.pair_counts + (b % kCountCopies) * (kMaxPasses * kMaxRadix);
-    for (uint32_t x = tid; x < a.pair_passes * PR; x += kPreBlock) {
-        const uint32_t v = L.pair[x / PR][x % PR];
-        if (v) atomicAdd(&pcounts[x], v);
-    }
+}
+
+void launch_frame_items(const FrameArgs& f, hipStream_t s) {
+    const uint32_t chunks = (f.n + kPreBlock - 1) / kPreBlock;
+    if (chunks == 0) return;
+    hipLaunchKernelGGL(k_frame_items, dim3(chunks < kFrameBlocks ? chunks : kFrameBlocks), dim3(kPreBlock), 0, s, f);
 }
 
 void launch_batch_items(const BatchArgs& a, hipStream_t s) {
@@ -244,46 +316,47 @@ void launch_batch_items(const BatchArgs& a, hipStream_t s) {
 
 // ------------------------------------------------------------------ pair emission in depth order
 
-// Blocks take partitions of kEmitItems depth-sorted items (kEmitPerThread consecutive ones per
-// thread, so that a thread has that many independent record loads in flight) from an atomic
-// ticket; item i's pairs go to base + the exclusive scan of the tile counts over the sorted items
-// (decoupled look-back over the partitions, as the plain preprocess), key = global tile, value =
-// item.  Items with at most kOwnTiles tiles write their own pairs; the larger ones are spread over
-// the block (pair j of them belongs to the item whose inclusive count of large tiles first exceeds
-// j).  The last partition stores the pair total and the overflow flag.
-constexpr uint32_t kEmitItems = kEmitBlockItems;
+// Blocks take partitions of 512 x PT depth-sorted items (PT consecutive ones per thread, so that a
+// thread has that many independent record loads in flight) from an atomic ticket; item i's pairs go to
+// base + the exclusive scan of the tile counts over the sorted items (decoupled look-back over the
+// partitions), key = global tile, value = item.  Items with at most kOwnTiles tiles write their own
+// pairs; the larger ones are spread over the block (pair j of them belongs to the item whose inclusive
+// count of large tiles first exceeds j).  The last partition stores the pair total and the overflow
+// flag (unless a.totals_known).
 constexpr uint32_t kEmitThreads = 512;
-constexpr uint32_t kEmitPerThread = kEmitItems / kEmitThreads;
-static_assert(kEmitPerThread % 4 == 0, "items are loaded four at a time");
 
 // Pairs of the block's small rectangles staged per chunk before they are written out: the large
 // items' tables (start, rectangle; their values are re-read from the sorted items) are done with
-// by then and lend their space.
-// 2 x 4,096 - 512 pairs: with the large items' tables (48 KB) in the same space, the kernel's LDS
-// stays under 80 KB, two blocks of 512 threads per CU.
-constexpr uint32_t kEmitStage = 2 * kEmitItems - kEmitThreads;
+// by then and lend their space.  For PT = 8, 2 x 4,096 - 512 pairs: with the large items' tables
+// (48 KB) in the same space, the kernel's LDS stays under 80 KB, two blocks of 512 threads per CU.
 constexpr uint32_t kEmitMaxChunks = 4;
 constexpr uint32_t kNoPair = 0xFFFFFFFFu;  // an empty staging slot (no item has this index)
+template <uint32_t PT>
 union EmitLds {
+    static constexpr uint32_t kItems = kEmitThreads * PT;
+    static constexpr uint32_t kStage = 2 * kItems - kEmitThreads;
     struct {
-        uint32_t start[kEmitItems];
-        uint64_t rect[kEmitItems];
+        uint32_t start[kItems];
+        uint64_t rect[kItems];
     } big;
     struct {
-        uint32_t key[kEmitStage], val[kEmitStage];
+        uint32_t key[kStage], val[kStage];
     } stage;
 };
 
+template <uint32_t PT>
 __global__ __launch_bounds__(kEmitThreads) void k_batch_emit(const BatchArgs a) {
     __shared__ uint32_t s_part;
     __shared__ uint32_t s_wave_sum[kEmitThreads / kWave], s_wave_big[kEmitThreads / kWave];
+    constexpr uint32_t kEmitPerThread = PT, kEmitItems = EmitLds<PT>::kItems, kEmitStage = EmitLds<PT>::kStage;
     __shared__ uint32_t s_big_incl[kEmitItems];
-    __shared__ EmitLds L;
+    __shared__ EmitLds<PT> L;
     __shared__ uint64_t s_base;
     uint32_t* const s_start = L.big.start;
     uint64_t* const s_rect = L.big.rect;
 
     const uint32_t tid = threadIdx.x, wave = tid / kWave, lane = __lane_id();
+    if (a.totals_known && a.counters[kCtrOverflow]) return;  // the frame is rendered again
     // the pair sort's counts come from the item kernel: its first pass's descriptors (which the
     // item sort's last pass may have used) and the tickets are cleared here
     for (uint32_t x = blockIdx.x * kEmitThreads + tid; x < a.pair_desc0_words; x += gridDim.x * kEmitThreads)
@@ -297,7 +370,7 @@ __global__ __launch_bounds__(kEmitThreads) void k_batch_emit(const BatchArgs a) 
         __builtin_amdgcn_readfirstlane(a.kept_items ? min(*a.kept_items, a.nitems) : a.nitems);
     const uint32_t nparts = (nitems + kEmitItems - 1) / kEmitItems;
     if (blockIdx.x >= nparts) {
-        if (blockIdx.x == 0 && tid == 0) {  // no visible item: the totals the last partition would store
+        if (blockIdx.x == 0 && tid == 0 && !a.totals_known) {  // no visible item: the totals the last partition would store
             a.counters[kCtrPairs] = 0u;
             a.counters[kCtrOverflow] = 0u;
             a.counters[kCtrSortPairs] = 0u;
@@ -314,12 +387,20 @@ __global__ __launch_bounds__(kEmitThreads) void k_batch_emit(const BatchArgs a) 
     uint64_t rect[kEmitPerThread];
     if (i0 + kEmitPerThread <= nitems) {
 #pragma unroll
-        for (uint32_t j = 0; j < kEmitPerThread; j += 4) {  // i0 is a multiple of 4
-            const uint4 v = *reinterpret_cast<const uint4*>(a.sorted_items + i0 + j);
-            item[j] = v.x; item[j + 1] = v.y; item[j + 2] = v.z; item[j + 3] = v.w;
-            const ulonglong2* k2 = reinterpret_cast<const ulonglong2*>(a.sorted_keys64 + i0 + j);
-            const ulonglong2 k01 = k2[0], k23 = k2[1];
-            rect[j] = k01.x; rect[j + 1] = k01.y; rect[j + 2] = k23.x; rect[j + 3] = k23.y;
+        for (uint32_t j = 0; j < kEmitPerThread; j += 2) {  // i0 is a multiple of PT, which is even
+            const ulonglong2 k = *reinterpret_cast<const ulonglong2*>(a.sorted_keys64 + i0 + j);
+            rect[j] = k.x; rect[j + 1] = k.y;
+        }
+        if constexpr (PT % 4 == 0) {
+#pragma unroll
+            for (uint32_t j = 0; j < kEmitPerThread; j += 4) {
+                const uint4 v = *reinterpret_cast<const uint4*>(a.sorted_items + i0 + j);
+                item[j] = v.x; item[j + 1] = v.y; item[j + 2] = v.z; item[j + 3] = v.w;
+            }
+        } else {
+            static_assert(PT == 2, "items per thread");
+            const uint2 v = *reinterpret_cast<const uint2*>(a.sorted_items + i0);
+            item[0] = v.x; item[1] = v.y;
         }
     } else {
 #pragma unroll
@@ -374,7 +455,7 @@ __global__ __launch_bounds__(kEmitThreads) void k_batch_emit(const BatchArgs a) 
         if (lane == 0) {
             if (part > 0) store_relaxed(&a.scan_desc[part], kDescP | (excl + block_total));
             s_base = excl;
-            if (part == nparts - 1) {
+            if (part == nparts - 1 && !a.totals_known) {
                 const uint64_t total = excl + block_total;
                 a.counters[kCtrPairs] = total > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)total;
                 a.counters[kCtrOverflow] = total > a.cap ? 1u : 0u;
@@ -419,8 +500,9 @@ __global__ __launch_bounds__(kEmitThreads) void k_batch_emit(const BatchArgs a) 
 
 // For frames kept for a backward: the exclusive scan of the items' tile counts in item order,
 // where the backward keeps each item's per-pair partial sums (consecutive Gaussians of a view then
-// have adjacent partials, which the parameter-gradient pass reads item by item).  kEmitPerThread
-// items per thread, decoupled look-back over the second half of the scan descriptors.
+// have adjacent partials, which the parameter-gradient pass reads item by item).  Partitions of
+// kOffsetItems items, decoupled look-back over a.scan_desc2.
+constexpr uint32_t kOffsetPerThread = 8, kOffsetItems = kEmitThreads * kOffsetPerThread;
 __global__ __launch_bounds__(kEmitThreads) void k_batch_item_offsets(const BatchArgs a) {
     __shared__ uint32_t s_part;
     __shared__ uint32_t s_wave_sum[kEmitThreads / kWave];
@@ -429,23 +511,23 @@ __global__ __launch_bounds__(kEmitThreads) void k_batch_item_offsets(const Batch
     if (tid == 0) s_part = atomicAdd(&a.counters[kCtrScanTicket2], 1u);
     __syncthreads();
     const uint32_t part = __builtin_amdgcn_readfirstlane(s_part);
-    const uint32_t nparts = (a.nitems + kEmitItems - 1) / kEmitItems;
+    const uint32_t nparts = (a.nitems + kOffsetItems - 1) / kOffsetItems;
     if (part >= nparts) return;
-    uint64_t* desc = a.scan_desc + nparts;
-    const uint32_t i0 = part * kEmitItems + tid * kEmitPerThread;
-    uint32_t t[kEmitPerThread], mine = 0;
-    if (i0 + kEmitPerThread <= a.nitems) {
+    uint64_t* desc = a.scan_desc2;
+    const uint32_t i0 = part * kOffsetItems + tid * kOffsetPerThread;
+    uint32_t t[kOffsetPerThread], mine = 0;
+    if (i0 + kOffsetPerThread <= a.nitems) {
 #pragma unroll
-        for (uint32_t j = 0; j < kEmitPerThread; j += 4) {  // i0 is a multiple of 4
+        for (uint32_t j = 0; j < kOffsetPerThread; j += 4) {  // i0 is a multiple of 4
             const uint4 v = *reinterpret_cast<const uint4*>(a.tiles + i0 + j);
             t[j] = v.x; t[j + 1] = v.y; t[j + 2] = v.z; t[j + 3] = v.w;
         }
     } else {
 #pragma unroll
-        for (uint32_t j = 0; j < kEmitPerThread; ++j) t[j] = i0 + j < a.nitems ? a.tiles[i0 + j] : 0u;
+        for (uint32_t j = 0; j < kOffsetPerThread; ++j) t[j] = i0 + j < a.nitems ? a.tiles[i0 + j] : 0u;
     }
 #pragma unroll
-    for (uint32_t j = 0; j < kEmitPerThread; ++j) mine += t[j];
+    for (uint32_t j = 0; j < kOffsetPerThread; ++j) mine += t[j];
     const uint32_t incl_w = wave_incl_scan(mine);
     if (lane == kWave - 1) s_wave_sum[wave] = incl_w;
     __syncthreads();
@@ -467,33 +549,48 @@ __global__ __launch_bounds__(kEmitThreads) void k_batch_item_offsets(const Batch
     }
     __syncthreads();
     uint32_t off = (uint32_t)(s_base + wave_off + incl_w - mine);
-    uint32_t o[kEmitPerThread];
+    uint32_t o[kOffsetPerThread];
 #pragma unroll
-    for (uint32_t j = 0; j < kEmitPerThread; ++j) {
+    for (uint32_t j = 0; j < kOffsetPerThread; ++j) {
         o[j] = off;
         off += t[j];
     }
-    if (i0 + kEmitPerThread <= a.nitems) {
+    if (i0 + kOffsetPerThread <= a.nitems) {
 #pragma unroll
-        for (uint32_t j = 0; j < kEmitPerThread; j += 4)
+        for (uint32_t j = 0; j < kOffsetPerThread; j += 4)
             *reinterpret_cast<uint4*>(a.offsets + i0 + j) = make_uint4(o[j], o[j + 1], o[j + 2], o[j + 3]);
     } else {
 #pragma unroll
-        for (uint32_t j = 0; j < kEmitPerThread; ++j)
+        for (uint32_t j = 0; j < kOffsetPerThread; ++j)
             if (i0 + j < a.nitems) a.offsets[i0 + j] = o[j];
     }
 }
 
+uint32_t item_offset_parts(uint32_t nitems) { return (nitems + kOffsetItems - 1) / kOffsetItems; }
+
 void launch_batch_item_offsets(const BatchArgs& a, hipStream_t s) {
-    const uint32_t nparts = (a.nitems + kEmitItems - 1) / kEmitItems;
+    const uint32_t nparts = item_offset_parts(a.nitems);
     if (nparts == 0 || !a.offsets || !a.tiles) return;
     hipLaunchKernelGGL(k_batch_item_offsets, dim3(nparts), dim3(kEmitThreads), 0, s, a);
 }
 
+// Items per thread of the emission: smaller partitions where the larger would leave CUs without a block.
+static uint32_t emit_per_thread(uint32_t nitems) {
+    return nitems >= 512u * 8u * kEmitThreads ? 8u : nitems >= 512u * 4u * kEmitThreads ? 4u : 2u;
+}
+
+uint32_t emit_parts(uint32_t nitems) {
+    const uint32_t n = emit_per_thread(nitems) * kEmitThreads;
+    return (nitems + n - 1) / n;
+}
+
 void launch_batch_emit(const BatchArgs& a, hipStream_t s) {
-    const uint32_t nparts = (a.nitems + kEmitItems - 1) / kEmitItems;
+    const uint32_t nparts = emit_parts(a.nitems);
     if (nparts == 0) return;
-    hipLaunchKernelGGL(k_batch_emit, dim3(nparts), dim3(kEmitThreads), 0, s, a);
+    const auto kernel = emit_per_thread(a.nitems) == 8u   ? k_batch_emit<8>
+                        : emit_per_thread(a.nitems) == 4u ? k_batch_emit<4>
+                                                          : k_batch_emit<2>;
+    hipLaunchKernelGGL(kernel, dim3(nparts), dim3(kEmitThreads), 0, s, a);
 }
 
 // ------------------------------------------------------------------ blend, forward and backward

@@ -1,8 +1,8 @@
-// Forward path kernels: entity matrices, fused preprocess + look-back scan + duplicate,
-// tile ranges, and the front-to-back blend.
+// Forward path kernels of a frame besides its items and their pairs (k_batch.hip): entity matrices,
+// tile ranges, tile order, and the front-to-back blend.
 //
-// Reference: torpedo/volumetric/assets/gaussian/{project,prefix,keygen,range,blend}.slang and the
-// dispatch sequence of GaussianEngine::recordSplat/recordBlend (GaussianEngine.cpp:777-863).
+// Reference: torpedo/volumetric/assets/gaussian/{project,range,blend}.slang and the dispatch sequence
+// of GaussianEngine::recordSplat/recordBlend (GaussianEngine.cpp:777-863).
 #include "tpd_blend.hpp"
 #include "tpd_kernels.hpp"
 
@@ -23,184 +23,22 @@ void launch_entity_mats(const float* models, uint32_t n_ent, const CameraParams&
     hipLaunchKernelGGL(k_entity_mats, dim3((ne + 63) / 64), dim3(64), 0, s, models, ne, cam, out);
 }
 
-// ------------------------------------------------------------------ preprocess + scan + duplicate
-
-// Gaussians per preprocess partition: one per thread, 1,024 threads (a quarter of the look-backs of
-// 256; 24 KB of LDS).
-constexpr uint32_t kDupBlock = 1024;
-
-__global__ __launch_bounds__(kDupBlock) void k_preprocess_dup(const ForwardArgs a) {
-    __shared__ uint32_t s_part;
-    __shared__ uint32_t s_wave_sum[kDupBlock / kWave], s_wave_big[kDupBlock / kWave];
-    __shared__ uint32_t s_big_incl[kDupBlock], s_start[kDupBlock];
-    __shared__ int32_t s_x0[kDupBlock], s_y0[kDupBlock], s_w[kDupBlock];
-    __shared__ uint32_t s_depth[kDupBlock];
-    __shared__ uint64_t s_base;
-
-    const uint32_t tid = threadIdx.x;
-    if (tid == 0) s_part = atomicAdd(&a.counters[kCtrScanTicket], 1u);
-    // Tile ranges are cleared here (every block strides over them) so that the ranges kernel,
-    // which runs after the sort, only writes the non-empty tiles.
-    for (uint32_t t = blockIdx.x * kDupBlock + tid; t < a.ntiles; t += gridDim.x * kDupBlock)
-        a.ranges[t] = make_uint2(0u, 0u);
-    __syncthreads();
-    const uint32_t part = __builtin_amdgcn_readfirstlane(s_part);  // block-uniform: keep it scalar
-    if (part >= gridDim.x) return;  // tickets are reset every frame; never true in a consistent state
-    const uint32_t i = part * kDupBlock + tid;
-
-    Projected p;
-    p.tiles = 0;
-    p.radius = 0.0f;
-    if (i < a.n) {
-        const uint32_t e = a.ent_idx ? a.ent_idx[i] : 0u;
-        // The record into registers at once, 16-byte loads when the records are 16-byte aligned (read
-        // field by field as the projection needs them, each load waited for in turn, the kernel took
-        // a quarter longer, at 63 instead of 78 VGPRs).
-        const float* g = a.gauss + (size_t)i * 60;
-        float rec[60];
-        if ((reinterpret_cast<uintptr_t>(a.gauss) & 15u) == 0u) {  // uniform
-            const float4* r4 = reinterpret_cast<const float4*>(g);
-#pragma unroll
-            for (int q = 0; q < 15; ++q) {
-                const float4 t = r4[q];
-                rec[4 * q + 0] = t.x; rec[4 * q + 1] = t.y; rec[4 * q + 2] = t.z; rec[4 * q + 3] = t.w;
-            }
-        } else {
-#pragma unroll
-            for (int q = 0; q < 60; ++q) rec[q] = g[q];
-        }
-        const bool vis = project_gaussian(rec, a.ent[e].vm, a.ent[e].pvm, a.cam.view,
-                                          (0.5f * (float)a.cam.width) * a.cam.focal_ndc[0],
-                                          (0.5f * (float)a.cam.height) * a.cam.focal_ndc[1], a.cam.width,
-                                          a.cam.height, a.gx, a.gy, a.sh_degree, p);
-        store_splat(a.splats + i, vis, p);
-        a.tiles[i] = p.tiles;
-    }
-
-    // Block-wide inclusive scans of the tile counts and of the counts above kOwnTiles.
-    const uint32_t wave = tid / kWave, lane = __lane_id();
-    // Depths that will be emitted but lie outside the sort's depth window: the host then sorts the
-    // frame on the wider key.
-    if (ballot(p.tiles != 0 && depth_outside_window(p.vz)) != 0 && lane == 0)
-        atomicOr(&a.counters[kCtrDepthOut], 1u);
-    const uint32_t t = p.tiles, big = t > kOwnTiles ? t : 0u;
-    const uint32_t incl_w = wave_incl_scan(t), big_w = wave_incl_scan(big);
-    if (lane == kWave - 1) {
-        s_wave_sum[wave] = incl_w;
-        s_wave_big[wave] = big_w;
-    }
-    __syncthreads();
-    uint32_t wave_off = 0, block_total = 0, big_off = 0, big_total = 0;
-#pragma unroll
-    for (uint32_t w = 0; w < kDupBlock / kWave; ++w) {
-        const uint32_t v = s_wave_sum[w], vb = s_wave_big[w];
-        wave_off += (w < wave) ? v : 0u;
-        block_total += v;
-        big_off += (w < wave) ? vb : 0u;
-        big_total += vb;
-    }
-    const uint32_t excl_in_block = wave_off + incl_w - t;
-    s_big_incl[tid] = big_off + big_w;
-    if (big) {
-        s_start[tid] = excl_in_block;
-        s_x0[tid] = p.x0;
-        s_y0[tid] = p.y0;
-        s_w[tid] = p.x1 - p.x0;
-        s_depth[tid] = as_uint(p.vz);
-    }
-
-    // Decoupled look-back (atomic ticket order guarantees the predecessors are running).
-    if (wave == 0) {
-        if (lane == 0) store_relaxed(&a.scan_desc[part], (part == 0 ? kDescP : kDescA) | (uint64_t)block_total);
-        uint64_t excl = 0;
-        if (part > 0) excl = scan_lookback(a.scan_desc, part);
-        if (lane == 0) {
-            if (part > 0) store_relaxed(&a.scan_desc[part], kDescP | (excl + block_total));
-            s_base = excl;
-            const uint32_t nparts = (a.n + kDupBlock - 1) / kDupBlock;
-            if (part == nparts - 1) {
-                const uint64_t total = excl + block_total;
-                a.counters[kCtrPairs] = total > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)total;
-                a.counters[kCtrOverflow] = total > a.cap ? 1u : 0u;
-            }
-        }
-    }
-    __syncthreads();
-    const uint64_t base = s_base;
-    if (i < a.n) a.offsets[i] = (uint32_t)(base + excl_in_block);
-    if (t && !big)
-        emit_own_pairs(t, p.x0, p.y0, p.x1, as_uint(p.vz), base + excl_in_block, a.gx, 0u, a.cap, a.keys, a.vals,
-                       a.val_base + i);
-    emit_large_pairs<kDupBlock>(s_big_incl, s_start, s_x0, s_y0, s_w, s_depth, big_total, base, a.gx, 0u, a.cap, a.keys, a.vals,
-                     a.val_base + part * kDupBlock);
-}
-
-void launch_preprocess_dup(const ForwardArgs& a, hipStream_t s) {
-    const uint32_t nb = (a.n + kDupBlock - 1) / kDupBlock;
-    if (nb == 0) return;
-    hipLaunchKernelGGL(k_preprocess_dup, dim3(nb), dim3(kDupBlock), 0, s, a);
-}
-
 // ------------------------------------------------------------------ ranges
 
 // Each thread takes runs of kRangeRun consecutive sorted keys, read with 16-byte loads, and
-// compares each key's tile with the one before it (the key before the run is one more load).
+// compares each key (a tile) with the one before it (the key before the run is one more load).
 constexpr uint32_t kRangeRun = 8;
 
-template <typename KT>
-__device__ __forceinline__ uint32_t range_tile(KT k, uint32_t tshift) {
-    return (uint32_t)(k >> tshift);
-}
-
-template <typename KT>
-__device__ __forceinline__ void ranges_of_run(const KT* __restrict__ keys, uint32_t i0, uint32_t P, uint32_t tshift,
-                                              uint32_t* __restrict__ r) {
-    uint32_t t[kRangeRun];
-    const uint32_t n = min(kRangeRun, P - i0);
-    if (n == kRangeRun) {
-        const uint4* v = reinterpret_cast<const uint4*>(keys + i0);  // i0 is a multiple of 8 keys
-        if constexpr (sizeof(KT) == 4) {
-            const uint4 x = v[0], y = v[1];
-            t[0] = x.x >> tshift; t[1] = x.y >> tshift; t[2] = x.z >> tshift; t[3] = x.w >> tshift;
-            t[4] = y.x >> tshift; t[5] = y.y >> tshift; t[6] = y.z >> tshift; t[7] = y.w >> tshift;
-        } else {  // 64-bit keys: the tile is the high word
-#pragma unroll
-            for (uint32_t q = 0; q < 4; ++q) {
-                const uint4 x = v[q];
-                t[2 * q] = x.y;
-                t[2 * q + 1] = x.w;
-            }
-        }
-    } else {
-#pragma unroll
-        for (uint32_t j = 0; j < kRangeRun; ++j) t[j] = j < n ? range_tile(keys[i0 + j], tshift) : 0u;
-    }
-    uint32_t prev = i0 > 0 ? range_tile(keys[i0 - 1], tshift) : 0u;
-#pragma unroll
-    for (uint32_t j = 0; j < kRangeRun; ++j) {
-        if (j >= n) break;
-        const uint32_t idx = i0 + j, cur = t[j];
-        if (idx == 0) {
-            r[2 * cur] = 0;
-        } else if (cur != prev) {
-            r[2 * prev + 1] = idx;
-            r[2 * cur] = idx;
-        }
-        if (idx == P - 1) r[2 * cur + 1] = P;
-        prev = cur;
-    }
-}
-
-// range.slang:16-35.  Empty tiles keep the (0, 0) written by the preprocess kernel (the
-// reference clears with fillBuffer, GaussianEngine.cpp:843-848).  The kernel also re-zeroes the
-// scan descriptors and the scan ticket for the next frame.  A frame sorted on the depth-window key
-// although one of its depths lies outside the window (kCtrDepthOut) has some pairs out of depth
-// order inside their tiles (never in the wrong tile: the key's tile bits are kept); it is marked
-// overflowed, so that every later kernel skips it and the host renders it again on the wider key.
-__global__ void k_ranges(const void* keys, uint32_t* __restrict__ counters, uint32_t cap,
+// range.slang:16-35.  Empty tiles keep the (0, 0) written by the item kernel (the reference clears
+// with fillBuffer, GaussianEngine.cpp:843-848).  The kernel also re-zeroes the scan descriptors and
+// the scan tickets for the next frame.  A batch frame whose items were sorted on the depth-window key
+// although one of its depths lies outside the window (kCtrDepthOut) has some pairs out of depth order
+// inside their tiles (never in the wrong tile); it is marked overflowed, so that every later kernel
+// skips it and the host renders it again on the wider key.
+__global__ void k_ranges(const uint32_t* __restrict__ keys, uint32_t* __restrict__ counters, uint32_t cap,
                          uint2* __restrict__ ranges, uint64_t* scan_desc, uint32_t n_scan_desc, uint32_t* ticket,
-                         uint32_t key_drop, uint32_t lo_bits, uint32_t count_slot) {
-    const uint32_t P = min(counters[count_slot], cap);
+                         uint32_t lo_bits) {
+    const uint32_t P = min(counters[kCtrSortPairs], cap);
     const uint32_t gid = blockIdx.x * blockDim.x + threadIdx.x;
     const uint32_t nthreads = gridDim.x * blockDim.x;
     for (uint32_t d = gid; d < n_scan_desc; d += nthreads) scan_desc[d] = 0;
@@ -211,39 +49,83 @@ __global__ void k_ranges(const void* keys, uint32_t* __restrict__ counters, uint
     }
     uint32_t* r = reinterpret_cast<uint32_t*>(ranges);
     const uint32_t runs = (P + kRangeRun - 1) / kRangeRun;
-    if (key_drop == kKeysWide) {
-        for (uint32_t run = gid; run < runs; run += nthreads)
-            ranges_of_run(static_cast<const uint64_t*>(keys), run * kRangeRun, P, 32u, r);
-    } else {
-        for (uint32_t run = gid; run < runs; run += nthreads)
-            ranges_of_run(static_cast<const uint32_t*>(keys), run * kRangeRun, P, lo_bits - key_drop, r);
+    for (uint32_t run = gid; run < runs; run += nthreads) {
+        const uint32_t i0 = run * kRangeRun, n = min(kRangeRun, P - i0);
+        uint32_t t[kRangeRun];
+        if (n == kRangeRun) {
+            const uint4* v = reinterpret_cast<const uint4*>(keys + i0);
+            const uint4 x = v[0], y = v[1];
+            t[0] = x.x; t[1] = x.y; t[2] = x.z; t[3] = x.w;
+            t[4] = y.x; t[5] = y.y; t[6] = y.z; t[7] = y.w;
+        } else {
+#pragma unroll
+            for (uint32_t j = 0; j < kRangeRun; ++j) t[j] = j < n ? keys[i0 + j] : 0u;
+        }
+        uint32_t prev = i0 > 0 ? keys[i0 - 1] : 0u;
+#pragma unroll
+        for (uint32_t j = 0; j < kRangeRun; ++j) {
+            if (j >= n) break;
+            const uint32_t idx = i0 + j, cur = t[j];
+            if (idx == 0) {
+                r[2 * cur] = 0;
+            } else if (cur != prev) {
+                r[2 * prev + 1] = idx;
+                r[2 * cur] = idx;
+            }
+            if (idx == P - 1) r[2 * cur + 1] = P;
+            prev = cur;
+        }
     }
 }
 
-void launch_ranges(const void* keys, uint32_t* counters, uint32_t P_hint, uint32_t ntiles, uint2* ranges,
-                   uint64_t* scan_desc, uint32_t n_scan_desc, uint32_t* ticket, hipStream_t s, uint32_t cap,
-                   uint32_t key_drop, uint32_t lo_bits, uint32_t count_slot) {
-    (void)ntiles;
+void launch_ranges(const uint32_t* keys, uint32_t* counters, uint32_t P_hint, uint2* ranges, uint64_t* scan_desc,
+                   uint32_t n_scan_desc, uint32_t* ticket, hipStream_t s, uint32_t cap, uint32_t lo_bits) {
     uint32_t work = (P_hint + kRangeRun - 1) / kRangeRun;
     work = work > n_scan_desc ? work : n_scan_desc;
     uint32_t nb = (work + 255) / 256;
     nb = nb < 1 ? 1 : (nb > 8192 ? 8192 : nb);
     hipLaunchKernelGGL(k_ranges, dim3(nb), dim3(256), 0, s, keys, counters, cap, ranges, scan_desc, n_scan_desc, ticket,
-                       key_drop, lo_bits, count_slot);
+                       lo_bits);
 }
 
-__global__ void k_full_keys(const uint32_t* __restrict__ keys32, uint32_t tshift, const uint32_t* __restrict__ vals,
+// ------------------------------------------------------------------ the reference's keys, for readers
+
+__global__ void k_full_keys(const uint32_t* __restrict__ keys, const uint32_t* __restrict__ vals,
                             const Splat* __restrict__ splats, uint32_t n, uint64_t* __restrict__ out) {
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
-        out[i] = ((uint64_t)(keys32[i] >> tshift) << 32) | as_uint(splats[vals[i]].xyzr.z);
+        out[i] = ((uint64_t)keys[i] << 32) | as_uint(splats[vals[i]].xyzr.z);
 }
 
-void launch_full_keys(const uint32_t* keys32, uint32_t drop, uint32_t lo_bits, const uint32_t* vals,
-                      const Splat* splats, uint32_t n, uint64_t* out, hipStream_t s) {
+void launch_full_keys(const uint32_t* keys, const uint32_t* vals, const Splat* splats, uint32_t n, uint64_t* out,
+                      hipStream_t s) {
     if (n == 0) return;
     uint32_t nb = (n + 255) / 256;
     nb = nb > 8192 ? 8192 : nb;
-    hipLaunchKernelGGL(k_full_keys, dim3(nb), dim3(256), 0, s, keys32, lo_bits - drop, vals, splats, n, out);
+    hipLaunchKernelGGL(k_full_keys, dim3(nb), dim3(256), 0, s, keys, vals, splats, n, out);
+}
+
+// keygen.slang:21-54.
+__global__ void k_unsorted_pairs(const Splat* __restrict__ splats, const uint32_t* __restrict__ tiles,
+                                 const uint32_t* __restrict__ offsets, uint32_t n, uint32_t gx, uint32_t gy,
+                                 uint64_t* __restrict__ keys, uint32_t* __restrict__ vals) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n || tiles[i] == 0) return;
+    const float4 c = splats[i].xyzr;
+    int32_t x0, y0, x1, y1;
+    bounding_rect(c.x, c.y, c.w, gx, gy, x0, y0, x1, y1);
+    uint32_t pos = offsets[i];
+    for (int32_t y = y0; y < y1; ++y)
+        for (int32_t x = x0; x < x1; ++x, ++pos) {
+            keys[pos] = ((uint64_t)((uint32_t)y * gx + (uint32_t)x) << 32) | as_uint(c.z);
+            vals[pos] = i;
+        }
+}
+
+void launch_unsorted_pairs(const Splat* splats, const uint32_t* tiles, const uint32_t* offsets, uint32_t n, uint32_t gx,
+                           uint32_t gy, uint64_t* keys, uint32_t* vals, hipStream_t s) {
+    if (n == 0) return;
+    hipLaunchKernelGGL(k_unsorted_pairs, dim3((n + 255) / 256), dim3(256), 0, s, splats, tiles, offsets, n, gx, gy, keys,
+                       vals);
 }
 
 // ------------------------------------------------------------------ tile order
@@ -360,7 +242,8 @@ void launch_tile_order(const uint2* ranges, uint32_t ntiles, const uint32_t* cou
 template <bool COUNT>
 __global__ __launch_bounds__(kTilePixels) void k_blend(const BlendArgs a) {
     __shared__ BlendLds lds;
-    const TileJob j = a.jobs[blockIdx.x];
+    const TileJob j = a.jobs[blockIdx.x];  // loaded beside the flag (meaningless after an overflow)
+    if (a.counters[kCtrOverflow]) return;  // the frame is rendered again
     const TileView tv{j.txy & 0xFFFFu, j.txy >> 16, a.width, a.height, a.gx, 0, 0};
     blend_tile<COUNT>(lds, tv, make_uint2(j.start, j.end), a.vals, a.splats, a.image, a.rgba8, a.eval_count, a.final_T,
                       a.final_last, a.tile_last + 4 * (size_t)blockIdx.x);

@@ -21,20 +21,11 @@ namespace tpd {
 constexpr uint32_t kFlagA = 1u << 30;
 constexpr uint32_t kFlagP = 2u << 30;
 constexpr uint32_t kValMask = (1u << 30) - 1u;
-constexpr uint32_t kNoSlot = 0xFFFFFFFFu;  // kWideDrop: the rank of a dropped key
+constexpr uint32_t kNoSlot = 0xFFFFFFFFu;  // kKeys64Drop: the rank of a dropped key
 
-template <uint32_t BITS, typename KT>
-__device__ __forceinline__ uint32_t digit_of(KT k, uint32_t shift) {
-    return (uint32_t)(k >> shift) & ((1u << BITS) - 1u);
-}
-
-// Keys are (high word << 32) | low word.  When every low word is known to lie in
-// [lo_base, lo_base + 2^lo_bits) (a positive float depth has bit 31 clear; a depth in the window
-// has bits in [kDepthBase, kDepthBase + 2^27)), the sort runs on the compacted key
-// (high << lo_bits) | (low - lo_base), which orders exactly as the full key and can need fewer
-// passes.  The difference is masked to lo_bits bits, so the high word's bits survive any key.
-__device__ __forceinline__ uint64_t compact_key(uint64_t k, uint32_t lo_bits, uint32_t lo_base) {
-    return ((k >> 32) << lo_bits) | ((uint64_t)((uint32_t)k - lo_base) & ((1ull << lo_bits) - 1ull));
+template <typename KT>
+__device__ __forceinline__ uint32_t digit_of(KT k, uint32_t shift, uint32_t mask) {
+    return (uint32_t)(k >> shift) & mask;
 }
 
 // ------------------------------------------------------------------ histograms
@@ -62,19 +53,16 @@ __device__ __forceinline__ uint32_t key_of_lane_below(uint32_t k) {
     return (uint32_t)__builtin_amdgcn_update_dpp((int)k, (int)k, kWaveShr1, 0xF, 0xF, false);
 }
 
-// KT = uint64_t: (tile | depth) keys, histogrammed on their compacted form; KT = uint32_t: keys
-// sorted as they are (lo_bits and lo_base unused).
-// Only the key's low key_bits bits (key_mask) order it; bits above ride along.
 template <uint32_t BITS, typename KT>
 __global__ __launch_bounds__(256) void k_sort_hist(const KT* __restrict__ keys, const uint32_t* count_ptr,
-                                                   uint32_t n_imm, uint32_t passes, uint32_t lo_bits, uint32_t lo_base,
-                                                   KT key_mask, uint32_t tile_keys,
+                                                   uint32_t n_imm, const DigitPlan plan, uint32_t tile_keys,
                                                    uint32_t* __restrict__ counts, uint32_t* __restrict__ desc0,
                                                    uint32_t* __restrict__ tickets) {
     constexpr uint32_t R = 1u << BITS;
     __shared__ uint32_t h[kMaxPasses][R];
     const uint32_t n = count_ptr ? min(*count_ptr, n_imm) : n_imm;  // device count, capped by the capacity
     const uint32_t tid = threadIdx.x, lane = __lane_id();
+    const uint32_t passes = plan.passes;
     for (uint32_t x = tid; x < kMaxPasses * R; x += 256) (&h[0][0])[x] = 0;
     // The first onesweep pass needs region 0 of the look-back descriptors and all tickets at zero.
     const uint32_t nparts = (n + tile_keys - 1) / tile_keys;
@@ -91,12 +79,6 @@ __global__ __launch_bounds__(256) void k_sort_hist(const KT* __restrict__ keys, 
             const uint32_t i = c0 + u * 256 + tid;
             k[u] = i < n ? keys[i] : KT(0);
         }
-        if constexpr (sizeof(KT) == 8) {
-#pragma unroll
-            for (uint32_t u = 0; u < kHistUnroll; ++u) k[u] = compact_key(k[u], lo_bits, lo_base);
-        }
-#pragma unroll
-        for (uint32_t u = 0; u < kHistUnroll; ++u) k[u] &= key_mask;
 #pragma unroll
         for (uint32_t u = 0; u < kHistUnroll; ++u) {
             const uint32_t i = c0 + u * 256 + tid;
@@ -106,8 +88,9 @@ __global__ __launch_bounds__(256) void k_sort_hist(const KT* __restrict__ keys, 
 #pragma unroll
             for (uint32_t p = 0; p < kMaxPasses; ++p) {
                 if (p >= passes) break;
-                const uint32_t d = digit_of<BITS>(k[u], p * BITS);
-                const uint32_t prev = digit_of<BITS>(below, p * BITS);
+                const uint32_t mask = (1u << (plan.shift[p + 1] - plan.shift[p])) - 1u;
+                const uint32_t d = digit_of(k[u], plan.shift[p], mask);
+                const uint32_t prev = digit_of(below, plan.shift[p], mask);
                 const bool head = valid && (lane == 0 || prev != d);
                 const uint64_t heads = ballot(head) | ~vmask;  // invalid lanes end runs
                 if (head) {
@@ -126,51 +109,78 @@ __global__ __launch_bounds__(256) void k_sort_hist(const KT* __restrict__ keys, 
         }
 }
 
-// One block per pass: exclusive scan of the 2^BITS digit counts summed over their kCountCopies
-// copies (each thread takes a contiguous run of digits); every copy is then re-zeroed.  With
-// total_out, pass 0's block stores the number of keys counted there.
-template <uint32_t BITS>
-__global__ __launch_bounds__(256) void k_sort_offsets(uint32_t* __restrict__ counts, uint32_t* __restrict__ offsets,
-                                                      uint32_t* __restrict__ total_out) {
-    constexpr uint32_t R = 1u << BITS;
-    constexpr uint32_t DPT = R / 256;
-    __shared__ uint32_t s_w[4];
-    const uint32_t p = blockIdx.x, t = threadIdx.x;
-    uint32_t c[DPT], local = 0;
-#pragma unroll
-    for (uint32_t i = 0; i < DPT; ++i) {
-        c[i] = 0;
+// Exclusive scan of one pass's 2^bits digit counts (bits 8 or 9) summed over their kCountCopies copies,
+// by a block of 256 threads (each takes a contiguous run of digits); every copy is then re-zeroed.
+// Returns, in thread 255, the number of keys counted.
+__device__ __forceinline__ uint32_t scan_digit_counts(uint32_t* __restrict__ counts, uint32_t* __restrict__ offsets,
+                                                      uint32_t bits, uint32_t* s_w) {
+    const uint32_t t = threadIdx.x, dpt = bits == 9 ? 2u : 1u;
+    uint32_t c[2] = {0u, 0u};
+    for (uint32_t i = 0; i < dpt; ++i) {
 #pragma unroll
         for (uint32_t k = 0; k < kCountCopies; ++k) {
-            uint32_t* q = counts + k * (kMaxPasses * kMaxRadix) + p * R + t * DPT + i;
+            uint32_t* q = counts + k * (kMaxPasses * kMaxRadix) + t * dpt + i;
             c[i] += *q;
             *q = 0;
         }
-        local += c[i];
     }
+    const uint32_t local = c[0] + c[1];
     const uint32_t incl = wave_incl_scan(local);
     const uint32_t w = t / kWave;
     if (__lane_id() == kWave - 1) s_w[w] = incl;
     __syncthreads();
     uint32_t off = incl - local;
     for (uint32_t q = 0; q < w; ++q) off += s_w[q];
-#pragma unroll
-    for (uint32_t i = 0; i < DPT; ++i) {
-        offsets[p * R + t * DPT + i] = off;
+    for (uint32_t i = 0; i < dpt; ++i) {
+        offsets[t * dpt + i] = off;
         off += c[i];
     }
-    if (total_out && p == 0 && t == 255) *total_out = off;
+    return off;
+}
+
+__global__ __launch_bounds__(256) void k_sort_offsets(uint32_t* __restrict__ counts, uint32_t* __restrict__ offsets,
+                                                      uint32_t bits) {
+    __shared__ uint32_t s_w[4];
+    const uint32_t row = blockIdx.x << bits;
+    (void)scan_digit_counts(counts + row, offsets + row, bits, s_w);
+}
+
+// The frame's two sorts at once, one block per pass of either (launch_sort_offsets).
+__global__ __launch_bounds__(256) void k_frame_offsets(uint32_t* __restrict__ counts, uint32_t* __restrict__ offsets,
+                                                       uint32_t ibits, uint32_t ipasses, uint32_t pbits,
+                                                       uint32_t* __restrict__ counters, const FrameTotals totals) {
+    __shared__ uint32_t s_w[4];
+    const uint32_t b = blockIdx.x;
+    const bool items = b < ipasses;
+    const uint32_t row = items ? b << ibits : kPairCountRow + ((b - ipasses) << pbits);
+    const uint32_t n = scan_digit_counts(counts + row, offsets + row, items ? ibits : pbits, s_w);
+    if (b == 0 && items && threadIdx.x == 255) counters[kCtrItemsKept] = n;
+    if (totals.host && b == gridDim.x - 1 && threadIdx.x == 0) {
+        // the 64-bit total, as the digit counts may have wrapped
+        uint64_t* const t64 = reinterpret_cast<uint64_t*>(counters + kCtrTotal64);
+        const uint64_t total = *t64;
+        const uint32_t P = total > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)total;
+        const uint32_t depth_out = counters[kCtrDepthOut];
+        const bool over = total > totals.cap || (totals.lo_bits == kDepthWindowBits && depth_out != 0);
+        *t64 = 0;
+        counters[kCtrDepthOut] = 0;
+        counters[kCtrPairs] = P;
+        counters[kCtrOverflow] = over ? 1u : 0u;
+        counters[kCtrSortPairs] = over ? 0u : P;
+        totals.host[kHostPairs] = P;
+        totals.host[kHostOverflow] = over ? 1u : 0u;
+        totals.host[kHostDepthOut] = depth_out;
+        __hip_atomic_store(&totals.host[kHostSeq], totals.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
 }
 
 // ------------------------------------------------------------------ one pass
 
-// Key widths of a pass: kWide reads and writes 64-bit keys; kNarrow reads 64-bit keys and writes
-// the 32-bit key (compacted key >> drop), possible once the passes before it have consumed the bits
-// below `drop` and the rest fit in 32 bits; kNarrowed reads and writes such 32-bit keys.
-// kWideDrop is kWide that also drops the keys whose high word is zero (the batch's culled items,
-// which the digit counts leave out): they take no part in the ranking, get no LDS slot and are
-// never written.  Its values are the keys' indices (the batch's items), generated rather than read.
-enum : uint32_t { kWide = 0, kNarrow = 1, kNarrowed = 2, kWideDrop = 3 };
+// Key widths of a pass: kKeys64 and kKeys32 read and write 64- and 32-bit keys.  kKeys64Drop is kKeys64
+// that also drops the keys whose high word is zero (the culled items, which the digit counts leave
+// out): they take no part in the ranking, get no LDS slot and are never written.  Its values are the
+// keys' indices (the items), generated rather than read.
+enum : uint32_t { kKeys64 = 0, kKeys32 = 1, kKeys64Drop = 2 };
 
 struct OnesweepArgs {
     const void* keys_in;
@@ -179,11 +189,7 @@ struct OnesweepArgs {
     uint32_t* vals_out;
     const uint32_t* count_ptr;
     uint32_t n_imm;
-    uint32_t shift;
-    uint32_t lo_bits;          // bits of the key's low word (32; 31 for positive depths; 27 in the depth window)
-    uint32_t lo_base;          // subtracted from the low word before compaction
-    uint32_t drop;             // kNarrow / kNarrowed: low bits of the compacted key left out of the 32-bit key
-    uint32_t digit_mask;       // this pass's digit bits below key_bits (bits at and above it do not order)
+    uint32_t shift, digit_mask;  // this pass's digit
     const uint32_t* offsets;   // 2^BITS global exclusive offsets of this pass's digits
     uint32_t* desc;            // this pass's look-back region (parts x 2^BITS), zero on entry
     uint32_t* desc_next;       // the other region, cleared here for the next pass
@@ -200,7 +206,7 @@ struct OnesweepLds {
     uint32_t bstart[R];
     uint32_t adj[R];
     uint32_t wtot[8];
-    uint32_t nkeep;             // kWideDrop: the partition's kept keys
+    uint32_t nkeep;             // kKeys64Drop: the partition's kept keys
     uint32_t part;
     KT keys[kTileKeys];         // the partition reordered by digit (then its values)
 };
@@ -245,8 +251,8 @@ __device__ __forceinline__ uint32_t onesweep_lookback(const uint32_t* desc, uint
 // bookkeeping and the look-back.
 template <uint32_t BITS, uint32_t BLOCK, uint32_t ITEMS, uint32_t MODE>
 __global__ __launch_bounds__(BLOCK) void k_onesweep(const OnesweepArgs a) {
-    constexpr bool DROP = MODE == kWideDrop;
-    constexpr bool WIDE = MODE == kWide || DROP;
+    constexpr bool DROP = MODE == kKeys64Drop;
+    constexpr bool WIDE = MODE != kKeys32;
     using KT = typename std::conditional<WIDE, uint64_t, uint32_t>::type;  // key type after the load
     using Lds = OnesweepLds<BITS, BLOCK, ITEMS, KT>;
     constexpr uint32_t R = Lds::R;
@@ -261,6 +267,9 @@ __global__ __launch_bounds__(BLOCK) void k_onesweep(const OnesweepArgs a) {
     const uint32_t n = a.count_ptr ? min(*a.count_ptr, a.n_imm) : a.n_imm;
     const uint32_t nparts = (n + kTileKeys - 1) / kTileKeys;
     const uint32_t tid = threadIdx.x, wave = tid / kWave, lane = __lane_id();
+    // The grid covers the most keys there may be: the blocks past the partitions leave before they
+    // take a ticket, so that exactly nparts blocks share nparts tickets.
+    if (blockIdx.x >= nparts) return;
     if (tid == 0) L.part = atomicAdd(a.ticket, 1u);
     for (uint32_t x = tid; x < kWaves * R / 2; x += BLOCK) reinterpret_cast<uint32_t*>(&L.whist[0][0])[x] = 0;
     __syncthreads();
@@ -270,16 +279,13 @@ __global__ __launch_bounds__(BLOCK) void k_onesweep(const OnesweepArgs a) {
         for (uint32_t d = tid; d < R; d += BLOCK) a.desc_next[part * R + d] = 0;
 
     // Load ITEMS keys and values per thread, wave-striped: element e = wave*(ITEMS*64) + j*64 +
-    // lane; past the end keys are all ones (kWideDrop: zero, i.e. dropped).  Every partition but the
+    // lane; past the end keys are all ones (kKeys64Drop: zero, i.e. dropped).  Every partition but the
     // last is full: its loads (and, without dropped keys, its stores) need no bounds checks.
     const uint32_t base = part * kTileKeys;
     const uint32_t wbase = base + wave * (ITEMS * kWave) + lane;
     const bool full = base + kTileKeys <= n;
     const auto load_key = [&](uint32_t idx) -> KT {
-        if constexpr (WIDE) return static_cast<const uint64_t*>(a.keys_in)[idx];
-        if constexpr (MODE == kNarrow)
-            return (uint32_t)(compact_key(static_cast<const uint64_t*>(a.keys_in)[idx], a.lo_bits, a.lo_base) >> a.drop);
-        return static_cast<const uint32_t*>(a.keys_in)[idx];
+        return static_cast<const KT*>(a.keys_in)[idx];
     };
     KT k[ITEMS];
     uint32_t v[ITEMS];
@@ -305,8 +311,7 @@ __global__ __launch_bounds__(BLOCK) void k_onesweep(const OnesweepArgs a) {
     // each group advances the wave's running digit counter.  Digits are recomputed from the keys
     // wherever they are needed (a few instructions) rather than kept in registers or LDS.
     const auto digit = [&](KT key) -> uint32_t {
-        if constexpr (WIDE) return digit_of<BITS>(compact_key(key, a.lo_bits, a.lo_base), a.shift) & a.digit_mask;
-        else return (uint32_t)(key >> (a.shift - a.drop)) & a.digit_mask;
+        return digit_of(key, a.shift, a.digit_mask);
     };
     const uint64_t lt = lanemask_lt();
     const auto dropped = [&](KT key) { return DROP && (uint32_t)((uint64_t)key >> 32) == 0u; };
@@ -425,18 +430,14 @@ __global__ __launch_bounds__(BLOCK) void k_onesweep(const OnesweepArgs a) {
     }
 }
 
-// Shapes the tuner chooses from: {digit bits, threads, keys per thread}.
-// kernel[mode] for the key widths kWide, kNarrow, kNarrowed and kWideDrop.
+// Shapes the tuner chooses from: {digit bits, threads, keys per thread}; kernel[mode].
 struct SortShape {
     uint32_t bits, block, items;
-    void (*kernel[4])(const OnesweepArgs);
+    void (*kernel[3])(const OnesweepArgs);
 };
-#define TPD_SHAPE(B, T, I)                                                                              \
-    {                                                                                                   \
-        B, T, I, {                                                                                      \
-            k_onesweep<B, T, I, kWide>, k_onesweep<B, T, I, kNarrow>, k_onesweep<B, T, I, kNarrowed>, \
-                k_onesweep<B, T, I, kWideDrop>                                                          \
-        }                                                                                               \
+#define TPD_SHAPE(B, T, I)                                                                                \
+    {                                                                                                     \
+        B, T, I, { k_onesweep<B, T, I, kKeys64>, k_onesweep<B, T, I, kKeys32>, k_onesweep<B, T, I, kKeys64Drop> } \
     }
 static const SortShape kShapes[] = {
     TPD_SHAPE(8, 256, 16), TPD_SHAPE(8, 256, 8),  TPD_SHAPE(8, 256, 12), TPD_SHAPE(8, 512, 8),
@@ -453,21 +454,18 @@ uint32_t sort_shape_passes(uint32_t shape, uint32_t key_bits) {
     const uint32_t b = sort_shape_bits(shape);
     return (key_bits + b - 1) / b;
 }
-
-template <uint32_t BITS, typename KT>
-static void launch_hist(uint32_t hb, uint32_t passes, hipStream_t s, const KT* keys, const uint32_t* count_ptr,
-                        uint32_t n_max, uint32_t lo_bits, uint32_t lo_base, uint32_t key_bits, uint32_t tile,
-                        SortWorkspace& ws) {
-    const KT key_mask = key_bits >= 8 * sizeof(KT) ? ~KT(0) : (KT(1) << key_bits) - KT(1);
-    hipLaunchKernelGGL((k_sort_hist<BITS, KT>), dim3(hb), dim3(256), 0, s, keys, count_ptr, n_max, passes, lo_bits,
-                       lo_base, key_mask, tile, ws.partials, ws.desc, ws.tickets);
-    hipLaunchKernelGGL(k_sort_offsets<BITS>, dim3(passes), dim3(256), 0, s, ws.partials, ws.offsets, nullptr);
+DigitPlan sort_digit_plan(uint32_t shape, uint32_t key_bits) {
+    DigitPlan p{};
+    p.passes = sort_shape_passes(shape, key_bits);
+    for (uint32_t i = 0; i <= p.passes && i <= kMaxPasses; ++i) p.shift[i] = key_bits * i / (p.passes ? p.passes : 1u);
+    return p;
 }
 
-// The digit bits of the pass at `shift` that lie below key_bits.
-static uint32_t pass_digit_mask(uint32_t bits, uint32_t key_bits, uint32_t shift) {
-    const uint32_t w = key_bits - shift < bits ? key_bits - shift : bits;
-    return (1u << w) - 1u;
+uint32_t sort_shape_for(uint32_t shape, uint32_t n, uint32_t key_bytes) {
+    if (shape != kShapeAuto) return shape % kNumShapes;
+    (void)n;
+    (void)key_bytes;
+    return 0;
 }
 
 static uint32_t hist_blocks(uint32_t n_max) {
@@ -475,108 +473,81 @@ static uint32_t hist_blocks(uint32_t n_max) {
     return hb < 1 ? 1 : (hb > kHistBlocks ? kHistBlocks : hb);
 }
 
-bool launch_sort_pairs(SortWorkspace& ws, uint64_t* keys, uint32_t* vals, uint64_t* keys_alt, uint32_t* vals_alt,
-                       const uint32_t* count_ptr, uint32_t n_max, uint32_t key_bits, hipStream_t s,
-                       hipEvent_t after_hist, uint32_t lo_bits, uint32_t* narrow_drop, uint32_t lo_base, bool counted,
-                       uint32_t* kept) {
-    const SortShape& sh = kShapes[ws.shape % kNumShapes];
-    const uint32_t R = 1u << sh.bits;
-    const uint32_t tile = sh.block * sh.items;
-    const uint32_t passes = (key_bits + sh.bits - 1) / sh.bits;
-    const uint32_t parts = (n_max + tile - 1) / tile;
-    if (parts == 0 || passes == 0 || passes > kMaxPasses) return false;
+// Counts the digits of every pass and scans them (offsets from word 0 of ws.offsets).
+template <typename KT>
+static void launch_count(SortWorkspace& ws, uint32_t shape, const DigitPlan& plan, const KT* keys,
+                         const uint32_t* count_ptr, uint32_t n_max, hipStream_t s) {
+    const uint32_t hb = hist_blocks(n_max), bits = sort_shape_bits(shape), tile = sort_shape_keys(shape);
+    if (bits == 8)
+        hipLaunchKernelGGL((k_sort_hist<8, KT>), dim3(hb), dim3(256), 0, s, keys, count_ptr, n_max, plan, tile,
+                           ws.partials, ws.desc, ws.tickets);
+    else
+        hipLaunchKernelGGL((k_sort_hist<9, KT>), dim3(hb), dim3(256), 0, s, keys, count_ptr, n_max, plan, tile,
+                           ws.partials, ws.desc, ws.tickets);
+    hipLaunchKernelGGL(k_sort_offsets, dim3(plan.passes), dim3(256), 0, s, ws.partials, ws.offsets, bits);
+}
 
-    const uint32_t hb = hist_blocks(n_max);
-    if (!counted) kept = nullptr;  // the histogram pass counts every key
-    if (counted) {
-        if (sh.bits == 8) hipLaunchKernelGGL(k_sort_offsets<8>, dim3(passes), dim3(256), 0, s, ws.partials, ws.offsets, kept);
-        else hipLaunchKernelGGL(k_sort_offsets<9>, dim3(passes), dim3(256), 0, s, ws.partials, ws.offsets, kept);
-    } else if (sh.bits == 8) {
-        launch_hist<8>(hb, passes, s, keys, count_ptr, n_max, lo_bits, lo_base, key_bits, tile, ws);
-    } else {
-        launch_hist<9>(hb, passes, s, keys, count_ptr, n_max, lo_bits, lo_base, key_bits, tile, ws);
-    }
-    if (after_hist) hipEventRecord(after_hist, s);
-    // With narrow_drop, the first pass whose digit starts at or above key_bits - 32 writes 32-bit
-    // keys (the bits from its digit up) and the later passes move 8 instead of 12 bytes per pair.
-    uint32_t narrow_pass = passes;
-    if (narrow_drop) {
-        for (uint32_t p = 0; p < passes; ++p)
-            if (key_bits <= p * sh.bits + 32) {
-                narrow_pass = p;
-                break;
-            }
-        *narrow_drop = narrow_pass < passes ? narrow_pass * sh.bits : kKeysWide;
-    }
-    if (narrow_pass == 0) kept = nullptr;  // the dropping pass reads and writes 64-bit keys
-    const uint64_t* kin = keys;
+// The passes of one sort, its digit offsets in `offsets`.  kept (optional): the first pass drops the
+// keys whose high word is zero, the later ones run on the *kept others.
+template <typename KT>
+static bool launch_passes(SortWorkspace& ws, uint32_t shape, const DigitPlan& plan, const uint32_t* offsets, KT* keys,
+                          uint32_t* vals, KT* keys_alt, uint32_t* vals_alt, const uint32_t* count_ptr, uint32_t n_max,
+                          const uint32_t* kept, hipStream_t s) {
+    const SortShape& sh = kShapes[shape];
+    const uint32_t R = 1u << sh.bits, tile = sh.block * sh.items, parts = (n_max + tile - 1) / tile;
+    const KT* kin = keys;
     const uint32_t* vin = vals;
-    uint64_t* kout = keys_alt;
+    KT* kout = keys_alt;
     uint32_t* vout = vals_alt;
-    for (uint32_t p = 0; p < passes; ++p) {
+    for (uint32_t p = 0; p < plan.passes; ++p) {
         OnesweepArgs o;
         o.keys_in = kin; o.vals_in = vin; o.keys_out = kout; o.vals_out = vout;
         o.count_ptr = (kept && p > 0) ? kept : count_ptr;
         o.n_imm = n_max;
-        o.shift = p * sh.bits;
-        o.lo_bits = lo_bits;
-        o.lo_base = lo_base;
-        o.drop = narrow_pass < passes ? narrow_pass * sh.bits : 0u;
-        o.digit_mask = pass_digit_mask(sh.bits, key_bits, o.shift);
-        const uint32_t mode = p < narrow_pass ? ((kept && p == 0) ? kWideDrop : kWide) : (p == narrow_pass ? kNarrow : kNarrowed);
-        o.offsets = ws.offsets + p * R;
+        o.shift = plan.shift[p];
+        o.digit_mask = (1u << (plan.shift[p + 1] - plan.shift[p])) - 1u;
+        o.offsets = offsets + p * R;
         o.desc = ws.desc + (size_t)(p & 1u) * ws.parts_cap * R;
         o.desc_next = ws.desc + (size_t)((p + 1) & 1u) * ws.parts_cap * R;
         o.ticket = ws.tickets + p;
+        const uint32_t mode = sizeof(KT) == 4 ? kKeys32 : (kept && p == 0) ? kKeys64Drop : kKeys64;
         hipLaunchKernelGGL(sh.kernel[mode], dim3(parts), dim3(sh.block), 0, s, o);
-        const uint64_t* tk = kout; kout = const_cast<uint64_t*>(kin); kin = tk;
-        const uint32_t* tv = vout; vout = const_cast<uint32_t*>(vin); vin = tv;
+        KT* const tk = kout; kout = const_cast<KT*>(kin); kin = tk;
+        uint32_t* const tv = vout; vout = const_cast<uint32_t*>(vin); vin = tv;
     }
-    return (passes & 1u) != 0;
+    return (plan.passes & 1u) != 0;
 }
 
-bool launch_sort_pairs32(SortWorkspace& ws, uint32_t* keys, uint32_t* vals, uint32_t* keys_alt, uint32_t* vals_alt,
-                         const uint32_t* count_ptr, uint32_t n_max, uint32_t key_bits, hipStream_t s,
-                         hipEvent_t after_hist, bool counted) {
-    const SortShape& sh = kShapes[ws.shape % kNumShapes];
-    const uint32_t R = 1u << sh.bits;
-    const uint32_t tile = sh.block * sh.items;
-    const uint32_t passes = (key_bits + sh.bits - 1) / sh.bits;
-    const uint32_t parts = (n_max + tile - 1) / tile;
-    if (parts == 0 || passes == 0 || passes > kMaxPasses) return false;
-    const uint32_t hb = hist_blocks(n_max);
-    if (counted) {
-        uint32_t* counts = ws.partials + kPairCountRow;
-        if (sh.bits == 8) hipLaunchKernelGGL(k_sort_offsets<8>, dim3(passes), dim3(256), 0, s, counts, ws.offsets, nullptr);
-        else hipLaunchKernelGGL(k_sort_offsets<9>, dim3(passes), dim3(256), 0, s, counts, ws.offsets, nullptr);
-    } else if (sh.bits == 8) {
-        launch_hist<8>(hb, passes, s, (const uint32_t*)keys, count_ptr, n_max, 32u, 0u, key_bits, tile, ws);
-    } else {
-        launch_hist<9>(hb, passes, s, (const uint32_t*)keys, count_ptr, n_max, 32u, 0u, key_bits, tile, ws);
-    }
-    if (after_hist) hipEventRecord(after_hist, s);
-    const uint32_t* kin = keys;
-    const uint32_t* vin = vals;
-    uint32_t* kout = keys_alt;
-    uint32_t* vout = vals_alt;
-    for (uint32_t p = 0; p < passes; ++p) {
-        OnesweepArgs o;
-        o.keys_in = kin; o.vals_in = vin; o.keys_out = kout; o.vals_out = vout;
-        o.count_ptr = count_ptr; o.n_imm = n_max;
-        o.shift = p * sh.bits;
-        o.lo_bits = 32u;
-        o.lo_base = 0u;
-        o.drop = 0u;
-        o.digit_mask = pass_digit_mask(sh.bits, key_bits, o.shift);
-        o.offsets = ws.offsets + p * R;
-        o.desc = ws.desc + (size_t)(p & 1u) * ws.parts_cap * R;
-        o.desc_next = ws.desc + (size_t)((p + 1) & 1u) * ws.parts_cap * R;
-        o.ticket = ws.tickets + p;
-        hipLaunchKernelGGL(sh.kernel[kNarrowed], dim3(parts), dim3(sh.block), 0, s, o);
-        const uint32_t* tk = kout; kout = const_cast<uint32_t*>(kin); kin = tk;
-        const uint32_t* tv = vout; vout = const_cast<uint32_t*>(vin); vin = tv;
-    }
-    return (passes & 1u) != 0;
+bool launch_sort_pairs(SortWorkspace& ws, uint64_t* keys, uint32_t* vals, uint64_t* keys_alt, uint32_t* vals_alt,
+                       uint32_t n, uint32_t key_bits, hipStream_t s) {
+    const uint32_t shape = sort_shape_for(ws.shape, n, 8);
+    const DigitPlan plan = sort_digit_plan(shape, key_bits);
+    if (n == 0 || plan.passes == 0 || plan.passes > kMaxPasses) return false;
+    launch_count(ws, shape, plan, (const uint64_t*)keys, nullptr, n, s);
+    return launch_passes(ws, shape, plan, ws.offsets, keys, vals, keys_alt, vals_alt, nullptr, n, nullptr, s);
+}
+
+void launch_sort_offsets(SortWorkspace& ws, uint32_t item_shape, uint32_t ipasses, uint32_t pair_shape, uint32_t ppasses,
+                         uint32_t* counters, const FrameTotals* totals, hipStream_t s) {
+    hipLaunchKernelGGL(k_frame_offsets, dim3(ipasses + ppasses), dim3(256), 0, s, ws.partials, ws.offsets,
+                       sort_shape_bits(item_shape), ipasses, sort_shape_bits(pair_shape), counters,
+                       totals ? *totals : FrameTotals{});
+}
+
+bool launch_sort_items(SortWorkspace& ws, uint32_t shape, uint64_t* keys, uint32_t* vals, uint64_t* keys_alt,
+                       uint32_t* vals_alt, uint32_t n, uint32_t lo_bits, const uint32_t* kept, hipStream_t s) {
+    return launch_passes(ws, shape, sort_digit_plan(shape, lo_bits), ws.offsets, keys, vals, keys_alt, vals_alt, nullptr,
+                         n, kept, s);
+}
+
+bool launch_sort_pairs32(SortWorkspace& ws, uint32_t shape, uint32_t* keys, uint32_t* vals, uint32_t* keys_alt,
+                         uint32_t* vals_alt, const uint32_t* count_ptr, uint32_t n_max, uint32_t key_bits, hipStream_t s,
+                         bool counted) {
+    const DigitPlan plan = sort_digit_plan(shape, key_bits);
+    if (n_max == 0 || plan.passes == 0 || plan.passes > kMaxPasses) return false;
+    if (!counted) launch_count(ws, shape, plan, (const uint32_t*)keys, count_ptr, n_max, s);
+    return launch_passes(ws, shape, plan, ws.offsets + (counted ? kPairCountRow : 0u), keys, vals, keys_alt, vals_alt,
+                         count_ptr, n_max, nullptr, s);
 }
 
 }  // namespace tpd

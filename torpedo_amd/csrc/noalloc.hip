@@ -82,7 +82,7 @@ extern "C" int tpd_sort_pairs_noalloc(tpd_ctx* c, uint64_t* d_keys, uint32_t* d_
     // The histogram kernel adds into the digit counts, which must start at zero.
     hipLaunchKernelGGL(k_clear_words, dim3((uint32_t)((kNaCountWords + 255) / 256)), dim3(256), 0, s, ws.partials,
                        (uint32_t)kNaCountWords);
-    *in_alt = launch_sort_pairs(ws, d_keys, d_vals, d_keys_alt, d_vals_alt, nullptr, n, key_bits, s) ? 1 : 0;
+    *in_alt = launch_sort_pairs(ws, d_keys, d_vals, d_keys_alt, d_vals_alt, n, key_bits, s) ? 1 : 0;
     e = hipGetLastError();
     if (e != hipSuccess) return hip_fail(e, "tpd_sort_pairs_noalloc: launch");
     return TPD_OK;

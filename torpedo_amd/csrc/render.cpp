@@ -1,15 +1,150 @@
 // The plain forward frame (GaussianEngine::rasterFrame, GaussianEngine.cpp:621-712).
+//
+// The reference sorts its (tile, Gaussian) pairs by (tile, depth).  Here the Gaussians are sorted by
+// depth first (stable, so equal depths keep Gaussian order), their pairs are emitted in that order and
+// sorted by tile alone (stable): the same order, (tile, depth, Gaussian), with the depth's digits
+// sorted once per visible Gaussian instead of once per pair, and 8-byte pairs instead of 12-byte ones.
+//
+// The whole frame is issued at once: its launches cover the pair capacity and read the pair count on
+// the device.  The count reaches the host while the frame's sorts still run; a frame that turns out to
+// have more pairs than the capacity, or a depth outside the window it was sorted on, stops there (every
+// later kernel returns) and is issued again.
 #include "tpd_ctx.hpp"
 
 #include <algorithm>
 
 namespace tpd {
 
-static int clear_frame_state(tpd_ctx* c, hipStream_t s) {
-    const size_t nd = (std::max<uint32_t>(c->n, 1u) + kPreBlock - 1) / kPreBlock;
-    hipError_t e = hipMemsetAsync(c->d_scan_desc, 0, nd * sizeof(uint64_t), s);
-    if (e == hipSuccess) e = hipMemsetAsync(c->d_counters, 0, sizeof(uint32_t) * kCtrCount, s);
-    return e == hipSuccess ? TPD_OK : hip_fail(e, "clear frame state");
+// The arguments shared by the frame's item kernel, its emission and the item offsets.
+static BatchArgs item_args(tpd_ctx* c) {
+    BatchArgs a{};
+    a.nitems = c->n;
+    a.scan_desc = c->d_scan_desc;
+    a.scan_desc2 = c->d_scan_desc2;
+    a.counters = c->d_counters;
+    a.splats = c->d_splats;
+    a.tiles = c->d_tiles;
+    a.offsets = c->d_offsets;
+    a.rects = c->d_rects;
+    a.item_keys = c->d_ikeys;
+    a.keys = c->d_keys;
+    a.vals = c->d_vals;
+    a.totals_known = 1u;
+    return a;
+}
+
+// Where each Gaussian's pairs lie in emission order: the exclusive scan of the tile counts, made for
+// the frames whose backward or tile readback asks for it.
+int ensure_offsets(tpd_ctx* c, hipStream_t s) {
+    if (c->have_offsets || c->n == 0) return TPD_OK;
+    hipError_t e = hipMemsetAsync(c->d_scan_desc2, 0, item_offset_parts(c->n) * sizeof(uint64_t), s);
+    if (e != hipSuccess) return hip_fail(e, "item offsets");
+    launch_batch_item_offsets(item_args(c), s);
+    e = hipGetLastError();
+    if (e != hipSuccess) return hip_fail(e, "item offsets");
+    c->have_offsets = true;
+    return TPD_OK;
+}
+
+// Waits until the frame's totals have reached h_counters (k_frame_offsets stores seq last).
+static int wait_totals(tpd_ctx* c, hipStream_t s, uint32_t seq) {
+    volatile uint32_t* const at = &c->h_counters[kHostSeq];
+    for (uint32_t spins = 1; __atomic_load_n(at, __ATOMIC_ACQUIRE) != seq; ++spins) {
+        if (spins % 4096u) continue;
+        const hipError_t e = hipStreamQuery(s);
+        if (e == hipErrorNotReady) {
+            (void)hipGetLastError();  // not an error to be found by a later check
+            continue;
+        }
+        if (e != hipSuccess) return hip_fail(e, "frame");
+        if (__atomic_load_n(at, __ATOMIC_ACQUIRE) != seq) return fail(TPD_ERR_STATE, "tpd_render: the frame ended without its totals");
+    }
+    return TPD_OK;
+}
+
+// Issues the frame once; c->frame_cap is the pair capacity it runs with.
+static int issue_frame(tpd_ctx* c, hipStream_t s, uint32_t gx, uint32_t gy) {
+    const uint32_t ntiles = gx * gy, W = c->cam.width, H = c->cam.height;
+    const uint32_t cap = (uint32_t)std::min<size_t>(c->cap_keys, kMaxSortKeys);
+    if (c->profile) hipEventRecord(c->ev[0], s);
+    if (c->d_ent_idx)
+        launch_entity_mats(c->d_models, c->n_ent, c->cam, c->d_ent_mats, s);
+    else
+        entity_mats(c->h_models.data(), c->cam, c->mats0);
+
+    const uint32_t lo_bits = c->depth_wide ? kDepthWideBits : kDepthWindowBits;
+    const uint32_t key_bits = bit_length(ntiles > 1 ? ntiles - 1 : 1);
+    const uint32_t ishape = sort_shape_for(c->item_shape, c->n, 8), pshape = sort_shape_for(c->ws.shape, cap, 4);
+    FrameArgs f{};
+    f.b = item_args(c);
+    BatchArgs& a = f.b;
+    a.cap = cap;
+    a.lo_bits = lo_bits;
+    a.lo_base = c->depth_wide ? 0u : kDepthBase;
+    a.hist_counts = c->ws.partials;
+    a.hist_desc0 = c->ws.desc;
+    a.hist_tickets = c->ws.tickets;
+    a.hist_bits = sort_shape_bits(ishape);
+    a.hist_plan = sort_digit_plan(ishape, lo_bits);
+    a.hist_desc0_words = ((c->n + sort_shape_keys(ishape) - 1) / sort_shape_keys(ishape)) << a.hist_bits;
+    a.pair_counts = c->ws.partials + kPairCountRow;
+    a.pair_bits = sort_shape_bits(pshape);
+    a.pair_plan = sort_digit_plan(pshape, key_bits);
+    a.pair_desc0_words = ((cap + sort_shape_keys(pshape) - 1) / sort_shape_keys(pshape)) << a.pair_bits;
+    a.ranges = c->d_ranges;
+    a.ntiles = ntiles;
+    f.gauss = c->d_gauss;
+    f.ent_idx = c->d_ent_idx;
+    f.ent = c->d_ent_mats;
+    f.mats0 = c->mats0;
+    f.cam = c->cam;
+    f.n = c->n;
+    f.sh_degree = c->sh_degree;
+    f.gx = gx;
+    f.gy = gy;
+    launch_frame_items(f, s);
+    if (c->profile) hipEventRecord(c->ev[1], s);
+    const FrameTotals totals{cap, lo_bits, ++c->frame_seq, c->d_host_counters};
+    launch_sort_offsets(c->ws, ishape, a.hist_plan.passes, pshape, a.pair_plan.passes, c->d_counters, &totals, s);
+    if (c->profile) hipEventRecord(c->ev[2], s);
+    const bool items_alt = launch_sort_items(c->ws, ishape, c->d_ikeys, c->d_ivals, c->d_ikeys_alt, c->d_ivals_alt, c->n,
+                                             lo_bits, &c->d_counters[kCtrItemsKept], s);
+    if (c->profile) hipEventRecord(c->ev[3], s);
+    a.kept_items = &c->d_counters[kCtrItemsKept];
+    a.sorted_items = items_alt ? c->d_ivals_alt : c->d_ivals;
+    a.sorted_keys64 = items_alt ? c->d_ikeys_alt : c->d_ikeys;
+    launch_batch_emit(a, s);
+    if (c->profile) hipEventRecord(c->ev[4], s);
+    const bool in_alt = launch_sort_pairs32(c->ws, pshape, c->d_keys, c->d_vals, c->d_keys_alt, c->d_vals_alt,
+                                            &c->d_counters[kCtrSortPairs], cap, key_bits, s, true);
+    if (c->profile) hipEventRecord(c->ev[5], s);
+    c->sorted_keys = in_alt ? c->d_keys_alt : c->d_keys;
+    c->sorted_vals = in_alt ? c->d_vals_alt : c->d_vals;
+    c->last_passes = a.hist_plan.passes + a.pair_plan.passes;
+    launch_ranges(c->sorted_keys, c->d_counters, cap, c->d_ranges, c->d_scan_desc,
+                  emit_parts(c->n), &c->d_counters[kCtrScanTicket], s, cap, kDepthWideBits);
+    launch_tile_order(c->d_ranges, ntiles, c->d_counters, c->d_tile_hist, c->d_jobs, gx, nullptr, nullptr, s);
+    if (c->profile) hipEventRecord(c->ev[6], s);
+    BlendArgs b{};
+    b.counters = c->d_counters;
+    b.jobs = c->d_jobs;
+    b.vals = c->sorted_vals;
+    b.splats = c->d_splats;
+    b.width = W;
+    b.height = H;
+    b.gx = gx;
+    b.ntiles = ntiles;
+    b.image = c->d_image;
+    b.rgba8 = c->d_rgba8;
+    b.eval_count = nullptr;  // counted on request, by blending the frame once more
+    b.final_T = c->d_final_T;  // kept for a backward of this frame
+    b.final_last = c->d_final_last;
+    b.tile_last = c->d_tile_last;
+    launch_blend(b, s);
+    c->last_blend = b;
+    if (c->profile) hipEventRecord(c->ev[7], s);
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? TPD_OK : hip_fail(e, "forward launch");
 }
 
 int render_forward(tpd_ctx* c, hipStream_t s) {
@@ -20,6 +155,7 @@ int render_forward(tpd_ctx* c, hipStream_t s) {
     int rc;
     if ((rc = ensure_scene_buffers(c)) != TPD_OK) return rc;
     if ((rc = ensure_image_buffers(c)) != TPD_OK) return rc;
+    c->have_offsets = false;
 
     if (c->n == 0) {
         // Empty scene: black image, empty ranges (GaussianEngine.cpp:362-365 renders nothing).
@@ -36,107 +172,37 @@ int render_forward(tpd_ctx* c, hipStream_t s) {
         c->last_pairs = 0;
         c->sorted_keys = c->d_keys;
         c->sorted_vals = c->d_vals;
-        c->key_drop = kKeysWide;
         return TPD_OK;
     }
 
-    if (c->profile) hipEventRecord(c->ev[0], s);
-    launch_entity_mats(c->d_models, c->n_ent, c->cam, c->d_ent_mats, s);
     if (c->cap_keys == 0 && (rc = ensure_pair_buffers(c, std::max<size_t>(4 * (size_t)c->n, 1u << 20))) != TPD_OK)
         return rc;
+    if ((rc = ensure_sort_workspace(c, std::max<size_t>(c->n, c->cap_keys))) != TPD_OK) return rc;
 
     uint32_t P = 0;
     for (int attempt = 0;; ++attempt) {
-        ForwardArgs a{};
-        a.gauss = c->d_gauss;
-        a.ent_idx = c->d_ent_idx;
-        a.ent = c->d_ent_mats;
-        a.cam = c->cam;
-        a.n = c->n;
-        a.sh_degree = c->sh_degree;
-        a.gx = gx;
-        a.gy = gy;
-        a.cap = (uint32_t)std::min<size_t>(c->cap_keys, kMaxSortKeys);
-        a.splats = c->d_splats;
-        a.tiles = c->d_tiles;
-        a.offsets = c->d_offsets;
-        a.scan_desc = c->d_scan_desc;
-        a.counters = c->d_counters;
-        a.keys = c->d_keys;
-        a.vals = c->d_vals;
-        a.ranges = c->d_ranges;
-        a.ntiles = ntiles;
-        launch_preprocess_dup(a, s);
-        if (c->profile) hipEventRecord(c->ev[1], s);
-        // The reference reads tilesRendered back here (GaussianEngine.cpp:659-674) to size its
-        // buffers; this read also detects a capacity overflow, which is replayed after growing.
-        e = hipMemcpyAsync(c->h_counters, c->d_counters, sizeof(uint32_t) * kCtrCount, hipMemcpyDeviceToHost, s);
-        if (e == hipSuccess) e = hipStreamSynchronize(s);
-        if (e != hipSuccess) return hip_fail(e, "preprocess");
-        P = c->h_counters[kCtrPairs];
-        if (P > kMaxSortKeys) {
-            clear_frame_state(c, s);
-            return fail(TPD_ERR_CAPACITY, "tpd_render: more than 2^30 - 1 tile/Gaussian pairs");
-        }
-        if (!c->h_counters[kCtrOverflow]) break;
-        if ((rc = clear_frame_state(c, s)) != TPD_OK) return rc;
-        if ((rc = ensure_pair_buffers(c, P)) != TPD_OK) return rc;
+        if ((rc = issue_frame(c, s, gx, gy)) != TPD_OK) return rc;
+        if ((rc = wait_totals(c, s, c->frame_seq)) != TPD_OK) return rc;
+        P = c->h_counters[kHostPairs];
+        const bool depth_out = c->h_counters[kHostDepthOut] != 0, was_wide = c->depth_wide;
+        if (P > kMaxSortKeys) return fail(TPD_ERR_CAPACITY, "tpd_render: more than 2^30 - 1 tile/Gaussian pairs");
+        c->depth_wide = depth_out;  // the next frame's key: the wider one only while a depth needs it
+        if (!c->h_counters[kHostOverflow]) break;
         if (attempt > 2) return fail(TPD_ERR_STATE, "tpd_render: pair buffers did not converge");
+        if (!(depth_out && !was_wide) || P > c->cap_keys) {
+            if ((rc = ensure_pair_buffers(c, P)) != TPD_OK) return rc;
+        }
     }
     c->last_pairs = P;
-    if (c->keep_unsorted && P) {
-        if ((rc = ensure_pair_buffers(c, P)) != TPD_OK) return rc;
-        e = hipMemcpyAsync(c->d_keys_dbg, c->d_keys, sizeof(uint64_t) * P, hipMemcpyDeviceToDevice, s);
-        if (e == hipSuccess) e = hipMemcpyAsync(c->d_vals_dbg, c->d_vals, sizeof(uint32_t) * P, hipMemcpyDeviceToDevice, s);
-        if (e != hipSuccess) return hip_fail(e, "copy unsorted pairs");
-    }
-
-    bool in_alt = false;
-    // Emitted depths are positive floats (view z > 0), so bit 31 of every key's low word is clear
-    // and the sort may run on the compacted (tile << 31) | depth key: same order, one bit less;
-    // when the preprocess saw no depth outside [2^-8, 2^8), on (tile << 27) | (depth - 2^-8 bits).
-    const bool depth_out = c->h_counters[kCtrDepthOut] != 0;
-    c->lo_bits = depth_out ? kDepthWideBits : kDepthWindowBits;
-    c->lo_base = depth_out ? 0u : kDepthBase;
-    if (depth_out && (e = hipMemsetAsync(&c->d_counters[kCtrDepthOut], 0, sizeof(uint32_t), s)) != hipSuccess)
-        return hip_fail(e, "clear depth flag");
-    const uint32_t key_bits = bit_length(ntiles > 1 ? ntiles - 1 : 1) + c->lo_bits;
-    c->last_passes = P > 0 ? sort_shape_passes(c->ws.shape, key_bits) : 0;
-    if (c->profile) hipEventRecord(c->ev[2], s);
-    if (P > 0)
-        in_alt = launch_sort_pairs(c->ws, c->d_keys, c->d_vals, c->d_keys_alt, c->d_vals_alt, nullptr, P, key_bits, s,
-                                   c->profile ? c->ev[3] : nullptr, c->lo_bits, &c->key_drop, c->lo_base);
-    else
-        c->key_drop = kKeysWide;
-    if (P == 0 && c->profile) hipEventRecord(c->ev[3], s);
-    if (c->profile) hipEventRecord(c->ev[4], s);
-    c->sorted_keys = in_alt ? c->d_keys_alt : c->d_keys;
-    c->sorted_vals = in_alt ? c->d_vals_alt : c->d_vals;
-    const uint32_t nd = (c->n + kPreBlock - 1) / kPreBlock;
-    launch_ranges(c->sorted_keys, c->d_counters, P, ntiles, c->d_ranges, c->d_scan_desc, nd,
-                  &c->d_counters[kCtrScanTicket], s, 0xFFFFFFFFu, c->key_drop, c->lo_bits);
-    launch_tile_order(c->d_ranges, ntiles, nullptr, c->d_tile_hist, c->d_jobs, gx, nullptr, nullptr, s);
-    if (c->profile) hipEventRecord(c->ev[5], s);
-    BlendArgs b{};
-    b.jobs = c->d_jobs;
-    b.vals = c->sorted_vals;
-    b.splats = c->d_splats;
-    b.width = W;
-    b.height = H;
-    b.gx = gx;
-    b.ntiles = ntiles;
-    b.image = c->d_image;
-    b.rgba8 = c->d_rgba8;
-    b.eval_count = nullptr;  // counted on request, by blending the frame once more
-    b.final_T = c->d_final_T;  // kept for a backward of this frame
-    b.final_last = c->d_final_last;
-    b.tile_last = c->d_tile_last;
-    launch_blend(b, s);
-    c->last_blend = b;
     c->has_blend = true;
-    if (c->profile) hipEventRecord(c->ev[6], s);
-    e = hipGetLastError();
-    if (e != hipSuccess) return hip_fail(e, "forward launch");
+    if (c->keep_unsorted && P) {
+        if ((rc = ensure_offsets(c, s)) != TPD_OK) return rc;
+        if ((e = grow(c->d_keys_dbg, c->cap_keys_dbg, P, 1.25)) != hipSuccess ||
+            (e = grow(c->d_vals_dbg, c->cap_vals_dbg, P, 1.25)) != hipSuccess)
+            return hip_fail(e, "alloc unsorted pairs");
+        launch_unsorted_pairs(c->d_splats, c->d_tiles, c->d_offsets, c->n, gx, gy, c->d_keys_dbg, c->d_vals_dbg, s);
+        if ((e = hipGetLastError()) != hipSuccess) return hip_fail(e, "unsorted pairs");
+    }
     return TPD_OK;
 }
 

@@ -37,24 +37,36 @@ struct tpd_ctx {
     tpd::Splat* d_splats = nullptr; size_t cap_splats = 0;
     uint32_t* d_tiles = nullptr; size_t cap_tiles = 0;
     uint32_t* d_offsets = nullptr; size_t cap_offsets = 0;
-    uint64_t* d_scan_desc = nullptr; size_t cap_scan_desc = 0;
+    uint64_t* d_scan_desc = nullptr; size_t cap_scan_desc = 0;    // the emission's, zero between frames
+    uint64_t* d_scan_desc2 = nullptr; size_t cap_scan_desc2 = 0;  // the item offsets', cleared before use
     uint32_t* d_counters = nullptr;
-    uint32_t* h_counters = nullptr;  // pinned
+    uint32_t* h_counters = nullptr;  // pinned: the frame's totals (kHost*), written by the device
+    uint32_t* d_host_counters = nullptr;  // the same memory as the device addresses it
 
-    // pairs + sort
-    uint64_t* d_keys = nullptr; size_t cap_keys = 0;
+    uint64_t* d_ikeys = nullptr; size_t cap_ikeys = 0;   // item sort: depth keys (+ tile rectangles) and
+    uint64_t* d_ikeys_alt = nullptr; size_t cap_ikeys_alt = 0;  // Gaussian indices, ping-pong
+    uint32_t* d_ivals = nullptr; size_t cap_ivals = 0;
+    uint32_t* d_ivals_alt = nullptr; size_t cap_ivals_alt = 0;
+    uint64_t* d_rects = nullptr; size_t cap_rects = 0;   // rectangles that do not fit their item's key
+    tpd::EntityMats mats0{};                             // scene without entity indices: its one model
+    bool have_offsets = false;                           // d_offsets is that of the last frame
+    uint32_t frame_seq = 0;                              // of the totals in h_counters
+
+    // pairs (tiles and Gaussian indices) + sort
+    uint32_t* d_keys = nullptr; size_t cap_keys = 0;
     uint32_t* d_vals = nullptr; size_t cap_vals = 0;
-    uint64_t* d_keys_alt = nullptr; size_t cap_keys_alt = 0;
+    uint32_t* d_keys_alt = nullptr; size_t cap_keys_alt = 0;
     uint32_t* d_vals_alt = nullptr; size_t cap_vals_alt = 0;
     uint64_t* d_keys_dbg = nullptr; size_t cap_keys_dbg = 0;
     uint32_t* d_vals_dbg = nullptr; size_t cap_vals_dbg = 0;
-    tpd::SortWorkspace ws;
-    const uint64_t* sorted_keys = nullptr;   // 64-bit keys, or 32-bit ones when key_drop != kKeysWide
-    uint32_t key_drop = tpd::kKeysWide;
-    // The last frame's sort key: (tile << lo_bits) | (depth bits - lo_base), the depth window
-    // (27, kDepthBase) or the positive-float form (31, 0).
-    uint32_t lo_bits = tpd::kDepthWideBits, lo_base = 0;
+    uint64_t* d_full_keys = nullptr; size_t cap_full_keys = 0;  // 64-bit keys rebuilt for readers
+    tpd::SortWorkspace ws;                       // shared by both sorts; ws.shape: that of the pair sort
+    uint32_t item_shape = tpd::kShapeAuto;
+    const uint32_t* sorted_keys = nullptr;
     const uint32_t* sorted_vals = nullptr;
+    // Depth key of the next frame's item sort: the depth window unless the last frame had a depth
+    // outside it.
+    bool depth_wide = false;
 
     // image
     uint2* d_ranges = nullptr; size_t cap_ranges = 0;
@@ -93,6 +105,7 @@ int ensure_image_buffers(tpd_ctx* c);
 int ensure_pair_buffers(tpd_ctx* c, size_t pairs);
 int ensure_sort_workspace(tpd_ctx* c, size_t pairs);
 int render_forward(tpd_ctx* c, hipStream_t s);
+int ensure_offsets(tpd_ctx* c, hipStream_t s);
 void backward_release(tpd_ctx* c);
 void batch_release(tpd_ctx* c);
 void batch_set_sort_shape(tpd_ctx* c, uint32_t shape);

@@ -388,25 +388,17 @@ __device__ __forceinline__ OpacityTerms opacity_terms(float o) {
     return OpacityTerms{__logf(1.0f / (255.0f * o)) - 0.01f, mask_q0(o)};
 }
 
-// Writes one splat record: the projected values (and the tile-independent part of the blend's
-// sub-block mask), or zeros for a culled Gaussian.  ot = opacity_terms(p.opacity).
-__device__ __forceinline__ void store_splat(Splat* dst, bool vis, const Projected& p, const OpacityTerms& ot) {
+// Writes one visible Gaussian's splat record: the projected values and the tile-independent part of
+// the blend's sub-block mask.  ot = opacity_terms(p.opacity).
+__device__ __forceinline__ void store_splat(Splat* dst, const Projected& p, const OpacityTerms& ot) {
+    const SubBlockReach r = sub_block_reach_q0(p.con_a, p.con_b, p.con_c, p.opacity, ot.q0);
     Splat s;
-    if (vis) {
-        const SubBlockReach r = sub_block_reach_q0(p.con_a, p.con_b, p.con_c, p.opacity, ot.q0);
-        s.xyzr = make_float4(p.px, p.py, p.vz, p.radius);
-        s.conop = make_float4(p.con_a, p.con_b, p.con_c, p.opacity);
-        s.rgb = make_float4(p.r, p.g, p.b, r.inva);
-        s.aux = make_float4(ot.skip, r.ey, r.vstar, r.aq0);
-    } else {
-        s.xyzr = s.conop = s.rgb = s.aux = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    }
+    s.xyzr = make_float4(p.px, p.py, p.vz, p.radius);
+    s.conop = make_float4(p.con_a, p.con_b, p.con_c, p.opacity);
+    s.rgb = make_float4(p.r, p.g, p.b, r.inva);
+    s.aux = make_float4(ot.skip, r.ey, r.vstar, r.aq0);
     *dst = s;
 }
-__device__ __forceinline__ void store_splat(Splat* dst, bool vis, const Projected& p) {
-    store_splat(dst, vis, p, vis ? opacity_terms(p.opacity) : OpacityTerms{0.0f, 0.0f});
-}
-
 
 // ------------------------------------------------------------------ wave64 helpers
 
@@ -502,7 +494,7 @@ __host__ __device__ __forceinline__ uint32_t xcd_unmap(uint32_t r, uint32_t nb) 
 
 // VM = view * model, PVM = projView * model (Slang mul order: each entry summed k = 0..3 left to
 // right; project.slang:48/57 via common.slang:102,106).  models null = identity.
-__device__ __forceinline__ void entity_mats(const float* __restrict__ model, const CameraParams& cam, EntityMats& out) {
+__host__ __device__ inline void entity_mats(const float* __restrict__ model, const CameraParams& cam, EntityMats& out) {
     float M[16];
     if (model) {
         for (int i = 0; i < 16; ++i) M[i] = model[i];
@@ -550,69 +542,11 @@ __device__ __forceinline__ uint64_t scan_lookback(uint64_t* desc, uint32_t part)
     }
 }
 
-// Pair emission of one block of 256 Gaussians for one view (keygen.slang:21-54): Gaussian i's
-// pairs go to positions base + excl_i + k, k row-major over its tile rectangle, with key
-// ((tile_base + tile) << 32) | depth bits and value val_first + i; positions at or past cap are
-// dropped (the frame overflowed).  A Gaussian with at most kOwnTiles tiles writes its pairs from
-// its own thread (emit_own_pairs, no search); the larger ones are spread over the block
-// (emit_large_pairs): pair j of the large ones belongs to the thread whose inclusive count of large
-// tiles s_big_incl first exceeds j, which balances footprints of thousands of tiles.
+// Rectangles of at most kOwnTiles tiles are emitted by their item's own thread, larger ones by the
+// whole block.
 constexpr uint32_t kOwnTiles = 4;
 
-__device__ __forceinline__ void emit_own_pairs(uint32_t tiles, int32_t x0, int32_t y0, int32_t x1, uint32_t depth,
-                                               uint64_t pos, uint32_t gx, uint32_t tile_base, uint64_t cap,
-                                               uint64_t* __restrict__ keys, uint32_t* __restrict__ vals,
-                                               uint32_t val) {
-    int32_t x = x0, y = y0;
-    for (uint32_t k = 0; k < tiles; ++k) {
-        if (pos + k < cap) {
-            keys[pos + k] = ((uint64_t)(tile_base + (uint32_t)y * gx + (uint32_t)x) << 32) | depth;
-            vals[pos + k] = val;
-        }
-        if (++x == x1) {
-            x = x0;
-            ++y;
-        }
-    }
-}
-
-template <uint32_t NB>  // threads of the block, one Gaussian each
-__device__ __forceinline__ void emit_large_pairs(const uint32_t* s_big_incl, const uint32_t* s_start,
-                                                 const int32_t* s_x0, const int32_t* s_y0, const int32_t* s_w,
-                                                 const uint32_t* s_depth, uint32_t big_total, uint64_t base,
-                                                 uint32_t gx, uint32_t tile_base, uint64_t cap,
-                                                 uint64_t* __restrict__ keys, uint32_t* __restrict__ vals,
-                                                 uint32_t val_first) {
-    for (uint32_t j = threadIdx.x; j < big_total; j += NB) {
-        uint32_t lo = 0, hi = NB - 1;
-        while (lo < hi) {
-            const uint32_t mid = (lo + hi) >> 1;
-            if (s_big_incl[mid] > j) hi = mid; else lo = mid + 1;
-        }
-        const uint32_t owner = lo;
-        const uint32_t k = j - (owner ? s_big_incl[owner - 1] : 0u);
-        const uint32_t w = (uint32_t)s_w[owner];
-        // k / w through a float reciprocal, corrected by one step either way (exact below 2^22)
-        uint32_t ry, rx;
-        if (k < (1u << 22)) {
-            int32_t q = (int32_t)((float)k * (1.0f / (float)w));
-            int32_t r = (int32_t)k - q * (int32_t)w;
-            if (r < 0) { --q; r += (int32_t)w; }
-            if (r >= (int32_t)w) { ++q; r -= (int32_t)w; }
-            ry = (uint32_t)q; rx = (uint32_t)r;
-        } else {
-            ry = k / w; rx = k - ry * w;
-        }
-        const uint32_t tile = tile_base + ((uint32_t)s_y0[owner] + ry) * gx + ((uint32_t)s_x0[owner] + rx);
-        const uint64_t gpos = base + s_start[owner] + k;
-        if (gpos < cap) {
-            keys[gpos] = ((uint64_t)tile << 32) | s_depth[owner];
-            vals[gpos] = val_first + owner;
-        }
-    }
-}
-
-// Pair emission of the batch, in depth order (k_batch_emit).  Each item carries one 64-bit
+// Pair emission in depth order (k_batch_emit).  Each item carries one 64-bit
 // emission record: the global tile of its rectangle's first tile (31 bits: global tiles stay below
 // 2^31), its view's tile-grid width and its rectangle's width and height in tiles (11 bits each:
 // grids are at most 1024 tiles wide and high); zero for an item without tiles.  Its k-th pair

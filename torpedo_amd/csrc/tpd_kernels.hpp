@@ -12,9 +12,11 @@ enum : uint32_t {
     kCtrOverflow = 2,     // 1 when P exceeded the key/value capacity
     kCtrDepthOut = 3,     // non-zero when an emitted depth lies outside the sort's depth window
     kCtrScanTicket2 = 4,  // partition ticket of a second scan in the frame (the batch's item offsets)
-    kCtrSortPairs = 5,    // the batch's pair count for its pair sort and ranges: P, or 0 when P exceeded
-                          // the capacity (that frame is rendered again)
-    kCtrItemsKept = 32,   // the batch's visible items: those the item sort keeps (its later passes and
+    kCtrSortPairs = 5,    // pair count for the pair sort and the ranges: P, or 0 when the frame overflowed
+                          // (it is rendered again)
+    kCtrTotal64 = 6,      // (two words) the plain frame's pair count, summed by its item kernel; zero between
+                          // frames
+    kCtrItemsKept = 32,   // the visible items: those the item sort keeps (its later passes and
                           // the emission run on them).  128 bytes past the tickets: every emission
                           // block reads it right after its ticket atomic, and on the tickets' L2
                           // line that read would queue behind the other blocks' atomics
@@ -22,10 +24,10 @@ enum : uint32_t {
 };
 
 // The sort's depth window.  Culling keeps view depths inside [near, far], and depths in
-// [2^-8, 2^8) have float bit patterns in [kDepthBase, kDepthBase + 2^27): for such frames the sort
-// may key on (tile << 27) | (depth bits - kDepthBase), in the same order as (tile << 32) | depth
-// bits and with 4 bits less than the positive-float form (tile << 31) | depth bits.  A frame with
-// any depth outside the window (flagged by its preprocess in kCtrDepthOut) sorts that 31-bit form.
+// [2^-8, 2^8) have float bit patterns in [kDepthBase, kDepthBase + 2^27): such frames sort their items
+// by the 27 bits (depth bits - kDepthBase), in the same order as the depth bits and with 4 bits less
+// than a positive float.  A frame with any depth outside the window (flagged by its item kernel in
+// kCtrDepthOut) sorts the 31-bit form.
 constexpr uint32_t kDepthBase = 0x3B800000u;  // floatbits(2^-8)
 constexpr uint32_t kDepthWindowBits = 27;
 constexpr uint32_t kDepthWideBits = 31;
@@ -33,24 +35,13 @@ __device__ __forceinline__ bool depth_outside_window(float vz) {
     return __float_as_uint(vz) - kDepthBase >= (1u << kDepthWindowBits);
 }
 
-struct ForwardArgs {
-    const float* gauss;          // N x 60 floats (GaussianPoint records)
-    const uint32_t* ent_idx;     // N entity indices, or null (entity 0 for all)
-    const EntityMats* ent;       // per-entity matrices
-    CameraParams cam;
-    uint32_t n, sh_degree, gx, gy;
-    uint32_t cap;                // pair capacity of keys/vals
-    Splat* splats;               // per Gaussian (zeros when culled)
-    uint32_t* tiles;             // tile count per Gaussian
-    uint32_t* offsets;           // exclusive scan of tiles
-    uint64_t* scan_desc;         // look-back descriptors, one per partition of the preprocess (the
-                                 // buffer holds ceil(N/256)), zero on entry
-    uint32_t* counters;          // kCtr* block
-    uint64_t* keys;
-    uint32_t* vals;
-    uint32_t val_base;           // value written for Gaussian i is val_base + i
-    uint2* ranges;               // zeroed here for the ranges kernel
-    uint32_t ntiles;
+// The digits of an LSD radix sort's passes: pass p orders the bits [shift[p], shift[p + 1]) of the key.
+// The key's bits are shared out evenly (13 bits in two passes: 6 and 7, not 8 and 5): fewer digits in
+// a pass mean longer runs of equal digits, and the length of the runs it writes bounds a pass.
+constexpr uint32_t kMaxPasses = 8;
+struct DigitPlan {
+    uint32_t passes;
+    uint32_t shift[kMaxPasses + 1];
 };
 
 // A block of the blend: one tile, its sorted pairs and (in a batch) its view, in the launch order of
@@ -62,6 +53,7 @@ struct alignas(16) TileJob {
 };
 
 struct BlendArgs {
+    const uint32_t* counters;    // the frame's kCtr* block: nothing is done after an overflow
     const TileJob* jobs;         // per block (heaviest tiles first)
     const uint32_t* vals;
     const Splat* splats;
@@ -90,8 +82,9 @@ struct BackwardArgs {
 
 struct PreBackwardArgs {
     const float* gauss;
-    const uint32_t* ent_idx;
-    const EntityMats* ent;
+    const uint32_t* ent_idx;     // N entity indices, or null: every Gaussian uses mats0
+    const EntityMats* ent;       // per entity (with ent_idx)
+    EntityMats mats0;
     CameraParams cam;
     uint32_t n, sh_degree;
     const uint32_t* tiles;
@@ -110,22 +103,19 @@ void launch_blend_bwd(const BackwardArgs& a, hipStream_t s);
 void launch_preprocess_bwd(const PreBackwardArgs& a, hipStream_t s);
 
 void launch_entity_mats(const float* models, uint32_t n_ent, const CameraParams& cam, EntityMats* out, hipStream_t s);
-void launch_preprocess_dup(const ForwardArgs& a, hipStream_t s);
-// Sorted keys are 64-bit (tile << 32) | depth, or, after a sort that narrowed them, 32-bit
-// (compacted key (tile << lo_bits) | (depth - lo_base)) >> drop; key_drop = kKeysWide marks the
-// first form.
-constexpr uint32_t kKeysWide = 0xFFFFFFFFu;
-// Tile ranges of the sorted keys; P = min(counters[count_slot], cap).  Also re-zeroes the scan
-// descriptors and the scan ticket for the next frame, and sets kCtrOverflow when a frame sorted
-// on the depth-window key (lo_bits = kDepthWindowBits) has kCtrDepthOut set.
-void launch_ranges(const void* keys, uint32_t* counters, uint32_t P_hint, uint32_t ntiles, uint2* ranges,
-                   uint64_t* scan_desc, uint32_t n_scan_desc, uint32_t* ticket, hipStream_t s,
-                   uint32_t cap = 0xFFFFFFFFu, uint32_t key_drop = kKeysWide, uint32_t lo_bits = kDepthWideBits,
-                   uint32_t count_slot = kCtrPairs);
-// The 64-bit keys (tile << 32) | floatbits(view depth) of n sorted 32-bit keys, the tile from the
-// key and the depth from the splat of each value (for readers of the sorted pairs).
-void launch_full_keys(const uint32_t* keys32, uint32_t drop, uint32_t lo_bits, const uint32_t* vals,
-                      const Splat* splats, uint32_t n, uint64_t* out, hipStream_t s);
+// Tile ranges of the P = min(counters[count_slot], cap) sorted keys (tiles).  Also re-zeroes the scan
+// descriptors and the scan tickets for the next frame, and sets kCtrOverflow when a frame whose items
+// were sorted on the depth-window key (lo_bits = kDepthWindowBits) has kCtrDepthOut set.
+void launch_ranges(const uint32_t* keys, uint32_t* counters, uint32_t P_hint, uint2* ranges, uint64_t* scan_desc,
+                   uint32_t n_scan_desc, uint32_t* ticket, hipStream_t s, uint32_t cap, uint32_t lo_bits);
+// The 64-bit keys (tile << 32) | floatbits(view depth) of n sorted tile keys, the depth from the splat
+// of each value (for readers of the sorted pairs).
+void launch_full_keys(const uint32_t* keys, const uint32_t* vals, const Splat* splats, uint32_t n, uint64_t* out,
+                      hipStream_t s);
+// The plain frame's pairs in the reference's emission order (Gaussian by Gaussian, row-major over each
+// one's rectangle), 64-bit keys, at the scan of the tile counts (for readers of the unsorted pairs).
+void launch_unsorted_pairs(const Splat* splats, const uint32_t* tiles, const uint32_t* offsets, uint32_t n, uint32_t gx,
+                           uint32_t gy, uint64_t* keys, uint32_t* vals, hipStream_t s);
 void launch_blend(const BlendArgs& a, hipStream_t s);
 // The tiles in launch order for the blend: classes of pair count (bit length) from the heaviest
 // down, empty tiles last, so that the longest tiles start first and the short ones fill the tail.
@@ -180,8 +170,8 @@ struct BatchArgs {
     const uint32_t* block_scene;  // scene of each preprocess block
     uint32_t nblocks, nviews, nitems;
     const EntityMats* mats;
-    uint64_t* scan_desc;          // 2 x ceil(nitems / kEmitBlockItems) look-back descriptors, zero on entry: the
-                                  // emission's, then the item offsets
+    uint64_t* scan_desc;          // look-back descriptors, zero on entry: one per emission partition ...
+    uint64_t* scan_desc2;         // ... and one per partition of the item offsets
     uint32_t* counters;           // kCtr* block
     uint32_t cap;                 // pair capacity
     Splat* splats;                // per item (written for visible items only)
@@ -202,13 +192,16 @@ struct BatchArgs {
     uint32_t* hist_counts;
     uint32_t* hist_desc0;
     uint32_t* hist_tickets;
-    uint32_t hist_bits, hist_passes, hist_desc0_words;
+    uint32_t hist_bits, hist_desc0_words;
+    DigitPlan hist_plan;
     // the pair sort's digit histograms, counted by the item kernel from each visible item's tile
     // rectangle (needs hist_counts): counts from row kPairCountRow of the sort's digit counts, digit
     // width and passes of the pair sort's shape; the emission clears the pair sort's first-pass
     // descriptors (pair_desc0_words, for the pair capacity) and the tickets
     uint32_t* pair_counts;
-    uint32_t pair_bits, pair_passes, pair_desc0_words;
+    uint32_t pair_bits, pair_desc0_words;
+    DigitPlan pair_plan;
+    uint32_t totals_known;          // the emission finds P and the overflow flag in the counters (plain frame)
     const uint32_t* kept_items;     // emission input: the number of sorted items (the visible ones) ...
     const uint64_t* sorted_keys64;  // ... the item keys in depth order ...
     const uint32_t* sorted_items;   // ... and their items
@@ -216,6 +209,17 @@ struct BatchArgs {
     uint32_t* vals;               //        item
     uint2* ranges;                // all views' tiles, cleared by the item kernel
     uint32_t ntiles;
+};
+
+// The plain frame's items: one view of one scene, its tables in the kernel's arguments.
+struct FrameArgs {
+    BatchArgs b;
+    const float* gauss;           // N x 60 records (any alignment)
+    const uint32_t* ent_idx;      // N entity indices, or null: every Gaussian uses mats0
+    const EntityMats* ent;
+    EntityMats mats0;
+    CameraParams cam;
+    uint32_t n, sh_degree, gx, gy;
 };
 
 struct BatchBlendArgs {
@@ -262,9 +266,12 @@ struct BatchPreBwdArgs {
 void launch_batch_mats(const BatchSceneDev* scenes, const BatchViewDev* views, uint32_t nviews, uint32_t max_ent,
                        EntityMats* mats, uint32_t* counters, hipStream_t s);
 void launch_batch_items(const BatchArgs& a, hipStream_t s);
+void launch_frame_items(const FrameArgs& a, hipStream_t s);
 void launch_batch_emit(const BatchArgs& a, hipStream_t s);
 void launch_batch_item_offsets(const BatchArgs& a, hipStream_t s);
-constexpr uint32_t kEmitBlockItems = 4096;  // sorted items per emission partition (k_batch_emit)
+// Partitions of the emission (smaller ones for fewer items) and of the item offsets.
+uint32_t emit_parts(uint32_t nitems);
+uint32_t item_offset_parts(uint32_t nitems);
 void launch_batch_blend(const BatchBlendArgs& a, hipStream_t s);
 void launch_batch_blend_bwd(const BatchBlendArgs& a, hipStream_t s);
 void launch_batch_preprocess_bwd(const BatchPreBwdArgs& a, hipStream_t s);
@@ -274,10 +281,11 @@ void launch_batch_preprocess_bwd(const BatchPreBwdArgs& a, hipStream_t s);
 constexpr uint32_t kMaxRadixBits = 9;                      // digit widths 8 and 9 bits
 constexpr uint32_t kMaxRadix = 1u << kMaxRadixBits;
 constexpr uint32_t kSortMinTile = 2048;                    // smallest partition of any block shape
-constexpr uint32_t kMaxPasses = 8;
 constexpr uint32_t kCountCopies = 8;  // copies of the digit counts, block b adds into copy b mod 8
 constexpr uint32_t kHistBlocks = 1024;                      // blocks of the digit-histogram kernel
 constexpr uint32_t kMaxSortKeys = (1u << 30) - 1;          // 30-bit look-back values
+
+constexpr uint32_t kShapeAuto = 0xFFFFFFFFu;  // the shape the key count and width ask for (sort_shape_for)
 
 struct SortWorkspace {
     uint32_t* desc = nullptr;      // 2 regions x parts_cap x kMaxRadix look-back descriptors
@@ -285,49 +293,52 @@ struct SortWorkspace {
     uint32_t* partials = nullptr;  // kCountCopies x kMaxPasses x kMaxRadix digit counts (zero between sorts)
     uint32_t* offsets = nullptr;   // kMaxPasses x kMaxRadix global exclusive digit offsets
     uint32_t* tickets = nullptr;   // kMaxPasses partition tickets
-    uint32_t shape = 0;            // onesweep block shape (index into the tuner's table)
+    uint32_t shape = kShapeAuto;   // onesweep block shape (index into the tuner's table), or kShapeAuto
 };
 
 // Partitions for n keys at the smallest partition size (descriptor capacity for every shape).
 __host__ __device__ inline uint32_t sort_parts(uint32_t n) { return (n + kSortMinTile - 1) / kSortMinTile; }
 uint32_t sort_num_shapes();
+// The shape itself, or for kShapeAuto the one for n keys of key_bytes.
+uint32_t sort_shape_for(uint32_t shape, uint32_t n, uint32_t key_bytes);
 uint32_t sort_shape_keys(uint32_t shape);
-uint32_t sort_shape_bits(uint32_t shape);                      // digit width of a shape
+uint32_t sort_shape_bits(uint32_t shape);                       // digit width of a shape
 uint32_t sort_shape_passes(uint32_t shape, uint32_t key_bits);  // passes for key_bits bits
+DigitPlan sort_digit_plan(uint32_t shape, uint32_t key_bits);
 
-// Stable LSD sort of (keys, vals) by the low key_bits bits of the keys.  n comes from *count_ptr
-// when count_ptr is non-null (device-resident count capped at n_max, grids sized by n_max), else
-// from n_max.
-// Returns true when the sorted data ended in the alternate buffers.
-// after_hist (optional) is recorded between the histogram kernels and the first onesweep pass.
-// lo_bits < 32 sorts the compacted key (high word << lo_bits) | (low word - lo_base), valid when
-// every key's low word lies in [lo_base, lo_base + 2^lo_bits); key_bits then counts the compacted
-// key's bits.  A low word outside that range cannot change the high word's bits in the compacted
-// key (the difference is masked to lo_bits bits), only the order among keys of equal high word.
-// narrow_drop (optional) lets the later passes move 32-bit keys: *narrow_drop receives the number
-// of low compacted-key bits the sorted 32-bit keys leave out, or kKeysWide if the keys stayed
-// 64-bit (see launch_ranges).
+// Stable LSD sort of n (64-bit key, value) pairs by the low key_bits bits of the keys.  Returns true
+// when the sorted data ended in the alternate buffers.
 bool launch_sort_pairs(SortWorkspace& ws, uint64_t* keys, uint32_t* vals, uint64_t* keys_alt, uint32_t* vals_alt,
-                       const uint32_t* count_ptr, uint32_t n_max, uint32_t key_bits, hipStream_t s,
-                       hipEvent_t after_hist = nullptr, uint32_t lo_bits = 32, uint32_t* narrow_drop = nullptr,
-                       uint32_t lo_base = 0, bool counted = false, uint32_t* kept = nullptr);
-// With counted, the digit counts are already in ws.partials and the first pass's descriptors and the
-// tickets already cleared (by the kernel that made the keys): the histogram kernel is not launched.
-// With kept as well (and 64-bit keys in the first pass), the counts leave out the keys whose high
-// word is zero and the first pass drops those keys: *kept receives the number of keys kept, the
-// later passes sort those, and the result holds the kept keys in order (stable), nothing after.
-// The first pass then also takes each key's index as its value: vals is not read, only used as
-// the later passes' buffer.
-constexpr uint32_t kMaxCountedPasses = 4;  // passes whose counts the item kernel can make
-// The same sort of 32-bit keys (key bits at and above key_bits zero) with 32-bit values: every pass
-// moves 8 bytes per pair.  Returns true when the result is in keys_alt / vals_alt.  With counted,
-// the digit counts are in ws.partials from word kPairCountRow of each copy on, and the first pass's
-// descriptors and the tickets are already cleared.
-bool launch_sort_pairs32(SortWorkspace& ws, uint32_t* keys, uint32_t* vals, uint32_t* keys_alt, uint32_t* vals_alt,
-                         const uint32_t* count_ptr, uint32_t n_max, uint32_t key_bits, hipStream_t s,
-                         hipEvent_t after_hist = nullptr, bool counted = false);
-constexpr uint32_t kPairCountRow = kMaxCountedPasses * kMaxRadix;  // after the item sort's counted rows
+                       uint32_t n, uint32_t key_bits, hipStream_t s);
+
+// The frame's sorts, whose digit counts the item kernel has made (it also cleared the first pass's
+// descriptors and the tickets): items in ws.partials from word 0 of each copy, pairs from word
+// kPairCountRow.  launch_sort_offsets turns both into digit offsets (items from word 0 of ws.offsets,
+// pairs from kPairCountRow) and re-zeroes the counts.  pair_shape with ppasses = 0: no counted pairs.
+// With a frame (totals non-null) it also settles the frame's totals from the item kernel's: kCtrPairs,
+// kCtrOverflow (more pairs than cap, or a depth outside the window of an item sort on it), kCtrSortPairs,
+// and tells the host.
+constexpr uint32_t kMaxCountedPasses = 4;      // item passes whose counts the item kernel can make
 constexpr uint32_t kMaxCountedPairPasses = 3;
+constexpr uint32_t kPairCountRow = kMaxCountedPasses * kMaxRadix;
 static_assert(kPairCountRow + kMaxCountedPairPasses * kMaxRadix <= kMaxPasses * kMaxRadix, "pair count rows");
+enum : uint32_t { kHostPairs = 0, kHostOverflow = 1, kHostDepthOut = 2, kHostSeq = 3 };  // words of FrameTotals::host
+struct FrameTotals {
+    uint32_t cap, lo_bits;
+    uint32_t seq;      // stored last, when the other words are there
+    uint32_t* host;    // pinned host memory
+};
+void launch_sort_offsets(SortWorkspace& ws, uint32_t item_shape, uint32_t ipasses, uint32_t pair_shape, uint32_t ppasses,
+                         uint32_t* counters, const FrameTotals* totals, hipStream_t s);
+// Sorts the n items by the low lo_bits bits of their keys.  The first pass drops the keys whose high
+// word is zero (the counts leave them out) and takes each key's index as its value; the later ones
+// sort the *kept others.
+bool launch_sort_items(SortWorkspace& ws, uint32_t shape, uint64_t* keys, uint32_t* vals, uint64_t* keys_alt,
+                       uint32_t* vals_alt, uint32_t n, uint32_t lo_bits, const uint32_t* kept, hipStream_t s);
+// Sorts the min(*count_ptr, n_max) pairs by the low key_bits bits of their 32-bit keys; without
+// counted, their digits are counted first.
+bool launch_sort_pairs32(SortWorkspace& ws, uint32_t shape, uint32_t* keys, uint32_t* vals, uint32_t* keys_alt,
+                         uint32_t* vals_alt, const uint32_t* count_ptr, uint32_t n_max, uint32_t key_bits, hipStream_t s,
+                         bool counted);
 
 }  // namespace tpd

@@ -6,40 +6,6 @@
 #include <algorithm>
 #include <vector>
 
-namespace tpd {
-
-static int rerun_duplicate(tpd_ctx* c, hipStream_t s) {
-    const uint32_t W = c->cam.width, H = c->cam.height;
-    const uint32_t gx = (W + kTile - 1) / kTile, gy = (H + kTile - 1) / kTile;
-    ForwardArgs a{};
-    a.gauss = c->d_gauss;
-    a.ent_idx = c->d_ent_idx;
-    a.ent = c->d_ent_mats;
-    a.cam = c->cam;
-    a.n = c->n;
-    a.sh_degree = c->sh_degree;
-    a.gx = gx;
-    a.gy = gy;
-    a.cap = (uint32_t)std::min<size_t>(c->cap_keys, kMaxSortKeys);
-    a.splats = c->d_splats;
-    a.tiles = c->d_tiles;
-    a.offsets = c->d_offsets;
-    a.scan_desc = c->d_scan_desc;
-    a.counters = c->d_counters;
-    a.keys = c->d_keys;
-    a.vals = c->d_vals;
-    a.ranges = c->d_ranges;
-    a.ntiles = gx * gy;
-    launch_preprocess_dup(a, s);
-    const size_t nd = (c->n + kPreBlock - 1) / kPreBlock;
-    hipError_t e = hipMemsetAsync(c->d_scan_desc, 0, nd * sizeof(uint64_t), s);
-    if (e == hipSuccess) e = hipMemsetAsync(&c->d_counters[kCtrScanTicket], 0, sizeof(uint32_t), s);
-    if (e == hipSuccess) e = hipMemsetAsync(&c->d_counters[kCtrDepthOut], 0, sizeof(uint32_t), s);
-    return e == hipSuccess ? TPD_OK : hip_fail(e, "autotune");
-}
-
-}  // namespace tpd
-
 using namespace tpd;
 
 extern "C" {
@@ -48,10 +14,13 @@ int tpd_set_sort_shape(tpd_ctx* c, uint32_t shape) {
     if (!c) return fail(TPD_ERR_INVALID, "null context");
     if (shape >= sort_num_shapes()) return fail(TPD_ERR_INVALID, "tpd_set_sort_shape: no such shape");
     c->ws.shape = shape;
+    c->item_shape = shape;
     batch_set_sort_shape(c, shape);
     return TPD_OK;
 }
 
+// Times both sorts (items by depth, pairs by tile) of whole frames per shape and keeps the fastest
+// shape for each; sort_ms[shape] = both sorts' time, *best = the pair sort's shape.
 int tpd_autotune(tpd_ctx* c, float* sort_ms, uint32_t capacity, uint32_t* n_shapes, uint32_t* best) {
     if (!c) return fail(TPD_ERR_INVALID, "null context");
     hipSetDevice(c->device);
@@ -60,49 +29,50 @@ int tpd_autotune(tpd_ctx* c, float* sort_ms, uint32_t capacity, uint32_t* n_shap
     if (!c->rendered || c->n == 0 || c->last_pairs == 0)
         return fail(TPD_ERR_STATE, "tpd_autotune: render a non-empty frame first");
     hipStream_t s = c->stream;
-    const uint32_t W = c->cam.width, H = c->cam.height;
-    const uint32_t ntiles = ((W + kTile - 1) / kTile) * ((H + kTile - 1) / kTile);
-    const uint32_t key_bits = bit_length(ntiles > 1 ? ntiles - 1 : 1) + c->lo_bits;  // the last frame's key
-    hipEvent_t e0, e1;
-    if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess)
-        return fail(TPD_ERR_HIP, "tpd_autotune: hipEventCreate");
-    const uint32_t keep = c->ws.shape;
-    std::vector<float> med(ns, 0.0f);
-    int rc = TPD_OK;
+    const uint32_t keep_items = c->item_shape, keep_pairs = c->ws.shape;
+    const bool keep_profile = c->profile;
+    int rc = tpd_set_profiling(c, 1);
+    std::vector<float> med(ns, 0.0f), items(ns, 0.0f), pairs(ns, 0.0f);
     for (uint32_t sh = 0; sh < ns && rc == TPD_OK; ++sh) {
-        c->ws.shape = sh;
-        std::vector<float> t;
+        c->item_shape = c->ws.shape = sh;
+        std::vector<float> ti, tp, t;
         for (int rep = 0; rep < 4 && rc == TPD_OK; ++rep) {
-            if ((rc = rerun_duplicate(c, s)) != TPD_OK) break;
-            hipEventRecord(e0, s);
-            uint32_t drop = kKeysWide;  // with the narrowed passes, as render_forward sorts
-            launch_sort_pairs(c->ws, c->d_keys, c->d_vals, c->d_keys_alt, c->d_vals_alt, nullptr, c->last_pairs,
-                              key_bits, s, nullptr, c->lo_bits, &drop, c->lo_base);
-            hipEventRecord(e1, s);
-            if (hipEventSynchronize(e1) != hipSuccess) {
-                rc = fail(TPD_ERR_HIP, "tpd_autotune: sort failed");
+            if ((rc = render_forward(c, s)) != TPD_OK) break;
+            float mi = 0.0f, mp = 0.0f;
+            if (hipEventSynchronize(c->ev[5]) != hipSuccess ||
+                hipEventElapsedTime(&mi, c->ev[2], c->ev[3]) != hipSuccess ||
+                hipEventElapsedTime(&mp, c->ev[4], c->ev[5]) != hipSuccess) {
+                rc = fail(TPD_ERR_HIP, "tpd_autotune: timing");
                 break;
             }
-            float ms = 0.0f;
-            hipEventElapsedTime(&ms, e0, e1);
-            if (rep > 0) t.push_back(ms);  // first run warms up
+            if (rep > 0) {  // first run warms up
+                ti.push_back(mi);
+                tp.push_back(mp);
+                t.push_back(mi + mp);
+            }
         }
-        if (!t.empty()) {
-            std::sort(t.begin(), t.end());
-            med[sh] = t[t.size() / 2];
-        }
+        const auto median = [](std::vector<float>& v) {
+            std::sort(v.begin(), v.end());
+            return v.empty() ? 0.0f : v[v.size() / 2];
+        };
+        items[sh] = median(ti);
+        pairs[sh] = median(tp);
+        med[sh] = median(t);
     }
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
+    c->profile = keep_profile;
     if (rc != TPD_OK) {
-        c->ws.shape = keep;
+        c->item_shape = keep_items;
+        c->ws.shape = keep_pairs;
         return rc;
     }
-    uint32_t b = 0;
-    for (uint32_t sh = 1; sh < ns; ++sh)
-        if (med[sh] < med[b]) b = sh;
-    c->ws.shape = b;
-    if (best) *best = b;
+    uint32_t bi = 0, bp = 0;
+    for (uint32_t sh = 1; sh < ns; ++sh) {
+        if (items[sh] < items[bi]) bi = sh;
+        if (pairs[sh] < pairs[bp]) bp = sh;
+    }
+    c->item_shape = bi;
+    c->ws.shape = bp;
+    if (best) *best = bp;
     if (sort_ms)
         for (uint32_t sh = 0; sh < ns && sh < capacity; ++sh) sort_ms[sh] = med[sh];
     // Leave a consistent frame behind (keys/ranges/image of the current camera).
