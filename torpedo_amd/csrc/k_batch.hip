@@ -316,45 +316,35 @@ void launch_batch_items(const BatchArgs& a, hipStream_t s) {
 
 // ------------------------------------------------------------------ pair emission in depth order
 
-// Blocks take partitions of 512 x PT depth-sorted items (PT consecutive ones per thread, so that a
-// thread has that many independent record loads in flight) from an atomic ticket; item i's pairs go to
-// base + the exclusive scan of the tile counts over the sorted items (decoupled look-back over the
-// partitions), key = global tile, value = item.  Items with at most kOwnTiles tiles write their own
-// pairs; the larger ones are spread over the block (pair j of them belongs to the item whose inclusive
-// count of large tiles first exceeds j).  The last partition stores the pair total and the overflow
-// flag (unless a.totals_known).
+// Blocks take partitions of 512 x PT depth-sorted items (PT consecutive ones per thread) from an atomic
+// ticket; item i's pairs go to base + the exclusive scan of the tile counts over the sorted items
+// (decoupled look-back over the partitions), key = global tile, value = item.  The last partition
+// stores the pair total and the overflow flag (unless a.totals_known).
+//
+// The pairs are made position by position: a thread takes 8 consecutive places of the output, aligned
+// so that it stores them with 16-byte stores, and needs the item each belongs to.  Items mark the place
+// of their first pair in LDS and a maximum scan (thread, wave, block) spreads the marks, so every place
+// costs the same whatever the rectangles' sizes: bound by the stores.  (Small rectangles written by
+// their own thread and the places of large ones found by a binary search over the block's items, 13
+// dependent LDS reads each: 534 us for 22M pairs of 1M items, 500 us for 61M pairs of 32M items;
+// this way @EMIT_DENSE@ and @EMIT_BATCH@ us.)
 constexpr uint32_t kEmitThreads = 512;
+constexpr uint32_t kEmitRun = 8;                              // places per thread
+constexpr uint32_t kEmitChunk = kEmitThreads * kEmitRun;      // places per round of the block
 
-// Pairs of the block's small rectangles staged per chunk before they are written out: the large
-// items' tables (start, rectangle; their values are re-read from the sorted items) are done with
-// by then and lend their space.  For PT = 8, 2 x 4,096 - 512 pairs: with the large items' tables
-// (48 KB) in the same space, the kernel's LDS stays under 80 KB, two blocks of 512 threads per CU.
-constexpr uint32_t kEmitMaxChunks = 4;
-constexpr uint32_t kNoPair = 0xFFFFFFFFu;  // an empty staging slot (no item has this index)
 template <uint32_t PT>
-union EmitLds {
-    static constexpr uint32_t kItems = kEmitThreads * PT;
-    static constexpr uint32_t kStage = 2 * kItems - kEmitThreads;
-    struct {
-        uint32_t start[kItems];
-        uint64_t rect[kItems];
-    } big;
-    struct {
-        uint32_t key[kStage], val[kStage];
-    } stage;
+struct EmitLds {
+    uint4 item[kEmitThreads * PT];  // first place, first tile, width | grid width << 16, item
+    alignas(16) uint16_t own[kEmitChunk];  // 1 + the block's item whose pairs begin at the place, else 0
+    uint32_t wave_sum[kEmitThreads / kWave], wave_max[kEmitThreads / kWave];
+    uint64_t base;
+    uint32_t part;
 };
 
 template <uint32_t PT>
 __global__ __launch_bounds__(kEmitThreads) void k_batch_emit(const BatchArgs a) {
-    __shared__ uint32_t s_part;
-    __shared__ uint32_t s_wave_sum[kEmitThreads / kWave], s_wave_big[kEmitThreads / kWave];
-    constexpr uint32_t kEmitPerThread = PT, kEmitItems = EmitLds<PT>::kItems, kEmitStage = EmitLds<PT>::kStage;
-    __shared__ uint32_t s_big_incl[kEmitItems];
+    constexpr uint32_t kItems = kEmitThreads * PT;
     __shared__ EmitLds<PT> L;
-    __shared__ uint64_t s_base;
-    uint32_t* const s_start = L.big.start;
-    uint64_t* const s_rect = L.big.rect;
-
     const uint32_t tid = threadIdx.x, wave = tid / kWave, lane = __lane_id();
     if (a.totals_known && a.counters[kCtrOverflow]) return;  // the frame is rendered again
     // the pair sort's counts come from the item kernel: its first pass's descriptors (which the
@@ -368,7 +358,7 @@ __global__ __launch_bounds__(kEmitThreads) void k_batch_emit(const BatchArgs a) 
     // first nparts blocks take tickets 0 .. nparts - 1.
     const uint32_t nitems =
         __builtin_amdgcn_readfirstlane(a.kept_items ? min(*a.kept_items, a.nitems) : a.nitems);
-    const uint32_t nparts = (nitems + kEmitItems - 1) / kEmitItems;
+    const uint32_t nparts = (nitems + kItems - 1) / kItems;
     if (blockIdx.x >= nparts) {
         if (blockIdx.x == 0 && tid == 0 && !a.totals_known) {  // no visible item: the totals the last partition would store
             a.counters[kCtrPairs] = 0u;
@@ -377,23 +367,22 @@ __global__ __launch_bounds__(kEmitThreads) void k_batch_emit(const BatchArgs a) 
         }
         return;
     }
-    if (tid == 0) s_part = atomicAdd(&a.counters[kCtrScanTicket], 1u);
+    if (tid == 0) L.part = atomicAdd(&a.counters[kCtrScanTicket], 1u);
     __syncthreads();
-    const uint32_t part = __builtin_amdgcn_readfirstlane(s_part);
+    const uint32_t part = __builtin_amdgcn_readfirstlane(L.part);
     if (part >= nparts) return;  // never: the first nparts blocks share nparts tickets
-    const uint32_t i0 = part * kEmitItems + tid * kEmitPerThread;
+    const uint32_t i0 = part * kItems + tid * PT;
 
-    uint32_t item[kEmitPerThread];
-    uint64_t rect[kEmitPerThread];
-    if (i0 + kEmitPerThread <= nitems) {
+    uint32_t item[PT], rect[PT];  // rect: the key's high word (inline_rect)
+    if (i0 + PT <= nitems) {
 #pragma unroll
-        for (uint32_t j = 0; j < kEmitPerThread; j += 2) {  // i0 is a multiple of PT, which is even
+        for (uint32_t j = 0; j < PT; j += 2) {  // i0 is a multiple of PT, which is even
             const ulonglong2 k = *reinterpret_cast<const ulonglong2*>(a.sorted_keys64 + i0 + j);
-            rect[j] = k.x; rect[j + 1] = k.y;
+            rect[j] = (uint32_t)(k.x >> 32); rect[j + 1] = (uint32_t)(k.y >> 32);
         }
         if constexpr (PT % 4 == 0) {
 #pragma unroll
-            for (uint32_t j = 0; j < kEmitPerThread; j += 4) {
+            for (uint32_t j = 0; j < PT; j += 4) {
                 const uint4 v = *reinterpret_cast<const uint4*>(a.sorted_items + i0 + j);
                 item[j] = v.x; item[j + 1] = v.y; item[j + 2] = v.z; item[j + 3] = v.w;
             }
@@ -404,49 +393,37 @@ __global__ __launch_bounds__(kEmitThreads) void k_batch_emit(const BatchArgs a) 
         }
     } else {
 #pragma unroll
-        for (uint32_t j = 0; j < kEmitPerThread; ++j) {
+        for (uint32_t j = 0; j < PT; ++j) {
             item[j] = i0 + j < nitems ? a.sorted_items[i0 + j] : 0u;
-            rect[j] = i0 + j < nitems ? a.sorted_keys64[i0 + j] : 0ull;
+            rect[j] = i0 + j < nitems ? (uint32_t)(a.sorted_keys64[i0 + j] >> 32) : 0u;
         }
     }
+    // The items' tile counts, and the places of their first pairs in the block.
+    uint32_t t[PT], mine = 0;
+    uint4 rec[PT];
 #pragma unroll
-    for (uint32_t j = 0; j < kEmitPerThread; ++j) rect[j] = rect_of((uint32_t)(rect[j] >> 32), a.rects, item[j]);
-    uint32_t t[kEmitPerThread], mine = 0, mine_big = 0;
-#pragma unroll
-    for (uint32_t j = 0; j < kEmitPerThread; ++j) {
-        t[j] = emit_rect_w(rect[j]) * emit_rect_h(rect[j]);
+    for (uint32_t j = 0; j < PT; ++j) {
+        const uint64_t r = rect_of(rect[j], a.rects, item[j]);
+        t[j] = rect[j] ? emit_rect_w(r) * emit_rect_h(r) : 0u;  // 0: past the end
+        rec[j] = make_uint4(mine, emit_rect_tile0(r), emit_rect_w(r) | emit_rect_gx(r) << 16, item[j]);
         mine += t[j];
-        mine_big += t[j] > kOwnTiles ? t[j] : 0u;
     }
-    const uint32_t incl_w = wave_incl_scan(mine), big_w = wave_incl_scan(mine_big);
-    if (lane == kWave - 1) {
-        s_wave_sum[wave] = incl_w;
-        s_wave_big[wave] = big_w;
-    }
+    const uint32_t incl_w = wave_incl_scan(mine);
+    if (lane == kWave - 1) L.wave_sum[wave] = incl_w;
+    *reinterpret_cast<uint4*>(&L.own[tid * kEmitRun]) = make_uint4(0u, 0u, 0u, 0u);
     __syncthreads();
-    uint32_t wave_off = 0, block_total = 0, big_off = 0, big_total = 0;
+    uint32_t wave_off = 0, block_total = 0;
 #pragma unroll
     for (uint32_t w = 0; w < kEmitThreads / kWave; ++w) {
-        const uint32_t v = s_wave_sum[w], vb = s_wave_big[w];
+        const uint32_t v = L.wave_sum[w];
         wave_off += (w < wave) ? v : 0u;
         block_total += v;
-        big_off += (w < wave) ? vb : 0u;
-        big_total += vb;
     }
-    // this thread's items: their block-local starts, and their inclusive counts of large tiles
-    uint32_t start = wave_off + incl_w - mine, big_incl = big_off + big_w - mine_big;
-    uint32_t first[kEmitPerThread];
+    const uint32_t start = wave_off + incl_w - mine;
 #pragma unroll
-    for (uint32_t j = 0; j < kEmitPerThread; ++j) {
-        const uint32_t o = tid * kEmitPerThread + j;
-        first[j] = start;
-        if (t[j] > kOwnTiles) {
-            big_incl += t[j];
-            s_start[o] = start;
-            s_rect[o] = rect[j];
-        }
-        s_big_incl[o] = big_incl;
-        start += t[j];
+    for (uint32_t j = 0; j < PT; ++j) {
+        rec[j].x += start;
+        L.item[tid * PT + j] = rec[j];
     }
     if (wave == 0) {
         if (lane == 0) store_relaxed(&a.scan_desc[part], (part == 0 ? kDescP : kDescA) | (uint64_t)block_total);
@@ -454,7 +431,7 @@ __global__ __launch_bounds__(kEmitThreads) void k_batch_emit(const BatchArgs a) 
         if (part > 0) excl = scan_lookback(a.scan_desc, part);
         if (lane == 0) {
             if (part > 0) store_relaxed(&a.scan_desc[part], kDescP | (excl + block_total));
-            s_base = excl;
+            L.base = excl;
             if (part == nparts - 1 && !a.totals_known) {
                 const uint64_t total = excl + block_total;
                 a.counters[kCtrPairs] = total > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)total;
@@ -464,36 +441,68 @@ __global__ __launch_bounds__(kEmitThreads) void k_batch_emit(const BatchArgs a) 
         }
     }
     __syncthreads();
-    const uint64_t base = s_base;
-    // (a large item's value is read back from the sorted items, which this block has just read)
-    emit_large_rects(s_big_incl, s_start, s_rect, a.sorted_items + part * kEmitItems, kEmitItems, big_total, base,
-                     a.cap, a.keys, a.vals);
-    // The small rectangles' pairs (at most kOwnTiles per item, written by the item's thread) go
-    // through LDS, chunk by chunk of the block's output range, so that the stores to HBM are
-    // consecutive across lanes; slots of the large items' pairs stay empty and are skipped.  A
-    // block whose large items make its range longer than kEmitMaxChunks chunks writes them directly.
-    if (block_total > kEmitMaxChunks * kEmitStage) {
+    const uint64_t base = L.base;
+    // Places are counted from the output position at or below base that is a multiple of 8: place p is
+    // position base - lead + p, and the block's pairs are places [lead, lead + block_total).
+    const uint32_t lead = (uint32_t)base & (kEmitRun - 1u), end = lead + block_total;
+    const uint64_t pos0 = base - lead;
+    uint32_t carry = 0;  // 1 + the last item whose pairs began before this round
+    for (uint32_t c0 = 0; c0 < end; c0 += kEmitChunk) {
 #pragma unroll
-        for (uint32_t j = 0; j < kEmitPerThread; ++j)
-            if (t[j] && t[j] <= kOwnTiles) emit_own_rect(t[j], rect[j], base + first[j], a.cap, a.keys, a.vals, item[j]);
-        return;
-    }
-    for (uint32_t c0 = 0; c0 < block_total; c0 += kEmitStage) {
-        const uint32_t n = min(block_total - c0, kEmitStage);
-        __syncthreads();  // the large items' tables, or the previous chunk, are done with
-        for (uint32_t p = tid; p < n; p += kEmitThreads) L.stage.val[p] = kNoPair;
+        for (uint32_t j = 0; j < PT; ++j) {
+            const uint32_t p = lead + rec[j].x - c0;  // wraps below c0: then not < kEmitChunk
+            if (t[j] != 0u && p < kEmitChunk) L.own[p] = (uint16_t)(tid * PT + j + 1u);
+        }
         __syncthreads();
+        uint4* const mark = reinterpret_cast<uint4*>(&L.own[tid * kEmitRun]);
+        const uint4 m = *mark;
+        *mark = make_uint4(0u, 0u, 0u, 0u);
+        uint32_t o[kEmitRun] = {m.x & 0xFFFFu, m.x >> 16, m.y & 0xFFFFu, m.y >> 16,
+                                m.z & 0xFFFFu, m.z >> 16, m.w & 0xFFFFu, m.w >> 16};
 #pragma unroll
-        for (uint32_t j = 0; j < kEmitPerThread; ++j)
-            if (t[j] && t[j] <= kOwnTiles) stage_own_rect(t[j], rect[j], first[j], c0, n, L.stage.key, L.stage.val, item[j]);
+        for (uint32_t q = 1; q < kEmitRun; ++q) o[q] = max(o[q], o[q - 1]);
+        const uint32_t scan = wave_incl_max(o[kEmitRun - 1]);
+        if (lane == kWave - 1) L.wave_max[wave] = scan;
         __syncthreads();
-        for (uint32_t p = tid; p < n; p += kEmitThreads) {
-            const uint32_t v = L.stage.val[p];
-            const uint64_t g = base + c0 + p;
-            if (v != kNoPair && g < a.cap) {
-                a.keys[g] = L.stage.key[p];
-                a.vals[g] = v;
-            }
+        uint32_t before = max(carry, wave_below(scan));
+#pragma unroll
+        for (uint32_t w = 0; w < kEmitThreads / kWave; ++w) {
+            const uint32_t v = L.wave_max[w];
+            before = w < wave ? max(before, v) : before;
+            carry = max(carry, v);
+        }
+        const uint32_t p0 = c0 + tid * kEmitRun;
+        if (p0 >= end) continue;
+        uint32_t key[kEmitRun], val[kEmitRun];
+#pragma unroll
+        for (uint32_t q = 0; q < kEmitRun; ++q) {
+            const uint32_t owner = max(max(o[q], before), 1u) - 1u;  // (item 0 for the places before the first)
+            const uint4 r = L.item[owner];
+            // row and column of the pair in the rectangle: k / w through an approximate reciprocal,
+            // corrected by one step either way (k < 2^22: grids are at most 2048 x 2048 tiles)
+            const uint32_t k = p0 + q - lead - r.x, w = r.z & 0xFFFFu;
+            int32_t ry = (int32_t)((float)k * __builtin_amdgcn_rcpf((float)w));
+            int32_t rx = (int32_t)k - ry * (int32_t)w;
+            if (rx < 0) { --ry; rx += (int32_t)w; }
+            if (rx >= (int32_t)w) { ++ry; rx -= (int32_t)w; }
+            key[q] = r.y + (uint32_t)ry * (r.z >> 16) + (uint32_t)rx;
+            val[q] = r.w;
+        }
+        const uint64_t pos = pos0 + p0;
+        if (p0 >= lead && p0 + kEmitRun <= end && pos + kEmitRun <= a.cap) {
+            uint4* const dk = reinterpret_cast<uint4*>(a.keys + pos);
+            uint4* const dv = reinterpret_cast<uint4*>(a.vals + pos);
+            dk[0] = make_uint4(key[0], key[1], key[2], key[3]);
+            dk[1] = make_uint4(key[4], key[5], key[6], key[7]);
+            dv[0] = make_uint4(val[0], val[1], val[2], val[3]);
+            dv[1] = make_uint4(val[4], val[5], val[6], val[7]);
+        } else {
+#pragma unroll
+            for (uint32_t q = 0; q < kEmitRun; ++q)
+                if (p0 + q >= lead && p0 + q < end && pos + q < a.cap) {
+                    a.keys[pos + q] = key[q];
+                    a.vals[pos + q] = val[q];
+                }
         }
     }
 }

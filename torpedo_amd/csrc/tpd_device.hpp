@@ -434,6 +434,23 @@ __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v) {
     return (uint32_t)x;
 }
 
+// The same with the maximum (lanes without a source read 0).
+__device__ __forceinline__ uint32_t wave_incl_max(uint32_t v) {
+    const auto step = [&](auto x) { v = max(v, (uint32_t)x); };
+    step(__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xF, 0xF, true));
+    step(__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xF, 0xF, true));
+    step(__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xF, 0xF, true));
+    step(__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xF, 0xF, true));
+    step(__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xA, 0xF, false));
+    step(__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, false));
+    return v;
+}
+
+// The value of the lane below; 0 in lane 0.
+__device__ __forceinline__ uint32_t wave_below(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x138, 0xF, 0xF, true);  // wave_shr:1
+}
+
 __device__ __forceinline__ uint64_t wave_sum_u64(uint64_t v) {
 #pragma unroll
     for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d, 64);
@@ -542,23 +559,19 @@ __device__ __forceinline__ uint64_t scan_lookback(uint64_t* desc, uint32_t part)
     }
 }
 
-// Rectangles of at most kOwnTiles tiles are emitted by their item's own thread, larger ones by the
-// whole block.
-constexpr uint32_t kOwnTiles = 4;
-
-// Pair emission in depth order (k_batch_emit).  Each item carries one 64-bit
-// emission record: the global tile of its rectangle's first tile (31 bits: global tiles stay below
-// 2^31), its view's tile-grid width and its rectangle's width and height in tiles (11 bits each:
-// grids are at most 1024 tiles wide and high); zero for an item without tiles.  Its k-th pair
-// (row-major over the rectangle) has key tile0 + (k / w) gx + k % w and value the item; positions
-// at or past cap are dropped (the frame overflowed).
+// Pair emission in depth order (k_batch_emit).  Each item carries one 64-bit emission record: the
+// global tile of its rectangle's first tile (31 bits: global tiles stay below 2^31), its view's
+// tile-grid width and its rectangle's width and height in tiles, each less one (11 bits: grids are at
+// most 2048 tiles wide and high).  Its k-th pair (row-major over the rectangle) has key
+// tile0 + (k / w) gx + k % w and value the item; positions at or past cap are dropped (the frame
+// overflowed).
 __host__ __device__ inline uint64_t pack_emit_rect(uint32_t tile0, uint32_t gx, uint32_t w, uint32_t h) {
-    return (uint64_t)tile0 | ((uint64_t)gx << 31) | ((uint64_t)w << 42) | ((uint64_t)h << 53);
+    return (uint64_t)tile0 | ((uint64_t)(gx - 1u) << 31) | ((uint64_t)(w - 1u) << 42) | ((uint64_t)(h - 1u) << 53);
 }
 __host__ __device__ inline uint32_t emit_rect_tile0(uint64_t r) { return (uint32_t)(r & 0x7FFFFFFFull); }
-__host__ __device__ inline uint32_t emit_rect_gx(uint64_t r) { return (uint32_t)(r >> 31) & 0x7FFu; }
-__host__ __device__ inline uint32_t emit_rect_w(uint64_t r) { return (uint32_t)(r >> 42) & 0x7FFu; }
-__host__ __device__ inline uint32_t emit_rect_h(uint64_t r) { return (uint32_t)(r >> 53) & 0x7FFu; }
+__host__ __device__ inline uint32_t emit_rect_gx(uint64_t r) { return ((uint32_t)(r >> 31) & 0x7FFu) + 1u; }
+__host__ __device__ inline uint32_t emit_rect_w(uint64_t r) { return ((uint32_t)(r >> 42) & 0x7FFu) + 1u; }
+__host__ __device__ inline uint32_t emit_rect_h(uint64_t r) { return ((uint32_t)(r >> 53) & 0x7FFu) + 1u; }
 
 // An item's emission record as carried through the item sort in the high word of its 64-bit key
 // (the sort orders by the low word alone): 0 for a culled item; for a rectangle of at most 4 x 4
@@ -571,82 +584,10 @@ __host__ __device__ inline uint32_t inline_rect(uint32_t tile0, uint32_t gx, uin
                ? tile0 | ((w - 1u) << 21) | ((h - 1u) << 23) | (gx << 25)
                : kRectLookup;
 }
+// The record of a visible item (u its key's high word).
 __device__ __forceinline__ uint64_t rect_of(uint32_t u, const uint64_t* __restrict__ rects, uint32_t item) {
-    if (u == 0u) return 0ull;
     if ((u >> 25) == 0u) return rects[item];
     return pack_emit_rect(u & 0x1FFFFFu, u >> 25, ((u >> 21) & 3u) + 1u, ((u >> 23) & 3u) + 1u);
-}
-
-__device__ __forceinline__ void emit_own_rect(uint32_t tiles, uint64_t rect, uint64_t pos, uint64_t cap,
-                                              uint32_t* __restrict__ keys, uint32_t* __restrict__ vals, uint32_t val) {
-    const uint32_t w = emit_rect_w(rect), gx = emit_rect_gx(rect);
-    uint32_t row = emit_rect_tile0(rect), x = 0;
-    for (uint32_t k = 0; k < tiles; ++k) {
-        if (pos + k < cap) {
-            keys[pos + k] = row + x;
-            vals[pos + k] = val;
-        }
-        if (++x == w) {
-            x = 0;
-            row += gx;
-        }
-    }
-}
-
-// The same pairs into a staging chunk: pair k (block-local position first + k) is placed at slot
-// first + k - c0 when that lies in [0, n).
-__device__ __forceinline__ void stage_own_rect(uint32_t tiles, uint64_t rect, uint32_t first, uint32_t c0,
-                                               uint32_t n, uint32_t* keys, uint32_t* vals, uint32_t val) {
-    if (first + tiles <= c0 || first >= c0 + n) return;
-    const uint32_t w = emit_rect_w(rect), gx = emit_rect_gx(rect);
-    uint32_t row = emit_rect_tile0(rect), x = 0;
-    for (uint32_t k = 0; k < tiles; ++k) {
-        const uint32_t slot = first + k - c0;  // wraps past 2^32 below c0: then >= n
-        if (slot < n) {
-            keys[slot] = row + x;
-            vals[slot] = val;
-        }
-        if (++x == w) {
-            x = 0;
-            row += gx;
-        }
-    }
-}
-
-// The large items of a block: s_big_incl[o] is the inclusive count of large tiles over the block's
-// items 0..o (n of them), s_start/s_rect the block-local first pair and the record of a large item
-// o, item_vals[o] its value (the block's sorted items).
-__device__ __forceinline__ void emit_large_rects(const uint32_t* s_big_incl, const uint32_t* s_start,
-                                                 const uint64_t* s_rect, const uint32_t* __restrict__ item_vals,
-                                                 uint32_t n,
-                                                 uint32_t big_total, uint64_t base, uint64_t cap,
-                                                 uint32_t* __restrict__ keys, uint32_t* __restrict__ vals) {
-    for (uint32_t j = threadIdx.x; j < big_total; j += blockDim.x) {
-        uint32_t lo = 0, hi = n - 1;
-        while (lo < hi) {
-            const uint32_t mid = (lo + hi) >> 1;
-            if (s_big_incl[mid] > j) hi = mid; else lo = mid + 1;
-        }
-        const uint32_t owner = lo;
-        const uint32_t k = j - (owner ? s_big_incl[owner - 1] : 0u);
-        const uint64_t rect = s_rect[owner];
-        const uint32_t w = emit_rect_w(rect);
-        uint32_t ry, rx;
-        if (k < (1u << 22)) {  // k / w through a float reciprocal, corrected by one step
-            int32_t q = (int32_t)((float)k * (1.0f / (float)w));
-            int32_t r = (int32_t)k - q * (int32_t)w;
-            if (r < 0) { --q; r += (int32_t)w; }
-            if (r >= (int32_t)w) { ++q; r -= (int32_t)w; }
-            ry = (uint32_t)q; rx = (uint32_t)r;
-        } else {
-            ry = k / w; rx = k - ry * w;
-        }
-        const uint64_t gpos = base + s_start[owner] + k;
-        if (gpos < cap) {
-            keys[gpos] = emit_rect_tile0(rect) + ry * emit_rect_gx(rect) + rx;
-            vals[gpos] = item_vals[owner];
-        }
-    }
 }
 
 }  // namespace tpd
