@@ -17,15 +17,15 @@ def eng():
     e.close()
 
 
-# Gaussians per emission partition: 1,024 below 1,048,576 items, 2,048 below 2,097,152, then 4,096; the item
-# kernel's grid strides from 262,144 on.
-@pytest.mark.parametrize("n", [1, 2, 511, 1023, 1024, 1025, 2049, 262_145])
+# Gaussians per emission partition: 512 below 262,144 (and wherever there is room for 8 pairs each), 1,024
+# below 524,288, 2,048 below 8,388,608, then 4,096; the item kernel's grid strides from 262,144 on.
+@pytest.mark.parametrize("n", [1, 2, 511, 512, 513, 1023, 1024, 1025, 2049, 262_143, 262_145, 524_289])
 def test_partition_edges(eng, orc, n):
     compare_frame(eng, orc, small_scene(n, seed=n, log_scale_mean=-3.5), c1_camera(orc, 200, 120), 3,
                   f"emission n={n}", check_f64=False)
 
 
-@pytest.mark.parametrize("n", [1_048_577, 2_100_001])
+@pytest.mark.parametrize("n", [1_048_577, 2_100_001, 8_388_611])
 def test_larger_partitions(eng, orc, n):
     from torpedo_amd import scenes
     compare_frame(eng, orc, scenes.uniform_scene(n, seed=7, log_scale_mean=-6.0), c1_camera(orc, 640, 360), 0,

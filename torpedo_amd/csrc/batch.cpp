@@ -262,8 +262,8 @@ static int build_layout(tpd_ctx* c, BatchState* b) {
         (e = grow(b->d_final_last, b->cap_final_last, std::max<size_t>(pix, 1))) != hipSuccess ||
         (e = grow(b->d_rgba8, b->cap_rgba8, std::max<size_t>(4 * pix, 1))) != hipSuccess)
         return hip_fail(e, "tpd_batch: alloc");
-    // look-back descriptors: the emission's, then the item offsets' (frames kept for a backward)
-    const size_t nparts = std::max<size_t>(emit_parts((uint32_t)items) + item_offset_parts((uint32_t)items), 1);
+    // look-back descriptors: the item offsets' (frames kept for a backward), then the emission's
+    const size_t nparts = std::max<size_t>(emit_max_parts((uint32_t)items) + item_offset_parts((uint32_t)items), 1);
     if (!b->d_scan_desc || b->cap_scan_desc < nparts) {
         if ((e = grow(b->d_scan_desc, b->cap_scan_desc, nparts)) != hipSuccess) return hip_fail(e, "tpd_batch: alloc");
     }
@@ -379,8 +379,8 @@ static BatchArgs forward_args(BatchState* b, bool keep_bwd) {
     a.nviews = (uint32_t)b->views.size();
     a.nitems = b->nitems;
     a.mats = b->d_mats;
-    a.scan_desc = b->d_scan_desc;
-    a.scan_desc2 = b->d_scan_desc + emit_parts(b->nitems);
+    a.scan_desc = b->d_scan_desc + item_offset_parts(b->nitems);
+    a.scan_desc2 = b->d_scan_desc;
     a.counters = b->d_counters;
     a.cap = b->cap;
     a.splats = b->d_splats;
@@ -475,7 +475,7 @@ static void record_forward(BatchState* b, bool keep_bwd, hipStream_t s, bool eve
     if (events) hipEventRecord(b->ev[4], s);
     // lo_bits tells the ranges kernel whether the items were sorted on the depth window
     launch_ranges(b->sorted_keys, b->d_counters, b->cap, b->d_ranges, b->d_scan_desc,
-                  emit_parts(b->nitems) + item_offset_parts(b->nitems), &b->d_counters[kCtrScanTicket], s, b->cap,
+                  emit_parts(b->nitems, b->cap) + item_offset_parts(b->nitems), &b->d_counters[kCtrScanTicket], s, b->cap,
                   b->lo_bits());
     launch_tile_order(b->d_ranges, b->ntiles, b->d_counters, b->d_tile_hist, b->d_jobs, 0, b->d_tile_view, b->d_views, s);
     if (events) hipEventRecord(b->ev[5], s);

@@ -46,7 +46,7 @@ int ensure_scene_buffers(tpd_ctx* c) {
         return hip_fail(e, "alloc items");
     if ((e = grow(c->d_scan_desc2, c->cap_scan_desc2, item_offset_parts((uint32_t)n))) != hipSuccess)
         return hip_fail(e, "alloc scan desc");
-    const size_t nd = emit_parts((uint32_t)n);
+    const size_t nd = emit_max_parts((uint32_t)n);
     if (!c->d_scan_desc || c->cap_scan_desc < nd) {
         if ((e = grow(c->d_scan_desc, c->cap_scan_desc, nd)) != hipSuccess) return hip_fail(e, "alloc scan desc");
         if ((e = hipMemset(c->d_scan_desc, 0, c->cap_scan_desc * sizeof(uint64_t))) != hipSuccess)

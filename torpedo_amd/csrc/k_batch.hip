@@ -374,9 +374,9 @@ __global__ __launch_bounds__(kEmitThreads) void k_batch_emit(const BatchArgs a) 
     const uint32_t i0 = part * kItems + tid * PT;
 
     uint32_t item[PT], rect[PT];  // rect: the key's high word (inline_rect)
-    if (i0 + PT <= nitems) {
+    if (PT > 1 && i0 + PT <= nitems) {
 #pragma unroll
-        for (uint32_t j = 0; j < PT; j += 2) {  // i0 is a multiple of PT, which is even
+        for (uint32_t j = 0; j + 1 < PT; j += 2) {  // i0 is a multiple of PT, which is even
             const ulonglong2 k = *reinterpret_cast<const ulonglong2*>(a.sorted_keys64 + i0 + j);
             rect[j] = (uint32_t)(k.x >> 32); rect[j + 1] = (uint32_t)(k.y >> 32);
         }
@@ -386,8 +386,7 @@ __global__ __launch_bounds__(kEmitThreads) void k_batch_emit(const BatchArgs a) 
                 const uint4 v = *reinterpret_cast<const uint4*>(a.sorted_items + i0 + j);
                 item[j] = v.x; item[j + 1] = v.y; item[j + 2] = v.z; item[j + 3] = v.w;
             }
-        } else {
-            static_assert(PT == 2, "items per thread");
+        } else if constexpr (PT == 2) {
             const uint2 v = *reinterpret_cast<const uint2*>(a.sorted_items + i0);
             item[0] = v.x; item[1] = v.y;
         }
@@ -583,22 +582,32 @@ void launch_batch_item_offsets(const BatchArgs& a, hipStream_t s) {
     hipLaunchKernelGGL(k_batch_item_offsets, dim3(nparts), dim3(kEmitThreads), 0, s, a);
 }
 
-// Items per thread of the emission: smaller partitions where the larger would leave CUs without a block.
-static uint32_t emit_per_thread(uint32_t nitems) {
-    return nitems >= 512u * 8u * kEmitThreads ? 8u : nitems >= 512u * 4u * kEmitThreads ? 4u : 2u;
+// Items per thread of the emission, by the items and the room for their pairs.  The partitions finish at
+// the rate of the look-back, so many items want large ones; few items want enough blocks; and items of
+// many pairs each (the nearest partition of 1,024 then holds six times the mean) want the smallest, as
+// the block with the most pairs ends last.  Measured, us at 1 / 2 / 4 / 8 items per thread:
+//     100k items, 2.4 pairs each    10 /  12 /  15 /  25
+//     0.8M items, 1.5 pairs         37 /  27 /  21 /  24
+//     1M items, 2.8 pairs           38 /  29 /  29 /  41
+//     1M items, 22 pairs            80 / 117 / 176 / 312
+//     3M items, 2 pairs             82 /  56 /  46 /  58
+//     32M items, 2 pairs           619 / 411 / 300 / 254
+static uint32_t emit_per_thread(uint32_t nitems, uint32_t cap) {
+    if (nitems < (1u << 18) || cap / 8u >= nitems) return 1u;
+    return nitems < (1u << 19) ? 2u : nitems < (1u << 23) ? 4u : 8u;
 }
 
-uint32_t emit_parts(uint32_t nitems) {
-    const uint32_t n = emit_per_thread(nitems) * kEmitThreads;
+uint32_t emit_max_parts(uint32_t nitems) { return (nitems + kEmitThreads - 1) / kEmitThreads; }
+
+uint32_t emit_parts(uint32_t nitems, uint32_t cap) {
+    const uint32_t n = emit_per_thread(nitems, cap) * kEmitThreads;
     return (nitems + n - 1) / n;
 }
 
 void launch_batch_emit(const BatchArgs& a, hipStream_t s) {
-    const uint32_t nparts = emit_parts(a.nitems);
+    const uint32_t nparts = emit_parts(a.nitems, a.cap), per = emit_per_thread(a.nitems, a.cap);
     if (nparts == 0) return;
-    const auto kernel = emit_per_thread(a.nitems) == 8u   ? k_batch_emit<8>
-                        : emit_per_thread(a.nitems) == 4u ? k_batch_emit<4>
-                                                          : k_batch_emit<2>;
+    const auto kernel = per == 8u ? k_batch_emit<8> : per == 4u ? k_batch_emit<4> : per == 2u ? k_batch_emit<2> : k_batch_emit<1>;
     hipLaunchKernelGGL(kernel, dim3(nparts), dim3(kEmitThreads), 0, s, a);
 }
 

@@ -122,7 +122,7 @@ static int issue_frame(tpd_ctx* c, hipStream_t s, uint32_t gx, uint32_t gy) {
     c->sorted_vals = in_alt ? c->d_vals_alt : c->d_vals;
     c->last_passes = a.hist_plan.passes + a.pair_plan.passes;
     launch_ranges(c->sorted_keys, c->d_counters, cap, c->d_ranges, c->d_scan_desc,
-                  emit_parts(c->n), &c->d_counters[kCtrScanTicket], s, cap, kDepthWideBits);
+                  emit_parts(c->n, cap), &c->d_counters[kCtrScanTicket], s, cap, kDepthWideBits);
     launch_tile_order(c->d_ranges, ntiles, c->d_counters, c->d_tile_hist, c->d_jobs, gx, nullptr, nullptr, s);
     if (c->profile) hipEventRecord(c->ev[6], s);
     BlendArgs b{};

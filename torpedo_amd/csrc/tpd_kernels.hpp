@@ -269,8 +269,10 @@ void launch_batch_items(const BatchArgs& a, hipStream_t s);
 void launch_frame_items(const FrameArgs& a, hipStream_t s);
 void launch_batch_emit(const BatchArgs& a, hipStream_t s);
 void launch_batch_item_offsets(const BatchArgs& a, hipStream_t s);
-// Partitions of the emission (smaller ones for fewer items) and of the item offsets.
-uint32_t emit_parts(uint32_t nitems);
+// Partitions of the emission (of a frame with room for `cap` pairs, and the most of any) and of the item
+// offsets.
+uint32_t emit_parts(uint32_t nitems, uint32_t cap);
+uint32_t emit_max_parts(uint32_t nitems);
 uint32_t item_offset_parts(uint32_t nitems);
 void launch_batch_blend(const BatchBlendArgs& a, hipStream_t s);
 void launch_batch_blend_bwd(const BatchBlendArgs& a, hipStream_t s);
