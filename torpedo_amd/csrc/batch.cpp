@@ -366,8 +366,10 @@ static int ensure_partials(BatchState* b, size_t pairs) {
 
 static uint32_t tile_key_bits(const BatchState* b) { return bit_length(b->ntiles > 1 ? b->ntiles - 1 : 1); }
 
-static uint32_t item_shape_of(const BatchState* b) { return sort_shape_for(b->item_shape, b->nitems, 8); }
-static uint32_t pair_shape_of(const BatchState* b) { return sort_shape_for(b->ws.shape, b->cap, 4); }
+static uint32_t item_shape_of(const BatchState* b) { return sort_shape_for(b->item_shape, b->nitems, b->lo_bits(), 8); }
+static uint32_t pair_shape_of(const BatchState* b) {
+    return sort_shape_for(b->ws.shape, expected_pairs(b->nitems, b->cap), tile_key_bits(b), 4);
+}
 
 static BatchArgs forward_args(BatchState* b, bool keep_bwd) {
     BatchArgs a{};

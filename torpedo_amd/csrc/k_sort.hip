@@ -461,11 +461,26 @@ DigitPlan sort_digit_plan(uint32_t shape, uint32_t key_bits) {
     return p;
 }
 
-uint32_t sort_shape_for(uint32_t shape, uint32_t n, uint32_t key_bytes) {
+// Wide digits where they save a pass (27-bit depths 3 passes for 4, 45-bit keys 5 for 6, 17-bit tiles 2
+// for 3), and blocks as large as still fill the chip: few keys want many small partitions, many keys
+// few look-back steps and long digit runs.  us a pass:
+//   64-bit keys       8-bit 256x8  512x8  512x12  1024x12    9-bit 512x8  512x12  1024x12  1024x16
+//     3k                      6.5    6.9     8.2     11.5          7.0     9.3     12.9     17.0
+//     100k                    8.8    8.7    11.2     14.8         10.9    12.5     16.2     23.0
+//     1M                       21     16      16       19           18      19       21       27
+//     3M                       42     31      27       23           35      29       26       33
+//     20M                     214    156     137      135          200     165      150      180
+//   32-bit keys
+//     0.24M                    16     13      14       16           15      15       17       20
+//     2.8M                     48     32      26       23           36      29       25       27
+//     22M                     191    137     120      118          158     132      127      130
+//     62M                     497    370     318      315          474     384      358      330
+uint32_t sort_shape_for(uint32_t shape, uint32_t n, uint32_t key_bits, uint32_t key_bytes) {
     if (shape != kShapeAuto) return shape % kNumShapes;
-    (void)n;
-    (void)key_bytes;
-    return 0;
+    constexpr uint32_t k8_256x8 = 1, k8_512x8 = 3, k8_512x12 = 4, k9_512x8 = 7, k9_1024x16 = 9, k9_1024x12 = 10, k8_1024x12 = 11;
+    if ((key_bits + 8) / 9 < (key_bits + 7) / 8)
+        return n < 1500000u ? k9_512x8 : key_bytes == 4 && n >= (1u << 24) ? k9_1024x16 : k9_1024x12;
+    return n < (1u << 16) ? k8_256x8 : n < (1u << 19) ? k8_512x8 : n < 1500000u ? k8_512x12 : k8_1024x12;
 }
 
 static uint32_t hist_blocks(uint32_t n_max) {
@@ -520,7 +535,7 @@ static bool launch_passes(SortWorkspace& ws, uint32_t shape, const DigitPlan& pl
 
 bool launch_sort_pairs(SortWorkspace& ws, uint64_t* keys, uint32_t* vals, uint64_t* keys_alt, uint32_t* vals_alt,
                        uint32_t n, uint32_t key_bits, hipStream_t s) {
-    const uint32_t shape = sort_shape_for(ws.shape, n, 8);
+    const uint32_t shape = sort_shape_for(ws.shape, n, key_bits, 8);
     const DigitPlan plan = sort_digit_plan(shape, key_bits);
     if (n == 0 || plan.passes == 0 || plan.passes > kMaxPasses) return false;
     launch_count(ws, shape, plan, (const uint64_t*)keys, nullptr, n, s);

@@ -74,7 +74,8 @@ static int issue_frame(tpd_ctx* c, hipStream_t s, uint32_t gx, uint32_t gy) {
 
     const uint32_t lo_bits = c->depth_wide ? kDepthWideBits : kDepthWindowBits;
     const uint32_t key_bits = bit_length(ntiles > 1 ? ntiles - 1 : 1);
-    const uint32_t ishape = sort_shape_for(c->item_shape, c->n, 8), pshape = sort_shape_for(c->ws.shape, cap, 4);
+    const uint32_t ishape = sort_shape_for(c->item_shape, c->n, lo_bits, 8);
+    const uint32_t pshape = sort_shape_for(c->ws.shape, expected_pairs(c->n, cap), key_bits, 4);
     FrameArgs f{};
     f.b = item_args(c);
     BatchArgs& a = f.b;

@@ -301,8 +301,11 @@ struct SortWorkspace {
 // Partitions for n keys at the smallest partition size (descriptor capacity for every shape).
 __host__ __device__ inline uint32_t sort_parts(uint32_t n) { return (n + kSortMinTile - 1) / kSortMinTile; }
 uint32_t sort_num_shapes();
-// The shape itself, or for kShapeAuto the one for n keys of key_bytes.
-uint32_t sort_shape_for(uint32_t shape, uint32_t n, uint32_t key_bytes);
+// The shape itself, or for kShapeAuto the one for n keys of key_bytes with key_bits sorted.
+uint32_t sort_shape_for(uint32_t shape, uint32_t n, uint32_t key_bits, uint32_t key_bytes);
+// The pair count a shape is chosen for before the pairs are counted: most frames have 1.5 to 4 pairs a
+// Gaussian, and buffers keep the room of larger frames.
+inline uint32_t expected_pairs(uint32_t nitems, uint32_t cap) { return nitems < cap / 4u ? 4u * nitems : cap; }
 uint32_t sort_shape_keys(uint32_t shape);
 uint32_t sort_shape_bits(uint32_t shape);                       // digit width of a shape
 uint32_t sort_shape_passes(uint32_t shape, uint32_t key_bits);  // passes for key_bits bits
