@@ -38,29 +38,21 @@ void launch_blend_bwd(const BackwardArgs& a, hipStream_t s) {
 // ------------------------------------------------------------------ preprocess backward
 
 // Per Gaussian: sums its per-tile partials (contiguous, in tile order: deterministic) and applies
-// the chain rule of accumulate_param_grads.  The block's 256 records (240 B each, consecutive) are
-// staged in LDS by consecutive loads of the whole block (one thread's record at a time would make
-// every load touch 64 cache lines): 16-byte loads when the records are 16-byte aligned, else 4-byte
-// ones.  A stride of 61 floats keeps the lanes' reads of one field on distinct banks.  The same LDS
+// the chain rule of accumulate_param_grads.  The block's records (240 B each, consecutive) are
+// staged in LDS (load_records_block; by 4-byte loads when they are not 16-byte aligned).  The same LDS
 // then holds the block's SH gradients (48 floats per Gaussian), stored to HBM the same way when
 // the gradient buffer is 16-byte aligned (else by each thread).
-constexpr uint32_t kPreBwdBlock = 256;
-constexpr uint32_t kRecStride = 61;
-__global__ __launch_bounds__(kPreBwdBlock) void k_preprocess_bwd(const PreBackwardArgs a) {
-    __shared__ alignas(16) float s_rec[kPreBwdBlock * kRecStride];
-    const uint32_t i0 = blockIdx.x * kPreBwdBlock, i = i0 + threadIdx.x;
-    const uint32_t nvalid = min(kPreBwdBlock, a.n - i0);  // >= 1: the grid covers n
+__global__ __launch_bounds__(kGradBlock) void k_preprocess_bwd(const PreBackwardArgs a) {
+    __shared__ alignas(16) float s_rec[kGradBlock * kRecStride];
+    const uint32_t i0 = blockIdx.x * kGradBlock, i = i0 + threadIdx.x;
+    const uint32_t nvalid = min(kGradBlock, a.n - i0);  // >= 1: the grid covers n
     const bool valid = threadIdx.x < nvalid;             // every thread stays for the barriers
+    const uint32_t tiles = valid ? a.tiles[i] : 0u, off = valid ? a.offsets[i] : 0u;
     const float* src = a.gauss + (size_t)i0 * 60;
     if ((reinterpret_cast<uintptr_t>(src) & 15u) == 0u) {  // block-uniform
-        const float4* src4 = reinterpret_cast<const float4*>(src);
-        for (uint32_t x = threadIdx.x; x < nvalid * 15u; x += kPreBwdBlock) {
-            const float4 v = src4[x];
-            float* d = s_rec + (x / 15u) * kRecStride + 4u * (x % 15u);
-            d[0] = v.x; d[1] = v.y; d[2] = v.z; d[3] = v.w;
-        }
+        load_records_block(reinterpret_cast<const float4*>(src), nvalid, s_rec);
     } else {
-        for (uint32_t x = threadIdx.x; x < nvalid * 60u; x += kPreBwdBlock)
+        for (uint32_t x = threadIdx.x; x < nvalid * 60u; x += kGradBlock)
             s_rec[(x / 60u) * kRecStride + x % 60u] = src[x];
     }
     __syncthreads();
@@ -71,9 +63,8 @@ __global__ __launch_bounds__(kPreBwdBlock) void k_preprocess_bwd(const PreBackwa
     float gr[9];
 #pragma unroll
     for (int q = 0; q < 9; ++q) gr[q] = 0.0f;
-    const uint32_t tiles = valid ? a.tiles[i] : 0u;
     if (tiles > 0) {
-        sum_pair_partials(a.partials + (size_t)a.offsets[i] * 9, tiles, gr);
+        sum_pair_partials(a.partials + (size_t)off * 9, tiles, gr);
         const float* const rec = s_rec + threadIdx.x * kRecStride;
         if (a.ent_idx) {
             const EntityMats& m = a.ent[a.ent_idx[i]];
@@ -110,7 +101,7 @@ __global__ __launch_bounds__(kPreBwdBlock) void k_preprocess_bwd(const PreBackwa
 
 void launch_preprocess_bwd(const PreBackwardArgs& a, hipStream_t s) {
     if (a.n == 0) return;
-    hipLaunchKernelGGL(k_preprocess_bwd, dim3((a.n + kPreBwdBlock - 1) / kPreBwdBlock), dim3(kPreBwdBlock), 0, s, a);
+    hipLaunchKernelGGL(k_preprocess_bwd, dim3((a.n + kGradBlock - 1) / kGradBlock), dim3(kGradBlock), 0, s, a);
 }
 
 }  // namespace tpd

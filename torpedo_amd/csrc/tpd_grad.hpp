@@ -10,6 +10,33 @@
 
 namespace tpd {
 
+// Gaussians per block of the parameter-gradient passes.  Their records fill the LDS (244 bytes each): blocks
+// of 128 let ten waves stand on a CU and load, compute and store by turns, where blocks of 256 left room for
+// eight in two blocks (3M Gaussians 580 -> 499 us, 64 views of 16 scenes 2645 -> 2178; blocks of 64: 502, 2261).
+constexpr uint32_t kGradBlock = 128;
+
+// The block's n <= kGradBlock records (60 floats each, 16-byte aligned) to LDS rows of kRecStride floats, as
+// consecutive 16-byte loads of the whole block, all of a thread's in flight together (one at a time, each
+// waited for before the next, took 3M Gaussians 499 us; this way 392, where their 1.65 GB take 310).  One
+// thread's record at a time would make every load touch 64 cache lines.  A row of 61 floats keeps the lanes'
+// reads of one field on distinct banks.
+constexpr uint32_t kRecStride = 61;
+__device__ __forceinline__ void load_records_block(const float4* __restrict__ src, uint32_t n, float* rec) {
+    float4 v[15];
+#pragma unroll
+    for (uint32_t u = 0; u < 15u; ++u) {
+        const uint32_t x = threadIdx.x + u * kGradBlock;
+        v[u] = src[x < n * 15u ? x : 0u];
+    }
+#pragma unroll
+    for (uint32_t u = 0; u < 15u; ++u) {
+        const uint32_t x = threadIdx.x + u * kGradBlock;
+        if (x >= n * 15u) continue;
+        float* d = rec + (x / 15u) * kRecStride + 4u * (x % 15u);
+        d[0] = v[u].x; d[1] = v[u].y; d[2] = v[u].z; d[3] = v[u].w;
+    }
+}
+
 // gr[q] += the tiles' partial sums src[t * 9 + q], t = 0 .. tiles - 1, in that order (the sums are
 // the same floats as a loop over t).  Four tiles' 36 loads are issued together: one at a time, each
 // pair waited for its loads, and a lane walked as many pairs as the largest footprint of its wave.
@@ -249,13 +276,27 @@ __device__ __forceinline__ void store_param_grads_but_sh(uint32_t i, bool accumu
 // The SH gradients of n consecutive Gaussians (48 floats each, src in LDS, Gaussian-major) to dst,
 // as consecutive 16-byte stores by the whole block (accumulate: dst + src).
 __device__ __forceinline__ void store_sh_grads_block(const float4* src, uint32_t n, bool accumulate, float4* dst) {
-    for (uint32_t x = threadIdx.x; x < n * 12u; x += blockDim.x) {
-        float4 v = src[x];
-        if (accumulate) {
-            const float4 o = dst[x];
-            v = make_float4(o.x + v.x, o.y + v.y, o.z + v.z, o.w + v.w);
+    float4 v[12];
+#pragma unroll
+    for (uint32_t u = 0; u < 12u; ++u) {
+        const uint32_t x = threadIdx.x + u * kGradBlock;
+        v[u] = src[x];
+    }
+    if (accumulate) {
+        float4 o[12];
+#pragma unroll
+        for (uint32_t u = 0; u < 12u; ++u) {
+            const uint32_t x = threadIdx.x + u * kGradBlock;
+            o[u] = dst[x < n * 12u ? x : 0u];
         }
-        dst[x] = v;
+#pragma unroll
+        for (uint32_t u = 0; u < 12u; ++u)
+            v[u] = make_float4(o[u].x + v[u].x, o[u].y + v[u].y, o[u].z + v[u].z, o[u].w + v[u].w);
+    }
+#pragma unroll
+    for (uint32_t u = 0; u < 12u; ++u) {
+        const uint32_t x = threadIdx.x + u * kGradBlock;
+        if (x < n * 12u) dst[x] = v[u];
     }
 }
 
