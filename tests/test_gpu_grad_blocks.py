@@ -1,6 +1,7 @@
 """Parameter gradients where the blocks of 128 Gaussians end: a full block, one more and one less, and the
 half blocks past a scene's end in a batch.  Plain gradients against the FP64 reference, batched ones against
-the sum of plain ones bit for bit, nothing written beyond a buffer's end."""
+the sum of plain ones bit for bit, nothing written beyond a buffer's end.  And blends whose tiles end at a
+staging round's edge: 184 splats in the backward, 256 in the forward."""
 import numpy as np
 import pytest
 
@@ -23,6 +24,20 @@ def eng():
 @pytest.mark.parametrize("n", [1, 127, 128, 129, 257])
 def test_plain_blocks(eng, orc, n):
     run_case(eng, orc, n, 48, 40, 3, seed=n, log_scale_mean=-2.0)
+
+
+@pytest.mark.parametrize("n", [183, 184, 185, 255, 256, 257, 368, 369, 553])
+def test_blend_rounds(eng, orc, monkeypatch, n):
+    """Faint Gaussians that all cover the one tile: every pixel blends to the end of a list of n."""
+    import test_gpu_backward
+
+    def faint(n, seed, log_scale_mean):
+        g = small_scene(n, seed=seed, log_scale_mean=log_scale_mean)
+        g[:, 3] = 0.012 + 0.006 * np.random.default_rng(seed).random(n, dtype=np.float32)
+        return g
+
+    monkeypatch.setattr(test_gpu_backward, "small_scene", faint)
+    run_case(eng, orc, n, 16, 16, 1, seed=n, log_scale_mean=0.0)
 
 
 @pytest.mark.parametrize("n", [1, 127, 128, 129, 256, 257, 385])

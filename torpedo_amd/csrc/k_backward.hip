@@ -21,7 +21,7 @@ namespace tpd {
 
 // ------------------------------------------------------------------ blend backward
 
-__global__ __launch_bounds__(kTilePixels) void k_blend_bwd(const BackwardArgs a) {
+__global__ __launch_bounds__(kTilePixels, 6) void k_blend_bwd(const BackwardArgs a) {
     __shared__ BlendBwdLds lds;
     const TileJob j = a.jobs[blockIdx.x];
     const int4 last = reinterpret_cast<const int4*>(a.tile_last)[blockIdx.x];

@@ -621,9 +621,9 @@ __device__ __forceinline__ TileView batch_tile_view(const BatchViewDev* __restri
 // COUNT: also adds the evaluated pixel-splat pairs to a.eval_count (a separate launch for the
 // FLOP count, so that the frame's own blend is timed without the counting).
 template <bool COUNT>
-__global__ __launch_bounds__(kTilePixels) void k_batch_blend(const BatchBlendArgs a,
+__global__ __launch_bounds__(kTilePixels, 8) void k_batch_blend(const BatchBlendArgs a,
                                                              const BatchViewDev* __restrict__ views) {
-    __shared__ BlendLds lds;
+    __shared__ BlendFwdLds lds;
     const TileJob j = a.jobs[blockIdx.x];  // loaded beside the flag (meaningless after an overflow)
     if (a.counters[kCtrOverflow]) return;  // the frame is rendered again with larger buffers
     const TileView tv = batch_tile_view(views, j);
@@ -639,7 +639,7 @@ void launch_batch_blend(const BatchBlendArgs& a, hipStream_t s) {
         hipLaunchKernelGGL(k_batch_blend<false>, dim3(a.ntiles), dim3(kTilePixels), 0, s, a, a.views);
 }
 
-__global__ __launch_bounds__(kTilePixels) void k_batch_blend_bwd(const BatchBlendArgs a,
+__global__ __launch_bounds__(kTilePixels, 6) void k_batch_blend_bwd(const BatchBlendArgs a,
                                                                  const BatchViewDev* __restrict__ views) {
     __shared__ BlendBwdLds lds;
     const TileJob j = a.jobs[blockIdx.x];

@@ -240,8 +240,8 @@ void launch_tile_order(const uint2* ranges, uint32_t ntiles, const uint32_t* cou
 
 // blend.slang:22-105.  One 16x16 tile per 256-thread block (blend_tile).
 template <bool COUNT>
-__global__ __launch_bounds__(kTilePixels) void k_blend(const BlendArgs a) {
-    __shared__ BlendLds lds;
+__global__ __launch_bounds__(kTilePixels, 8) void k_blend(const BlendArgs a) {
+    __shared__ BlendFwdLds lds;
     const TileJob j = a.jobs[blockIdx.x];  // loaded beside the flag (meaningless after an overflow)
     if (a.counters[kCtrOverflow]) return;  // the frame is rendered again
     const TileView tv{j.txy & 0xFFFFu, j.txy >> 16, a.width, a.height, a.gx, 0, 0};

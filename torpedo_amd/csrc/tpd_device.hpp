@@ -349,9 +349,9 @@ __host__ __device__ inline SubBlockReach sub_block_reach(float a, float b, float
 }
 
 // The per-tile part: the band extents of the splat at (gx, gy) with conic (a, b, c) against the
-// tile with top-left pixel (ox, oy).
-__host__ __device__ inline uint32_t sub_block_mask(float gx, float gy, float a, float b, float c,
-                                                   const SubBlockReach& r, float ox, float oy) {
+// tile with left pixel ox, whose bands' top pixel rows are band_y.
+__host__ __device__ inline uint32_t sub_block_mask_bands(float gx, float gy, float a, float b, float c,
+                                                         const SubBlockReach& r, float ox, const float band_y[4]) {
     if (r.ey < 0.0f) return 0u;
     if (!(r.ey == r.ey)) return 0xFFFFu;
     const float det = a * c - b * b;
@@ -360,7 +360,7 @@ __host__ __device__ inline uint32_t sub_block_mask(float gx, float gy, float a, 
     uint32_t mask = 0;
 #pragma unroll
     for (uint32_t band = 0; band < 4; ++band) {
-        const float lo = (oy + 4.0f * (float)band) - gy, hi = lo + 3.0f;
+        const float lo = band_y[band] - gy, hi = lo + 3.0f;
         if (hi < -ey - sy || lo > ey + sy) continue;
         const float vlo = fmaxf(lo, -ey), vhi = fminf(hi, ey);
         const float vr = fminf(fmaxf(vstar, vlo), vhi), vl = fminf(fmaxf(-vstar, vlo), vhi);
@@ -372,6 +372,13 @@ __host__ __device__ inline uint32_t sub_block_mask(float gx, float gy, float a, 
         mask |= (((2u << c1) - 1u) & ~((1u << c0) - 1u)) << (4u * band);
     }
     return mask;
+}
+
+// The same for the tile with top-left pixel (ox, oy).
+__host__ __device__ inline uint32_t sub_block_mask(float gx, float gy, float a, float b, float c,
+                                                   const SubBlockReach& r, float ox, float oy) {
+    const float band_y[4] = {oy, oy + 4.0f, oy + 8.0f, oy + 12.0f};
+    return sub_block_mask_bands(gx, gy, a, b, c, r, ox, band_y);
 }
 
 __host__ __device__ inline uint32_t splat_sub_block_mask(float gx, float gy, float a, float b, float c, float o,
