@@ -9,7 +9,7 @@ from torpedo_amd.engine import GaussianEngine, sort_pairs_device
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n", [65_535, 65_537, 524_287, 524_289, 1_499_999, 1_500_001])
+@pytest.mark.parametrize("n", [65_535, 65_537, 524_287, 524_289, 1_499_999, 1_500_001, 3_145_728, 3_145_729])
 @pytest.mark.parametrize("bits", [17, 27, 32, 64])  # 9-bit digits save a pass at 17 and 27 bits
 def test_chosen_shape(n, bits):
     rng = np.random.default_rng(n + bits)

@@ -288,56 +288,54 @@ __global__ __launch_bounds__(BLOCK) void k_onesweep(const OnesweepArgs a) {
         return static_cast<const KT*>(a.keys_in)[idx];
     };
     KT k[ITEMS];
-    uint32_t v[ITEMS];
     if (full) {
 #pragma unroll
         for (uint32_t j = 0; j < ITEMS; ++j) k[j] = load_key(wbase + j * kWave);
-#pragma unroll
-        for (uint32_t j = 0; j < ITEMS; ++j) v[j] = DROP ? wbase + j * kWave : a.vals_in[wbase + j * kWave];
     } else {
 #pragma unroll
         for (uint32_t j = 0; j < ITEMS; ++j) {
             const uint32_t idx = wbase + j * kWave;
             k[j] = idx < n ? load_key(idx) : (DROP ? KT(0) : ~KT(0));
         }
-#pragma unroll
-        for (uint32_t j = 0; j < ITEMS; ++j) {
-            const uint32_t idx = wbase + j * kWave;
-            v[j] = idx < n ? (DROP ? idx : a.vals_in[idx]) : 0u;
-        }
     }
 
     // Rank within the wave: peers with the same digit found with BITS ballots; the lowest lane of
-    // each group advances the wave's running digit counter.  Digits are recomputed from the keys
+    // each group advances the wave's running digit counter.  This matching is most of the pass's
+    // arithmetic, and arithmetic and LDS are most of its time: a bit costs four instructions (nine
+    // as peers &= bit ? bal : ~bal; a pass over 62.9M 32-bit keys 326 -> 285 us, 20M 64-bit 150 -> 126).  Digits are recomputed from the keys
     // wherever they are needed (a few instructions) rather than kept in registers or LDS.
     const auto digit = [&](KT key) -> uint32_t {
         return digit_of(key, a.shift, a.digit_mask);
     };
-    const uint64_t lt = lanemask_lt();
     const auto dropped = [&](KT key) { return DROP && (uint32_t)((uint64_t)key >> 32) == 0u; };
     uint32_t rank[ITEMS];
 #pragma unroll
     for (uint32_t j = 0; j < ITEMS; ++j) {
         const uint32_t d = digit(k[j]);
-        uint64_t peers = ~0ull;
+        uint32_t plo = ~0u, phi = ~0u;
+        constexpr uint32_t kAndXnor = 0x90;  // a & ~(b ^ c)
 #pragma unroll
         for (uint32_t b = 0; b < BITS; ++b) {
-            const bool bit = (d >> b) & 1u;
-            const uint64_t bal = ballot(bit);
-            peers &= bit ? bal : ~bal;
+            uint32_t m = (uint32_t)((int32_t)(d << (31u - b)) >> 31);  // all ones where the bit is set
+            asm("" : "+v"(m));  // one value for the ballot and the masks
+            const uint64_t bal = ballot(m != 0u);
+            plo = __builtin_amdgcn_bitop3_b32(plo, (uint32_t)bal, m, kAndXnor);
+            phi = __builtin_amdgcn_bitop3_b32(phi, (uint32_t)(bal >> 32), m, kAndXnor);
         }
         if constexpr (DROP) {
             // a dropped key is nobody's peer and gets no rank (kNoSlot)
             const bool cull = dropped(k[j]);
-            peers &= ~ballot(cull);
-            const uint32_t below = (uint32_t)__popcll(peers & lt);
+            const uint64_t gone = ballot(cull);
+            plo &= ~(uint32_t)gone;
+            phi &= ~(uint32_t)(gone >> 32);
+            const uint32_t below = __builtin_amdgcn_mbcnt_hi(phi, __builtin_amdgcn_mbcnt_lo(plo, 0u));
             const uint32_t pre = L.whist[wave][d];
-            if (!cull && below == 0) L.whist[wave][d] = (uint16_t)(pre + (uint32_t)__popcll(peers));
+            if (!cull && below == 0) L.whist[wave][d] = (uint16_t)(pre + __popc(plo) + __popc(phi));
             rank[j] = cull ? kNoSlot : pre + below;
         } else {
-            const uint32_t below = (uint32_t)__popcll(peers & lt);
+            const uint32_t below = __builtin_amdgcn_mbcnt_hi(phi, __builtin_amdgcn_mbcnt_lo(plo, 0u));
             const uint32_t pre = L.whist[wave][d];
-            if (below == 0) L.whist[wave][d] = (uint16_t)(pre + (uint32_t)__popcll(peers));
+            if (below == 0) L.whist[wave][d] = (uint16_t)(pre + __popc(plo) + __popc(phi));
             rank[j] = pre + below;
         }
     }
@@ -387,6 +385,14 @@ __global__ __launch_bounds__(BLOCK) void k_onesweep(const OnesweepArgs a) {
         const uint32_t lp = L.bstart[d] + L.whist[wave][d] + rank[j];
         rank[j] = lp;
         L.keys[lp] = k[j];
+    }
+
+    // The values, wanted last: their registers are free only now that the keys are in LDS.
+    uint32_t v[ITEMS];
+#pragma unroll
+    for (uint32_t j = 0; j < ITEMS; ++j) {
+        const uint32_t idx = wbase + j * kWave;
+        v[j] = DROP ? idx : a.vals_in[full || idx < n ? idx : 0u];
     }
 
     // Look-back per digit, then the global position adjustment of each digit run.
@@ -463,24 +469,28 @@ DigitPlan sort_digit_plan(uint32_t shape, uint32_t key_bits) {
 
 // Wide digits where they save a pass (27-bit depths 3 passes for 4, 45-bit keys 5 for 6, 17-bit tiles 2
 // for 3), and blocks as large as still fill the chip: few keys want many small partitions, many keys
-// few look-back steps and long digit runs.  us a pass:
+// few look-back steps and long digit runs; 3 * 2^20 keys are the most whose partitions of 12,288 stand on
+// 256 CUs at once.  us a pass:
 //   64-bit keys       8-bit 256x8  512x8  512x12  1024x12    9-bit 512x8  512x12  1024x12  1024x16
-//     3k                      6.5    6.9     8.2     11.5          7.0     9.3     12.9     17.0
-//     100k                    8.8    8.7    11.2     14.8         10.9    12.5     16.2     23.0
-//     1M                       21     16      16       19           18      19       21       27
-//     3M                       42     31      27       23           35      29       26       33
-//     20M                     214    156     137      135          200     165      150      180
+//     3k                      6.2    6.1     7.1      9.7          6.8     7.7      9.7     12.1
+//     100k                    8.6    8.6    10.0     11.8          9.9    11.1     13.2     15.8
+//     1M                       21     16      16       16           17      17       18       20
+//     3M                       40     28      24       21           32      27       23       25
+//     4M                       54     37      33       31           43      37       35       27
+//     20M                     212    152     130      122          193     158      136      126
 //   32-bit keys
-//     0.24M                    16     13      14       16           15      15       17       20
-//     2.8M                     48     32      26       23           36      29       25       27
-//     22M                     191    137     120      118          158     132      127      130
-//     62M                     497    370     318      315          474     384      358      330
+//     0.24M                    16     12      13       13           14      14       14       16
+//     0.7M                     31     21      19       18           23      21       19       20
+//     2.8M                     45     29      24       20           32      26       21       23
+//     22M                     187    128     106      101          149     119      110      110
+//     62M                     490    347     271      270          461     364      313      286
 uint32_t sort_shape_for(uint32_t shape, uint32_t n, uint32_t key_bits, uint32_t key_bytes) {
     if (shape != kShapeAuto) return shape % kNumShapes;
-    constexpr uint32_t k8_256x8 = 1, k8_512x8 = 3, k8_512x12 = 4, k9_512x8 = 7, k9_1024x16 = 9, k9_1024x12 = 10, k8_1024x12 = 11;
+    constexpr uint32_t k8_256x8 = 1, k8_512x8 = 3, k9_512x8 = 7, k9_1024x16 = 9, k9_1024x12 = 10, k8_1024x12 = 11;
+    const uint32_t large = key_bytes == 4 ? 1u << 19 : 1500000u;
     if ((key_bits + 8) / 9 < (key_bits + 7) / 8)
-        return n < 1500000u ? k9_512x8 : key_bytes == 4 && n >= (1u << 24) ? k9_1024x16 : k9_1024x12;
-    return n < (1u << 16) ? k8_256x8 : n < (1u << 19) ? k8_512x8 : n < 1500000u ? k8_512x12 : k8_1024x12;
+        return n < large ? k9_512x8 : n <= (key_bytes == 4 ? 1u << 23 : 3u << 20) ? k9_1024x12 : k9_1024x16;
+    return n < (1u << 16) ? k8_256x8 : n < large ? k8_512x8 : k8_1024x12;
 }
 
 static uint32_t hist_blocks(uint32_t n_max) {
