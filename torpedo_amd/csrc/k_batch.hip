@@ -254,6 +254,8 @@ __global__ __launch_bounds__(kPreBlock) void k_frame_items(const FrameArgs f) {
     const BatchArgs& a = f.b;
     begin_items(a, L);
     const uint32_t tid = threadIdx.x;
+    // for a backward that may follow (a fill of its own costs it two launches)
+    for (uint32_t x = blockIdx.x * kPreBlock + tid; x < f.offset_parts; x += gridDim.x * kPreBlock) a.scan_desc2[x] = 0;
     uint32_t all0 = 0;
     uint64_t total = 0;
     bool depth_out = false;
@@ -509,9 +511,10 @@ __global__ __launch_bounds__(kEmitThreads) void k_batch_emit(const BatchArgs a) 
 // For frames kept for a backward: the exclusive scan of the items' tile counts in item order,
 // where the backward keeps each item's per-pair partial sums (consecutive Gaussians of a view then
 // have adjacent partials, which the parameter-gradient pass reads item by item).  Partitions of
-// kOffsetItems items, decoupled look-back over a.scan_desc2.
-constexpr uint32_t kOffsetPerThread = 8, kOffsetItems = kEmitThreads * kOffsetPerThread;
+// 512 x PT items, decoupled look-back over a.scan_desc2.
+template <uint32_t PT>
 __global__ __launch_bounds__(kEmitThreads) void k_batch_item_offsets(const BatchArgs a) {
+    constexpr uint32_t kItems = kEmitThreads * PT;
     __shared__ uint32_t s_part;
     __shared__ uint32_t s_wave_sum[kEmitThreads / kWave];
     __shared__ uint64_t s_base;
@@ -519,24 +522,33 @@ __global__ __launch_bounds__(kEmitThreads) void k_batch_item_offsets(const Batch
     if (tid == 0) s_part = atomicAdd(&a.counters[kCtrScanTicket2], 1u);
     __syncthreads();
     const uint32_t part = __builtin_amdgcn_readfirstlane(s_part);
-    const uint32_t nparts = (a.nitems + kOffsetItems - 1) / kOffsetItems;
+    const uint32_t nparts = (a.nitems + kItems - 1) / kItems;
     if (part >= nparts) return;
     uint64_t* desc = a.scan_desc2;
-    const uint32_t i0 = part * kOffsetItems + tid * kOffsetPerThread;
-    uint32_t t[kOffsetPerThread], mine = 0;
-    if (i0 + kOffsetPerThread <= a.nitems) {
+    // A wave takes PT / 4 rows of 256 consecutive items, a lane 4 of each row.
+    constexpr uint32_t kRows = PT / 4u;
+    const uint32_t i0 = part * kItems + wave * (kWave * PT) + 4u * lane;
+    const bool full = (part + 1u) * kItems <= a.nitems;
+    uint4 t[kRows];
 #pragma unroll
-        for (uint32_t j = 0; j < kOffsetPerThread; j += 4) {  // i0 is a multiple of 4
-            const uint4 v = *reinterpret_cast<const uint4*>(a.tiles + i0 + j);
-            t[j] = v.x; t[j + 1] = v.y; t[j + 2] = v.z; t[j + 3] = v.w;
+    for (uint32_t r = 0; r < kRows; ++r) {
+        const uint32_t i = i0 + r * 4u * kWave;
+        if (full) {
+            t[r] = *reinterpret_cast<const uint4*>(a.tiles + i);
+        } else {
+            t[r].x = i < a.nitems ? a.tiles[i] : 0u;
+            t[r].y = i + 1u < a.nitems ? a.tiles[i + 1u] : 0u;
+            t[r].z = i + 2u < a.nitems ? a.tiles[i + 2u] : 0u;
+            t[r].w = i + 3u < a.nitems ? a.tiles[i + 3u] : 0u;
         }
-    } else {
-#pragma unroll
-        for (uint32_t j = 0; j < kOffsetPerThread; ++j) t[j] = i0 + j < a.nitems ? a.tiles[i0 + j] : 0u;
     }
+    uint32_t before[kRows], incl_w = 0;  // the wave's tiles before the lane's items of a row; in all its rows
 #pragma unroll
-    for (uint32_t j = 0; j < kOffsetPerThread; ++j) mine += t[j];
-    const uint32_t incl_w = wave_incl_scan(mine);
+    for (uint32_t r = 0; r < kRows; ++r) {
+        const uint32_t own = (t[r].x + t[r].y) + (t[r].z + t[r].w), incl = wave_incl_scan(own);
+        before[r] = incl_w + incl - own;
+        incl_w += (uint32_t)__builtin_amdgcn_readlane(incl, kWave - 1);
+    }
     if (lane == kWave - 1) s_wave_sum[wave] = incl_w;
     __syncthreads();
     uint32_t wave_off = 0, block_total = 0;
@@ -556,30 +568,36 @@ __global__ __launch_bounds__(kEmitThreads) void k_batch_item_offsets(const Batch
         }
     }
     __syncthreads();
-    uint32_t off = (uint32_t)(s_base + wave_off + incl_w - mine);
-    uint32_t o[kOffsetPerThread];
+    const uint32_t base = (uint32_t)s_base + wave_off;
 #pragma unroll
-    for (uint32_t j = 0; j < kOffsetPerThread; ++j) {
-        o[j] = off;
-        off += t[j];
-    }
-    if (i0 + kOffsetPerThread <= a.nitems) {
-#pragma unroll
-        for (uint32_t j = 0; j < kOffsetPerThread; j += 4)
-            *reinterpret_cast<uint4*>(a.offsets + i0 + j) = make_uint4(o[j], o[j + 1], o[j + 2], o[j + 3]);
-    } else {
-#pragma unroll
-        for (uint32_t j = 0; j < kOffsetPerThread; ++j)
-            if (i0 + j < a.nitems) a.offsets[i0 + j] = o[j];
+    for (uint32_t r = 0; r < kRows; ++r) {
+        const uint32_t i = i0 + r * 4u * kWave, o = base + before[r];
+        const uint4 off = make_uint4(o, o + t[r].x, o + t[r].x + t[r].y, o + t[r].x + t[r].y + t[r].z);
+        if (full) {
+            *reinterpret_cast<uint4*>(a.offsets + i) = off;
+        } else {
+            if (i < a.nitems) a.offsets[i] = off.x;
+            if (i + 1u < a.nitems) a.offsets[i + 1u] = off.y;
+            if (i + 2u < a.nitems) a.offsets[i + 2u] = off.z;
+            if (i + 3u < a.nitems) a.offsets[i + 3u] = off.w;
+        }
     }
 }
 
-uint32_t item_offset_parts(uint32_t nitems) { return (nitems + kOffsetItems - 1) / kOffsetItems; }
+// Items per thread of the offsets' scan.  Its partitions finish at the rate of the look-back (about 16 ns
+// each), so many items want large ones: at 8 / 16 / 32 per thread 33.8M items take 125 / 95 / 85 us, 3M 19 / 13 / 11.
+static uint32_t offsets_per_thread(uint32_t nitems) { return nitems >= (1u << 21) ? 32u : 8u; }
+
+uint32_t item_offset_parts(uint32_t nitems) {
+    const uint32_t n = offsets_per_thread(nitems) * kEmitThreads;
+    return (nitems + n - 1) / n;
+}
 
 void launch_batch_item_offsets(const BatchArgs& a, hipStream_t s) {
     const uint32_t nparts = item_offset_parts(a.nitems);
     if (nparts == 0 || !a.offsets || !a.tiles) return;
-    hipLaunchKernelGGL(k_batch_item_offsets, dim3(nparts), dim3(kEmitThreads), 0, s, a);
+    const auto kernel = offsets_per_thread(a.nitems) == 32u ? k_batch_item_offsets<32> : k_batch_item_offsets<8>;
+    hipLaunchKernelGGL(kernel, dim3(nparts), dim3(kEmitThreads), 0, s, a);
 }
 
 // Items per thread of the emission, by the items and the room for their pairs.  The partitions finish at

@@ -37,10 +37,8 @@ static BatchArgs item_args(tpd_ctx* c) {
 // the frames whose backward or tile readback asks for it.
 int ensure_offsets(tpd_ctx* c, hipStream_t s) {
     if (c->have_offsets || c->n == 0) return TPD_OK;
-    hipError_t e = hipMemsetAsync(c->d_scan_desc2, 0, item_offset_parts(c->n) * sizeof(uint64_t), s);
-    if (e != hipSuccess) return hip_fail(e, "item offsets");
     launch_batch_item_offsets(item_args(c), s);
-    e = hipGetLastError();
+    const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return hip_fail(e, "item offsets");
     c->have_offsets = true;
     return TPD_OK;
@@ -103,6 +101,7 @@ static int issue_frame(tpd_ctx* c, hipStream_t s, uint32_t gx, uint32_t gy) {
     f.sh_degree = c->sh_degree;
     f.gx = gx;
     f.gy = gy;
+    f.offset_parts = item_offset_parts(c->n);
     launch_frame_items(f, s);
     if (c->profile) hipEventRecord(c->ev[1], s);
     const FrameTotals totals{cap, lo_bits, ++c->frame_seq, c->d_host_counters};

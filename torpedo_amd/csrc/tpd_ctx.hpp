@@ -38,7 +38,7 @@ struct tpd_ctx {
     uint32_t* d_tiles = nullptr; size_t cap_tiles = 0;
     uint32_t* d_offsets = nullptr; size_t cap_offsets = 0;
     uint64_t* d_scan_desc = nullptr; size_t cap_scan_desc = 0;    // the emission's, zero between frames
-    uint64_t* d_scan_desc2 = nullptr; size_t cap_scan_desc2 = 0;  // the item offsets', cleared before use
+    uint64_t* d_scan_desc2 = nullptr; size_t cap_scan_desc2 = 0;  // the item offsets', cleared by the frame
     uint32_t* d_counters = nullptr;
     uint32_t* h_counters = nullptr;  // pinned: the frame's totals (kHost*), written by the device
     uint32_t* d_host_counters = nullptr;  // the same memory as the device addresses it

@@ -220,6 +220,7 @@ struct FrameArgs {
     EntityMats mats0;
     CameraParams cam;
     uint32_t n, sh_degree, gx, gy;
+    uint32_t offset_parts;        // partitions of the item offsets, whose descriptors are cleared
 };
 
 struct BatchBlendArgs {
