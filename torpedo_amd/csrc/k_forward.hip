@@ -131,14 +131,17 @@ void launch_unsorted_pairs(const Splat* splats, const uint32_t* tiles, const uin
 // ------------------------------------------------------------------ tile order
 
 // Tiles are ordered by class (bit length of the pair count, 0 for an empty tile), heaviest class
-// first.  Two launches of one 1024-thread block per chunk of 1024 tiles: the first counts each
-// chunk's tiles per class into hist[class * chunks + chunk]; the second gives every chunk its
-// start in each class (the tiles of all heavier classes, then those of the class in earlier
-// chunks) and scatters its tiles.  Within a chunk and class the order is the order in which waves
-// claim slots.  Every wave combines its lanes of one class into one LDS atomic.  Inside each
+// first.  One 1024-thread block per chunk of 1024 tiles needs its start in each class (the tiles of all
+// heavier classes, then those of the class in earlier chunks) and scatters its tiles.  Up to
+// kOrderOwnChunks chunks every block counts all tiles itself, one launch; beyond, a launch before
+// counts each chunk's tiles per class into hist[class * chunks + chunk], as a block's own count
+// takes longer (both launches and the one, us: 144 tiles 8.5 and 5.1, 3,600 9.6 and 7.9, 8,160 11.3 and
+// 10.9).  Within a chunk and class the order is the order in which waves claim slots.  Every wave combines its lanes of one class into one LDS atomic.  Inside each
 // class's range of launch positions the tiles are placed by xcd_unmap, so that each XCD (blocks
 // go to the 8 XCDs round-robin) takes one contiguous run of the class's tiles, in index order by
 // chunks: neighbouring tiles, which share splats, then mostly meet in one L2.
+
+constexpr uint32_t kOrderOwnChunks = 4;
 
 __device__ __forceinline__ uint32_t tile_class(const uint2* __restrict__ ranges, uint32_t t) {
     const uint2 r = ranges[t];
@@ -180,6 +183,19 @@ __global__ __launch_bounds__(kOrderChunk) void k_tile_class_count(const uint2* _
     if (tid < kTileClasses) hist[tid * chunks + blockIdx.x] = cnt[tid];
 }
 
+// Adds the wave's tiles per class to count[class]: lanes of one class found with a ballot per bit of the
+// class, one LDS addition each; kTileClasses: no tile.
+__device__ __forceinline__ void count_classes(uint32_t* count, uint32_t cls) {
+    uint64_t peers = ~0ull;
+#pragma unroll
+    for (uint32_t b = 0; b < 6; ++b) {
+        const uint64_t bal = ballot((cls >> b) & 1u);
+        peers &= ((cls >> b) & 1u) ? bal : ~bal;
+    }
+    if (cls < kTileClasses && (peers & lanemask_lt()) == 0) atomicAdd(&count[cls], (uint32_t)__popcll(peers));
+}
+
+// hist: the chunks' counts, or null: every block counts them.
 __global__ __launch_bounds__(kOrderChunk) void k_tile_order(const uint2* __restrict__ ranges, uint32_t ntiles,
                                                             const uint32_t* counters, const uint32_t* __restrict__ hist,
                                                             TileJob* __restrict__ jobs, uint32_t grid_width,
@@ -188,18 +204,32 @@ __global__ __launch_bounds__(kOrderChunk) void k_tile_order(const uint2* __restr
     __shared__ uint32_t slot[kTileClasses], total[kTileClasses], cstart[kTileClasses];
     const uint32_t tid = threadIdx.x, lane = __lane_id(), wave = tid / kWave, chunks = gridDim.x;
     if (counters && counters[kCtrOverflow]) return;
-    for (uint32_t c = wave; c < kTileClasses; c += kOrderChunk / kWave) {
-        uint64_t all = 0, before = 0;
-        for (uint32_t k = lane; k < chunks; k += kWave) {
-            const uint32_t v = hist[c * chunks + k];
-            all += v;
-            before += k < blockIdx.x ? v : 0u;
-        }
-        all = wave_sum_u64(all);
-        before = wave_sum_u64(before);
-        if (lane == 0) {
-            total[c] = (uint32_t)all;
-            slot[c] = (uint32_t)before;
+    if (!hist) {
+        if (tid < kTileClasses) slot[tid] = total[tid] = 0;
+        __syncthreads();
+        uint32_t cls[kOrderOwnChunks];  // all loads in flight together
+#pragma unroll
+        for (uint32_t k = 0; k < kOrderOwnChunks; ++k)
+            cls[k] = k * kOrderChunk + tid < ntiles ? tile_class(ranges, k * kOrderChunk + tid) : kTileClasses;
+#pragma unroll
+        for (uint32_t k = 0; k < kOrderOwnChunks; ++k)  // total: of this chunk and the later ones, until below
+            if (k < chunks) count_classes(k < blockIdx.x ? slot : total, cls[k]);
+        __syncthreads();
+        if (tid < kTileClasses) total[tid] += slot[tid];
+    } else {
+        for (uint32_t c = wave; c < kTileClasses; c += kOrderChunk / kWave) {
+            uint64_t all = 0, before = 0;
+            for (uint32_t k = lane; k < chunks; k += kWave) {
+                const uint32_t v = hist[c * chunks + k];
+                all += v;
+                before += k < blockIdx.x ? v : 0u;
+            }
+            all = wave_sum_u64(all);
+            before = wave_sum_u64(before);
+            if (lane == 0) {
+                total[c] = (uint32_t)all;
+                slot[c] = (uint32_t)before;
+            }
         }
     }
     __syncthreads();
@@ -231,9 +261,11 @@ void launch_tile_order(const uint2* ranges, uint32_t ntiles, const uint32_t* cou
                        uint32_t grid_width, const uint32_t* tile_view, const BatchViewDev* views, hipStream_t s) {
     if (ntiles == 0) return;
     const uint32_t chunks = (ntiles + kOrderChunk - 1) / kOrderChunk;
-    hipLaunchKernelGGL(k_tile_class_count, dim3(chunks), dim3(kOrderChunk), 0, s, ranges, ntiles, counters, hist);
+    const bool own = chunks <= kOrderOwnChunks;
+    if (!own)
+        hipLaunchKernelGGL(k_tile_class_count, dim3(chunks), dim3(kOrderChunk), 0, s, ranges, ntiles, counters, hist);
     hipLaunchKernelGGL(k_tile_order, dim3(chunks), dim3(kOrderChunk), 0, s, ranges, ntiles, counters,
-                       (const uint32_t*)hist, jobs, grid_width, tile_view, views);
+                       own ? nullptr : (const uint32_t*)hist, jobs, grid_width, tile_view, views);
 }
 
 // ------------------------------------------------------------------ blend
