@@ -493,8 +493,10 @@ uint32_t sort_shape_for(uint32_t shape, uint32_t n, uint32_t key_bits, uint32_t 
     return n < (1u << 16) ? k8_256x8 : n < large ? k8_512x8 : k8_1024x12;
 }
 
+// A block per 2,048 keys, what its threads load at once: a block that takes four such chunks one after
+// the other is alone on its CU below 2M keys (200k keys 18.6 -> 8.2 us, 1M 19.1 -> 12.8, 4M 23.2 and 23.0).
 static uint32_t hist_blocks(uint32_t n_max) {
-    uint32_t hb = (n_max + 256 * kHistUnroll * 4 - 1) / (256 * kHistUnroll * 4);
+    uint32_t hb = (n_max + 256 * kHistUnroll - 1) / (256 * kHistUnroll);
     return hb < 1 ? 1 : (hb > kHistBlocks ? kHistBlocks : hb);
 }
 
