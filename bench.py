@@ -35,18 +35,12 @@ sys.path.insert(0, ROOT)
 
 METRIC = "views/s batched vs plain; fwd+bwd ms @3M Gaussians 1080p; sort % HBM peak"
 HBM_PEAK_GBS = 8000.0
-# HBM bytes per element per k_onesweep launch of the batched frame (32-bit keys and values; mean
-# over the frame's item and pair passes), per radix shape, from two rocprofv3 --pmc runs:
-# FETCH_SIZE x 2.0 + WRITE_SIZE x 1.0 (factors read off a plain copy kernel).
 # HBM bytes per k_onesweep launch of the batched frame (mean over its launches), measured with
 # FETCH_SIZE x 2 + WRITE_SIZE for the (item sort, pair sort) block shapes named; other shapes: null.
 ONESWEEP_TRAFFIC = {
-    (10, 9): {"bytes_per_launch": 779_200_000,
-              "source": "profiles/batch_frame-multiview32-clusters1M.md (item passes: first 614.2 MB, later "
-                        "2 x 626.1 MB; pair passes 2 x 1,014.9 MB; FETCH_SIZE x 2 + WRITE_SIZE)"},
-    (6, 8): {"bytes_per_launch": 893_200_000,
-             "source": "profiles/batch_frame-multiview32-clusters1M.md (item passes: first 731.9 MB, later "
-                       "2 x 708.0 MB; pair passes 2 x 1,159.1 MB; FETCH_SIZE x 2 + WRITE_SIZE)"},
+    (9, 9): {"bytes_per_launch": 773_700_000,
+             "source": "profiles/batch_frame-multiview32-clusters1M.md (item passes: first 598.3 MB, later "
+                       "2 x 615.5 MB; pair passes 2 x 1,019.5 MB; FETCH_SIZE x 2 + WRITE_SIZE)"},
 }
 VALU_PEAK_TFLOPS = 157.3
 
@@ -88,15 +82,18 @@ def shape_desc(i):
 
 
 def sort_keys_per_s(P, stage_ms):
-    """Pairs sorted per second over the whole sort: histogram pass plus every radix pass."""
+    """Pairs sorted per second over the whole sort: digit offsets plus every radix pass of both sorts."""
     t = (stage_ms["sort_histogram"] + stage_ms["sort_passes"]) / 1000.0
     return P / t if t > 0 else 0.0
 
 
-def onesweep_roofline(P, sort_passes_ms, passes):
-    t_launch = sort_passes_ms / 1000.0 / max(passes, 1)
-    achieved = 24.0 * P / t_launch / 1e9 if t_launch > 0 else 0.0
-    return achieved, t_launch
+def plain_sort_gbs(P, stage_ms, w, h, digit_bits=9):
+    """The sort metric of a plain frame: 24 B x P x ceil(K / d) over the time to order the pairs by (tile,
+    depth), i.e. both sorts' passes (the Gaussians by depth, their pairs by tile) and digit offsets;
+    K = tile bits + 27 depth bits, d the widest digit of the passes."""
+    t = (stage_ms["sort_histogram"] + stage_ms["sort_passes"]) / 1000.0
+    k = int(np.ceil(np.log2(max(((w + 15) // 16) * ((h + 15) // 16), 2)))) + 27
+    return 24.0 * P * ((k + digit_bits - 1) // digit_bits) / t / 1e9 if t > 0 else 0.0
 
 
 def time_multiview(eng, g, steps, warmup, tune=True):
@@ -469,10 +466,10 @@ def main():
     if args.only == "sort-load":
         g2 = scenes.cluster_scene(1_000_000, seed=2, log_scale_mean=-3.0)
         dt2, P2, st2 = time_plain(eng, g2, eye, W, H, args.steps, args.warmup, tune=tune)
-        ach, t_launch = onesweep_roofline(P2, st2["sort_passes"], st2["radix_passes"])
+        ach = plain_sort_gbs(P2, st2, W, H)
         copy_gbs = eng.measureCopy(256 << 20, 3)  # a plain copy of 256 MiB for counter calibration
         print(json.dumps({"workload": "clusters-1M-1920x1080 log-scale mean -3", "pairs": P2, "stage_ms": st2,
-                          "onesweep_avg_launch_us": round(t_launch * 1e6, 2), "onesweep_gbs": round(ach, 1),
+                          "sort_gbs": round(ach, 1),
                           "copy_256MiB_gbs": round(copy_gbs, 1)}), flush=True)
         eng.close()
         return
@@ -573,8 +570,7 @@ def main():
     sort_metric = 24.0 * mv["pairs"] * ((K + d - 1) // d) / t_sort / 1e9 if t_sort > 0 else 0.0
     roofline["sort_ms"] = round(t_sort * 1000.0, 4)
     roofline["sort_gkeys_per_s"] = round(mv["pairs"] / t_sort / 1e9, 3) if t_sort > 0 else 0.0
-    ach2, t2 = onesweep_roofline(P2, st2["sort_passes"], st2["radix_passes"])
-    ach1, _ = onesweep_roofline(P, st["sort_passes"], st["radix_passes"])
+    ach2, ach1 = plain_sort_gbs(P2, st2, W, H), plain_sort_gbs(P, st, W, H)
 
     log("[bench] forward + backward, 3M Gaussians 1920x1080")
     fb = time_fwd_bwd(eng, max(5, args.steps // 2), 2)
@@ -628,6 +624,8 @@ def main():
                           "multiview_32_key_bits": K,
                           "sort_load_variant": round(ach2 / HBM_PEAK_GBS, 4), "pairs_sort_load": P2,
                           "plain_1080p": round(ach1 / HBM_PEAK_GBS, 4), "pairs_plain_1080p": P,
+                          "metric": "24 B x pairs x ceil(K / d) over both sorts' time: the bytes of a sort of the "
+                                    "pairs by their whole key; Gaussians sorted by depth first move fewer",
                           "gkeys_per_s": {"multiview_32": roofline["sort_gkeys_per_s"],
                                           "sort_load_variant": round(sort_keys_per_s(P2, st2) / 1e9, 3),
                                           "plain_1080p": round(sort_keys_per_s(P, st) / 1e9, 3)}},

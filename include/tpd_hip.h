@@ -142,8 +142,9 @@ int tpd_memcpy(tpd_ctx* ctx, void* dst, const void* src, uint64_t bytes, int kin
 
 /* ----- stage timing (the reference has none; SurfaceRenderer only measures whole frames) -----
  * With profiling on, tpd_render records HIP events on its stream between stages; ms[0..5]
- * receive the last frame's preprocess+scan+duplicate, sort histograms, all radix passes, ranges,
- * blend and whole-frame times in milliseconds; *passes the number of radix passes. */
+ * receive the last frame's projection + pair emission, digit offsets, radix passes of both sorts
+ * (Gaussians by depth, pairs by tile), ranges + tile order, blend and whole-frame times in milliseconds;
+ * *passes the number of radix passes of both sorts. */
 int tpd_set_profiling(tpd_ctx* ctx, int enable);
 int tpd_get_stage_times(tpd_ctx* ctx, float* ms, uint32_t* passes);
 /* Pixel-splat pairs whose power the blend of the last rendered frame evaluates (counted by blending
@@ -182,11 +183,13 @@ int tpd_sort_pairs_noalloc(tpd_ctx* ctx, uint64_t* d_keys, uint32_t* d_vals, uin
                            uint32_t* d_vals_alt, uint32_t n, uint32_t key_bits, void* stream, int* in_alt);
 
 /* ----- autotuning (the reference's shapes are compile-time constants, GaussianEngine.h:121-124) -----
- * Times every radix-pass block shape on the last rendered frame's pairs and keeps the fastest
- * (results are identical for every shape).  sort_ms[0..capacity) receives the median time of a
- * full sort per shape; *n_shapes the number of shapes; *best the chosen one.  Re-renders the frame. */
+ * Times every radix-pass block shape on frames of the last rendered scene and camera and keeps the
+ * fastest for each of the two sorts (results are identical for every shape).  sort_ms[0..capacity)
+ * receives the median time of both sorts per shape; *n_shapes the number of shapes; *best the pair
+ * sort's.  Re-renders the frame. */
 int tpd_autotune(tpd_ctx* ctx, float* sort_ms, uint32_t capacity, uint32_t* n_shapes, uint32_t* best);
-/* Selects a radix-pass block shape by index (0 = default) for the plain and the batched frame. */
+/* Selects a radix-pass block shape by index for the plain and the batched frame and the stand-alone
+ * sorts; until then, or until an autotune, each sort's shape follows from its key count and width. */
 int tpd_set_sort_shape(tpd_ctx* ctx, uint32_t shape);
 
 /* ----- batched rendering -------------------------------------------------------------------------

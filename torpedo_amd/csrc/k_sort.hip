@@ -1,10 +1,12 @@
-// Stable LSD radix sort of (64-bit key, 32-bit value) pairs, one pass per digit of BITS bits
-// (8 or 9; the autotuner picks the shape, digit width included).
+// Stable LSD radix sort of (32- or 64-bit key, 32-bit value) pairs, one pass per digit of BITS bits
+// (8 or 9; sort_shape_for or an autotuner picks the shape, digit width included).  A frame sorts its
+// items by depth with 64-bit keys, then their pairs by tile with 32-bit ones.
 //
 // Replaces the reference's 2-bit "4-way" sorter (radix-shuffle/-prefixA/-prefixB/-mapping.slang,
 // 4 dispatches per 2 bits, GaussianEngine.cpp:819-841) with:
 //   k_sort_hist + k_sort_offsets  one read of the keys computes the digit histograms of every pass
-//                                 and their global exclusive offsets;
+//                                 and their global exclusive offsets (a frame's counts come from
+//                                 its item kernel, k_frame_offsets scans those of both sorts);
 //   k_onesweep (once per pass)    each block takes the next partition of BLOCK x ITEMS keys from an
 //                                 atomic ticket, ranks its keys by digit with wave64 ballot
 //                                 matching (stable: element order inside a wave, then waves in

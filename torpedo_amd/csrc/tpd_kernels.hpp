@@ -11,7 +11,7 @@ enum : uint32_t {
     kCtrPairs = 1,        // pair count P written by the last preprocess partition
     kCtrOverflow = 2,     // 1 when P exceeded the key/value capacity
     kCtrDepthOut = 3,     // non-zero when an emitted depth lies outside the sort's depth window
-    kCtrScanTicket2 = 4,  // partition ticket of a second scan in the frame (the batch's item offsets)
+    kCtrScanTicket2 = 4,  // partition ticket of a second scan in the frame (the item offsets)
     kCtrSortPairs = 5,    // pair count for the pair sort and the ranges: P, or 0 when the frame overflowed
                           // (it is rendered again)
     kCtrTotal64 = 6,      // (two words) the plain frame's pair count, summed by its item kernel; zero between
