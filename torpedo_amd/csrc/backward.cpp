@@ -57,7 +57,7 @@ extern "C" int tpd_backward(tpd_ctx* c, const float* d_dL_dimage, float* d_grad_
         b->cap_partials = want;
     }
     if (c->n == 0) return TPD_OK;
-    const int rc = ensure_offsets(c, s);
+    const int rc = launch_offsets(c, s);
     if (rc != TPD_OK) return rc;
     if (c->profile) {
         for (auto& ev : b->ev)
@@ -89,7 +89,6 @@ extern "C" int tpd_backward(tpd_ctx* c, const float* d_dL_dimage, float* d_grad_
     p.gauss = c->d_gauss;
     p.ent_idx = c->d_ent_idx;
     p.ent = c->d_ent_mats;
-    p.mats0 = c->mats0;
     p.cam = c->cam;
     p.n = c->n;
     p.sh_degree = c->sh_degree;

@@ -383,8 +383,9 @@ int tpd_read_tiles(tpd_ctx* c, uint32_t* counts, uint32_t* offsets) {
     if (!check_ctx(c) || !counts) return fail(TPD_ERR_INVALID, "tpd_read_tiles: bad argument");
     if (!c->rendered) return fail(TPD_ERR_STATE, "tpd_read_tiles: nothing rendered");
     int rc = copy_back(c, counts, c->d_tiles, sizeof(uint32_t) * (size_t)c->n);
-    if (rc == TPD_OK && offsets) rc = ensure_offsets(c, c->stream);
-    if (rc == TPD_OK && offsets) rc = copy_back(c, offsets, c->d_offsets, sizeof(uint32_t) * (size_t)c->n);
+    // summed here: a scan on the context's stream would not be ordered with the stream the frame ran on
+    uint32_t sum = 0;
+    for (uint32_t i = 0; rc == TPD_OK && offsets && i < c->n; sum += counts[i++]) offsets[i] = sum;
     return rc;
 }
 

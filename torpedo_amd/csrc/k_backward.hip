@@ -69,8 +69,8 @@ __global__ __launch_bounds__(kGradBlock) void k_preprocess_bwd(const PreBackward
         if (a.ent_idx) {
             const EntityMats& m = a.ent[a.ent_idx[i]];
             accumulate_param_grads(rec, m.vm, m.pvm, a.cam, a.sh_degree, gr, gm, gls, gq, gop, gsh);
-        } else {
-            accumulate_param_grads(rec, a.mats0.vm, a.mats0.pvm, a.cam, a.sh_degree, gr, gm, gls, gq, gop, gsh);
+        } else {  // a block-uniform address: scalar loads
+            accumulate_param_grads(rec, a.ent[0].vm, a.ent[0].pvm, a.cam, a.sh_degree, gr, gm, gls, gq, gop, gsh);
         }
     }
     if (valid && a.g2d)

@@ -232,7 +232,10 @@ __global__ __launch_bounds__(kPreBlock) void k_batch_items(const BatchArgs a, co
     __shared__ ItemCountLds L;
     begin_items(a, L);
     const uint32_t b = blockIdx.x;
-    if (b == 0 && threadIdx.x == 0) a.counters[kCtrSortPairs] = 0u;  // set by the emission
+    if (b == 0 && threadIdx.x == 0) {
+        a.counters[kCtrSortPairs] = 0u;    // set by the emission
+        a.counters[kCtrScanTicket2] = 0u;  // of the item offsets
+    }
     if (b >= a.nblocks) return;  // the one block of a batch without Gaussians only clears
     const BatchSceneDev& sc = scenes[block_scene[b]];
     const uint32_t g = (b - sc.first_block) * kPreBlock + threadIdx.x;
@@ -257,7 +260,13 @@ __global__ __launch_bounds__(kPreBlock) void k_frame_items(const FrameArgs f) {
     const BatchArgs& a = f.b;
     begin_items(a, L);
     const uint32_t tid = threadIdx.x;
-    // for a backward that may follow (a fill of its own costs it two launches)
+    // for a backward that may follow (a fill of its own costs it two launches): the offsets' ticket and
+    // descriptors, and the matrices of a scene without entity indices
+    if (blockIdx.x == 0) {
+        if (tid == 0) a.counters[kCtrScanTicket2] = 0u;
+        if (!f.ent_idx && tid < sizeof(EntityMats) / sizeof(float))
+            reinterpret_cast<float*>(f.ent)[tid] = reinterpret_cast<const float*>(&f.mats0)[tid];
+    }
     for (uint32_t x = blockIdx.x * kPreBlock + tid; x < f.offset_parts; x += gridDim.x * kPreBlock) a.scan_desc2[x] = 0;
     uint32_t all0 = 0;
     uint64_t total = 0;

@@ -31,7 +31,7 @@ constexpr uint32_t kRangeRun = 8;
 
 // range.slang:16-35.  Empty tiles keep the (0, 0) written by the item kernel (the reference clears
 // with fillBuffer, GaussianEngine.cpp:843-848).  The kernel also re-zeroes the scan descriptors and
-// the scan tickets for the next frame.  A batch frame whose items were sorted on the depth-window key
+// the scan ticket for the next frame.  A batch frame whose items were sorted on the depth-window key
 // although one of its depths lies outside the window (kCtrDepthOut) has some pairs out of depth order
 // inside their tiles (never in the wrong tile); it is marked overflowed, so that every later kernel
 // skips it and the host renders it again on the wider key.
@@ -44,7 +44,6 @@ __global__ void k_ranges(const uint32_t* __restrict__ keys, uint32_t* __restrict
     for (uint32_t d = gid; d < n_scan_desc; d += nthreads) scan_desc[d] = 0;
     if (gid == 0) {
         *ticket = 0;
-        counters[kCtrScanTicket2] = 0;
         if (lo_bits == kDepthWindowBits && counters[kCtrDepthOut]) counters[kCtrOverflow] = 1u;
     }
     uint32_t* r = reinterpret_cast<uint32_t*>(ranges);

@@ -33,15 +33,15 @@ static BatchArgs item_args(tpd_ctx* c) {
     return a;
 }
 
-// Where each Gaussian's pairs lie in emission order: the exclusive scan of the tile counts, made for
-// the frames whose backward or tile readback asks for it.
-int ensure_offsets(tpd_ctx* c, hipStream_t s) {
-    if (c->have_offsets || c->n == 0) return TPD_OK;
+// Where each Gaussian's pairs lie in emission order: the exclusive scan of the tile counts, for a backward
+// on the stream it runs on.  The frame's item kernel, complete when tpd_render returns, clears the scan's
+// ticket and descriptors, and nothing else does: a second scan of one frame finds no partition left and
+// keeps the first one's offsets, so every backward launches it, recorded into a caller's graph or not.
+int launch_offsets(tpd_ctx* c, hipStream_t s) {
+    if (c->n == 0) return TPD_OK;
     launch_batch_item_offsets(item_args(c), s);
     const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return hip_fail(e, "item offsets");
-    c->have_offsets = true;
-    return TPD_OK;
+    return e == hipSuccess ? TPD_OK : hip_fail(e, "item offsets");
 }
 
 // Waits until the frame's totals have reached h_counters (k_frame_offsets stores seq last).
@@ -60,15 +60,16 @@ static int wait_totals(tpd_ctx* c, hipStream_t s, uint32_t seq) {
     return TPD_OK;
 }
 
-// Issues the frame once; c->frame_cap is the pair capacity it runs with.
+// Issues the frame once, with the room of the pair buffers.
 static int issue_frame(tpd_ctx* c, hipStream_t s, uint32_t gx, uint32_t gy) {
     const uint32_t ntiles = gx * gy, W = c->cam.width, H = c->cam.height;
     const uint32_t cap = (uint32_t)std::min<size_t>(c->cap_keys, kMaxSortKeys);
     if (c->profile) hipEventRecord(c->ev[0], s);
+    EntityMats mats0{};  // of a scene without entity indices
     if (c->d_ent_idx)
         launch_entity_mats(c->d_models, c->n_ent, c->cam, c->d_ent_mats, s);
     else
-        entity_mats(c->h_models.data(), c->cam, c->mats0);
+        entity_mats(c->h_models.data(), c->cam, mats0);
 
     const uint32_t lo_bits = c->depth_wide ? kDepthWideBits : kDepthWindowBits;
     const uint32_t key_bits = bit_length(ntiles > 1 ? ntiles - 1 : 1);
@@ -95,7 +96,7 @@ static int issue_frame(tpd_ctx* c, hipStream_t s, uint32_t gx, uint32_t gy) {
     f.gauss = c->d_gauss;
     f.ent_idx = c->d_ent_idx;
     f.ent = c->d_ent_mats;
-    f.mats0 = c->mats0;
+    f.mats0 = mats0;
     f.cam = c->cam;
     f.n = c->n;
     f.sh_degree = c->sh_degree;
@@ -155,7 +156,6 @@ int render_forward(tpd_ctx* c, hipStream_t s) {
     int rc;
     if ((rc = ensure_scene_buffers(c)) != TPD_OK) return rc;
     if ((rc = ensure_image_buffers(c)) != TPD_OK) return rc;
-    c->have_offsets = false;
 
     if (c->n == 0) {
         // Empty scene: black image, empty ranges (GaussianEngine.cpp:362-365 renders nothing).
@@ -196,7 +196,7 @@ int render_forward(tpd_ctx* c, hipStream_t s) {
     c->last_pairs = P;
     c->has_blend = true;
     if (c->keep_unsorted && P) {
-        if ((rc = ensure_offsets(c, s)) != TPD_OK) return rc;
+        if ((rc = launch_offsets(c, s)) != TPD_OK) return rc;
         if ((e = grow(c->d_keys_dbg, c->cap_keys_dbg, P, 1.25)) != hipSuccess ||
             (e = grow(c->d_vals_dbg, c->cap_vals_dbg, P, 1.25)) != hipSuccess)
             return hip_fail(e, "alloc unsorted pairs");

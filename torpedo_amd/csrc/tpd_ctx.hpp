@@ -48,8 +48,6 @@ struct tpd_ctx {
     uint32_t* d_ivals = nullptr; size_t cap_ivals = 0;
     uint32_t* d_ivals_alt = nullptr; size_t cap_ivals_alt = 0;
     uint64_t* d_rects = nullptr; size_t cap_rects = 0;   // rectangles that do not fit their item's key
-    tpd::EntityMats mats0{};                             // scene without entity indices: its one model
-    bool have_offsets = false;                           // d_offsets is that of the last frame
     uint32_t frame_seq = 0;                              // of the totals in h_counters
 
     // pairs (tiles and Gaussian indices) + sort
@@ -105,7 +103,7 @@ int ensure_image_buffers(tpd_ctx* c);
 int ensure_pair_buffers(tpd_ctx* c, size_t pairs);
 int ensure_sort_workspace(tpd_ctx* c, size_t pairs);
 int render_forward(tpd_ctx* c, hipStream_t s);
-int ensure_offsets(tpd_ctx* c, hipStream_t s);
+int launch_offsets(tpd_ctx* c, hipStream_t s);
 void backward_release(tpd_ctx* c);
 void batch_release(tpd_ctx* c);
 void batch_set_sort_shape(tpd_ctx* c, uint32_t shape);

@@ -11,7 +11,8 @@ enum : uint32_t {
     kCtrPairs = 1,        // pair count P written by the last preprocess partition
     kCtrOverflow = 2,     // 1 when P exceeded the key/value capacity
     kCtrDepthOut = 3,     // non-zero when an emitted depth lies outside the sort's depth window
-    kCtrScanTicket2 = 4,  // partition ticket of a second scan in the frame (the item offsets)
+    kCtrScanTicket2 = 4,  // partition ticket of a second scan in the frame (the item offsets), cleared by
+                          // the item kernel
     kCtrSortPairs = 5,    // pair count for the pair sort and the ranges: P, or 0 when the frame overflowed
                           // (it is rendered again)
     kCtrTotal64 = 6,      // (two words) the plain frame's pair count, summed by its item kernel; zero between
@@ -82,9 +83,8 @@ struct BackwardArgs {
 
 struct PreBackwardArgs {
     const float* gauss;
-    const uint32_t* ent_idx;     // N entity indices, or null: every Gaussian uses mats0
-    const EntityMats* ent;       // per entity (with ent_idx)
-    EntityMats mats0;
+    const uint32_t* ent_idx;     // N entity indices, or null: every Gaussian uses the first
+    const EntityMats* ent;       // per entity
     CameraParams cam;
     uint32_t n, sh_degree;
     const uint32_t* tiles;
@@ -104,7 +104,7 @@ void launch_preprocess_bwd(const PreBackwardArgs& a, hipStream_t s);
 
 void launch_entity_mats(const float* models, uint32_t n_ent, const CameraParams& cam, EntityMats* out, hipStream_t s);
 // Tile ranges of the P = min(counters[count_slot], cap) sorted keys (tiles).  Also re-zeroes the scan
-// descriptors and the scan tickets for the next frame, and sets kCtrOverflow when a frame whose items
+// descriptors and the emission's ticket for the next frame, and sets kCtrOverflow when a frame whose items
 // were sorted on the depth-window key (lo_bits = kDepthWindowBits) has kCtrDepthOut set.
 void launch_ranges(const uint32_t* keys, uint32_t* counters, uint32_t P_hint, uint2* ranges, uint64_t* scan_desc,
                    uint32_t n_scan_desc, uint32_t* ticket, hipStream_t s, uint32_t cap, uint32_t lo_bits);
@@ -216,7 +216,7 @@ struct FrameArgs {
     BatchArgs b;
     const float* gauss;           // N x 60 records (any alignment)
     const uint32_t* ent_idx;      // N entity indices, or null: every Gaussian uses mats0
-    const EntityMats* ent;
+    EntityMats* ent;              // per entity; without ent_idx the kernel stores mats0 there, for the backward
     EntityMats mats0;
     CameraParams cam;
     uint32_t n, sh_degree, gx, gy;
