@@ -268,7 +268,7 @@ static int build_layout(tpd_ctx* c, BatchState* b) {
         if ((e = grow(b->d_scan_desc, b->cap_scan_desc, nparts)) != hipSuccess) return hip_fail(e, "tpd_batch: alloc");
     }
     // look-back descriptors and counters start at zero; afterwards every frame leaves them so
-    if ((e = hipMemset(b->d_scan_desc, 0, b->cap_scan_desc * sizeof(uint64_t))) != hipSuccess)
+    if ((e = clear_now(b->d_scan_desc, b->cap_scan_desc * sizeof(uint64_t))) != hipSuccess)
         return hip_fail(e, "tpd_batch: clear");
     if (!b->d_counters) {
         if ((e = hipMalloc(&b->d_counters, sizeof(uint32_t) * kCtrCount)) != hipSuccess)
@@ -277,7 +277,7 @@ static int build_layout(tpd_ctx* c, BatchState* b) {
                                hipHostMallocDefault)) != hipSuccess)
             return hip_fail(e, "tpd_batch: alloc");
     }
-    if ((e = hipMemset(b->d_counters, 0, sizeof(uint32_t) * kCtrCount)) != hipSuccess)
+    if ((e = clear_now(b->d_counters, sizeof(uint32_t) * kCtrCount)) != hipSuccess)
         return hip_fail(e, "tpd_batch: clear");
     if (nv) {
         e = hipMemcpy(b->d_scene_views, b->h_scene_views.data(), nv * sizeof(uint32_t), hipMemcpyHostToDevice);
@@ -314,7 +314,7 @@ static int ensure_sort_ws(BatchState* b) {
     hipError_t e;
     if (!b->ws.partials) {
         if ((e = hipMalloc(&b->ws.partials, sizeof(uint32_t) * kCountCopies * kMaxPasses * kMaxRadix)) != hipSuccess ||
-            (e = hipMemset(b->ws.partials, 0, sizeof(uint32_t) * kCountCopies * kMaxPasses * kMaxRadix)) != hipSuccess ||
+            (e = clear_now(b->ws.partials, sizeof(uint32_t) * kCountCopies * kMaxPasses * kMaxRadix)) != hipSuccess ||
             (e = hipMalloc(&b->ws.offsets, sizeof(uint32_t) * kMaxPasses * kMaxRadix)) != hipSuccess ||
             (e = hipMalloc(&b->ws.tickets, sizeof(uint32_t) * kMaxPasses)) != hipSuccess)
             return hip_fail(e, "tpd_batch: alloc sort workspace");

@@ -49,7 +49,7 @@ int ensure_scene_buffers(tpd_ctx* c) {
     const size_t nd = emit_max_parts((uint32_t)n);
     if (!c->d_scan_desc || c->cap_scan_desc < nd) {
         if ((e = grow(c->d_scan_desc, c->cap_scan_desc, nd)) != hipSuccess) return hip_fail(e, "alloc scan desc");
-        if ((e = hipMemset(c->d_scan_desc, 0, c->cap_scan_desc * sizeof(uint64_t))) != hipSuccess)
+        if ((e = clear_now(c->d_scan_desc, c->cap_scan_desc * sizeof(uint64_t))) != hipSuccess)
             return hip_fail(e, "clear scan desc");
     }
     const size_t ne = std::max<uint32_t>(c->n_ent, 1u);
@@ -96,7 +96,7 @@ int ensure_sort_workspace(tpd_ctx* c, size_t pairs) {
     hipError_t e;
     if (!c->ws.partials) {
         if ((e = hipMalloc(&c->ws.partials, sizeof(uint32_t) * kCountCopies * kMaxPasses * kMaxRadix)) != hipSuccess ||
-            (e = hipMemset(c->ws.partials, 0, sizeof(uint32_t) * kCountCopies * kMaxPasses * kMaxRadix)) != hipSuccess)
+            (e = clear_now(c->ws.partials, sizeof(uint32_t) * kCountCopies * kMaxPasses * kMaxRadix)) != hipSuccess)
             return hip_fail(e, "alloc sort counts");
         if ((e = hipMalloc(&c->ws.offsets, sizeof(uint32_t) * kMaxPasses * kMaxRadix)) != hipSuccess)
             return hip_fail(e, "alloc sort offsets");
@@ -157,7 +157,7 @@ int tpd_create(tpd_ctx** out, const tpd_config* cfg) {
         return hip_fail(e, "hipHostMalloc");
     }
     if ((e = hipMalloc(&c->d_counters, sizeof(uint32_t) * kCtrCount)) != hipSuccess ||
-        (e = hipMemset(c->d_counters, 0, sizeof(uint32_t) * kCtrCount)) != hipSuccess) {
+        (e = clear_now(c->d_counters, sizeof(uint32_t) * kCtrCount)) != hipSuccess) {
         tpd_destroy(c);
         return hip_fail(e, "alloc counters");
     }

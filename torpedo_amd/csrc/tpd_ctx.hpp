@@ -132,6 +132,13 @@ inline hipError_t grow(T*& p, size_t& cap, size_t count, double headroom = 1.0) 
     return hipSuccess;
 }
 
+// Zeroes device memory before anything uses it.  hipMemset goes to the null stream and may return before it
+// has run (8 GiB: 3 us, then 1.4 ms of work), and the streams frames run on do not wait for the null stream.
+inline hipError_t clear_now(void* p, size_t bytes) {
+    const hipError_t e = hipMemset(p, 0, bytes);
+    return e == hipSuccess ? hipStreamSynchronize(nullptr) : e;
+}
+
 template <typename T>
 inline void release(T*& p) {
     if (p) (void)hipFree(p);
