@@ -260,7 +260,7 @@ int tpd_upload(tpd_ctx* c, const float* gaussians, uint32_t n, const uint32_t* e
     }
     c->have_scene = true;
     c->rendered = false;
-    c->depth_wide = false;
+    c->wide_frames = 0;
     return ensure_scene_buffers(c);
 }
 
@@ -425,6 +425,12 @@ int tpd_read_tile_order(tpd_ctx* c, uint32_t* order) {
     const uint32_t gx = (c->cam.width + 15) / 16;
     for (size_t t = 0; rc == TPD_OK && t < ntiles; ++t) order[t] = (jobs[t].txy >> 16) * gx + (jobs[t].txy & 0xFFFFu);
     return rc;
+}
+
+int tpd_get_frame_issues(tpd_ctx* c, uint64_t* issues) {
+    if (!check_ctx(c) || !issues) return fail(TPD_ERR_INVALID, "tpd_get_frame_issues: bad argument");
+    *issues = c->issues;
+    return TPD_OK;
 }
 
 int tpd_synchronize(tpd_ctx* c) {

@@ -44,7 +44,10 @@ __global__ void k_ranges(const uint32_t* __restrict__ keys, uint32_t* __restrict
     for (uint32_t d = gid; d < n_scan_desc; d += nthreads) scan_desc[d] = 0;
     if (gid == 0) {
         *ticket = 0;
-        if (lo_bits == kDepthWindowBits && counters[kCtrDepthOut]) counters[kCtrOverflow] = 1u;
+        if (lo_bits != kDepthWindowBits)
+            counters[kCtrDepthOut] = 0;  // (always, in a plain frame: the host has it)
+        else if (counters[kCtrDepthOut])
+            counters[kCtrOverflow] = 1u;
     }
     uint32_t* r = reinterpret_cast<uint32_t*>(ranges);
     const uint32_t runs = (P + kRangeRun - 1) / kRangeRun;

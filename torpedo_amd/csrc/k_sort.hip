@@ -156,16 +156,20 @@ __global__ __launch_bounds__(256) void k_frame_offsets(uint32_t* __restrict__ co
     const bool items = b < ipasses;
     const uint32_t row = items ? b << ibits : kPairCountRow + ((b - ipasses) << pbits);
     const uint32_t n = scan_digit_counts(counts + row, offsets + row, items ? ibits : pbits, s_w);
-    if (b == 0 && items && threadIdx.x == 255) counters[kCtrItemsKept] = n;
+    const bool depth_over = totals.host && totals.lo_bits == kDepthWindowBits && counters[kCtrDepthOut] != 0;
+    // (no item is sorted on a window that does not hold its depth: the frame is issued again)
+    if (b == 0 && items && threadIdx.x == 255) {
+        counters[kCtrItemsKept] = depth_over ? 0u : n;
+        counters[kCtrSortItems] = depth_over ? 0u : totals.items;
+    }
     if (totals.host && b == gridDim.x - 1 && threadIdx.x == 0) {
         // the 64-bit total, as the digit counts may have wrapped
         uint64_t* const t64 = reinterpret_cast<uint64_t*>(counters + kCtrTotal64);
         const uint64_t total = *t64;
         const uint32_t P = total > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)total;
         const uint32_t depth_out = counters[kCtrDepthOut];
-        const bool over = total > totals.cap || (totals.lo_bits == kDepthWindowBits && depth_out != 0);
+        const bool over = total > totals.cap || depth_over;
         *t64 = 0;
-        counters[kCtrDepthOut] = 0;
         counters[kCtrPairs] = P;
         counters[kCtrOverflow] = over ? 1u : 0u;
         counters[kCtrSortPairs] = over ? 0u : P;
@@ -564,8 +568,9 @@ void launch_sort_offsets(SortWorkspace& ws, uint32_t item_shape, uint32_t ipasse
 }
 
 bool launch_sort_items(SortWorkspace& ws, uint32_t shape, uint64_t* keys, uint32_t* vals, uint64_t* keys_alt,
-                       uint32_t* vals_alt, uint32_t n, uint32_t lo_bits, const uint32_t* kept, hipStream_t s) {
-    return launch_passes(ws, shape, sort_digit_plan(shape, lo_bits), ws.offsets, keys, vals, keys_alt, vals_alt, nullptr,
+                       uint32_t* vals_alt, uint32_t n, uint32_t lo_bits, const uint32_t* kept, hipStream_t s,
+                       const uint32_t* count_ptr) {
+    return launch_passes(ws, shape, sort_digit_plan(shape, lo_bits), ws.offsets, keys, vals, keys_alt, vals_alt, count_ptr,
                          n, kept, s);
 }
 

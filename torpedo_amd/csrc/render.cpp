@@ -15,6 +15,12 @@
 
 namespace tpd {
 
+// A frame sorted on the depth window although one of its depths lies outside is issued again on the wide
+// key (1M Gaussians at 1920x1080: 125 us beside the frame's 405), where that key costs 10 us (one more pass
+// of the item sort).  So it is kept for some frames after the last such depth: a camera whose farthest depth
+// moves in and out by turns, 957 -> 780 us for two frames.
+constexpr uint32_t kDepthHold = 64;
+
 // The arguments shared by the frame's item kernel, its emission and the item offsets.
 static BatchArgs item_args(tpd_ctx* c) {
     BatchArgs a{};
@@ -71,7 +77,7 @@ static int issue_frame(tpd_ctx* c, hipStream_t s, uint32_t gx, uint32_t gy) {
     else
         entity_mats(c->h_models.data(), c->cam, mats0);
 
-    const uint32_t lo_bits = c->depth_wide ? kDepthWideBits : kDepthWindowBits;
+    const uint32_t lo_bits = c->wide_frames ? kDepthWideBits : kDepthWindowBits;
     const uint32_t key_bits = bit_length(ntiles > 1 ? ntiles - 1 : 1);
     const uint32_t ishape = sort_shape_for(c->item_shape, c->n, lo_bits, 8);
     const uint32_t pshape = sort_shape_for(c->ws.shape, expected_pairs(c->n, cap), key_bits, 4);
@@ -80,7 +86,7 @@ static int issue_frame(tpd_ctx* c, hipStream_t s, uint32_t gx, uint32_t gy) {
     BatchArgs& a = f.b;
     a.cap = cap;
     a.lo_bits = lo_bits;
-    a.lo_base = c->depth_wide ? 0u : kDepthBase;
+    a.lo_base = c->wide_frames ? 0u : kDepthBase;
     a.hist_counts = c->ws.partials;
     a.hist_desc0 = c->ws.desc;
     a.hist_tickets = c->ws.tickets;
@@ -103,13 +109,14 @@ static int issue_frame(tpd_ctx* c, hipStream_t s, uint32_t gx, uint32_t gy) {
     f.gx = gx;
     f.gy = gy;
     f.offset_parts = item_offset_parts(c->n);
+    ++c->issues;
     launch_frame_items(f, s);
     if (c->profile) hipEventRecord(c->ev[1], s);
-    const FrameTotals totals{cap, lo_bits, ++c->frame_seq, c->d_host_counters};
+    const FrameTotals totals{cap, lo_bits, c->n, ++c->frame_seq, c->d_host_counters};
     launch_sort_offsets(c->ws, ishape, a.hist_plan.passes, pshape, a.pair_plan.passes, c->d_counters, &totals, s);
     if (c->profile) hipEventRecord(c->ev[2], s);
     const bool items_alt = launch_sort_items(c->ws, ishape, c->d_ikeys, c->d_ivals, c->d_ikeys_alt, c->d_ivals_alt, c->n,
-                                             lo_bits, &c->d_counters[kCtrItemsKept], s);
+                                             lo_bits, &c->d_counters[kCtrItemsKept], s, &c->d_counters[kCtrSortItems]);
     if (c->profile) hipEventRecord(c->ev[3], s);
     a.kept_items = &c->d_counters[kCtrItemsKept];
     a.sorted_items = items_alt ? c->d_ivals_alt : c->d_ivals;
@@ -184,9 +191,12 @@ int render_forward(tpd_ctx* c, hipStream_t s) {
         if ((rc = issue_frame(c, s, gx, gy)) != TPD_OK) return rc;
         if ((rc = wait_totals(c, s, c->frame_seq)) != TPD_OK) return rc;
         P = c->h_counters[kHostPairs];
-        const bool depth_out = c->h_counters[kHostDepthOut] != 0, was_wide = c->depth_wide;
+        const bool depth_out = c->h_counters[kHostDepthOut] != 0, was_wide = c->wide_frames != 0;
         if (P > kMaxSortKeys) return fail(TPD_ERR_CAPACITY, "tpd_render: more than 2^30 - 1 tile/Gaussian pairs");
-        c->depth_wide = depth_out;  // the next frame's key: the wider one only while a depth needs it
+        if (depth_out)
+            c->wide_frames = kDepthHold;
+        else if (was_wide && !c->h_counters[kHostOverflow])
+            --c->wide_frames;
         if (!c->h_counters[kHostOverflow]) break;
         if (attempt > 2) return fail(TPD_ERR_STATE, "tpd_render: pair buffers did not converge");
         if (!(depth_out && !was_wide) || P > c->cap_keys) {

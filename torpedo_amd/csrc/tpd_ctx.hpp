@@ -62,9 +62,8 @@ struct tpd_ctx {
     uint32_t item_shape = tpd::kShapeAuto;
     const uint32_t* sorted_keys = nullptr;
     const uint32_t* sorted_vals = nullptr;
-    // Depth key of the next frame's item sort: the depth window unless the last frame had a depth
-    // outside it.
-    bool depth_wide = false;
+    uint32_t wide_frames = 0;   // frames still to be sorted on the wide depth key (kDepthHold, render.cpp)
+    uint64_t issues = 0;        // item launches of all frames: one a frame, two where a depth left the window
 
     // image
     uint2* d_ranges = nullptr; size_t cap_ranges = 0;

@@ -17,6 +17,8 @@ enum : uint32_t {
                           // (it is rendered again)
     kCtrTotal64 = 6,      // (two words) the plain frame's pair count, summed by its item kernel; zero between
                           // frames
+    kCtrSortItems = 8,    // the plain frame's items as its item sort's first pass counts them: all, or 0 when
+                          // a depth lies outside the window that they would be sorted on
     kCtrItemsKept = 32,   // the visible items: those the item sort keeps (its later passes and
                           // the emission run on them).  128 bytes past the tickets: every emission
                           // block reads it right after its ticket atomic, and on the tickets' L2
@@ -105,7 +107,8 @@ void launch_preprocess_bwd(const PreBackwardArgs& a, hipStream_t s);
 void launch_entity_mats(const float* models, uint32_t n_ent, const CameraParams& cam, EntityMats* out, hipStream_t s);
 // Tile ranges of the P = min(counters[count_slot], cap) sorted keys (tiles).  Also re-zeroes the scan
 // descriptors and the emission's ticket for the next frame, and sets kCtrOverflow when a frame whose items
-// were sorted on the depth-window key (lo_bits = kDepthWindowBits) has kCtrDepthOut set.
+// were sorted on the depth-window key (lo_bits = kDepthWindowBits) has kCtrDepthOut set, which it clears
+// otherwise.
 void launch_ranges(const uint32_t* keys, uint32_t* counters, uint32_t P_hint, uint2* ranges, uint64_t* scan_desc,
                    uint32_t n_scan_desc, uint32_t* ticket, hipStream_t s, uint32_t cap, uint32_t lo_bits);
 // The 64-bit keys (tile << 32) | floatbits(view depth) of n sorted tile keys, the depth from the splat
@@ -323,14 +326,14 @@ bool launch_sort_pairs(SortWorkspace& ws, uint64_t* keys, uint32_t* vals, uint64
 // pairs from kPairCountRow) and re-zeroes the counts.  pair_shape with ppasses = 0: no counted pairs.
 // With a frame (totals non-null) it also settles the frame's totals from the item kernel's: kCtrPairs,
 // kCtrOverflow (more pairs than cap, or a depth outside the window of an item sort on it), kCtrSortPairs,
-// and tells the host.
+// kCtrSortItems, and tells the host.
 constexpr uint32_t kMaxCountedPasses = 4;      // item passes whose counts the item kernel can make
 constexpr uint32_t kMaxCountedPairPasses = 3;
 constexpr uint32_t kPairCountRow = kMaxCountedPasses * kMaxRadix;
 static_assert(kPairCountRow + kMaxCountedPairPasses * kMaxRadix <= kMaxPasses * kMaxRadix, "pair count rows");
 enum : uint32_t { kHostPairs = 0, kHostOverflow = 1, kHostDepthOut = 2, kHostSeq = 3 };  // words of FrameTotals::host
 struct FrameTotals {
-    uint32_t cap, lo_bits;
+    uint32_t cap, lo_bits, items;
     uint32_t seq;      // stored last, when the other words are there
     uint32_t* host;    // pinned host memory
 };
@@ -338,9 +341,10 @@ void launch_sort_offsets(SortWorkspace& ws, uint32_t item_shape, uint32_t ipasse
                          uint32_t* counters, const FrameTotals* totals, hipStream_t s);
 // Sorts the n items by the low lo_bits bits of their keys.  The first pass drops the keys whose high
 // word is zero (the counts leave them out) and takes each key's index as its value; the later ones
-// sort the *kept others.
+// sort the *kept others.  count_ptr (optional): the first pass takes *count_ptr of the n.
 bool launch_sort_items(SortWorkspace& ws, uint32_t shape, uint64_t* keys, uint32_t* vals, uint64_t* keys_alt,
-                       uint32_t* vals_alt, uint32_t n, uint32_t lo_bits, const uint32_t* kept, hipStream_t s);
+                       uint32_t* vals_alt, uint32_t n, uint32_t lo_bits, const uint32_t* kept, hipStream_t s,
+                       const uint32_t* count_ptr = nullptr);
 // Sorts the min(*count_ptr, n_max) pairs by the low key_bits bits of their 32-bit keys; without
 // counted, their digits are counted first.
 bool launch_sort_pairs32(SortWorkspace& ws, uint32_t shape, uint32_t* keys, uint32_t* vals, uint32_t* keys_alt,
