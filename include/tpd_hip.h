@@ -147,9 +147,10 @@ int tpd_memcpy(tpd_ctx* ctx, void* dst, const void* src, uint64_t bytes, int kin
  * *passes the number of radix passes of both sorts. */
 int tpd_set_profiling(tpd_ctx* ctx, int enable);
 int tpd_get_stage_times(tpd_ctx* ctx, float* ms, uint32_t* passes);
-/* How many times the context has projected a plain frame's Gaussians: once per tpd_render, and once more
- * for a frame that met a depth outside the sort's depth window. */
-int tpd_get_frame_issues(tpd_ctx* ctx, uint64_t* issues);
+/* How many times the context has projected a plain frame's Gaussians (once per tpd_render, and once more
+ * for a frame that met a depth outside the sort's depth window), and how many frames emitted their pairs
+ * once more because there was no room for them. */
+int tpd_get_frame_issues(tpd_ctx* ctx, uint64_t* issues, uint64_t* resumes);
 /* Pixel-splat pairs whose power the blend of the last rendered frame evaluates (counted by blending
  * that frame once more with a counting kernel; same image). */
 int tpd_get_blend_evaluations(tpd_ctx* ctx, uint64_t* evaluations);

@@ -19,7 +19,7 @@ def eng():
 
 
 def frame(eng, orc, g, cam):
-    """One frame, checked; returns how often it was issued."""
+    """One frame, checked; returns how often it was issued, and its pairs issued again."""
     before = eng.frameIssues()
     eng.setCamera(cam.view, cam.proj_view, cam.focal_ndc, cam.width, cam.height)
     eng.render()
@@ -27,7 +27,7 @@ def frame(eng, orc, g, cam):
     ref = orc.render(g, cam, 3)
     assert np.array_equal(keys, ref["keys"]) and np.array_equal(vals, ref["vals"])
     assert np.abs(eng.readImage() - ref["image"]).max() <= 1e-5
-    return eng.frameIssues() - before
+    return tuple(a - b for a, b in zip(eng.frameIssues(), before))
 
 
 def test_depths_moving_across_the_window(eng, orc):
@@ -44,11 +44,66 @@ def test_depths_moving_across_the_window(eng, orc):
     eng.uploadRecords(g, 3)
     eng.setSortShape(6)
     eng.setProfiling(True)
-    assert frame(eng, orc, g, inside) == 1 and eng.stageTimes()["radix_passes"] == 4
-    assert frame(eng, orc, g, outside) == 2 and eng.stageTimes()["radix_passes"] == 5
+    assert frame(eng, orc, g, inside) == (1, 0) and eng.stageTimes()["radix_passes"] == 4
+    assert frame(eng, orc, g, outside) == (2, 0) and eng.stageTimes()["radix_passes"] == 5
     for k in range(12):
-        assert frame(eng, orc, g, (inside, outside)[k % 2]) == 1, k
+        assert frame(eng, orc, g, (inside, outside)[k % 2]) == (1, 0), k
     for k in range(64):
-        assert frame(eng, orc, g, inside) == 1 and eng.stageTimes()["radix_passes"] == 5, k
-    assert frame(eng, orc, g, inside) == 1 and eng.stageTimes()["radix_passes"] == 4
-    assert frame(eng, orc, g, outside) == 2
+        assert frame(eng, orc, g, inside) == (1, 0) and eng.stageTimes()["radix_passes"] == 5, k
+    assert frame(eng, orc, g, inside) == (1, 0) and eng.stageTimes()["radix_passes"] == 4
+    assert frame(eng, orc, g, outside) == (2, 0)
+
+
+def crowd(n, seed, scale, far=None):
+    """n Gaussians of n x some hundred pairs at 320x200; far: and one at that depth."""
+    g = small_scene(n, seed=seed, log_scale_mean=scale)
+    if far is not None:
+        from torpedo_amd.engine import gaussian_point
+        g = np.concatenate([g, gaussian_point([0, 0, far], 0.8, (0, 0, 0, 1), (2.0,) * 3, np.full(48, 0.3, np.float32))[None]])
+    return g
+
+
+@pytest.mark.parametrize("shape", [None, 0, 6, 9])
+def test_first_frame_over_the_room(orc, shape):
+    """More pairs than max(4 n, 2^20) with headroom: the Gaussians are projected and sorted once, their pairs
+    emitted again with room for them; then the same frame, a backward and a small frame."""
+    from torpedo_amd.engine import GaussianEngine
+    cam = orc.make_camera([0.0, 0.0, -3.0], [0.0, 0.0, 0.0], [0.0, -1.0, 0.0], W, H)
+    g, small = crowd(8000, 11, -0.5), crowd(500, 12, -3.0)
+    with GaussianEngine() as eng:
+        if shape is not None:
+            eng.setSortShape(shape)
+        eng.uploadRecords(g, 3)
+        assert frame(eng, orc, g, cam) == (1, 1) and eng.pairCount > 5 * (1 << 18)
+        assert frame(eng, orc, g, cam) == (1, 0)
+        counts, offs = eng.readTiles()
+        assert counts.sum() == eng.pairCount and np.array_equal(offs[1:], np.cumsum(counts)[:-1])
+        eng.uploadRecords(small, 3)
+        assert frame(eng, orc, small, cam) == (1, 0)
+
+
+def test_first_frame_over_the_room_and_the_window(orc, eng):
+    """A first frame with neither room for its pairs nor its depths in the window."""
+    cam = orc.make_camera([0.0, 0.0, -3.0], [0.0, 0.0, 0.0], [0.0, -1.0, 0.0], W, H, near=0.01, far=1000.0)
+    g = crowd(8000, 13, -0.5, far=300.0)
+    eng.uploadRecords(g, 3)
+    assert frame(eng, orc, g, cam) == (2, 0) and eng.pairCount > 5 * (1 << 18)
+    assert frame(eng, orc, g, cam) == (1, 0)
+
+
+def test_backward_of_a_resumed_frame(orc):
+    """The gradients of a frame whose pairs were emitted twice are those of the frame issued with room."""
+    import torch
+    from torpedo_amd.engine import GaussianEngine
+    cam = orc.make_camera([0.0, 0.0, -3.0], [0.0, 0.0, 0.0], [0.0, -1.0, 0.0], W, H)
+    g = crowd(8000, 14, -0.5)
+    with GaussianEngine() as eng:
+        up = torch.randn(H, W, 3, device="cuda", generator=torch.Generator("cuda").manual_seed(3))
+        sets = [[torch.empty(g.shape[0], k, device="cuda") for k in (3, 3, 4, 1, 48)] for _ in range(2)]
+        torch.cuda.synchronize()
+        eng.uploadRecords(g, 3)
+        for k, out in enumerate(sets):
+            assert frame(eng, orc, g, cam) == (1, 1 - k)
+            eng.backward(up.data_ptr(), *[t.data_ptr() for t in out])
+            eng.waitIdle()
+        assert all(torch.equal(a, b) for a, b in zip(*sets))

@@ -70,7 +70,7 @@ SIGNATURES = {
     "tpd_memcpy": (_i32, [_vp, _vp, _vp, ctypes.c_uint64, _i32]),
     "tpd_set_profiling": (_i32, [_vp, _i32]),
     "tpd_get_stage_times": (_i32, [_vp, _vp, ctypes.POINTER(_u32)]),
-    "tpd_get_frame_issues": (_i32, [_vp, ctypes.POINTER(ctypes.c_uint64)]),
+    "tpd_get_frame_issues": (_i32, [_vp, ctypes.POINTER(ctypes.c_uint64), ctypes.POINTER(ctypes.c_uint64)]),
     "tpd_get_blend_evaluations": (_i32, [_vp, ctypes.POINTER(ctypes.c_uint64)]),
     "tpd_measure_copy": (_i32, [_vp, ctypes.c_uint64, _u32, ctypes.POINTER(_f32)]),
     "tpd_measure_bandwidth": (_i32, [_vp, _u32, ctypes.c_uint64, _u32, _u32, ctypes.POINTER(_f32)]),

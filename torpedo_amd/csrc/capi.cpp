@@ -427,9 +427,10 @@ int tpd_read_tile_order(tpd_ctx* c, uint32_t* order) {
     return rc;
 }
 
-int tpd_get_frame_issues(tpd_ctx* c, uint64_t* issues) {
-    if (!check_ctx(c) || !issues) return fail(TPD_ERR_INVALID, "tpd_get_frame_issues: bad argument");
+int tpd_get_frame_issues(tpd_ctx* c, uint64_t* issues, uint64_t* resumes) {
+    if (!check_ctx(c) || !issues || !resumes) return fail(TPD_ERR_INVALID, "tpd_get_frame_issues: bad argument");
     *issues = c->issues;
+    *resumes = c->resumes;
     return TPD_OK;
 }
 

@@ -180,6 +180,16 @@ __global__ __launch_bounds__(256) void k_frame_offsets(uint32_t* __restrict__ co
     }
 }
 
+// A frame whose pairs had no room, found room for meanwhile: its totals stand, its emission may run.
+__global__ void k_frame_resume(uint32_t* counters) {
+    counters[kCtrOverflow] = 0u;
+    counters[kCtrSortPairs] = counters[kCtrPairs];
+}
+
+void launch_frame_resume(uint32_t* counters, hipStream_t s) {
+    hipLaunchKernelGGL(k_frame_resume, dim3(1), dim3(1), 0, s, counters);
+}
+
 // ------------------------------------------------------------------ one pass
 
 // Key widths of a pass: kKeys64 and kKeys32 read and write 64- and 32-bit keys.  kKeys64Drop is kKeys64

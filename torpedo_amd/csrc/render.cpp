@@ -7,8 +7,8 @@
 //
 // The whole frame is issued at once: its launches cover the pair capacity and read the pair count on
 // the device.  The count reaches the host while the frame's sorts still run; a frame that turns out to
-// have more pairs than the capacity, or a depth outside the window it was sorted on, stops there (every
-// later kernel returns) and is issued again.
+// have more pairs than the capacity, or a depth outside the window it is to be sorted on, stops there (every
+// later kernel returns).  The first is issued again from its emission on, the second from the start.
 #include "tpd_ctx.hpp"
 
 #include <algorithm>
@@ -66,82 +66,107 @@ static int wait_totals(tpd_ctx* c, hipStream_t s, uint32_t seq) {
     return TPD_OK;
 }
 
-// Issues the frame once, with the room of the pair buffers.
-static int issue_frame(tpd_ctx* c, hipStream_t s, uint32_t gx, uint32_t gy) {
-    const uint32_t ntiles = gx * gy, W = c->cam.width, H = c->cam.height;
-    const uint32_t cap = (uint32_t)std::min<size_t>(c->cap_keys, kMaxSortKeys);
-    if (c->profile) hipEventRecord(c->ev[0], s);
-    EntityMats mats0{};  // of a scene without entity indices
-    if (c->d_ent_idx)
-        launch_entity_mats(c->d_models, c->n_ent, c->cam, c->d_ent_mats, s);
-    else
-        entity_mats(c->h_models.data(), c->cam, mats0);
-
-    const uint32_t lo_bits = c->wide_frames ? kDepthWideBits : kDepthWindowBits;
-    const uint32_t key_bits = bit_length(ntiles > 1 ? ntiles - 1 : 1);
-    const uint32_t ishape = sort_shape_for(c->item_shape, c->n, lo_bits, 8);
-    const uint32_t pshape = sort_shape_for(c->ws.shape, expected_pairs(c->n, cap), key_bits, 4);
+// What one frame is issued with.
+struct FrameIssue {
     FrameArgs f{};
+    uint32_t gx, gy, ntiles, lo_bits, key_bits, ishape, pshape;
+};
+
+// The pair buffers as they are, for all that follows the item sort.  The pair sort's shape stays the one
+// the pairs' digits were counted for.
+static void set_pair_room(tpd_ctx* c, FrameIssue& q) {
+    BatchArgs& a = q.f.b;
+    a.cap = (uint32_t)std::min<size_t>(c->cap_keys, kMaxSortKeys);
+    a.keys = c->d_keys;
+    a.vals = c->d_vals;
+    a.hist_desc0 = c->ws.desc;
+    a.pair_desc0_words = ((a.cap + sort_shape_keys(q.pshape) - 1) / sort_shape_keys(q.pshape)) << a.pair_bits;
+}
+
+static FrameIssue plan_frame(tpd_ctx* c, uint32_t gx, uint32_t gy) {
+    FrameIssue q;
+    q.gx = gx;
+    q.gy = gy;
+    q.ntiles = gx * gy;
+    q.lo_bits = c->wide_frames ? kDepthWideBits : kDepthWindowBits;
+    q.key_bits = bit_length(q.ntiles > 1 ? q.ntiles - 1 : 1);
+    q.ishape = sort_shape_for(c->item_shape, c->n, q.lo_bits, 8);
+    q.pshape = sort_shape_for(c->ws.shape, expected_pairs(c->n, (uint32_t)std::min<size_t>(c->cap_keys, kMaxSortKeys)),
+                              q.key_bits, 4);
+    FrameArgs& f = q.f;
     f.b = item_args(c);
     BatchArgs& a = f.b;
-    a.cap = cap;
-    a.lo_bits = lo_bits;
+    a.lo_bits = q.lo_bits;
     a.lo_base = c->wide_frames ? 0u : kDepthBase;
     a.hist_counts = c->ws.partials;
-    a.hist_desc0 = c->ws.desc;
     a.hist_tickets = c->ws.tickets;
-    a.hist_bits = sort_shape_bits(ishape);
-    a.hist_plan = sort_digit_plan(ishape, lo_bits);
-    a.hist_desc0_words = ((c->n + sort_shape_keys(ishape) - 1) / sort_shape_keys(ishape)) << a.hist_bits;
+    a.hist_bits = sort_shape_bits(q.ishape);
+    a.hist_plan = sort_digit_plan(q.ishape, q.lo_bits);
+    a.hist_desc0_words = ((c->n + sort_shape_keys(q.ishape) - 1) / sort_shape_keys(q.ishape)) << a.hist_bits;
     a.pair_counts = c->ws.partials + kPairCountRow;
-    a.pair_bits = sort_shape_bits(pshape);
-    a.pair_plan = sort_digit_plan(pshape, key_bits);
-    a.pair_desc0_words = ((cap + sort_shape_keys(pshape) - 1) / sort_shape_keys(pshape)) << a.pair_bits;
+    a.pair_bits = sort_shape_bits(q.pshape);
+    a.pair_plan = sort_digit_plan(q.pshape, q.key_bits);
     a.ranges = c->d_ranges;
-    a.ntiles = ntiles;
+    a.ntiles = q.ntiles;
     f.gauss = c->d_gauss;
     f.ent_idx = c->d_ent_idx;
     f.ent = c->d_ent_mats;
-    f.mats0 = mats0;
     f.cam = c->cam;
     f.n = c->n;
     f.sh_degree = c->sh_degree;
     f.gx = gx;
     f.gy = gy;
     f.offset_parts = item_offset_parts(c->n);
+    set_pair_room(c, q);
+    return q;
+}
+
+// The frame up to its Gaussians in depth order, and its totals on their way to the host.
+static void issue_items(tpd_ctx* c, FrameIssue& q, hipStream_t s) {
     ++c->issues;
-    launch_frame_items(f, s);
+    BatchArgs& a = q.f.b;
+    if (c->profile) hipEventRecord(c->ev[0], s);
+    if (c->d_ent_idx)
+        launch_entity_mats(c->d_models, c->n_ent, c->cam, c->d_ent_mats, s);
+    else
+        entity_mats(c->h_models.data(), c->cam, q.f.mats0);
+    launch_frame_items(q.f, s);
     if (c->profile) hipEventRecord(c->ev[1], s);
-    const FrameTotals totals{cap, lo_bits, c->n, ++c->frame_seq, c->d_host_counters};
-    launch_sort_offsets(c->ws, ishape, a.hist_plan.passes, pshape, a.pair_plan.passes, c->d_counters, &totals, s);
+    const FrameTotals totals{a.cap, q.lo_bits, c->n, ++c->frame_seq, c->d_host_counters};
+    launch_sort_offsets(c->ws, q.ishape, a.hist_plan.passes, q.pshape, a.pair_plan.passes, c->d_counters, &totals, s);
     if (c->profile) hipEventRecord(c->ev[2], s);
-    const bool items_alt = launch_sort_items(c->ws, ishape, c->d_ikeys, c->d_ivals, c->d_ikeys_alt, c->d_ivals_alt, c->n,
-                                             lo_bits, &c->d_counters[kCtrItemsKept], s, &c->d_counters[kCtrSortItems]);
-    if (c->profile) hipEventRecord(c->ev[3], s);
+    const bool items_alt = launch_sort_items(c->ws, q.ishape, c->d_ikeys, c->d_ivals, c->d_ikeys_alt, c->d_ivals_alt, c->n,
+                                             q.lo_bits, &c->d_counters[kCtrItemsKept], s, &c->d_counters[kCtrSortItems]);
     a.kept_items = &c->d_counters[kCtrItemsKept];
     a.sorted_items = items_alt ? c->d_ivals_alt : c->d_ivals;
     a.sorted_keys64 = items_alt ? c->d_ikeys_alt : c->d_ikeys;
+}
+
+// The rest: the pairs, their sort and ranges, and the blend.
+static int issue_pairs(tpd_ctx* c, const FrameIssue& q, hipStream_t s) {
+    const BatchArgs& a = q.f.b;
+    if (c->profile) hipEventRecord(c->ev[3], s);
     launch_batch_emit(a, s);
     if (c->profile) hipEventRecord(c->ev[4], s);
-    const bool in_alt = launch_sort_pairs32(c->ws, pshape, c->d_keys, c->d_vals, c->d_keys_alt, c->d_vals_alt,
-                                            &c->d_counters[kCtrSortPairs], cap, key_bits, s, true);
+    const bool in_alt = launch_sort_pairs32(c->ws, q.pshape, c->d_keys, c->d_vals, c->d_keys_alt, c->d_vals_alt,
+                                            &c->d_counters[kCtrSortPairs], a.cap, q.key_bits, s, true);
     if (c->profile) hipEventRecord(c->ev[5], s);
     c->sorted_keys = in_alt ? c->d_keys_alt : c->d_keys;
     c->sorted_vals = in_alt ? c->d_vals_alt : c->d_vals;
     c->last_passes = a.hist_plan.passes + a.pair_plan.passes;
-    launch_ranges(c->sorted_keys, c->d_counters, cap, c->d_ranges, c->d_scan_desc,
-                  emit_parts(c->n, cap), &c->d_counters[kCtrScanTicket], s, cap, kDepthWideBits);
-    launch_tile_order(c->d_ranges, ntiles, c->d_counters, c->d_tile_hist, c->d_jobs, gx, nullptr, nullptr, s);
+    launch_ranges(c->sorted_keys, c->d_counters, a.cap, c->d_ranges, c->d_scan_desc,
+                  emit_parts(c->n, a.cap), &c->d_counters[kCtrScanTicket], s, a.cap, kDepthWideBits);
+    launch_tile_order(c->d_ranges, q.ntiles, c->d_counters, c->d_tile_hist, c->d_jobs, q.gx, nullptr, nullptr, s);
     if (c->profile) hipEventRecord(c->ev[6], s);
     BlendArgs b{};
     b.counters = c->d_counters;
     b.jobs = c->d_jobs;
     b.vals = c->sorted_vals;
     b.splats = c->d_splats;
-    b.width = W;
-    b.height = H;
-    b.gx = gx;
-    b.ntiles = ntiles;
+    b.width = c->cam.width;
+    b.height = c->cam.height;
+    b.gx = q.gx;
+    b.ntiles = q.ntiles;
     b.image = c->d_image;
     b.rgba8 = c->d_rgba8;
     b.eval_count = nullptr;  // counted on request, by blending the frame once more
@@ -187,21 +212,27 @@ int render_forward(tpd_ctx* c, hipStream_t s) {
     if ((rc = ensure_sort_workspace(c, std::max<size_t>(c->n, c->cap_keys))) != TPD_OK) return rc;
 
     uint32_t P = 0;
-    for (int attempt = 0;; ++attempt) {
-        if ((rc = issue_frame(c, s, gx, gy)) != TPD_OK) return rc;
-        if ((rc = wait_totals(c, s, c->frame_seq)) != TPD_OK) return rc;
+    for (;;) {
+        FrameIssue q = plan_frame(c, gx, gy);
+        issue_items(c, q, s);
+        if ((rc = issue_pairs(c, q, s)) != TPD_OK || (rc = wait_totals(c, s, c->frame_seq)) != TPD_OK) return rc;
         P = c->h_counters[kHostPairs];
         const bool depth_out = c->h_counters[kHostDepthOut] != 0, was_wide = c->wide_frames != 0;
         if (P > kMaxSortKeys) return fail(TPD_ERR_CAPACITY, "tpd_render: more than 2^30 - 1 tile/Gaussian pairs");
-        if (depth_out)
+        if (P > c->cap_keys && (rc = ensure_pair_buffers(c, P)) != TPD_OK) return rc;
+        if (depth_out) {
             c->wide_frames = kDepthHold;
-        else if (was_wide && !c->h_counters[kHostOverflow])
+            if (!was_wide) continue;  // issued again on the wide key
+        } else if (was_wide) {
             --c->wide_frames;
-        if (!c->h_counters[kHostOverflow]) break;
-        if (attempt > 2) return fail(TPD_ERR_STATE, "tpd_render: pair buffers did not converge");
-        if (!(depth_out && !was_wide) || P > c->cap_keys) {
-            if ((rc = ensure_pair_buffers(c, P)) != TPD_OK) return rc;
         }
+        if (c->h_counters[kHostOverflow]) {  // the Gaussians are in order: their pairs once more, with room
+            ++c->resumes;
+            set_pair_room(c, q);
+            launch_frame_resume(c->d_counters, s);
+            if ((rc = issue_pairs(c, q, s)) != TPD_OK) return rc;
+        }
+        break;
     }
     c->last_pairs = P;
     c->has_blend = true;

@@ -64,6 +64,7 @@ struct tpd_ctx {
     const uint32_t* sorted_vals = nullptr;
     uint32_t wide_frames = 0;   // frames still to be sorted on the wide depth key (kDepthHold, render.cpp)
     uint64_t issues = 0;        // item launches of all frames: one a frame, two where a depth left the window
+    uint64_t resumes = 0;       // frames whose pairs were issued again with more room
 
     // image
     uint2* d_ranges = nullptr; size_t cap_ranges = 0;

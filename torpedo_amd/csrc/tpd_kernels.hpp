@@ -339,6 +339,8 @@ struct FrameTotals {
 };
 void launch_sort_offsets(SortWorkspace& ws, uint32_t item_shape, uint32_t ipasses, uint32_t pair_shape, uint32_t ppasses,
                          uint32_t* counters, const FrameTotals* totals, hipStream_t s);
+// Lets a frame that had no room for its pairs go on from its emission (the host has made room).
+void launch_frame_resume(uint32_t* counters, hipStream_t s);
 // Sorts the n items by the low lo_bits bits of their keys.  The first pass drops the keys whose high
 // word is zero (the counts leave them out) and takes each key's index as its value; the later ones
 // sort the *kept others.  count_ptr (optional): the first pass takes *count_ptr of the n.

@@ -458,12 +458,13 @@ class GaussianEngine:
         out["radix_passes"] = int(passes.value)
         return out
 
-    def frameIssues(self) -> int:
-        """How many times plain frames have been issued: once a frame, and once more for one that met a depth
-        outside the sort's depth window (tpd_get_frame_issues)."""
-        v = ctypes.c_uint64()
-        check(lib().tpd_get_frame_issues(self._ctx, ctypes.byref(v)))
-        return int(v.value)
+    def frameIssues(self) -> tuple:
+        """(issues, resumes): how many times plain frames have been issued (once a frame, and once more for
+        one that met a depth outside the sort's depth window), and how many emitted their pairs once more
+        because there was no room for them (tpd_get_frame_issues)."""
+        v, r = ctypes.c_uint64(), ctypes.c_uint64()
+        check(lib().tpd_get_frame_issues(self._ctx, ctypes.byref(v), ctypes.byref(r)))
+        return int(v.value), int(r.value)
 
     def blendEvaluations(self) -> int:
         """Pixel-splat pairs whose power the last rendered frame's blend evaluates
