@@ -78,7 +78,7 @@ int ensure_image_buffers(tpd_ctx* c) {
 }
 
 // Pair buffers and the sort workspace for `pairs` pairs (grown with 25% headroom).
-int ensure_pair_buffers(tpd_ctx* c, size_t pairs) {
+int ensure_pair_buffers(tpd_ctx* c, size_t pairs, hipStream_t s) {
     pairs = std::max<size_t>(pairs, 1);
     if (c->cap_keys >= pairs && c->cap_vals >= pairs && c->cap_keys_alt >= pairs && c->cap_vals_alt >= pairs)
         return TPD_OK;
@@ -88,15 +88,15 @@ int ensure_pair_buffers(tpd_ctx* c, size_t pairs) {
     if ((e = grow(c->d_vals, c->cap_vals, pairs, h)) != hipSuccess) return hip_fail(e, "alloc vals");
     if ((e = grow(c->d_keys_alt, c->cap_keys_alt, pairs, h)) != hipSuccess) return hip_fail(e, "alloc keys");
     if ((e = grow(c->d_vals_alt, c->cap_vals_alt, pairs, h)) != hipSuccess) return hip_fail(e, "alloc vals");
-    return ensure_sort_workspace(c, std::max<size_t>(c->cap_keys, c->n));
+    return ensure_sort_workspace(c, std::max<size_t>(c->cap_keys, c->n), s);
 }
 
-int ensure_sort_workspace(tpd_ctx* c, size_t pairs) {
+int ensure_sort_workspace(tpd_ctx* c, size_t pairs, hipStream_t s) {
     const uint32_t parts = sort_parts((uint32_t)std::min<size_t>(pairs, kMaxSortKeys));
     hipError_t e;
     if (!c->ws.partials) {
         if ((e = hipMalloc(&c->ws.partials, sizeof(uint32_t) * kCountCopies * kMaxPasses * kMaxRadix)) != hipSuccess ||
-            (e = clear_now(c->ws.partials, sizeof(uint32_t) * kCountCopies * kMaxPasses * kMaxRadix)) != hipSuccess)
+            (e = hipMemsetAsync(c->ws.partials, 0, sizeof(uint32_t) * kCountCopies * kMaxPasses * kMaxRadix, s)) != hipSuccess)
             return hip_fail(e, "alloc sort counts");
         if ((e = hipMalloc(&c->ws.offsets, sizeof(uint32_t) * kMaxPasses * kMaxRadix)) != hipSuccess)
             return hip_fail(e, "alloc sort offsets");
@@ -537,9 +537,9 @@ int tpd_sort_pairs(tpd_ctx* c, uint64_t* d_keys, uint32_t* d_vals, uint64_t* d_k
     *in_alt = 0;
     if (n == 0) return TPD_OK;
     if (!d_keys || !d_vals || !d_keys_alt || !d_vals_alt) return fail(TPD_ERR_INVALID, "tpd_sort_pairs: null pointer");
-    int rc = ensure_sort_workspace(c, n);
-    if (rc != TPD_OK) return rc;
     hipStream_t s = pick_stream(c, stream);
+    int rc = ensure_sort_workspace(c, n, s);
+    if (rc != TPD_OK) return rc;
     *in_alt = launch_sort_pairs(c->ws, d_keys, d_vals, d_keys_alt, d_vals_alt, n, key_bits, s) ? 1 : 0;
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return hip_fail(e, "sort launch");

@@ -207,9 +207,9 @@ int render_forward(tpd_ctx* c, hipStream_t s) {
         return TPD_OK;
     }
 
-    if (c->cap_keys == 0 && (rc = ensure_pair_buffers(c, std::max<size_t>(4 * (size_t)c->n, 1u << 20))) != TPD_OK)
+    if (c->cap_keys == 0 && (rc = ensure_pair_buffers(c, std::max<size_t>(4 * (size_t)c->n, 1u << 20), s)) != TPD_OK)
         return rc;
-    if ((rc = ensure_sort_workspace(c, std::max<size_t>(c->n, c->cap_keys))) != TPD_OK) return rc;
+    if ((rc = ensure_sort_workspace(c, std::max<size_t>(c->n, c->cap_keys), s)) != TPD_OK) return rc;
 
     uint32_t P = 0;
     for (;;) {
@@ -219,7 +219,7 @@ int render_forward(tpd_ctx* c, hipStream_t s) {
         P = c->h_counters[kHostPairs];
         const bool depth_out = c->h_counters[kHostDepthOut] != 0, was_wide = c->wide_frames != 0;
         if (P > kMaxSortKeys) return fail(TPD_ERR_CAPACITY, "tpd_render: more than 2^30 - 1 tile/Gaussian pairs");
-        if (P > c->cap_keys && (rc = ensure_pair_buffers(c, P)) != TPD_OK) return rc;
+        if (P > c->cap_keys && (rc = ensure_pair_buffers(c, P, s)) != TPD_OK) return rc;
         if (depth_out) {
             c->wide_frames = kDepthHold;
             if (!was_wide) continue;  // issued again on the wide key

@@ -100,8 +100,9 @@ int hip_fail(hipError_t e, const char* what);
 uint32_t bit_length(uint32_t v);
 int ensure_scene_buffers(tpd_ctx* c);
 int ensure_image_buffers(tpd_ctx* c);
-int ensure_pair_buffers(tpd_ctx* c, size_t pairs);
-int ensure_sort_workspace(tpd_ctx* c, size_t pairs);
+// s: the stream that uses them first
+int ensure_pair_buffers(tpd_ctx* c, size_t pairs, hipStream_t s);
+int ensure_sort_workspace(tpd_ctx* c, size_t pairs, hipStream_t s);
 int render_forward(tpd_ctx* c, hipStream_t s);
 int launch_offsets(tpd_ctx* c, hipStream_t s);
 void backward_release(tpd_ctx* c);
