@@ -107,3 +107,22 @@ def test_backward_of_a_resumed_frame(orc):
             eng.backward(up.data_ptr(), *[t.data_ptr() for t in out])
             eng.waitIdle()
         assert all(torch.equal(a, b) for a, b in zip(*sets))
+
+
+def test_room_follows_recent_frames(orc, eng):
+    """A large frame by turns with small ones keeps its room; forty small frames later it has to find it
+    again (and small frames no longer run over it)."""
+    cam = orc.make_camera([0.0, 0.0, -3.0], [0.0, 0.0, 0.0], [0.0, -1.0, 0.0], W, H)
+    large, small = crowd(8000, 15, -0.5), crowd(500, 16, -3.0)
+
+    def show(g):
+        eng.uploadRecords(g, 3)
+        return frame(eng, orc, g, cam)
+
+    assert show(large) == (1, 1) and show(large) == (1, 0)
+    for _ in range(3):
+        assert show(small) == (1, 0) and show(large) == (1, 0)
+    eng.uploadRecords(small, 3)
+    for _ in range(40):
+        assert frame(eng, orc, small, cam) == (1, 0)
+    assert show(large) == (1, 1) and show(large) == (1, 0) and show(small) == (1, 0)

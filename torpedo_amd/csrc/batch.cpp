@@ -402,13 +402,13 @@ static BatchArgs forward_args(BatchState* b, bool keep_bwd) {
         a.hist_plan = sort_digit_plan(ishape, a.lo_bits);
         a.hist_desc0_words = ((b->nitems + ikeys - 1) / ikeys) << a.hist_bits;
         // and the pair sort's from the items' tile rectangles, when its passes fit the LDS histograms
-        const uint32_t pshape = pair_shape_of(b), pkeys = sort_shape_keys(pshape);
+        const uint32_t pshape = pair_shape_of(b);
         const DigitPlan plan = sort_digit_plan(pshape, tile_key_bits(b));
         if (b->cap && plan.passes <= kMaxCountedPairPasses) {
             a.pair_counts = b->ws.partials + kPairCountRow;
             a.pair_bits = sort_shape_bits(pshape);
             a.pair_plan = plan;
-            a.pair_desc0_words = ((b->cap + pkeys - 1) / pkeys) << a.pair_bits;
+            a.pair_part_keys = sort_shape_keys(pshape);
         }
     }
     a.keys = b->d_keys;

@@ -362,10 +362,14 @@ __global__ __launch_bounds__(kEmitThreads) void k_batch_emit(const BatchArgs a) 
     const uint32_t tid = threadIdx.x, wave = tid / kWave, lane = __lane_id();
     if (a.totals_known && a.counters[kCtrOverflow]) return;  // the frame is rendered again
     // the pair sort's counts come from the item kernel: its first pass's descriptors (which the
-    // item sort's last pass may have used) and the tickets are cleared here
-    for (uint32_t x = blockIdx.x * kEmitThreads + tid; x < a.pair_desc0_words; x += gridDim.x * kEmitThreads)
-        a.hist_desc0[x] = 0u;
-    if (a.pair_desc0_words && blockIdx.x == 0 && tid < kMaxPasses) a.hist_tickets[tid] = 0u;
+    // item sort's last pass may have used) and the tickets are cleared here, for the pairs where their
+    // number is known, else for the room
+    if (a.pair_part_keys) {
+        const uint32_t pairs = a.totals_known ? a.counters[kCtrSortPairs] : a.cap;
+        const uint32_t words = ((pairs + a.pair_part_keys - 1) / a.pair_part_keys) << a.pair_bits;
+        for (uint32_t x = blockIdx.x * kEmitThreads + tid; x < words; x += gridDim.x * kEmitThreads) a.hist_desc0[x] = 0u;
+        if (blockIdx.x == 0 && tid < kMaxPasses) a.hist_tickets[tid] = 0u;
+    }
     // The sorted items are the visible ones (the item sort dropped the culled).  The grid is sized
     // for all items; the blocks past the visible items' partitions leave before taking a ticket
     // (the tickets, one atomic each on one address, pace the blocks' starts), so that exactly the

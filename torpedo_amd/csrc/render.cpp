@@ -21,6 +21,8 @@ namespace tpd {
 // moves in and out by turns, 957 -> 780 us for two frames.
 constexpr uint32_t kDepthHold = 64;
 
+constexpr size_t kMinPairRoom = 1u << 20;
+
 // The arguments shared by the frame's item kernel, its emission and the item offsets.
 static BatchArgs item_args(tpd_ctx* c) {
     BatchArgs a{};
@@ -72,15 +74,27 @@ struct FrameIssue {
     uint32_t gx, gy, ntiles, lo_bits, key_bits, ishape, pshape;
 };
 
-// The pair buffers as they are, for all that follows the item sort.  The pair sort's shape stays the one
-// the pairs' digits were counted for.
-static void set_pair_room(tpd_ctx* c, FrameIssue& q) {
+// The room for pairs that a frame is issued with: what recent frames of the context needed and a quarter
+// more, four pairs a Gaussian at least.  The grids of all that follows the item sort cover it and the
+// emission's partitions are chosen by it, so that a small frame does not pay for a large one long ago
+// (4k Gaussians at 256x144 after a frame of 17M pairs: 120 us with the buffers' whole room, 97 as without
+// that frame).  The buffers keep the room of the largest frame: where a frame needs more than it was given,
+// its pairs are issued once more (18 us).
+static uint32_t pair_room(const tpd_ctx* c) {
+    const size_t recent = (size_t)c->recent_pairs + c->recent_pairs / 4u;
+    const size_t room = std::max(std::max<size_t>(4 * (size_t)c->n, kMinPairRoom), recent);
+    return (uint32_t)std::min(std::min(room, c->cap_keys), (size_t)kMaxSortKeys);
+}
+
+// `room` pairs of the pair buffers as they are, for all that follows the item sort.  The pair sort's shape
+// stays the one the pairs' digits were counted for.
+static void set_pair_room(tpd_ctx* c, FrameIssue& q, uint32_t room) {
     BatchArgs& a = q.f.b;
-    a.cap = (uint32_t)std::min<size_t>(c->cap_keys, kMaxSortKeys);
+    a.cap = room;
     a.keys = c->d_keys;
     a.vals = c->d_vals;
     a.hist_desc0 = c->ws.desc;
-    a.pair_desc0_words = ((a.cap + sort_shape_keys(q.pshape) - 1) / sort_shape_keys(q.pshape)) << a.pair_bits;
+    a.pair_part_keys = sort_shape_keys(q.pshape);
 }
 
 static FrameIssue plan_frame(tpd_ctx* c, uint32_t gx, uint32_t gy) {
@@ -91,8 +105,8 @@ static FrameIssue plan_frame(tpd_ctx* c, uint32_t gx, uint32_t gy) {
     q.lo_bits = c->wide_frames ? kDepthWideBits : kDepthWindowBits;
     q.key_bits = bit_length(q.ntiles > 1 ? q.ntiles - 1 : 1);
     q.ishape = sort_shape_for(c->item_shape, c->n, q.lo_bits, 8);
-    q.pshape = sort_shape_for(c->ws.shape, expected_pairs(c->n, (uint32_t)std::min<size_t>(c->cap_keys, kMaxSortKeys)),
-                              q.key_bits, 4);
+    const uint32_t room = pair_room(c);
+    q.pshape = sort_shape_for(c->ws.shape, expected_pairs(c->n, room), q.key_bits, 4);
     FrameArgs& f = q.f;
     f.b = item_args(c);
     BatchArgs& a = f.b;
@@ -117,7 +131,7 @@ static FrameIssue plan_frame(tpd_ctx* c, uint32_t gx, uint32_t gy) {
     f.gx = gx;
     f.gy = gy;
     f.offset_parts = item_offset_parts(c->n);
-    set_pair_room(c, q);
+    set_pair_room(c, q, room);
     return q;
 }
 
@@ -207,7 +221,7 @@ int render_forward(tpd_ctx* c, hipStream_t s) {
         return TPD_OK;
     }
 
-    if (c->cap_keys == 0 && (rc = ensure_pair_buffers(c, std::max<size_t>(4 * (size_t)c->n, 1u << 20), s)) != TPD_OK)
+    if (c->cap_keys == 0 && (rc = ensure_pair_buffers(c, std::max<size_t>(4 * (size_t)c->n, kMinPairRoom), s)) != TPD_OK)
         return rc;
     if ((rc = ensure_sort_workspace(c, std::max<size_t>(c->n, c->cap_keys), s)) != TPD_OK) return rc;
 
@@ -219,6 +233,7 @@ int render_forward(tpd_ctx* c, hipStream_t s) {
         P = c->h_counters[kHostPairs];
         const bool depth_out = c->h_counters[kHostDepthOut] != 0, was_wide = c->wide_frames != 0;
         if (P > kMaxSortKeys) return fail(TPD_ERR_CAPACITY, "tpd_render: more than 2^30 - 1 tile/Gaussian pairs");
+        c->recent_pairs = std::max(P, c->recent_pairs - c->recent_pairs / 8u);
         if (P > c->cap_keys && (rc = ensure_pair_buffers(c, P, s)) != TPD_OK) return rc;
         if (depth_out) {
             c->wide_frames = kDepthHold;
@@ -228,7 +243,7 @@ int render_forward(tpd_ctx* c, hipStream_t s) {
         }
         if (c->h_counters[kHostOverflow]) {  // the Gaussians are in order: their pairs once more, with room
             ++c->resumes;
-            set_pair_room(c, q);
+            set_pair_room(c, q, pair_room(c));
             launch_frame_resume(c->d_counters, s);
             if ((rc = issue_pairs(c, q, s)) != TPD_OK) return rc;
         }

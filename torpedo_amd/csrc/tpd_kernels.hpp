@@ -200,9 +200,9 @@ struct BatchArgs {
     // the pair sort's digit histograms, counted by the item kernel from each visible item's tile
     // rectangle (needs hist_counts): counts from row kPairCountRow of the sort's digit counts, digit
     // width and passes of the pair sort's shape; the emission clears the pair sort's first-pass
-    // descriptors (pair_desc0_words, for the pair capacity) and the tickets
+    // descriptors (a partition has pair_part_keys pairs, 0: none to clear) and the tickets
     uint32_t* pair_counts;
-    uint32_t pair_bits, pair_desc0_words;
+    uint32_t pair_bits, pair_part_keys;
     DigitPlan pair_plan;
     uint32_t totals_known;          // the emission finds P and the overflow flag in the counters (plain frame)
     const uint32_t* kept_items;     // emission input: the number of sorted items (the visible ones) ...
