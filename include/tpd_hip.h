@@ -190,10 +190,11 @@ int tpd_sort_pairs_noalloc(tpd_ctx* ctx, uint64_t* d_keys, uint32_t* d_vals, uin
  * Times every radix-pass block shape on frames of the last rendered scene and camera and keeps the
  * fastest for each of the two sorts (results are identical for every shape).  sort_ms[0..capacity)
  * receives the median time of both sorts per shape; *n_shapes the number of shapes; *best the pair
- * sort's.  Re-renders the frame. */
+ * sort's.  Re-renders the frame.  The stand-alone sorts' shapes stay as they are. */
 int tpd_autotune(tpd_ctx* ctx, float* sort_ms, uint32_t capacity, uint32_t* n_shapes, uint32_t* best);
 /* Selects a radix-pass block shape by index for the plain and the batched frame and the stand-alone
- * sorts; until then, or until an autotune, each sort's shape follows from its key count and width. */
+ * sorts; until then, or for a frame's sorts an autotune, each sort's shape follows from its key count and
+ * width. */
 int tpd_set_sort_shape(tpd_ctx* ctx, uint32_t shape);
 
 /* ----- batched rendering -------------------------------------------------------------------------

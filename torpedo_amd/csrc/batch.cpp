@@ -150,7 +150,7 @@ void batch_release(tpd_ctx* c) {
 static BatchState* state(tpd_ctx* c) {
     if (!c->batch) {
         c->batch = new BatchState();
-        c->batch->ws.shape = c->ws.shape;  // the context's radix block shape until tuned separately
+        c->batch->ws.shape = c->pair_shape;  // the plain frame's radix block shapes until tuned separately
         c->batch->item_shape = c->item_shape;
     }
     return c->batch;

@@ -106,7 +106,7 @@ static FrameIssue plan_frame(tpd_ctx* c, uint32_t gx, uint32_t gy) {
     q.key_bits = bit_length(q.ntiles > 1 ? q.ntiles - 1 : 1);
     q.ishape = sort_shape_for(c->item_shape, c->n, q.lo_bits, 8);
     const uint32_t room = pair_room(c);
-    q.pshape = sort_shape_for(c->ws.shape, expected_pairs(c->n, room), q.key_bits, 4);
+    q.pshape = sort_shape_for(c->pair_shape, expected_pairs(c->n, room), q.key_bits, 4);
     FrameArgs& f = q.f;
     f.b = item_args(c);
     BatchArgs& a = f.b;

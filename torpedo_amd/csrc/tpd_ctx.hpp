@@ -58,8 +58,8 @@ struct tpd_ctx {
     uint64_t* d_keys_dbg = nullptr; size_t cap_keys_dbg = 0;
     uint32_t* d_vals_dbg = nullptr; size_t cap_vals_dbg = 0;
     uint64_t* d_full_keys = nullptr; size_t cap_full_keys = 0;  // 64-bit keys rebuilt for readers
-    tpd::SortWorkspace ws;                       // shared by both sorts; ws.shape: that of the pair sort
-    uint32_t item_shape = tpd::kShapeAuto;
+    tpd::SortWorkspace ws;  // shared by the frame's sorts and the stand-alone one; ws.shape: the latter's
+    uint32_t item_shape = tpd::kShapeAuto, pair_shape = tpd::kShapeAuto;  // of the frame's sorts
     const uint32_t* sorted_keys = nullptr;
     const uint32_t* sorted_vals = nullptr;
     uint32_t wide_frames = 0;   // frames still to be sorted on the wide depth key (kDepthHold, render.cpp)

@@ -13,14 +13,14 @@ extern "C" {
 int tpd_set_sort_shape(tpd_ctx* c, uint32_t shape) {
     if (!c) return fail(TPD_ERR_INVALID, "null context");
     if (shape >= sort_num_shapes()) return fail(TPD_ERR_INVALID, "tpd_set_sort_shape: no such shape");
-    c->ws.shape = shape;
-    c->item_shape = shape;
+    c->ws.shape = c->item_shape = c->pair_shape = shape;
     batch_set_sort_shape(c, shape);
     return TPD_OK;
 }
 
 // Times both sorts (items by depth, pairs by tile) of whole frames per shape and keeps the fastest
-// shape for each; sort_ms[shape] = both sorts' time, *best = the pair sort's shape.
+// shape for each; sort_ms[shape] = both sorts' time, *best = the pair sort's shape.  The stand-alone sorts,
+// of other keys and key counts, keep their own (200k 43-bit keys 84 us; with a frame's best 106).
 int tpd_autotune(tpd_ctx* c, float* sort_ms, uint32_t capacity, uint32_t* n_shapes, uint32_t* best) {
     if (!c) return fail(TPD_ERR_INVALID, "null context");
     hipSetDevice(c->device);
@@ -29,12 +29,12 @@ int tpd_autotune(tpd_ctx* c, float* sort_ms, uint32_t capacity, uint32_t* n_shap
     if (!c->rendered || c->n == 0 || c->last_pairs == 0)
         return fail(TPD_ERR_STATE, "tpd_autotune: render a non-empty frame first");
     hipStream_t s = c->stream;
-    const uint32_t keep_items = c->item_shape, keep_pairs = c->ws.shape;
+    const uint32_t keep_items = c->item_shape, keep_pairs = c->pair_shape;
     const bool keep_profile = c->profile;
     int rc = tpd_set_profiling(c, 1);
     std::vector<float> med(ns, 0.0f), items(ns, 0.0f), pairs(ns, 0.0f);
     for (uint32_t sh = 0; sh < ns && rc == TPD_OK; ++sh) {
-        c->item_shape = c->ws.shape = sh;
+        c->item_shape = c->pair_shape = sh;
         std::vector<float> ti, tp, t;
         for (int rep = 0; rep < 4 && rc == TPD_OK; ++rep) {
             if ((rc = render_forward(c, s)) != TPD_OK) break;
@@ -62,7 +62,7 @@ int tpd_autotune(tpd_ctx* c, float* sort_ms, uint32_t capacity, uint32_t* n_shap
     c->profile = keep_profile;
     if (rc != TPD_OK) {
         c->item_shape = keep_items;
-        c->ws.shape = keep_pairs;
+        c->pair_shape = keep_pairs;
         return rc;
     }
     uint32_t bi = 0, bp = 0;
@@ -71,7 +71,7 @@ int tpd_autotune(tpd_ctx* c, float* sort_ms, uint32_t capacity, uint32_t* n_shap
         if (pairs[sh] < pairs[bp]) bp = sh;
     }
     c->item_shape = bi;
-    c->ws.shape = bp;
+    c->pair_shape = bp;
     if (best) *best = bp;
     if (sort_ms)
         for (uint32_t sh = 0; sh < ns && sh < capacity; ++sh) sort_ms[sh] = med[sh];
