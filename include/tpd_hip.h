@@ -196,6 +196,8 @@ int tpd_autotune(tpd_ctx* ctx, float* sort_ms, uint32_t capacity, uint32_t* n_sh
  * sorts; until then, or for a frame's sorts an autotune, each sort's shape follows from its key count and
  * width. */
 int tpd_set_sort_shape(tpd_ctx* ctx, uint32_t shape);
+/* Back to shapes chosen by key count and width, for every sort, whatever was selected or tuned. */
+int tpd_reset_sort_shape(tpd_ctx* ctx);
 
 /* ----- batched rendering -------------------------------------------------------------------------
  * The reference renders one camera of one compiled scene per GaussianEngine::rasterFrame

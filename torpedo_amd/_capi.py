@@ -79,6 +79,7 @@ SIGNATURES = {
     "tpd_sort_pairs_noalloc": (_i32, [_vp, _vp, _vp, _vp, _vp, _u32, _u32, _vp, ctypes.POINTER(_i32)]),
     "tpd_autotune": (_i32, [_vp, _vp, _u32, ctypes.POINTER(_u32), ctypes.POINTER(_u32)]),
     "tpd_set_sort_shape": (_i32, [_vp, _u32]),
+    "tpd_reset_sort_shape": (_i32, [_vp]),
     "tpd_scene_add": (_i32, [_vp, _vp, _u32, _vp, _vp, _u32, _u32, ctypes.POINTER(_u32)]),
     "tpd_scene_add_device": (_i32, [_vp, _vp, _u32, _u32, ctypes.POINTER(_u32)]),
     "tpd_scene_set_transform": (_i32, [_vp, _u32, _u32, _vp]),

@@ -10,11 +10,21 @@ using namespace tpd;
 
 extern "C" {
 
+static void set_shapes(tpd_ctx* c, uint32_t shape) {
+    c->ws.shape = c->item_shape = c->pair_shape = shape;
+    batch_set_sort_shape(c, shape);
+}
+
 int tpd_set_sort_shape(tpd_ctx* c, uint32_t shape) {
     if (!c) return fail(TPD_ERR_INVALID, "null context");
     if (shape >= sort_num_shapes()) return fail(TPD_ERR_INVALID, "tpd_set_sort_shape: no such shape");
-    c->ws.shape = c->item_shape = c->pair_shape = shape;
-    batch_set_sort_shape(c, shape);
+    set_shapes(c, shape);
+    return TPD_OK;
+}
+
+int tpd_reset_sort_shape(tpd_ctx* c) {
+    if (!c) return fail(TPD_ERR_INVALID, "null context");
+    set_shapes(c, kShapeAuto);
     return TPD_OK;
 }
 

@@ -444,6 +444,10 @@ class GaussianEngine:
     def setSortShape(self, shape: int):
         check(lib().tpd_set_sort_shape(self._ctx, int(shape)))
 
+    def resetSortShape(self):
+        """Every sort's shape follows from its key count and width again (tpd_reset_sort_shape)."""
+        check(lib().tpd_reset_sort_shape(self._ctx))
+
     def setProfiling(self, enable: bool = True):
         check(lib().tpd_set_profiling(self._ctx, 1 if enable else 0))
 
