@@ -126,3 +126,27 @@ def test_room_follows_recent_frames(orc, eng):
     for _ in range(40):
         assert frame(eng, orc, small, cam) == (1, 0)
     assert show(large) == (1, 1) and show(large) == (1, 0) and show(small) == (1, 0)
+
+
+@pytest.mark.parametrize("n,scale", [(8_000, -0.5), (40_000, -0.5), (9_000, -1.7)])
+def test_first_batch_over_the_room(orc, n, scale):
+    """A batch's first frame with many times the pairs its buffers hold, blocks of it all past their end:
+    each view's pairs and image are the plain frame's."""
+    from torpedo_amd.engine import GaussianEngine, Settings
+    g = small_scene(n, seed=n, log_scale_mean=scale)
+    cams = [orc.make_camera([x, 0.0, -3.0], [0.0, 0.0, 0.0], [0.0, -1.0, 0.0], W, H) for x in (0.0, 0.4)]
+    with GaussianEngine() as eng, GaussianEngine() as plain:
+        sid = eng.addScene(g, Settings(3))
+        eng.setViews([(sid, c.view, c.proj_view, c.focal_ndc, c.width, c.height) for c in cams])
+        eng.rasterBatch()
+        keys, vals = eng.readBatchPairs()
+        plain.uploadRecords(g, 3)
+        for v, c in enumerate(cams):
+            plain.setCamera(c.view, c.proj_view, c.focal_ndc, c.width, c.height)
+            plain.render()
+            tile0, item0, _ = eng.batchViewLayout(v)
+            pk, pv = plain.readPairs()
+            mine = (vals >= item0) & (vals < item0 + n)
+            assert np.array_equal(vals[mine] - item0, pv)
+            assert np.array_equal(keys[mine] - (np.uint64(tile0) << np.uint64(32)), pk)
+            assert np.array_equal(eng.readBatchImage(v), plain.readImage())

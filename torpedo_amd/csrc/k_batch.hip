@@ -465,6 +465,7 @@ __global__ __launch_bounds__(kEmitThreads) void k_batch_emit(const BatchArgs a) 
     const uint64_t pos0 = base - lead;
     uint32_t carry = 0;  // 1 + the last item whose pairs began before this round
     for (uint32_t c0 = 0; c0 < end; c0 += kEmitChunk) {
+        if (pos0 + c0 >= a.cap) break;  // a batch without room: nothing that is left is stored
 #pragma unroll
         for (uint32_t j = 0; j < PT; ++j) {
             const uint32_t p = lead + rec[j].x - c0;  // wraps below c0: then not < kEmitChunk
