@@ -129,7 +129,7 @@ int tpd_backward(tpd_ctx* ctx, const float* d_dL_dimage, float* d_grad_means, fl
 /* Per-splat screen-space gradients of the last backward (N x 9 floats: image x, y, conic a, b, c,
  * colour r, g, b, opacity), for tests. */
 int tpd_read_splat_grads(tpd_ctx* ctx, float* g2d);
-/* Profiled backward: ms[0] splat-gradient pass, ms[1] parameter-gradient pass, ms[2] span from the
+/* Profiled backward: ms[0] splat-gradient pass (with the scan of the tile counts), ms[1] parameter-gradient pass, ms[2] span from the
  * start of the last profiled tpd_render to the end of this backward. */
 int tpd_get_backward_times(tpd_ctx* ctx, float* ms);
 
@@ -280,7 +280,8 @@ int tpd_batch_read_pairs(tpd_ctx* ctx, uint64_t* keys, uint32_t* vals, uint32_t 
  * (both sorts). */
 int tpd_batch_get_times(tpd_ctx* ctx, float* ms, uint32_t* passes);
 /* The last eager profiled forward frame's two sorts (items by depth, then pairs by tile): ms[4] =
- * item histogram, item radix passes, pair histogram, pair radix passes (milliseconds); counts[4]
+ * digit offsets (of both sorts where the item kernel counted the pairs' digits), item radix passes, pair
+ * histogram (0 where it did), pair radix passes (milliseconds); counts[4]
  * = items, item passes, pairs, pair passes. */
 int tpd_batch_get_sort_times(tpd_ctx* ctx, float* ms, uint32_t* counts);
 /* tpd_get_blend_evaluations for the last batch frame: the pixel-splat pairs whose power its blend

@@ -57,13 +57,13 @@ extern "C" int tpd_backward(tpd_ctx* c, const float* d_dL_dimage, float* d_grad_
         b->cap_partials = want;
     }
     if (c->n == 0) return TPD_OK;
-    const int rc = launch_offsets(c, s);
-    if (rc != TPD_OK) return rc;
     if (c->profile) {
         for (auto& ev : b->ev)
             if (!ev && (e = hipEventCreate(&ev)) != hipSuccess) return hip_fail(e, "hipEventCreate");
         hipEventRecord(b->ev[0], s);
     }
+    const int rc = launch_offsets(c, s);
+    if (rc != TPD_OK) return rc;
     const uint32_t W = c->cam.width, H = c->cam.height;
     const uint32_t gx = (W + kTile - 1) / kTile, gy = (H + kTile - 1) / kTile;
     if (c->last_pairs > 0) {
@@ -111,7 +111,7 @@ extern "C" int tpd_backward(tpd_ctx* c, const float* d_dL_dimage, float* d_grad_
     return e == hipSuccess ? TPD_OK : hip_fail(e, "backward launch");
 }
 
-// ms[0] = splat-gradient pass (blend backward, incl. clearing), ms[1] = parameter-gradient pass
+// ms[0] = splat-gradient pass (item offsets and blend backward), ms[1] = parameter-gradient pass
 // (preprocess backward), ms[2] = forward start -> backward end of the last profiled frame.
 extern "C" int tpd_get_backward_times(tpd_ctx* c, float* ms) {
     if (!c || !ms) return fail(TPD_ERR_INVALID, "tpd_get_backward_times: bad argument");

@@ -106,6 +106,7 @@ struct BatchState {
     bool rendered = false;      // last frame validated
     bool kept_bwd_state = false;
     uint32_t last_pairs = 0;
+    bool pairs_counted = false;  // the recorded frame's item kernel counts the pairs' digits
     uint32_t last_kept = 0;      // the last frame's items kept by its item sort (the visible ones)
     hipEvent_t ev[11] = {};  // eager stage events [0..6], frame bracket [7], [8], after each sort's histogram [9], [10]
     bool timed = false;
@@ -467,11 +468,12 @@ static void record_forward(BatchState* b, bool keep_bwd, hipStream_t s, bool eve
     a.sorted_keys64 = items_alt ? b->d_ikeys_alt : b->d_ikeys;
     launch_batch_emit(a, s);
     if (events) hipEventRecord(b->ev[3], s);
-    if (events) hipEventRecord(b->ev[10], s);
     // kCtrSortPairs is P, or 0 after an overflow: the counted digits then cover pairs that were
     // never written, and the sort and the ranges must not run on them
     const bool in_alt = launch_sort_pairs32(b->ws, pshape, b->d_keys, b->d_vals, b->d_keys_alt, b->d_vals_alt,
-                                            &b->d_counters[kCtrSortPairs], b->cap, key_bits, s, a.pair_counts != nullptr);
+                                            &b->d_counters[kCtrSortPairs], b->cap, key_bits, s, a.pair_counts != nullptr,
+                                            events && !a.pair_counts ? b->ev[10] : nullptr);
+    b->pairs_counted = a.pair_counts != nullptr;
     b->sorted_keys = in_alt ? b->d_keys_alt : b->d_keys;
     b->sorted_vals = in_alt ? b->d_vals_alt : b->d_vals;
     if (events) hipEventRecord(b->ev[4], s);
@@ -962,8 +964,9 @@ int tpd_batch_get_times(tpd_ctx* c, float* ms, uint32_t* passes) {
     return e == hipSuccess ? TPD_OK : hip_fail(e, "tpd_batch_get_times");
 }
 
-// The last eager profiled forward frame's two sorts: ms = {item histogram, item radix passes, pair
-// histogram, pair radix passes}; counts = {items, item passes, pairs, pair passes}.
+// The last eager profiled forward frame's two sorts: ms = {digit offsets (of both where the item kernel
+// counted the pairs' digits), item radix passes, pair histogram (0 where it did), pair radix passes};
+// counts = {items, item passes, pairs, pair passes}.
 int tpd_batch_get_sort_times(tpd_ctx* c, float* ms, uint32_t* counts) {
     if (!c || !ms) return fail(TPD_ERR_INVALID, "tpd_batch_get_sort_times: bad argument");
     hipSetDevice(c->device);
@@ -973,8 +976,9 @@ int tpd_batch_get_sort_times(tpd_ctx* c, float* ms, uint32_t* counts) {
     hipError_t e = hipEventSynchronize(b->ev[8]);
     if (e == hipSuccess) e = hipEventElapsedTime(&ms[0], b->ev[1], b->ev[9]);
     if (e == hipSuccess) e = hipEventElapsedTime(&ms[1], b->ev[9], b->ev[2]);
-    if (e == hipSuccess) e = hipEventElapsedTime(&ms[2], b->ev[3], b->ev[10]);
-    if (e == hipSuccess) e = hipEventElapsedTime(&ms[3], b->ev[10], b->ev[4]);
+    ms[2] = 0.0f;
+    if (e == hipSuccess && !b->pairs_counted) e = hipEventElapsedTime(&ms[2], b->ev[3], b->ev[10]);
+    if (e == hipSuccess) e = hipEventElapsedTime(&ms[3], b->ev[b->pairs_counted ? 3 : 10], b->ev[4]);
     if (counts) {
         counts[0] = b->nitems;
         counts[1] = b->item_passes;

@@ -586,10 +586,12 @@ bool launch_sort_items(SortWorkspace& ws, uint32_t shape, uint64_t* keys, uint32
 
 bool launch_sort_pairs32(SortWorkspace& ws, uint32_t shape, uint32_t* keys, uint32_t* vals, uint32_t* keys_alt,
                          uint32_t* vals_alt, const uint32_t* count_ptr, uint32_t n_max, uint32_t key_bits, hipStream_t s,
-                         bool counted) {
+                         bool counted, hipEvent_t after_count) {
     const DigitPlan plan = sort_digit_plan(shape, key_bits);
-    if (n_max == 0 || plan.passes == 0 || plan.passes > kMaxPasses) return false;
-    if (!counted) launch_count(ws, shape, plan, (const uint32_t*)keys, count_ptr, n_max, s);
+    const bool run = n_max != 0 && plan.passes != 0 && plan.passes <= kMaxPasses;
+    if (run && !counted) launch_count(ws, shape, plan, (const uint32_t*)keys, count_ptr, n_max, s);
+    if (after_count) hipEventRecord(after_count, s);
+    if (!run) return false;
     return launch_passes(ws, shape, plan, ws.offsets + (counted ? kPairCountRow : 0u), keys, vals, keys_alt, vals_alt,
                          count_ptr, n_max, nullptr, s);
 }

@@ -348,9 +348,9 @@ bool launch_sort_items(SortWorkspace& ws, uint32_t shape, uint64_t* keys, uint32
                        uint32_t* vals_alt, uint32_t n, uint32_t lo_bits, const uint32_t* kept, hipStream_t s,
                        const uint32_t* count_ptr = nullptr);
 // Sorts the min(*count_ptr, n_max) pairs by the low key_bits bits of their 32-bit keys; without
-// counted, their digits are counted first.
+// counted, their digits are counted first (after_count: recorded then).
 bool launch_sort_pairs32(SortWorkspace& ws, uint32_t shape, uint32_t* keys, uint32_t* vals, uint32_t* keys_alt,
                          uint32_t* vals_alt, const uint32_t* count_ptr, uint32_t n_max, uint32_t key_bits, hipStream_t s,
-                         bool counted);
+                         bool counted, hipEvent_t after_count = nullptr);
 
 }  // namespace tpd
