@@ -87,13 +87,23 @@ def sort_keys_per_s(P, stage_ms):
     return P / t if t > 0 else 0.0
 
 
-def plain_sort_gbs(P, stage_ms, w, h, digit_bits=9):
-    """The sort metric of a plain frame: 24 B x P x ceil(K / d) over the time to order the pairs by (tile,
-    depth), i.e. both sorts' passes (the Gaussians by depth, their pairs by tile) and digit offsets;
-    K = tile bits + 27 depth bits, d the widest digit of the passes."""
-    t = (stage_ms["sort_histogram"] + stage_ms["sort_passes"]) / 1000.0
-    k = int(np.ceil(np.log2(max(((w + 15) // 16) * ((h + 15) // 16), 2)))) + 27
-    return 24.0 * P * ((k + digit_bits - 1) // digit_bits) / t / 1e9 if t > 0 else 0.0
+def plain_sort_gbs(P, stage_ms, w, h, pair_shape):
+    """GB/s of a plain frame's radix passes: the bytes they read and write over their time.  The Gaussians'
+    first pass reads 8 B of each and writes 12 B of the visible ones, its later ones read and write 12 B of
+    those; each pass of the pairs reads and writes 8 B a pair."""
+    t = stage_ms["sort_passes"] / 1000.0
+    tile_bits = max(((w + 15) // 16) * ((h + 15) // 16) - 1, 1).bit_length()
+    digit = SORT_SHAPES[pair_shape][0]
+    pair_passes = (tile_bits + digit - 1) // digit
+    item_passes = int(stage_ms["radix_passes"]) - pair_passes
+    kept = stage_ms["items_kept"]
+    moved = 8.0 * stage_ms["items"] + (12.0 + 24.0 * (item_passes - 1)) * kept + 16.0 * P * pair_passes
+    return moved / t / 1e9 if t > 0 else 0.0
+
+
+def plain_pair_shape(stage_ms, fixed):
+    """The radix-pass block shape of a plain frame's pair sort: the tuned one, or the one given."""
+    return stage_ms["autotune"]["best_shape"] if "autotune" in stage_ms else fixed
 
 
 def time_multiview(eng, g, steps, warmup, tune=True):
@@ -192,6 +202,8 @@ def time_plain(eng, g, eye, w, h, steps, warmup, tune=False):
     P = eng.pairCount
     out = {k: med([s[k] for s in stages]) for k in stages[0]}
     out["blend_evaluations"] = eng.blendEvaluations()  # the last frame, blended once more, not timed
+    tiles = eng.readTiles()[0]
+    out["items"], out["items_kept"] = int(tiles.size), int(np.count_nonzero(tiles))
     if tuned is not None:
         out["autotune"] = tuned
     return dt, P, out
@@ -466,7 +478,7 @@ def main():
     if args.only == "sort-load":
         g2 = scenes.cluster_scene(1_000_000, seed=2, log_scale_mean=-3.0)
         dt2, P2, st2 = time_plain(eng, g2, eye, W, H, args.steps, args.warmup, tune=tune)
-        ach = plain_sort_gbs(P2, st2, W, H)
+        ach = plain_sort_gbs(P2, st2, W, H, plain_pair_shape(st2, args.sort_shape))
         copy_gbs = eng.measureCopy(256 << 20, 3)  # a plain copy of 256 MiB for counter calibration
         print(json.dumps({"workload": "clusters-1M-1920x1080 log-scale mean -3", "pairs": P2, "stage_ms": st2,
                           "sort_gbs": round(ach, 1),
@@ -570,7 +582,7 @@ def main():
     sort_metric = 24.0 * mv["pairs"] * ((K + d - 1) // d) / t_sort / 1e9 if t_sort > 0 else 0.0
     roofline["sort_ms"] = round(t_sort * 1000.0, 4)
     roofline["sort_gkeys_per_s"] = round(mv["pairs"] / t_sort / 1e9, 3) if t_sort > 0 else 0.0
-    ach2, ach1 = plain_sort_gbs(P2, st2, W, H), plain_sort_gbs(P, st, W, H)
+    ach2, ach1 = (plain_sort_gbs(p, s, W, H, plain_pair_shape(s, args.sort_shape)) for p, s in ((P2, st2), (P, st)))
 
     log("[bench] forward + backward, 3M Gaussians 1920x1080")
     fb = time_fwd_bwd(eng, max(5, args.steps // 2), 2)
@@ -618,14 +630,15 @@ def main():
         "multiview_32": mv,
         "plain_1080p": {"ms_per_frame": round(ms_plain, 4), "views_per_s": round(1000.0 / ms_plain, 2), "pairs": P,
                         "stage_ms": {k: round(v, 4) for k, v in st.items()
-                                     if k not in ("radix_passes", "autotune", "blend_evaluations")},
+                                     if k not in ("radix_passes", "autotune", "blend_evaluations", "items", "items_kept")},
                         "autotune": st.get("autotune")},
         "sort_hbm_frac": {"multiview_32": round(sort_metric / HBM_PEAK_GBS, 4), "pairs_multiview_32": mv["pairs"],
                           "multiview_32_key_bits": K,
                           "sort_load_variant": round(ach2 / HBM_PEAK_GBS, 4), "pairs_sort_load": P2,
                           "plain_1080p": round(ach1 / HBM_PEAK_GBS, 4), "pairs_plain_1080p": P,
-                          "metric": "24 B x pairs x ceil(K / d) over both sorts' time: the bytes of a sort of the "
-                                    "pairs by their whole key; Gaussians sorted by depth first move fewer",
+                          "metric": "multiview_32: 24 B x pairs x ceil(K / d) over both sorts' time, the bytes of a sort "
+                                    "of the pairs by their whole key (roofline: of the bytes moved); sort_load_variant, "
+                                    "plain_1080p: bytes read and written by both sorts' passes over the passes' time",
                           "gkeys_per_s": {"multiview_32": roofline["sort_gkeys_per_s"],
                                           "sort_load_variant": round(sort_keys_per_s(P2, st2) / 1e9, 3),
                                           "plain_1080p": round(sort_keys_per_s(P, st) / 1e9, 3)}},
