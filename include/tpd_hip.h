@@ -123,7 +123,7 @@ int tpd_write_png(const uint8_t* rgba, uint32_t width, uint32_t height, const ch
  * opacity logits (N, opacity = sigmoid(logit) as in GaussianGeometry.cpp:112) and SH (N x 48).
  * d_dL_dimage is the upstream gradient of the FP32 image (H x W x 3, device).  All gradient
  * pointers are device memory; with accumulate != 0 the results are added to their contents.
- * The per-pixel transmittance is recomputed, not stored by the forward. */
+ * It starts from the per-pixel final transmittance and last contributor that the frame stored. */
 int tpd_backward(tpd_ctx* ctx, const float* d_dL_dimage, float* d_grad_means, float* d_grad_log_scales,
                  float* d_grad_quats, float* d_grad_opacity_logits, float* d_grad_sh, int accumulate, void* stream);
 /* Per-splat screen-space gradients of the last backward (N x 9 floats: image x, y, conic a, b, c,

@@ -6,8 +6,8 @@ Parameters are CUDA (HIP) float tensors in the training parameterisation: means 
 log-scales (N, 3), quaternions (N, 4, xyzw, fed unnormalised as volume.slang:28-35 does),
 opacity logits (N,), SH (N, 48).  They are packed into the 60-float GaussianPoint records
 (GaussianGeometry.h:10-30: opacity = sigmoid(logit), scale = exp(log-scale), modifier 1) on the
-device, rendered by tpd_render, and differentiated by tpd_backward, which recomputes the per-pixel
-transmittance instead of storing it.  Returns the FP32 image (H, W, 3).
+device, rendered by tpd_render, and differentiated by tpd_backward, which starts from the per-pixel final
+transmittance that the frame stored.  Returns the FP32 image (H, W, 3).
 
 torch must be imported before the library is first loaded (torch carries its own HIP runtime and
 the library binds to it); importing this module does that.

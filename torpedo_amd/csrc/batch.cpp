@@ -479,8 +479,7 @@ static void record_forward(BatchState* b, bool keep_bwd, hipStream_t s, bool eve
     if (events) hipEventRecord(b->ev[4], s);
     // lo_bits tells the ranges kernel whether the items were sorted on the depth window
     launch_ranges(b->sorted_keys, b->d_counters, b->cap, b->d_ranges, b->d_scan_desc,
-                  emit_parts(b->nitems, b->cap) + item_offset_parts(b->nitems), &b->d_counters[kCtrScanTicket], s, b->cap,
-                  b->lo_bits());
+                  emit_parts(b->nitems, b->cap) + item_offset_parts(b->nitems), &b->d_counters[kCtrScanTicket], b->lo_bits(), s);
     launch_tile_order(b->d_ranges, b->ntiles, b->d_counters, b->d_tile_hist, b->d_jobs, 0, b->d_tile_view, b->d_views, s);
     if (events) hipEventRecord(b->ev[5], s);
     BatchBlendArgs ba = blend_args(b);

@@ -80,9 +80,9 @@ __global__ void k_ranges(const uint32_t* __restrict__ keys, uint32_t* __restrict
     }
 }
 
-void launch_ranges(const uint32_t* keys, uint32_t* counters, uint32_t P_hint, uint2* ranges, uint64_t* scan_desc,
-                   uint32_t n_scan_desc, uint32_t* ticket, hipStream_t s, uint32_t cap, uint32_t lo_bits) {
-    uint32_t work = (P_hint + kRangeRun - 1) / kRangeRun;
+void launch_ranges(const uint32_t* keys, uint32_t* counters, uint32_t cap, uint2* ranges, uint64_t* scan_desc,
+                   uint32_t n_scan_desc, uint32_t* ticket, uint32_t lo_bits, hipStream_t s) {
+    uint32_t work = (cap + kRangeRun - 1) / kRangeRun;
     work = work > n_scan_desc ? work : n_scan_desc;
     uint32_t nb = (work + 255) / 256;
     nb = nb < 1 ? 1 : (nb > 8192 ? 8192 : nb);

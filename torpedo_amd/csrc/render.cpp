@@ -169,7 +169,7 @@ static int issue_pairs(tpd_ctx* c, const FrameIssue& q, hipStream_t s) {
     c->sorted_vals = in_alt ? c->d_vals_alt : c->d_vals;
     c->last_passes = a.hist_plan.passes + a.pair_plan.passes;
     launch_ranges(c->sorted_keys, c->d_counters, a.cap, c->d_ranges, c->d_scan_desc,
-                  emit_parts(c->n, a.cap), &c->d_counters[kCtrScanTicket], s, a.cap, kDepthWideBits);
+                  emit_parts(c->n, a.cap), &c->d_counters[kCtrScanTicket], kDepthWideBits, s);
     launch_tile_order(c->d_ranges, q.ntiles, c->d_counters, c->d_tile_hist, c->d_jobs, q.gx, nullptr, nullptr, s);
     if (c->profile) hipEventRecord(c->ev[6], s);
     BlendArgs b{};

@@ -16,7 +16,6 @@ struct TileView {
     uint64_t pix_base;
 };
 
-constexpr uint32_t kQuad = 8;
 constexpr uint32_t kSub = 4;                              // 4x4-pixel sub-blocks ...
 constexpr uint32_t kSubBlocks = kTilePixels / (kSub * kSub);  // ... 16 per tile, one per 16-lane row
 constexpr uint32_t kSplatGrads = 9;  // dL/d(image x, y, conic a, b, c, r, g, b, opacity)

@@ -7,9 +7,10 @@ namespace tpd {
 
 // Indices into the per-context device counter block.
 enum : uint32_t {
-    kCtrScanTicket = 0,   // preprocess partition ticket
-    kCtrPairs = 1,        // pair count P written by the last preprocess partition
-    kCtrOverflow = 2,     // 1 when P exceeded the key/value capacity
+    kCtrScanTicket = 0,   // partition ticket of the emission
+    kCtrPairs = 1,        // pair count P: of the last emission partition, or in a plain frame of its totals
+    kCtrOverflow = 2,     // 1 when P exceeded the frame's room or a depth lay outside the window sorted on:
+                          // nothing that follows does anything
     kCtrDepthOut = 3,     // non-zero when an emitted depth lies outside the sort's depth window
     kCtrScanTicket2 = 4,  // partition ticket of a second scan in the frame (the item offsets), cleared by
                           // the item kernel
@@ -105,12 +106,12 @@ void launch_blend_bwd(const BackwardArgs& a, hipStream_t s);
 void launch_preprocess_bwd(const PreBackwardArgs& a, hipStream_t s);
 
 void launch_entity_mats(const float* models, uint32_t n_ent, const CameraParams& cam, EntityMats* out, hipStream_t s);
-// Tile ranges of the P = min(counters[count_slot], cap) sorted keys (tiles).  Also re-zeroes the scan
+// Tile ranges of the P = min(counters[kCtrSortPairs], cap) sorted keys (tiles).  Also re-zeroes the scan
 // descriptors and the emission's ticket for the next frame, and sets kCtrOverflow when a frame whose items
 // were sorted on the depth-window key (lo_bits = kDepthWindowBits) has kCtrDepthOut set, which it clears
 // otherwise.
-void launch_ranges(const uint32_t* keys, uint32_t* counters, uint32_t P_hint, uint2* ranges, uint64_t* scan_desc,
-                   uint32_t n_scan_desc, uint32_t* ticket, hipStream_t s, uint32_t cap, uint32_t lo_bits);
+void launch_ranges(const uint32_t* keys, uint32_t* counters, uint32_t cap, uint2* ranges, uint64_t* scan_desc,
+                   uint32_t n_scan_desc, uint32_t* ticket, uint32_t lo_bits, hipStream_t s);
 // The 64-bit keys (tile << 32) | floatbits(view depth) of n sorted tile keys, the depth from the splat
 // of each value (for readers of the sorted pairs).
 void launch_full_keys(const uint32_t* keys, const uint32_t* vals, const Splat* splats, uint32_t n, uint64_t* out,
@@ -186,7 +187,6 @@ struct BatchArgs {
     uint64_t* item_keys;          // per item: low word the depth key ((depth bits - lo_base) in lo_bits
                                   // bits, all ones within lo_bits when culled), high word the emission
                                   // record as inline_rect encodes it
-    uint32_t* item_vals;          // per item: the item itself (null when the item sort generates them)
     uint32_t lo_bits, lo_base;
     // the item sort's digit histograms, counted by the item kernel (the sort then skips its own):
     // counts as k_sort_hist leaves them (copy blockIdx mod kCountCopies), digit width and passes of
