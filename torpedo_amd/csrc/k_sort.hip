@@ -155,9 +155,10 @@ __global__ __launch_bounds__(256) void k_frame_offsets(uint32_t* __restrict__ co
     const uint32_t b = blockIdx.x;
     const bool items = b < ipasses;
     const uint32_t row = items ? b << ibits : kPairCountRow + ((b - ipasses) << pbits);
+    const uint32_t depth_out = counters[kCtrDepthOut];  // (loaded beside the counts)
     const uint32_t n = scan_digit_counts(counts + row, offsets + row, items ? ibits : pbits, s_w);
-    const bool depth_over = totals.host && totals.lo_bits == kDepthWindowBits && counters[kCtrDepthOut] != 0;
-    // (no item is sorted on a window that does not hold its depth: the frame is issued again)
+    // no item is sorted on a window that does not hold its depth: the frame is issued again
+    const bool depth_over = totals.host && totals.lo_bits == kDepthWindowBits && depth_out != 0;
     if (b == 0 && items && threadIdx.x == 255) {
         counters[kCtrItemsKept] = depth_over ? 0u : n;
         counters[kCtrSortItems] = depth_over ? 0u : totals.items;
@@ -167,7 +168,6 @@ __global__ __launch_bounds__(256) void k_frame_offsets(uint32_t* __restrict__ co
         uint64_t* const t64 = reinterpret_cast<uint64_t*>(counters + kCtrTotal64);
         const uint64_t total = *t64;
         const uint32_t P = total > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)total;
-        const uint32_t depth_out = counters[kCtrDepthOut];
         const bool over = total > totals.cap || depth_over;
         *t64 = 0;
         counters[kCtrPairs] = P;
@@ -203,7 +203,7 @@ struct OnesweepArgs {
     const uint32_t* vals_in;
     void* keys_out;
     uint32_t* vals_out;
-    const uint32_t* count_ptr;
+    const uint32_t* count_ptr;  // the key count, capped by n_imm (kKeys64Drop: n_imm keys, none when it is 0)
     uint32_t n_imm;
     uint32_t shift, digit_mask;  // this pass's digit
     const uint32_t* offsets;   // 2^BITS global exclusive offsets of this pass's digits
@@ -280,17 +280,18 @@ __global__ __launch_bounds__(BLOCK) void k_onesweep(const OnesweepArgs a) {
     static_assert(DTH / kWave <= 8, "at most 8 digit-owning waves");
     __shared__ Lds L;
 
-    const uint32_t n = a.count_ptr ? min(*a.count_ptr, a.n_imm) : a.n_imm;
+    const uint32_t n = a.count_ptr && !DROP ? min(*a.count_ptr, a.n_imm) : a.n_imm;
     const uint32_t nparts = (n + kTileKeys - 1) / kTileKeys;
     const uint32_t tid = threadIdx.x, wave = tid / kWave, lane = __lane_id();
     // The grid covers the most keys there may be: the blocks past the partitions leave before they
     // take a ticket, so that exactly nparts blocks share nparts tickets.
     if (blockIdx.x >= nparts) return;
     if (tid == 0) L.part = atomicAdd(a.ticket, 1u);
+    const uint32_t any = DROP && a.count_ptr ? *a.count_ptr : 1u;  // (on its way while the ticket is)
     for (uint32_t x = tid; x < kWaves * R / 2; x += BLOCK) reinterpret_cast<uint32_t*>(&L.whist[0][0])[x] = 0;
     __syncthreads();
     const uint32_t part = __builtin_amdgcn_readfirstlane(L.part);  // block-uniform: keep it scalar
-    if (part >= nparts) return;
+    if (part >= nparts || any == 0u) return;
     if (a.desc_next)
         for (uint32_t d = tid; d < R; d += BLOCK) a.desc_next[part * R + d] = 0;
 

@@ -18,8 +18,8 @@ enum : uint32_t {
                           // (it is rendered again)
     kCtrTotal64 = 6,      // (two words) the plain frame's pair count, summed by its item kernel; zero between
                           // frames
-    kCtrSortItems = 8,    // the plain frame's items as its item sort's first pass counts them: all, or 0 when
-                          // a depth lies outside the window that they would be sorted on
+    kCtrSortItems = 8,    // the plain frame's items to be sorted: all, or 0 when a depth lies outside the window
+                          // that they would be sorted on
     kCtrItemsKept = 32,   // the visible items: those the item sort keeps (its later passes and
                           // the emission run on them).  128 bytes past the tickets: every emission
                           // block reads it right after its ticket atomic, and on the tickets' L2
@@ -343,7 +343,7 @@ void launch_sort_offsets(SortWorkspace& ws, uint32_t item_shape, uint32_t ipasse
 void launch_frame_resume(uint32_t* counters, hipStream_t s);
 // Sorts the n items by the low lo_bits bits of their keys.  The first pass drops the keys whose high
 // word is zero (the counts leave them out) and takes each key's index as its value; the later ones
-// sort the *kept others.  count_ptr (optional): the first pass takes *count_ptr of the n.
+// sort the *kept others.  count_ptr (optional): nothing is sorted when *count_ptr is 0.
 bool launch_sort_items(SortWorkspace& ws, uint32_t shape, uint64_t* keys, uint32_t* vals, uint64_t* keys_alt,
                        uint32_t* vals_alt, uint32_t n, uint32_t lo_bits, const uint32_t* kept, hipStream_t s,
                        const uint32_t* count_ptr = nullptr);
