@@ -12,6 +12,8 @@
 #include "tpd_ctx.hpp"
 
 #include <algorithm>
+#include <chrono>
+#include <thread>
 
 namespace tpd {
 
@@ -52,14 +54,27 @@ int launch_offsets(tpd_ctx* c, hipStream_t s) {
     return e == hipSuccess ? TPD_OK : hip_fail(e, "item offsets");
 }
 
-// Waits until the frame's totals have reached h_counters (k_frame_offsets stores seq last).
+// Waits until the frame's totals have reached h_counters (k_frame_offsets stores seq last).  An ordinary
+// frame's are there within half a millisecond, looked for all the time; a frame behind long work on its
+// stream looks every 50 us after the first 2 ms and leaves its core to others meanwhile.
 static int wait_totals(tpd_ctx* c, hipStream_t s, uint32_t seq) {
+    using clock = std::chrono::steady_clock;
+    constexpr auto kSpin = std::chrono::milliseconds(2);
+    constexpr auto kNap = std::chrono::microseconds(50);
     volatile uint32_t* const at = &c->h_counters[kHostSeq];
+    clock::time_point begin{};
+    bool naps = false;
     for (uint32_t spins = 1; __atomic_load_n(at, __ATOMIC_ACQUIRE) != seq; ++spins) {
-        if (spins % 4096u) continue;
+        if (naps)
+            std::this_thread::sleep_for(kNap);
+        else if (spins % 4096u)
+            continue;
         const hipError_t e = hipStreamQuery(s);
         if (e == hipErrorNotReady) {
             (void)hipGetLastError();  // not an error to be found by a later check
+            const clock::time_point now = clock::now();
+            if (begin == clock::time_point{}) begin = now;
+            naps = now - begin >= kSpin;
             continue;
         }
         if (e != hipSuccess) return hip_fail(e, "frame");
