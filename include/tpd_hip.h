@@ -175,7 +175,8 @@ int tpd_measure_run_scatter(tpd_ctx* ctx, uint32_t key_bytes, uint32_t n, uint32
 /* ----- stand-alone stable radix sort (radix-*.slang, GaussianEngine.cpp:819-841) -----
  * Sorts n (key, value) pairs by the key's low key_bits bits (stable); bits at and above key_bits do
  * not take part in the order and are carried with the key.  d_keys_alt /
- * d_vals_alt are scratch of the same size; *in_alt is set to 1 when the result is there. */
+ * d_vals_alt are scratch of the same size; *in_alt is set to 1 when the result is there.  The context's
+ * first sort or frame allocates its workspace: under a stream capture that returns TPD_ERR_STATE. */
 int tpd_sort_pairs(tpd_ctx* ctx, uint64_t* d_keys, uint32_t* d_vals, uint64_t* d_keys_alt, uint32_t* d_vals_alt,
                    uint32_t n, uint32_t key_bits, void* stream, int* in_alt);
 /* As tpd_sort_pairs, allocating nothing: no counterpart in the reference.  For callers that cannot

@@ -94,9 +94,17 @@ int ensure_pair_buffers(tpd_ctx* c, size_t pairs, hipStream_t s) {
 int ensure_sort_workspace(tpd_ctx* c, size_t pairs, hipStream_t s) {
     const uint32_t parts = sort_parts((uint32_t)std::min<size_t>(pairs, kMaxSortKeys));
     hipError_t e;
-    if (!c->ws.partials) {
-        if ((e = hipMalloc(&c->ws.partials, sizeof(uint32_t) * kCountCopies * kMaxPasses * kMaxRadix)) != hipSuccess ||
-            (e = hipMemsetAsync(c->ws.partials, 0, sizeof(uint32_t) * kCountCopies * kMaxPasses * kMaxRadix, s)) != hipSuccess)
+    if (!c->ws.tickets) {  // allocated last: there once all of it is
+        // a capture would record the counts' clear instead of running it, and ends at the allocations
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        if ((e = hipStreamIsCapturing(s, &capture)) != hipSuccess) return hip_fail(e, "alloc sort counts");
+        if (capture != hipStreamCaptureStatusNone)
+            return fail(TPD_ERR_STATE, "sort workspace: sort or render once before a capture");
+        const size_t counts = sizeof(uint32_t) * kCountCopies * kMaxPasses * kMaxRadix;
+        release(c->ws.partials);
+        release(c->ws.offsets);
+        if ((e = hipMalloc(&c->ws.partials, counts)) != hipSuccess ||
+            (e = hipMemsetAsync(c->ws.partials, 0, counts, s)) != hipSuccess)
             return hip_fail(e, "alloc sort counts");
         if ((e = hipMalloc(&c->ws.offsets, sizeof(uint32_t) * kMaxPasses * kMaxRadix)) != hipSuccess)
             return hip_fail(e, "alloc sort offsets");
@@ -104,6 +112,7 @@ int ensure_sort_workspace(tpd_ctx* c, size_t pairs, hipStream_t s) {
             return hip_fail(e, "alloc sort tickets");
     }
     if (c->ws.parts_cap < parts) {
+        c->ws.parts_cap = 0;
         release(c->ws.desc);
         const uint32_t want = parts + parts / 4 + 1;
         if ((e = hipMalloc(&c->ws.desc, sizeof(uint32_t) * 2 * (size_t)want * kMaxRadix)) != hipSuccess)
