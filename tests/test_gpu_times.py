@@ -44,3 +44,26 @@ def test_backward_times(orc):
         fwd, bwd = eng.stageTimes(), eng.backwardTimes()
         assert min(bwd.values()) > 0.0 and np.isfinite(list(bwd.values())).all()
         assert fwd["frame"] + bwd["splat_grad_pass"] + bwd["param_grad_pass"] <= bwd["fwd_bwd_span"] + 1e-3
+
+
+def test_stage_times_of_a_frame_without_room(orc):
+    """A first frame of more pairs than there is room for emits them twice and grows its buffers between:
+    that is in no stage's time, only in the whole frame's."""
+    from torpedo_amd.engine import GaussianEngine
+    cam = c1_camera(orc, 320, 200)
+    with GaussianEngine() as eng:
+        eng.uploadRecords(small_scene(200_000, seed=3, log_scale_mean=-0.5), 3)
+        eng.setCamera(cam.view, cam.proj_view, cam.focal_ndc, cam.width, cam.height)
+        eng.setProfiling(True)
+        eng.render()
+        first = eng.stageTimes()
+        assert eng.frameIssues() == (1, 1) and eng.pairCount > 5 * 200_000
+        for _ in range(3):
+            eng.render()
+        then = eng.stageTimes()
+        assert eng.frameIssues() == (4, 1)
+        stages = [k for k in first if k not in ("frame", "radix_passes")]
+        gap = first["frame"] - sum(first[k] for k in stages)
+        assert gap > then["frame"] - sum(then[k] for k in stages)
+        # the item passes wait for nothing
+        assert first["sort_passes"] <= 2.0 * then["sort_passes"] + 0.2, (first, then)

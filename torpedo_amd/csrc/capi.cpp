@@ -469,7 +469,7 @@ int tpd_get_stage_times(tpd_ctx* c, float* ms, uint32_t* passes) {
     // items, digit offsets, item passes, emission, pair passes, ranges + tile order, blend
     float d[7];
     for (int k = 0; k < 7; ++k)
-        if ((e = hipEventElapsedTime(&d[k], c->ev[k], c->ev[k + 1])) != hipSuccess)
+        if ((e = hipEventElapsedTime(&d[k], c->ev[k == 3 ? c->emit_event : (uint32_t)k], c->ev[k + 1])) != hipSuccess)
             return hip_fail(e, "hipEventElapsedTime");
     ms[0] = d[0] + d[3];
     ms[1] = d[1];

@@ -169,12 +169,13 @@ static void issue_items(tpd_ctx* c, FrameIssue& q, hipStream_t s) {
     a.kept_items = &c->d_counters[kCtrItemsKept];
     a.sorted_items = items_alt ? c->d_ivals_alt : c->d_ivals;
     a.sorted_keys64 = items_alt ? c->d_ikeys_alt : c->d_ikeys;
+    if (c->profile) hipEventRecord(c->ev[3], s);
+    c->emit_event = 3;
 }
 
 // The rest: the pairs, their sort and ranges, and the blend.
 static int issue_pairs(tpd_ctx* c, const FrameIssue& q, hipStream_t s) {
     const BatchArgs& a = q.f.b;
-    if (c->profile) hipEventRecord(c->ev[3], s);
     launch_batch_emit(a, s);
     if (c->profile) hipEventRecord(c->ev[4], s);
     const bool in_alt = launch_sort_pairs32(c->ws, q.pshape, c->d_keys, c->d_vals, c->d_keys_alt, c->d_vals_alt,
@@ -260,6 +261,8 @@ int render_forward(tpd_ctx* c, hipStream_t s) {
             ++c->resumes;
             set_pair_room(c, q, pair_room(c));
             launch_frame_resume(c->d_counters, s);
+            if (c->profile) hipEventRecord(c->ev[8], s);
+            c->emit_event = 8;
             if ((rc = issue_pairs(c, q, s)) != TPD_OK) return rc;
         }
         break;

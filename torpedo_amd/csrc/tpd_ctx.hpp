@@ -84,7 +84,8 @@ struct tpd_ctx {
 
     // stage timing with HIP events on the render stream (tpd_set_profiling)
     bool profile = false;
-    hipEvent_t ev[8] = {};
+    hipEvent_t ev[9] = {};
+    uint32_t emit_event = 3;  // where the emission that made the frame's pairs began: 3, or 8 for a resumed frame
     uint64_t* d_eval_count = nullptr;  // blend evaluations, counted on request (tpd_get_blend_evaluations)
     tpd::BlendArgs last_blend{};       // the last rendered frame's blend, for that count
     bool has_blend = false;
