@@ -56,10 +56,11 @@ int launch_offsets(tpd_ctx* c, hipStream_t s) {
 
 // Waits until the frame's totals have reached h_counters (k_frame_offsets stores seq last).  An ordinary
 // frame's are there within half a millisecond, looked for all the time; a frame behind long work on its
-// stream looks every 50 us after the first 2 ms and leaves its core to others meanwhile.
+// stream looks every 50 us after the first 10 ms and leaves its core to others meanwhile (a look is up to
+// 110 us late with the kernel's timer slack: one part in a hundred of such a wait).
 static int wait_totals(tpd_ctx* c, hipStream_t s, uint32_t seq) {
     using clock = std::chrono::steady_clock;
-    constexpr auto kSpin = std::chrono::milliseconds(2);
+    constexpr auto kSpin = std::chrono::milliseconds(10);
     constexpr auto kNap = std::chrono::microseconds(50);
     volatile uint32_t* const at = &c->h_counters[kHostSeq];
     clock::time_point begin{};
