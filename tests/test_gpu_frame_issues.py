@@ -128,6 +128,21 @@ def test_room_follows_recent_frames(orc, eng):
     assert show(large) == (1, 1) and show(large) == (1, 0) and show(small) == (1, 0)
 
 
+def test_room_of_the_widest_view(orc, eng):
+    """One view in thirty with three times the others' pairs: it finds its room each time."""
+    g = crowd(8000, 15, -0.5)
+    near, far = (orc.make_camera([0.0, 0.0, z], [0.0, 0.0, 0.0], [0.0, -1.0, 0.0], W, H) for z in (-3.0, -40.0))
+    eng.uploadRecords(g, 3)
+    assert frame(eng, orc, g, near) == (1, 1)
+    pairs = eng.pairCount
+    for _ in range(3):
+        for k in range(29):
+            eng.setCamera(far.view, far.proj_view, far.focal_ndc, far.width, far.height)
+            eng.render()
+        assert 3 * eng.pairCount < pairs
+        assert frame(eng, orc, g, near) == (1, 0)
+
+
 @pytest.mark.parametrize("n,scale", [(8_000, -0.5), (40_000, -0.5), (9_000, -1.7)])
 def test_first_batch_over_the_room(orc, n, scale):
     """A batch's first frame with many times the pairs its buffers hold, blocks of it all past their end:

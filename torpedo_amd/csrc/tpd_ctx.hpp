@@ -78,7 +78,8 @@ struct tpd_ctx {
     int32_t* d_final_last = nullptr; size_t cap_final_last = 0;
 
     uint32_t last_pairs = 0;
-    uint32_t recent_pairs = 0;  // the most pairs of recent frames, an eighth less with each frame of fewer
+    uint32_t recent_pairs = 0;  // the most pairs of recent frames, after recent_hold frames of fewer an eighth less
+    uint32_t recent_hold = 0;   // with each
     uint32_t last_passes = 0;
     bool rendered = false;
 
